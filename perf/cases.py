@@ -16,8 +16,11 @@ Families (key "kind" of a case):
   marginal  all modes of a train but the first contracted against quadrature
             weights, then the cumulative distribution along the first.
 
-Cores are handed out as views of the library's own device buffers, indexed
-(r_k, n_k, r_{k+1}) over the column-major core memory.
+Cores are handed out indexed (r_k, n_k, r_{k+1}) over the column-major core
+memory, as views of the library's own device buffers or, after a rounding, as
+their magnitudes: the signs of singular vectors are free, so a program that
+compares or stores trains takes the magnitudes and an entry, which ties the
+signs together.
 """
 import ctypes as C
 import math
@@ -190,6 +193,11 @@ def _flux_coefficients(case, seed):
             for _ in range(case["d"])]
 
 
+def _index(case, seed):
+    rng = np.random.default_rng(int(seed))
+    return [int(i) for i in rng.integers(0, case["n"], case["d"])]
+
+
 DT_FLUX, DX_FLUX = 1.0e-4, 0.02
 
 
@@ -207,6 +215,7 @@ def prepare(case, seed):
         r = case["rx"] + case["ry"]
         s["z"] = P.DevTT([n] * d, _ranks(d, r))
         s["caps"] = _ranks(d, case["cap"] if case["cap"] else r)
+        s["index"] = _index(case, seed)
     elif kind == "rk4":
         L.paratt_amd_rxn_burgers_setup.argtypes = [C.c_double, C.c_double, C.c_double, C.c_int]
         pp = C.POINTER(P.Paratt)
@@ -269,8 +278,13 @@ def run(s):
         if case["mixed"]:
             P.set_leaf_precision(0)
         spec = P.last_round_spectra()[1:d]
-        return {"cores": _views(z), "ranks": np.array(z.r), "norm": P.last_round_stats().norm,
-                "sigma": np.concatenate([spec[:, 16:17], spec[:, :13]], axis=1)}
+        out = {"entry": P.entry(z, s["index"]), "ranks": np.array(z.r),
+               "norm": P.last_round_stats().norm,
+               "sigma": np.concatenate([spec[:, 16:17], spec[:, :13]], axis=1),
+               "cores": [v.abs() for v in _views(z)]}
+        # the library may reuse the cores from its next call on
+        torch.cuda.current_stream().synchronize()
+        return out
     if kind == "rk4":
         L.paratt_amd_rxn_burgers_setup(0.01, 2.0 * math.pi / case["n"], case["eps"], case["cap"])
         L.paratt_amd_rk4_st(s["u"].p, s["new"].p, s["field"], 1.0e-3, case["eps"], case["cap"])
@@ -361,8 +375,7 @@ def _sum_cores(xs, ys, beta):
 
 
 def _exact_round(case, seed):
-    """Ranks, norm and kept singular values by QR and SVD sweeps on the host (LAPACK).
-    Cores have signs that the factorisations are free to choose: no value for them."""
+    """The rounding by QR and SVD sweeps on the host (LAPACK)."""
     d, n = case["d"], case["n"]
     r = case["rx"] + case["ry"]
     if sum(float(n) * r * r * r * 6.0 for _ in range(d)) > 3.0e11:
@@ -396,8 +409,14 @@ def _exact_round(case, seed):
         for q in range(13):
             if 0 <= rho - 13 + q < len(sv):
                 sigma[k - 1, 1 + q] = sv[rho - 13 + q]
+        z[k] = vt[:rho].reshape(rho, n, -1)
         z[k - 1] = np.tensordot(z[k - 1], u[:, :rho] * sv[:rho], axes=(2, 0))
-    return {"cores": None, "ranks": np.array(ranks), "norm": nrm, "sigma": sigma}
+    z = [c * math.sqrt(n) for c in z]
+    entry = np.ones((1, 1))
+    for c, j in zip(z, _index(case, seed)):
+        entry = entry @ c[:, j, :]
+    return {"cores": [np.abs(c) for c in z], "ranks": np.array(ranks), "norm": nrm,
+            "sigma": sigma, "entry": float(entry[0, 0])}
 
 
 def exact(case, seed):
