@@ -96,6 +96,16 @@ void ptt_hip_scale(double *p, long count, double alpha);
 void ptt_hip_axpby_core(int kind, int n, int rx0, int rx1, const double *x,
                         int ry0, int ry1, const double *y, double a, double b,
                         double *z);
+/* The same for d cores in as few launches as their count allows: core k has
+ * kind[k], modes n[k] and ranks rx[k], rx[k+1] / ry[k], ry[k+1]. */
+void ptt_hip_axpby_train(int d, const int *kind, const int *n, const int *rx,
+                         double *const *x, const int *ry, double *const *y, double a,
+                         double b, double *const *z);
+/* S = sum_i D_i u as a rank-2r train of d cores: first [D u | u], interior
+ * [[u, 0], [D u, u]], last [u; D u] (d = 1: D u), D the periodic 3-point
+ * stencil of kind 0 below (host coefficients). */
+void ptt_hip_mode_sum_train(int d, const int *n, const int *r, double *const *u,
+                            const double *sten3, double *const *s);
 /* Kronecker of every mode slice: z[(ry0*ax+ay), j, (ry1*bx+by)]. */
 void ptt_hip_hadamard_core(int n, int rx0, int rx1, const double *x, int ry0,
                            int ry1, const double *y, double *z);
@@ -118,10 +128,6 @@ void ptt_hip_copy2d(int m, int n, const double *A, long lda, double *B, long ldb
 /* B (n x m) = alpha * A^T (A m x n). */
 void ptt_hip_transpose(int m, int n, const double *A, long lda, double *B,
                        long ldb, double alpha);
-/* Place src (sr0 x n x sr1) at row/col offset (ra, rb) of dst
- * (dr0 x n x dr1), scaled by alpha: dst[ra+a, j, rb+b] = alpha*src[a, j, b]. */
-void ptt_hip_block_place(double *dst, int dr0, int n, int dr1, int ra, int rb,
-                         const double *src, int sr0, int sr1, double alpha);
 /* p[0..count) = v. */
 void ptt_hip_fill(double *p, long count, double v);
 /* A[i + i*lda] = alpha for i < m (other entries untouched). */

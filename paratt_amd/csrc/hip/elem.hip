@@ -81,36 +81,115 @@ dim3 grid_core(long rows, long cols) {
     return dim3((unsigned)gx, gy < 1 ? 1 : gy);
 }
 
-// z = a*x (+) b*y, one core.  kind 0 first (cols concat), 1 interior
-// (block diagonal), 2 last (rows concat).  attac.c:81-112.
-__global__ void k_axpby_core(int kind, int n, int rx0, int rx1, const double *__restrict__ x,
-                             int ry0, int ry1, const double *__restrict__ y, double a,
-                             double b, double *__restrict__ z, FastDiv drz0) {
+// VW consecutive doubles moved as one 16-byte access (VW = 2).
+template <int VW>
+struct Vd {
+    double v[VW];
+};
+
+template <int VW>
+__device__ __forceinline__ Vd<VW> ld_vd(const double *p) {
+    Vd<VW> r;
+    if constexpr (VW == 2) {
+        const double2 t = *reinterpret_cast<const double2 *>(p);
+        r.v[0] = t.x;
+        r.v[1] = t.y;
+    } else {
+        r.v[0] = *p;
+    }
+    return r;
+}
+
+template <int VW>
+__device__ __forceinline__ void st_vd(double *p, const Vd<VW> &r) {
+    if constexpr (VW == 2)
+        *reinterpret_cast<double2 *>(p) = make_double2(r.v[0], r.v[1]);
+    else
+        *p = r.v[0];
+}
+
+// ---- whole trains per launch -------------------------------------------------
+// The formal sum, the Hadamard product and the stencil sum write every core of
+// a train independently: one launch takes up to TRAIN_CHUNK cores (descriptors
+// in the kernel arguments), with gridDim.z over the cores, y over a core's
+// columns and x over the rows of a column.  Trains of low rank are bound by
+// launches (about 3 us each on the stream), large ones by HBM.  Two rank
+// indices are moved per lane where ranks and addresses allow 16-byte accesses.
+// The headline sum (d = 40, n = 1024, 64 + 64 -> 128) is at the card's copy
+// rate (4.7 TB/s) either way.
+constexpr int TRAIN_CHUNK = 32;
+
+// Grid of a train launch: rows and cols are the largest of its cores; about
+// 16384 workgroups in all, each grid-stride.
+dim3 grid_train(long rows, long cols, int ncores, int vw) {
+    const unsigned gy = (unsigned)(cols < 1 ? 1 : cols < 65535 ? cols : 65535);
+    long gx = (rows + 256L * vw - 1) / (256L * vw);
+    const long cap = (16384L + (long)gy * ncores - 1) / ((long)gy * ncores);
+    if (gx > cap) gx = cap;
+    if (gx < 1) gx = 1;
+    return dim3((unsigned)gx, gy, (unsigned)ncores);
+}
+
+struct SumCore {
+    const double *x, *y;
+    double *z;
+    double a, b;
+    int kind, n, rx0, rx1, ry0, ry1;
+    FastDiv drz0;  // division by z's left rank
+};
+struct SumChunk {
+    SumCore c[TRAIN_CHUNK];
+};
+
+// z = a*x (+) b*y.  kind 0 first core (cols concat), 1 interior (block
+// diagonal), 2 last (rows concat).  attac.c:81-112.  VW rank indices per
+// thread (both left ranks even, 16-byte aligned cores).
+template <int VW>
+__global__ __launch_bounds__(256) void k_axpby_train(SumChunk ch) {
+    const SumCore &s = ch.c[blockIdx.z];
+    const int kind = s.kind, n = s.n, rx0 = s.rx0, rx1 = s.rx1, ry0 = s.ry0, ry1 = s.ry1;
+    const double *__restrict__ x = s.x;
+    const double *__restrict__ y = s.y;
     const int rz0 = (kind == 0) ? 1 : rx0 + ry0;
     const int rz1 = (kind == 2) ? 1 : rx1 + ry1;
     const unsigned rows = (unsigned)rz0 * (unsigned)n;
     for (int col = blockIdx.y; col < rz1; col += gridDim.y) {
-        double *zc = z + (long)col * rows;
-        for (unsigned m = blockIdx.x * blockDim.x + threadIdx.x; m < rows;
-             m += gridDim.x * blockDim.x) {
-            const int j = (int)fdiv(m, drz0);
+        double *__restrict__ zc = s.z + (long)col * rows;
+        for (unsigned m = VW * (blockIdx.x * blockDim.x + threadIdx.x); m < rows;
+             m += VW * gridDim.x * blockDim.x) {
+            const int j = (int)fdiv(m, s.drz0);
             const int al = (int)m - j * rz0;
-            double v = 0.0;
+            Vd<VW> v;
+#pragma unroll
+            for (int q = 0; q < VW; q++) v.v[q] = 0.0;
             if (kind == 0) {
-                v = (col < rx1) ? x[j + (long)n * col] * a
-                                : y[j + (long)n * (col - rx1)] * b;
+                const bool left = col < rx1;
+                v = ld_vd<VW>(left ? x + j + (long)n * col : y + j + (long)n * (col - rx1));
+#pragma unroll
+                for (int q = 0; q < VW; q++) v.v[q] = v.v[q] * (left ? s.a : s.b);
             } else if (kind == 2) {
-                v = (al < rx0) ? x[al + (long)rx0 * j] : y[(al - rx0) + (long)ry0 * j];
+                v = ld_vd<VW>((al < rx0) ? x + al + (long)rx0 * j : y + (al - rx0) + (long)ry0 * j);
             } else {
                 if (al < rx0 && col < rx1)
-                    v = x[al + (long)rx0 * (j + (long)n * col)];
+                    v = ld_vd<VW>(x + al + (long)rx0 * (j + (long)n * col));
                 else if (al >= rx0 && col >= rx1)
-                    v = y[(al - rx0) + (long)ry0 * (j + (long)n * (col - rx1))];
+                    v = ld_vd<VW>(y + (al - rx0) + (long)ry0 * (j + (long)n * (col - rx1)));
             }
-            zc[m] = v;
+            st_vd<VW>(zc + m, v);
         }
     }
 }
+
+struct ModeSumCore {
+    const double *u;
+    double *s;
+    int kind, r0, n, r1;  // kind 0 first, 1 interior, 2 last, 3 the only core
+    FastDiv ds0;          // division by s's left rank
+};
+struct ModeSumChunk {
+    ModeSumCore c[TRAIN_CHUNK];
+    double st[3];
+};
 
 // z[(ry0*ax+ay), j, (ry1*bx+by)] = x[ax,j,bx] * y[ay,j,by] (utilities.c:112-129)
 __global__ void k_hadamard_core(int n, int rx0, int rx1, const double *__restrict__ x,
@@ -149,24 +228,6 @@ __global__ void k_diag_core(int r0, int n, int r1, const double *__restrict__ v,
 // VW consecutive rank indices (same mode index) per thread, loaded and
 // stored as one vector when the leading rank is even: the arithmetic of each
 // is the scalar path's, in the same order.
-template <int VW>
-struct Vd {
-    double v[VW];
-};
-
-template <int VW>
-__device__ __forceinline__ Vd<VW> ld_vd(const double *p) {
-    Vd<VW> r;
-    if constexpr (VW == 2) {
-        const double2 t = *reinterpret_cast<const double2 *>(p);
-        r.v[0] = t.x;
-        r.v[1] = t.y;
-    } else {
-        r.v[0] = *p;
-    }
-    return r;
-}
-
 template <int VW>
 __global__ void k_stencil_core(int kind, int r0, int n, int r1,
                                const double *__restrict__ sten, int slen,
@@ -221,11 +282,58 @@ __global__ void k_stencil_core(int kind, int r0, int n, int r1,
                 add(sten[sc++], v);
             }
         }
-        if constexpr (VW == 2)
-            *reinterpret_cast<double2 *>(g + e) = make_double2(acc.v[0], acc.v[1]);
-        else
-            g[e] = acc.v[0];
+        st_vd<VW>(g + e, acc);
 #undef FV
+    }
+}
+
+// S = sum_i D_i u as a rank-2r train (first core [D u | u], interior
+// [[u, 0], [D u, u]], last [u; D u]), every block of S written in one pass
+// with the 3-point periodic stencil of kind 0 applied on the way (same order of
+// operations as k_stencil_core).  Written block by block (the stencil to a
+// buffer, a zero fill, three placements) S was passed over more than twice: the
+// whole operator at d = 20, n = 1024, r = 32 took 739 us and takes 252 us
+// (840 MB read and written once; bound by HBM and the final synchronisation).
+template <int VW>
+__global__ __launch_bounds__(256) void k_mode_sum_train(ModeSumChunk ch) {
+    const ModeSumCore &c = ch.c[blockIdx.z];
+    const int kind = c.kind, r0 = c.r0, n = c.n, r1 = c.r1;
+    const double *__restrict__ u = c.u;
+    const int s0 = (kind == 0 || kind == 3) ? r0 : 2 * r0;
+    const int s1 = (kind >= 2) ? r1 : 2 * r1;
+    const unsigned rows = (unsigned)s0 * (unsigned)n;
+    for (int col = blockIdx.y; col < s1; col += gridDim.y) {
+        double *__restrict__ sc = c.s + (long)col * rows;
+        const bool right = col >= r1;  // the right half of the columns
+        const double *uc = u + (long)(right ? col - r1 : col) * r0 * n;
+        for (unsigned m = VW * (blockIdx.x * blockDim.x + threadIdx.x); m < rows;
+             m += VW * gridDim.x * blockDim.x) {
+            const int j = (int)fdiv(m, c.ds0);
+            const int al = (int)m - j * s0;
+            const bool low = al >= r0;  // the lower half of the rows
+            const int a = low ? al - r0 : al;
+            Vd<VW> v;
+#pragma unroll
+            for (int q = 0; q < VW; q++) v.v[q] = 0.0;
+            const bool du = (kind == 0 || kind == 3) ? !right : (low && !right);
+            const double *fb = uc + a;
+            if (du) {
+                const int jl = (j > 0) ? j - 1 : n - 1, jr = (j + 1 < n) ? j + 1 : 0;
+                const Vd<VW> x = ld_vd<VW>(fb + (long)r0 * jl), y = ld_vd<VW>(fb + (long)r0 * j),
+                             z = ld_vd<VW>(fb + (long)r0 * jr);
+#pragma unroll
+                for (int q = 0; q < VW; q++) {
+                    double acc = 0.0;
+                    acc += ch.st[0] * x.v[q];
+                    acc += ch.st[1] * y.v[q];
+                    acc += ch.st[2] * z.v[q];
+                    v.v[q] = acc;
+                }
+            } else if (kind != 1 || low || !right) {
+                v = ld_vd<VW>(fb + (long)r0 * j);
+            }
+            st_vd<VW>(sc + m, v);
+        }
     }
 }
 
@@ -317,22 +425,6 @@ __global__ void k_transpose(int m, int n, const double *__restrict__ A, long lda
     }
 }
 
-__global__ void k_block_place(double *__restrict__ dst, int dr0, int n, int ra, int rb,
-                              const double *__restrict__ src, int sr0, int sr1, double alpha,
-                              FastDiv dsr0) {
-    const unsigned rows = (unsigned)sr0 * (unsigned)n;
-    for (int b = blockIdx.y; b < sr1; b += gridDim.y) {
-        const double *sc = src + (long)b * rows;
-        double *dc = dst + ra + (long)dr0 * n * (rb + b);
-        for (unsigned m = blockIdx.x * blockDim.x + threadIdx.x; m < rows;
-             m += gridDim.x * blockDim.x) {
-            const int j = (int)fdiv(m, dsr0);
-            const int a = (int)m - j * sr0;
-            dc[a + (long)dr0 * j] = alpha * sc[m];
-        }
-    }
-}
-
 __global__ void k_fill(double *p, long count, double v) {
     for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < count;
          e += (long)gridDim.x * blockDim.x)
@@ -410,15 +502,106 @@ void ptt_hip_scale(double *p, long count, double alpha) {
     PTT_LAUNCH("scale", k_scale, dim3(stream_blocks(count, 256)), dim3(256), 0, p, count, alpha);
 }
 
+void ptt_hip_axpby_train(int d, const int *kind, const int *n, const int *rx,
+                         double *const *x, const int *ry, double *const *y, double a, double b,
+                         double *const *z) {
+    ptt_hip_init();
+    // two chunks: cores that move in pairs and cores that do not
+    SumChunk ch[2];
+    int cnt[2] = {0, 0};
+    long rows[2] = {0, 0}, cols[2] = {0, 0};
+    double bytes[2] = {0.0, 0.0};
+    auto flush = [&](int v) {
+        if (!cnt[v]) return;
+        const dim3 grid = grid_train(rows[v], cols[v], cnt[v], v ? 2 : 1);
+        if (v)
+            PTT_LAUNCH_FB("axpby", 0.0, bytes[v], k_axpby_train<2>, grid, dim3(256), 0, ch[v]);
+        else
+            PTT_LAUNCH_FB("axpby", 0.0, bytes[v], k_axpby_train<1>, grid, dim3(256), 0, ch[v]);
+        cnt[v] = 0;
+        rows[v] = cols[v] = 0;
+        bytes[v] = 0.0;
+    };
+    for (int k = 0; k < d; k++) {
+        SumCore c;
+        c.kind = kind[k];
+        c.n = n[k];
+        c.rx0 = rx[k];
+        c.rx1 = rx[k + 1];
+        c.ry0 = ry[k];
+        c.ry1 = ry[k + 1];
+        c.x = x[k];
+        c.y = y[k];
+        c.z = z[k];
+        c.a = a;
+        c.b = b;
+        const long rz0 = (c.kind == 0) ? 1 : c.rx0 + c.ry0, rz1 = (c.kind == 2) ? 1 : c.rx1 + c.ry1;
+        const long total = rz0 * c.n * rz1;
+        if (total <= 0) continue;
+        c.drz0 = make_fastdiv((unsigned)rz0);
+        const bool even = c.kind == 0 ? (c.n & 1) == 0 : ((c.rx0 | c.ry0) & 1) == 0;
+        const int v =
+            (even && (((uintptr_t)c.x | (uintptr_t)c.y | (uintptr_t)c.z) & 15) == 0) ? 1 : 0;
+        ch[v].c[cnt[v]++] = c;
+        if (rz0 * c.n > rows[v]) rows[v] = rz0 * c.n;
+        if (rz1 > cols[v]) cols[v] = rz1;
+        bytes[v] += 8.0 * ((double)c.rx0 * c.n * c.rx1 + (double)c.ry0 * c.n * c.ry1 + (double)total);
+        if (cnt[v] == TRAIN_CHUNK) flush(v);
+    }
+    flush(0);
+    flush(1);
+}
+
 void ptt_hip_axpby_core(int kind, int n, int rx0, int rx1, const double *x, int ry0, int ry1,
                         const double *y, double a, double b, double *z) {
+    const int rx[2] = {rx0, rx1}, ry[2] = {ry0, ry1};
+    double *const xs = (double *)x, *const ys = (double *)y;
+    ptt_hip_axpby_train(1, &kind, &n, rx, &xs, ry, &ys, a, b, &z);
+}
+
+void ptt_hip_mode_sum_train(int d, const int *n, const int *r, double *const *u,
+                            const double *sten3, double *const *s) {
     ptt_hip_init();
-    long rz0 = (kind == 0) ? 1 : rx0 + ry0, rz1 = (kind == 2) ? 1 : rx1 + ry1;
-    long total = rz0 * n * rz1;
-    double bytes = 8.0 * ((double)rx0 * n * rx1 + (double)ry0 * n * ry1 + (double)total);
-    if (total <= 0) return;
-    PTT_LAUNCH_FB("axpby", 0.0, bytes, k_axpby_core, grid_core(rz0 * n, rz1), dim3(256), 0, kind,
-                  n, rx0, rx1, x, ry0, ry1, y, a, b, z, make_fastdiv((unsigned)rz0));
+    ModeSumChunk ch[2];
+    int cnt[2] = {0, 0};
+    long rows[2] = {0, 0}, cols[2] = {0, 0};
+    double bytes[2] = {0.0, 0.0};
+    for (int v = 0; v < 2; v++)
+        for (int q = 0; q < 3; q++) ch[v].st[q] = sten3[q];
+    auto flush = [&](int v) {
+        if (!cnt[v]) return;
+        const dim3 grid = grid_train(rows[v], cols[v], cnt[v], v ? 2 : 1);
+        if (v)
+            PTT_LAUNCH_FB("mode_sum", 0.0, bytes[v], k_mode_sum_train<2>, grid, dim3(256), 0, ch[v]);
+        else
+            PTT_LAUNCH_FB("mode_sum", 0.0, bytes[v], k_mode_sum_train<1>, grid, dim3(256), 0, ch[v]);
+        cnt[v] = 0;
+        rows[v] = cols[v] = 0;
+        bytes[v] = 0.0;
+    };
+    for (int k = 0; k < d; k++) {
+        ModeSumCore c;
+        c.kind = d == 1 ? 3 : k == 0 ? 0 : k == d - 1 ? 2 : 1;
+        c.r0 = r[k];
+        c.n = n[k];
+        c.r1 = r[k + 1];
+        c.u = u[k];
+        c.s = s[k];
+        const long s0 = (c.kind == 0 || c.kind == 3) ? c.r0 : 2L * c.r0;
+        const long s1 = (c.kind >= 2) ? c.r1 : 2L * c.r1;
+        const long total = s0 * c.n * s1;
+        if (total <= 0) continue;
+        c.ds0 = make_fastdiv((unsigned)s0);
+        const int v =
+            ((c.r0 & 1) == 0 && (((uintptr_t)c.u | (uintptr_t)c.s) & 15) == 0) ? 1 : 0;
+        ch[v].c[cnt[v]++] = c;
+        if (s0 * c.n > rows[v]) rows[v] = s0 * c.n;
+        if (s1 > cols[v]) cols[v] = s1;
+        bytes[v] += 8.0 * ((double)c.r0 * c.n * c.r1 + (double)total);
+        if (cnt[v] == TRAIN_CHUNK) flush(v);
+    }
+    flush(0);
+    flush(1);
 }
 
 void ptt_hip_hadamard_core(int n, int rx0, int rx1, const double *x, int ry0, int ry1,
@@ -491,20 +674,6 @@ void ptt_hip_transpose(int m, int n, const double *A, long lda, double *B, long 
     if (m <= 0 || n <= 0) return;
     PTT_LAUNCH("transpose", k_transpose, dim3(cdiv(m, 32), cdiv(n, 32)), dim3(256), 0, m, n, A,
                lda, B, ldb, alpha);
-}
-
-void ptt_hip_block_place(double *dst, int dr0, int n, int dr1, int ra, int rb, const double *src,
-                         int sr0, int sr1, double alpha) {
-    ptt_hip_init();
-    long total = (long)sr0 * n * sr1;
-    if (total <= 0) return;
-    if (ra + sr0 > dr0 || rb + sr1 > dr1) {
-        fprintf(stderr, "paratt_amd: block_place out of range\n");
-        exit(1);
-    }
-    PTT_LAUNCH_FB("block_place", 0.0, 16.0 * total, k_block_place, grid_core((long)sr0 * n, sr1),
-                  dim3(256), 0, dst, dr0, n, ra, rb, src, sr0, sr1, alpha,
-                  make_fastdiv((unsigned)sr0));
 }
 
 void ptt_hip_fill(double *p, long count, double v) {

@@ -210,30 +210,7 @@ void paratt_amd_mode_sum(paratt *u, const double *sten3, paratt *s) {
     int *rs = (int *)ptt_host_malloc(sizeof(int) * (d + 1));
     for (int k = 0; k <= d; k++) rs[k] = (k == 0 || k == d) ? 1 : 2 * u->x->ttRank[k];
     rank_change_tt(s->x, rs);
-    double *dst = ptt_host_coef(sten3, 3);
-    for (int k = 0; k < d; k++) {
-        int r0 = u->x->ttRank[k], r1 = u->x->ttRank[k + 1], n = u->dim[k];
-        int s0 = rs[k], s1 = rs[k + 1];
-        long cnt = (long)r0 * n * r1;
-        double *du = (double *)ptt_hip_scratch(PTT_WS_TMP2, sizeof(double) * (size_t)cnt);
-        ptt_hip_stencil_core(0, r0, n, r1, dst, 3, u->x->coreList[k], du);
-        double *sc = s->x->coreList[k];
-        const double *uk = u->x->coreList[k];
-        if (d == 1) {
-            ptt_hip_d2d(sc, du, sizeof(double) * (size_t)cnt);
-        } else if (k == 0) {
-            ptt_hip_block_place(sc, s0, n, s1, 0, 0, du, r0, r1, 1.0);
-            ptt_hip_block_place(sc, s0, n, s1, 0, r1, uk, r0, r1, 1.0);
-        } else if (k == d - 1) {
-            ptt_hip_block_place(sc, s0, n, s1, 0, 0, uk, r0, r1, 1.0);
-            ptt_hip_block_place(sc, s0, n, s1, r0, 0, du, r0, r1, 1.0);
-        } else {
-            ptt_hip_zero(sc, sizeof(double) * (size_t)s0 * n * s1);
-            ptt_hip_block_place(sc, s0, n, s1, 0, 0, uk, r0, r1, 1.0);
-            ptt_hip_block_place(sc, s0, n, s1, r0, 0, du, r0, r1, 1.0);
-            ptt_hip_block_place(sc, s0, n, s1, r0, r1, uk, r0, r1, 1.0);
-        }
-    }
+    ptt_hip_mode_sum_train(d, u->dim, u->x->ttRank, u->x->coreList, sten3, s->x->coreList);
     ptt_hip_sync();
     free(rs);
 }

@@ -26,11 +26,10 @@ void attacFormalAXPBY(const int d, const int *n, const double alpha, const int *
     rz[0] = 1;
     rz[d] = 1;
     for (int i = 1; i < d; i++) rz[i] = rx[i] + ry[i];
-    ptt_hip_axpby_core(0, n[0], rx[0], rx[1], x[0], ry[0], ry[1], y[0], alpha, beta, z[0]);
-    for (int i = 1; i < d - 1; i++)
-        ptt_hip_axpby_core(1, n[i], rx[i], rx[i + 1], x[i], ry[i], ry[i + 1], y[i], 1.0, 1.0, z[i]);
-    ptt_hip_axpby_core(2, n[d - 1], rx[d - 1], rx[d], x[d - 1], ry[d - 1], ry[d], y[d - 1], 1.0,
-                       1.0, z[d - 1]);
+    int *kind = (int *)ptt_host_malloc(sizeof(int) * (size_t)d);
+    for (int i = 0; i < d; i++) kind[i] = (i == 0) ? 0 : (i == d - 1) ? 2 : 1;
+    ptt_hip_axpby_train(d, kind, n, rx, x, ry, y, alpha, beta, z);
+    free(kind);
     ptt_hip_sync();
 }
 
