@@ -22,9 +22,17 @@ extern "C" {
 void ptt_hip_init(void);
 int ptt_hip_initialized(void);      /* 1 after ptt_hip_init */
 void ptt_hip_noalloc_setup(void);   /* part of ptt_hip_init: fixed workspace address */
+/* Device memory; freed blocks are kept for reuse (bounded, see runtime.hip)
+ * and given back to the device by ptt_hip_trim.  Freeing waits for all device
+ * work, once per call. */
 void *ptt_hip_malloc(size_t bytes);
 void ptt_hip_free(void *p);
+void ptt_hip_free_many(int count, void *const *p);
+void ptt_hip_trim(void);
 void ptt_hip_h2d(void *dst, const void *src, size_t bytes);       /* blocking */
+/* The same, stream-ordered: src is read before the call returns, dst is
+ * written in order with the main stream's work (up to 64 KiB; blocking above). */
+void ptt_hip_h2d_queued(void *dst, const void *src, size_t bytes);
 void ptt_hip_d2h(void *dst, const void *src, size_t bytes);       /* blocking */
 void ptt_hip_d2d(void *dst, const void *src, size_t bytes);       /* async */
 /* A device-to-host read of at most 64 KiB in two halves: begin queues the

@@ -4,7 +4,9 @@
 
 #include <chrono>
 #include <map>
+#include <mutex>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 namespace ptt {
@@ -18,11 +20,18 @@ hipStream_t g_launch = nullptr;
 static hipEvent_t g_fork_ev = nullptr, g_join_ev = nullptr, g_side_ev[2] = {nullptr, nullptr};
 static bool g_side_used[2] = {false, false};
 static bool g_side_on = true;
+// Side work queued since the main stream last joined the side stream.
+static bool g_side_dirty = false;
+// Small uploads queued since the main stream was last waited for (their
+// staging slots are free again after such a wait).
+static int g_h2d_inflight = 0;
 
 // Waits for both streams.
 static void sync_all() {
     HIPCHECK(hipStreamSynchronize(g_stream));
     if (g_side) HIPCHECK(hipStreamSynchronize(g_side));
+    g_side_dirty = false;
+    g_h2d_inflight = 0;
 }
 // Host-visible mode (environment PARATT_AMD_HOST_VISIBLE=1, read once at
 // init): every library allocation is pinned host memory that the GPU reads
@@ -61,6 +70,7 @@ static void host_mode_copy(void *dst, const void *src, size_t bytes) {
 // memory go through coherent pinned staging buffers moved by k_copy_bytes:
 // a one-wave kernel instead of the runtime's staged blit copy.
 constexpr size_t STAGE_BYTES = 64 * 1024;
+constexpr int H2D_SLOTS = 8;  // uploads in flight before one waits for the stream
 static unsigned char *g_stage_d2h = nullptr, *g_stage_h2d = nullptr;
 
 // Small reads by the host: one workgroup copies into the coherent staging
@@ -111,6 +121,12 @@ static void wait_published(unsigned long long seq) {
     }
 }
 
+// Waits for the main stream by publishing a sequence number behind its queued
+// work (which includes the side stream's once it is joined).
+__global__ void k_publish(unsigned long long *flag, unsigned long long seq) {
+    __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 static void launch_copy_bytes(void *dst, const void *src, size_t bytes) {
     unsigned blocks = (unsigned)((bytes / 8 + 255) / 256);
     blocks = blocks < 1 ? 1 : (blocks > 4096 ? 4096 : blocks);
@@ -122,6 +138,82 @@ void fatal_hip(hipError_t e, const char *what, const char *file, int line) {
     fprintf(stderr, "paratt_amd: HIP error '%s' (%d) in %s at %s:%d\n",
             hipGetErrorString(e), (int)e, what, file, line);
     exit(1);
+}
+
+// ---- device memory kept for reuse -------------------------------------------
+// Trains are made and dropped all the time (every stage of a time step, every
+// marginal), and hipMalloc / hipFree cost tens of microseconds a core.  Freed
+// blocks are kept, at most POOL_BYTES in all, and handed out again for requests
+// they fit within a quarter.  A block enters the pool only after the device has
+// finished everything queued so far (ptt_hip_free waits as hipFree does), so it
+// may be used on any stream by any thread.  The pool is emptied when an
+// allocation fails and by ptt_hip_trim.
+constexpr size_t POOL_BYTES = (size_t)8 << 30;
+static std::mutex g_pool_mutex;
+static std::multimap<size_t, void *> g_pool;            // cached blocks by size
+static std::unordered_map<void *, size_t> g_pool_live;  // sizes of blocks handed out
+static size_t g_pool_cached = 0;
+
+static size_t pool_round(size_t bytes) {
+    const size_t unit = bytes < ((size_t)1 << 20) ? 512 : (size_t)1 << 16;
+    return (bytes + unit - 1) / unit * unit;
+}
+
+// Gives cached blocks back to the device, largest first, until at most `keep`
+// bytes remain.  The mutex is held by the caller.
+static void pool_shrink(size_t keep) {
+    while (g_pool_cached > keep && !g_pool.empty()) {
+        auto it = std::prev(g_pool.end());
+        HIPCHECK(hipFree(it->second));
+        g_pool_cached -= it->first;
+        g_pool.erase(it);
+    }
+}
+
+static void *pool_alloc(size_t bytes) {
+    const size_t want = pool_round(bytes);
+    std::lock_guard<std::mutex> lock(g_pool_mutex);
+    auto it = g_pool.lower_bound(want);
+    if (it != g_pool.end() && it->first <= want + want / 4 + 4096) {
+        void *p = it->second;
+        g_pool_live[p] = it->first;
+        g_pool_cached -= it->first;
+        g_pool.erase(it);
+        return p;
+    }
+    void *p = nullptr;
+    hipError_t e = hipMalloc(&p, want);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        pool_shrink(0);
+        e = hipMalloc(&p, want);
+    }
+    if (e != hipSuccess) {
+        fprintf(stderr, "paratt_amd: hipMalloc(%zu bytes) failed: %s\n", bytes,
+                hipGetErrorString(e));
+        exit(1);
+    }
+    g_pool_live[p] = want;
+    return p;
+}
+
+// The device has finished all work that may use p.
+static void pool_free(void *p) {
+    std::lock_guard<std::mutex> lock(g_pool_mutex);
+    auto it = g_pool_live.find(p);
+    if (it == g_pool_live.end()) {
+        HIPCHECK(hipFree(p));  // not from pool_alloc
+        return;
+    }
+    const size_t size = it->second;
+    g_pool_live.erase(it);
+    if (size > POOL_BYTES / 2) {
+        HIPCHECK(hipFree(p));
+        return;
+    }
+    g_pool.emplace(size, p);
+    g_pool_cached += size;
+    pool_shrink(POOL_BYTES);
 }
 
 struct Slot {
@@ -215,7 +307,7 @@ void ptt_hip_init(void) {
     const char *hv = getenv("PARATT_AMD_HOST_VISIBLE");
     g_host_visible = hv != nullptr && hv[0] != '\0' && hv[0] != '0';
     HIPCHECK(hipHostMalloc((void **)&g_stage_d2h, STAGE_BYTES, hipHostMallocCoherent));
-    HIPCHECK(hipHostMalloc((void **)&g_stage_h2d, STAGE_BYTES, hipHostMallocCoherent));
+    HIPCHECK(hipHostMalloc((void **)&g_stage_h2d, H2D_SLOTS * STAGE_BYTES, hipHostMallocCoherent));
     HIPCHECK(hipHostMalloc((void **)&g_d2h_flag, 256, hipHostMallocCoherent));
     *g_d2h_flag = 0;
     ptt_hip_noalloc_setup();  // device address of the fixed workspace
@@ -226,25 +318,39 @@ int ptt_hip_initialized(void) { return g_init ? 1 : 0; }
 
 void *ptt_hip_malloc(size_t bytes) {
     ptt_hip_init();
-    void *p = nullptr;
     if (bytes == 0) bytes = 8;
-    hipError_t e = g_host_visible ? hipHostMalloc(&p, bytes, hipHostMallocCoherent)
-                                  : hipMalloc(&p, bytes);
+    if (!g_host_visible) return pool_alloc(bytes);
+    void *p = nullptr;
+    hipError_t e = hipHostMalloc(&p, bytes, hipHostMallocCoherent);
     if (e != hipSuccess) {
-        fprintf(stderr, "paratt_amd: %s(%zu bytes) failed: %s\n",
-                g_host_visible ? "hipHostMalloc" : "hipMalloc", bytes, hipGetErrorString(e));
+        fprintf(stderr, "paratt_amd: hipHostMalloc(%zu bytes) failed: %s\n", bytes,
+                hipGetErrorString(e));
         exit(1);
     }
     return p;
 }
 
-void ptt_hip_free(void *p) {
-    if (!p) return;
+void ptt_hip_free_many(int count, void *const *p) {
+    bool any = false;
+    for (int i = 0; i < count; i++) any = any || p[i] != nullptr;
+    if (!any) return;
     sync_all();
-    if (g_host_visible)
-        HIPCHECK(hipHostFree(p));
-    else
-        HIPCHECK(hipFree(p));
+    if (!g_host_visible) HIPCHECK(hipDeviceSynchronize());  // the caller's own streams
+    for (int i = 0; i < count; i++) {
+        if (!p[i]) continue;
+        if (g_host_visible)
+            HIPCHECK(hipHostFree(p[i]));
+        else
+            pool_free(p[i]);
+    }
+}
+
+void ptt_hip_free(void *p) { ptt_hip_free_many(1, &p); }
+
+void ptt_hip_trim(void) {
+    ptt_hip_init();
+    std::lock_guard<std::mutex> lock(g_pool_mutex);
+    pool_shrink(0);
 }
 
 int ptt_hip_host_visible(void) {
@@ -257,14 +363,31 @@ void ptt_hip_h2d(void *dst, const void *src, size_t bytes) {
     if (!bytes) return;
     if (g_host_visible) return host_mode_copy(dst, src, bytes);
     if (bytes <= STAGE_BYTES) {
-        // the previous small upload has completed (every h2d ends synchronised)
-        memcpy(g_stage_h2d, src, bytes);
-        launch_copy_bytes(dst, g_stage_h2d, bytes);
+        ptt_hip_h2d_queued(dst, src, bytes);
         HIPCHECK(hipStreamSynchronize(g_stream));
+        g_h2d_inflight = 0;
         return;
     }
     HIPCHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, g_stream));
     HIPCHECK(hipStreamSynchronize(g_stream));
+}
+
+void ptt_hip_h2d_queued(void *dst, const void *src, size_t bytes) {
+    ptt_hip_init();
+    if (!bytes) return;
+    if (g_host_visible) return host_mode_copy(dst, src, bytes);
+    if (bytes > STAGE_BYTES) return ptt_hip_h2d(dst, src, bytes);
+    if (g_h2d_inflight == H2D_SLOTS) {
+        HIPCHECK(hipStreamSynchronize(g_stream));
+        g_h2d_inflight = 0;
+    }
+    unsigned char *stage = g_stage_h2d + STAGE_BYTES * (size_t)g_h2d_inflight++;
+    memcpy(stage, src, bytes);
+    unsigned blocks = (unsigned)((bytes / 8 + 255) / 256);
+    ProfScope ps_("copy_bytes", 0.0, 2.0 * (double)bytes);
+    hipLaunchKernelGGL(k_copy_bytes, dim3(blocks < 1 ? 1 : blocks), dim3(256), 0, g_stream,
+                       (unsigned char *)dst, stage, bytes);
+    HIPCHECK(hipGetLastError());
 }
 
 void ptt_hip_d2h(void *dst, const void *src, size_t bytes) {
@@ -333,7 +456,14 @@ void ptt_hip_copy(void *dst, const void *src, size_t bytes) {
 
 void ptt_hip_sync(void) {
     ptt_hip_init();
-    sync_all();
+    // host-visible memory needs the stream's own end-of-work release; side
+    // work that the main stream has not joined is waited for by itself
+    if (g_host_visible || g_side_dirty) return sync_all();
+    const unsigned long long seq = ++g_d2h_seq;
+    hipLaunchKernelGGL(k_publish, dim3(1), dim3(1), 0, g_stream, g_d2h_flag, seq);
+    HIPCHECK(hipGetLastError());
+    wait_published(seq);
+    g_h2d_inflight = 0;
 }
 
 int ptt_hip_side_enabled(void) {
@@ -351,6 +481,7 @@ void ptt_hip_side_begin(void) {
     ptt_hip_init();
     HIPCHECK(hipEventRecord(g_fork_ev, g_stream));
     HIPCHECK(hipStreamWaitEvent(g_side, g_fork_ev, 0));
+    g_side_dirty = true;
     g_launch = g_side;
 }
 
@@ -369,6 +500,7 @@ void ptt_hip_side_join(void) {
     ptt_hip_init();
     HIPCHECK(hipEventRecord(g_join_ev, g_side));
     HIPCHECK(hipStreamWaitEvent(g_stream, g_join_ev, 0));
+    g_side_dirty = false;
 }
 
 void *ptt_hip_scratch(int slot, size_t bytes) {

@@ -164,7 +164,7 @@ static void round_rel_cap_role(paratt *x, double eps, int cap, int role) {
         int ns = d - 1;
         float *dX = (float *)ptt_hip_scratch(PTT_WS_COEF, sizeof(float) * (LN_FEAT + 1) * (size_t)ns + 64);
         float *dO = dX + LN_FEAT * ns;
-        ptt_hip_h2d(dX, feat, sizeof(float) * LN_FEAT * (size_t)ns);
+        ptt_hip_h2d_queued(dX, feat, sizeof(float) * LN_FEAT * (size_t)ns);
         ptt_hip_mlp_forward(ns, dX, g_learn.dP, dO);
         float *out = (float *)ptt_host_malloc(sizeof(float) * (size_t)ns);
         ptt_hip_d2h(out, dO, sizeof(float) * (size_t)ns);

@@ -52,13 +52,17 @@ void pattacFormalSum(const int d, const int *n, const int *rx, double *const *x,
 void attac_tt_axpby(double a, attac_tt *x, double b, attac_tt *y, attac_tt *z) {
     int d = z->numDim;
     if (z == x || z == y) ptt_host_fatal("attac_tt_axpby", "z must not alias x or y");
+    long *count = (long *)ptt_host_malloc(sizeof(long) * (size_t)d);
     for (int k = 0; k < d; k++) {
         int r0 = (k == 0) ? 1 : x->ttRank[k] + y->ttRank[k];
         int r1 = (k == d - 1) ? 1 : x->ttRank[k + 1] + y->ttRank[k + 1];
-        ptt_host_reserve_core(z, k, core_count3(r0, z->dim[k], r1));
-        z->ttRank[k] = r0;
+        count[k] = core_count3(r0, z->dim[k], r1);
     }
+    if (z->coreMem == NULL) ptt_host_fatal("paratt_amd", "borrowed core too small");
+    ptt_host_reserve_train(z, count);
+    for (int k = 0; k < d; k++) z->ttRank[k] = (k == 0) ? 1 : x->ttRank[k] + y->ttRank[k];
     z->ttRank[d] = 1;
+    free(count);
     attacFormalAXPBY(x->numDim, x->dim, a, x->ttRank, x->coreList, b, y->ttRank, y->coreList,
                      z->ttRank, z->coreList);
 }

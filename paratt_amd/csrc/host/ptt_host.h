@@ -14,8 +14,9 @@ void ptt_host_set_diag(double *A, int m, double alpha);
 /* Wrap raw (d, n, r, cores) arrays of the pattac* API as a borrowed TT. */
 void ptt_host_view(attac_tt *view, int d, int *n, int *r, double **x);
 void ptt_host_view_release(attac_tt *view, double **x);
-/* Ensure core k of x can hold `count` doubles (contents not preserved). */
-void ptt_host_reserve_core(attac_tt *x, int k, long count);
+/* Ensure core k of x can hold count[k] doubles, for every core (contents of
+ * cores that grow are not preserved). */
+void ptt_host_reserve_train(attac_tt *x, const long *count);
 /* Upload a small host coefficient vector to the COEF scratch slot. */
 double *ptt_host_coef(const double *host, long count);
 void ptt_host_fatal(const char *fn, const char *msg);

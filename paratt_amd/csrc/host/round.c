@@ -834,7 +834,7 @@ static int rtl_step_sketch(attac_tt *x, int i, const int *maxr, double delta,
     }
     if (rho > 0) {
         int h_rho = rho;
-        ptt_hip_h2d(sw.iinfo + 8, &h_rho, sizeof(int));
+        ptt_hip_h2d_queued(sw.iinfo + 8, &h_rho, sizeof(int));
         /* new core (rho x w) = sqrt(n_i) V_rho^T Q_B */
         double *tmp = (double *)ptt_hip_scratch(PTT_WS_TMP, sizeof(double) * (size_t)rho * w);
         ptt_hip_dgemm('T', 'N', rho, (int)w, l, nscale[i], sw.V, l, B, l, 0.0, tmp, rho);

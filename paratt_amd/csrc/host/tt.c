@@ -77,19 +77,23 @@ paratt *alloc_ptt(int ndims, int *d, int *ttR) {
 }
 
 attac_tt *rank_change_tt(attac_tt *x, int *ttR) {
+    void **old = (void **)xmalloc(sizeof(void *) * (size_t)x->numDim);
+    int nold = 0;
     for (int k = 0; k < x->numDim; k++) {
         long need = (long)x->dim[k] * ttR[k] * ttR[k + 1];
         if (x->coreMem[k] < need) {
             /* realloc semantics: keep the old contents */
             double *nb = (double *)ptt_hip_malloc(sizeof(double) * (size_t)need);
             ptt_hip_d2d(nb, x->coreList[k], sizeof(double) * (size_t)x->coreMem[k]);
-            ptt_hip_free(x->coreList[k]);
+            old[nold++] = x->coreList[k];
             x->coreList[k] = nb;
             x->coreMem[k] = (int)need;
         }
         x->ttRank[k] = ttR[k];
     }
     x->ttRank[x->numDim] = ttR[x->numDim];
+    ptt_hip_free_many(nold, old);
+    free(old);
     return x;
 }
 
@@ -103,7 +107,7 @@ void copy_rank_change_tt(attac_tt *dest, attac_tt *src) {
 
 void free_tt(attac_tt *x) {
     if (!x) return;
-    for (int k = 0; k < x->numDim; k++) ptt_hip_free(x->coreList[k]);
+    ptt_hip_free_many(x->numDim, (void *const *)x->coreList);
     free(x->dim);
     free(x->ttRank);
     free(x->coreList);
@@ -121,15 +125,18 @@ void free_ptt(paratt *p) {
     free(p);
 }
 
-void ptt_host_reserve_core(attac_tt *x, int k, long count) {
-    if (x->coreMem == NULL) {
-        ptt_host_fatal("paratt_amd", "borrowed core too small");
-    }
-    if (x->coreMem[k] < count) {
-        ptt_hip_free(x->coreList[k]);
-        x->coreList[k] = (double *)ptt_hip_malloc(sizeof(double) * (size_t)count);
-        x->coreMem[k] = (int)count;
-    }
+void ptt_host_reserve_train(attac_tt *x, const long *count) {
+    void **old = (void **)xmalloc(sizeof(void *) * (size_t)x->numDim);
+    int nold = 0;
+    for (int k = 0; k < x->numDim; k++)
+        if (x->coreMem[k] < count[k]) old[nold++] = x->coreList[k];
+    ptt_hip_free_many(nold, old);
+    free(old);
+    for (int k = 0; k < x->numDim; k++)
+        if (x->coreMem[k] < count[k]) {
+            x->coreList[k] = (double *)ptt_hip_malloc(sizeof(double) * (size_t)count[k]);
+            x->coreMem[k] = (int)count[k];
+        }
 }
 
 void ptt_host_swap_core_with_tmp(attac_tt *x, int k, long count) {
@@ -162,7 +169,7 @@ void ptt_host_view_release(attac_tt *view, double **x) { (void)view; (void)x; }
 
 double *ptt_host_coef(const double *host, long count) {
     double *d = (double *)ptt_hip_scratch(PTT_WS_COEF, sizeof(double) * (size_t)(count > 0 ? count : 1));
-    ptt_hip_h2d(d, host, sizeof(double) * (size_t)count);
+    ptt_hip_h2d_queued(d, host, sizeof(double) * (size_t)count);
     return d;
 }
 
