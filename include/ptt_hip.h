@@ -109,6 +109,8 @@ void ptt_hip_axpby_core(int kind, int n, int rx0, int rx1, const double *x,
 void ptt_hip_axpby_train(int d, const int *kind, const int *n, const int *rx,
                          double *const *x, const int *ry, double *const *y, double a,
                          double b, double *const *z);
+/* dst[k][0..count[k]) = src[k][0..count[k]) for d cores. */
+void ptt_hip_copy_train(int d, double *const *dst, double *const *src, const long *count);
 /* S = sum_i D_i u as a rank-2r train of d cores: first [D u | u], interior
  * [[u, 0], [D u, u]], last [u; D u] (d = 1: D u), D the periodic 3-point
  * stencil of kind 0 below (host coefficients). */

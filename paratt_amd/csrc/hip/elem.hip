@@ -180,6 +180,32 @@ __global__ __launch_bounds__(256) void k_axpby_train(SumChunk ch) {
     }
 }
 
+struct CopyCore {
+    const double *src;
+    double *dst;
+    long count;
+};
+struct CopyChunk {
+    CopyCore c[TRAIN_CHUNK];
+};
+
+// Copies of whole cores (y over the cores): 16 bytes a lane, the odd element by
+// the first lane.  Unaligned cores go element by element.
+__global__ __launch_bounds__(256) void k_copy_train(CopyChunk ch) {
+    const CopyCore &c = ch.c[blockIdx.y];
+    const long stride = (long)gridDim.x * blockDim.x;
+    const long t0 = blockIdx.x * (long)blockDim.x + threadIdx.x;
+    if ((((uintptr_t)c.src | (uintptr_t)c.dst) & 15) == 0) {
+        const double2 *s2 = reinterpret_cast<const double2 *>(c.src);
+        double2 *d2 = reinterpret_cast<double2 *>(c.dst);
+        const long half = c.count >> 1;
+        for (long e = t0; e < half; e += stride) d2[e] = s2[e];
+        if (t0 == 0 && (c.count & 1)) c.dst[c.count - 1] = c.src[c.count - 1];
+    } else {
+        for (long e = t0; e < c.count; e += stride) c.dst[e] = c.src[e];
+    }
+}
+
 struct ModeSumCore {
     const double *u;
     double *s;
@@ -550,6 +576,34 @@ void ptt_hip_axpby_train(int d, const int *kind, const int *n, const int *rx,
     }
     flush(0);
     flush(1);
+}
+
+void ptt_hip_copy_train(int d, double *const *dst, double *const *src, const long *count) {
+    ptt_hip_init();
+    CopyChunk ch;
+    int cnt = 0;
+    long most = 0;
+    double bytes = 0.0;
+    for (int k = 0; k <= d; k++) {
+        if (k < d && count[k] > 0 && dst[k] != src[k]) {
+            ch.c[cnt].src = src[k];
+            ch.c[cnt].dst = dst[k];
+            ch.c[cnt].count = count[k];
+            cnt++;
+            most = count[k] > most ? count[k] : most;
+            bytes += 16.0 * (double)count[k];
+        }
+        if (cnt == TRAIN_CHUNK || (k == d && cnt > 0)) {
+            long gx = (most + 511) / 512;
+            const long cap = (16384 + cnt - 1) / cnt;
+            gx = gx < 1 ? 1 : gx > cap ? cap : gx;
+            PTT_LAUNCH_FB("copy_train", 0.0, bytes, k_copy_train, dim3((unsigned)gx, (unsigned)cnt),
+                          dim3(256), 0, ch);
+            cnt = 0;
+            most = 0;
+            bytes = 0.0;
+        }
+    }
 }
 
 void ptt_hip_axpby_core(int kind, int n, int rx0, int rx1, const double *x, int ry0, int ry1,

@@ -65,7 +65,21 @@ __global__ void k_seq_gemm(int M, int N, int K, int batch, const double *__restr
         const double *a = A + i + sA * q;
         const double *bcol = B + ldb * j + sB * q;
         double acc = 0.0;
-        for (int k = 0; k < K; k++) acc = acc + a[lda * k] * bcol[k];
+        int k = 0;
+        // sixteen terms in flight, added in order: the sums of a marginal are
+        // a few hundred lanes at most, so the walk is bound by the latency of
+        // its loads (25 sums of 64 terms: 15.5 -> 8.1 us a launch)
+        for (; k + 16 <= K; k += 16) {
+            double av[16], bv[16];
+#pragma unroll
+            for (int u = 0; u < 16; u++) {
+                av[u] = a[lda * (k + u)];
+                bv[u] = bcol[k + u];
+            }
+#pragma unroll
+            for (int u = 0; u < 16; u++) acc = acc + av[u] * bv[u];
+        }
+        for (; k < K; k++) acc = acc + a[lda * k] * bcol[k];
         C[i + ldc * j + sC * q] = acc;
     }
 }
@@ -141,7 +155,7 @@ void ptt_hip_seq_gemm(int M, int N, int K, int batch, const double *A, long lda,
     long total = (long)M * N * batch;
     if (total <= 0) return;
     PTT_LAUNCH_FB("seq_gemm", 2.0 * total * K, 8.0 * total, k_seq_gemm,
-                  dim3(stream_blocks(total, 256)), dim3(256), 0, M, N, K, batch, A, lda, sA, B,
+                  dim3(stream_blocks(total, 64)), dim3(64), 0, M, N, K, batch, A, lda, sA, B,
                   ldb, sB, C, ldc, sC);
 }
 

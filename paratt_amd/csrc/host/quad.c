@@ -94,21 +94,24 @@ void pattac_apply_marginal(paratt *f_ptt, paratt **marginal_ptt_ptr, int mode,
         long cols = (long)nn[mode + 1] * r[mode + 2];
         ptt_hip_seq_gemm(r0, (int)cols, r1, 1, wk, r0, 0, x->coreList[mode + 1], r1, 0,
                          m->x->coreList[mode], r0, 0);
-        for (int k = 0; k < mode; k++)
-            ptt_hip_d2d(m->x->coreList[k], x->coreList[k],
-                        sizeof(double) * (size_t)r[k] * nn[k] * r[k + 1]);
-        for (int k = mode + 1; k < d - 1; k++)
-            ptt_hip_d2d(m->x->coreList[k], x->coreList[k + 1],
-                        sizeof(double) * (size_t)r[k + 1] * nn[k + 1] * r[k + 2]);
     } else {
         /* last mode: marginal core d-2 = X_{d-2} (r_{d-2} n_{d-2} x r_{d-1}) * wk */
         long rows = (long)r[mode - 1] * nn[mode - 1];
         ptt_hip_seq_gemm((int)rows, 1, r0, 1, x->coreList[mode - 1], rows, 0, wk, r0, 0,
                          m->x->coreList[mode - 1], rows, 0);
-        for (int k = 0; k < mode - 1; k++)
-            ptt_hip_d2d(m->x->coreList[k], x->coreList[k],
-                        sizeof(double) * (size_t)r[k] * nn[k] * r[k + 1]);
     }
+    /* the other cores are x's own, in order */
+    double **from = (double **)ptt_host_malloc(sizeof(double *) * (size_t)(d - 1));
+    long *count = (long *)ptt_host_malloc(sizeof(long) * (size_t)(d - 1));
+    const int made = mode < d - 1 ? mode : mode - 1; /* formed above */
+    for (int k = 0; k < d - 1; k++) {
+        const int q = k < mode ? k : k + 1;
+        from[k] = x->coreList[q];
+        count[k] = k == made ? 0 : (long)r[q] * nn[q] * r[q + 1];
+    }
+    ptt_hip_copy_train(d - 1, m->x->coreList, from, count);
+    free(from);
+    free(count);
     ptt_hip_sync();
     free(md);
     free(mr);

@@ -99,9 +99,10 @@ attac_tt *rank_change_tt(attac_tt *x, int *ttR) {
 
 void copy_rank_change_tt(attac_tt *dest, attac_tt *src) {
     rank_change_tt(dest, src->ttRank);
-    for (int k = 0; k < dest->numDim; k++)
-        ptt_hip_d2d(dest->coreList[k], src->coreList[k],
-                    sizeof(double) * (size_t)core_count(src->dim, src->ttRank, k));
+    long *count = (long *)xmalloc(sizeof(long) * (size_t)dest->numDim);
+    for (int k = 0; k < dest->numDim; k++) count[k] = core_count(src->dim, src->ttRank, k);
+    ptt_hip_copy_train(dest->numDim, dest->coreList, src->coreList, count);
+    free(count);
     ptt_hip_sync();
 }
 
