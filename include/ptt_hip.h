@@ -193,9 +193,8 @@ void ptt_hip_chol_qr_factor(int c, const double *G, double shift, double tiny,
  * against delta, capped by min(k, cap), floor 1: written to iout[0]=numrank,
  * iout[1]=rho, iout[2]=sweeps; iout needs 5 ints.  Exactly-zero columns of
  * A are excluded from the rotations (their sigma is 0).  A is not changed.
- * k <= 1024: one workgroup, columns in LDS where they fit; k > 1024: the
- * columns stay in HBM and each round of the circle schedule is one launch
- * (one workgroup per pair), with one host read of a convergence flag per
+ * Small k: one wave or one workgroup, columns in LDS; larger k: blocks of
+ * columns over many workgroups, with one host read of a convergence flag per
  * sweep. */
 void ptt_hip_svd_jacobi(int m, int k, double *A, long lda, double *sig,
                         double *U, long ldu, double *V, long ldv,

@@ -54,4 +54,45 @@ inline unsigned stream_blocks(long n, int threads) {
     return (unsigned)(b < 1 ? 1 : (b > cap ? cap : b));
 }
 
+// ---- sums across the lanes of a wave
+// DPP move of a double inside a quad / row (dpp_ctrl CTRL); every source lane
+// used below is a valid lane of the same row.
+template <int CTRL>
+__device__ __forceinline__ double dppd(double v) {
+    int lo = __double2loint(v), hi = __double2hiint(v);
+    lo = __builtin_amdgcn_mov_dpp(lo, CTRL, 0xF, 0xF, false);
+    hi = __builtin_amdgcn_mov_dpp(hi, CTRL, 0xF, 0xF, false);
+    return __hiloint2double(hi, lo);
+}
+// Sum over each aligned quad of lanes (xor 1, xor 2 quad permutations).
+__device__ __forceinline__ double quad_sum(double x) {
+    x += dppd<0xB1>(x);
+    x += dppd<0x4E>(x);
+    return x;
+}
+// x + (x of lane ^ 16) and x + (x of lane ^ 32): the gfx950 lane-swap
+// instructions exchange the 16-lane rows of each half / the two halves.
+__device__ __forceinline__ double xor16_sum(double x) {
+    const int lo = __double2loint(x), hi = __double2hiint(x);
+    const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+    return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
+}
+__device__ __forceinline__ double xor32_sum(double x) {
+    const int lo = __double2loint(x), hi = __double2hiint(x);
+    const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+    return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
+}
+// Sum over the 64 lanes of a wave (every lane receives it): quad
+// permutations, half-row and row mirrors inside each 16-lane row, then the
+// two cross-row swaps.
+__device__ __forceinline__ double wave_sum(double x) {
+    x = quad_sum(x);
+    x += dppd<0x141>(x);
+    x += dppd<0x140>(x);
+    x = xor16_sum(x);
+    return xor32_sum(x);
+}
+
 }  // namespace ptt

@@ -24,6 +24,11 @@ constexpr int LDS_DOUBLES = 17408;  // 136 KB dynamic + static arrays <= 160 KB 
 // The Jacobi kernel holds 24 KB of static LDS (sorting and packing tables),
 // so its dynamic budget is smaller: 17280 doubles + 24.1 KB < 160 KB.
 constexpr int SVD_LDS_DOUBLES = 17280;
+// Columns beyond which the Jacobi SVD runs over many workgroups.  Measured with
+// V (us; flat spectrum, square): k = 48: 658 on one workgroup, 760 on many;
+// 59: 942 / 826; 96: 1830 / 1315; 128: 2370 / 2030; 192: 37600 / 4140 (the
+// columns of one workgroup are then in HBM).
+constexpr int SVD_ONE_WG_MAX = 56;
 constexpr int SVD_NT = 1024;  // Jacobi SVD workgroup: at most 16 waves, four per SIMD
 constexpr int SVD_RV = 8;     // rows per lane held in registers by a Jacobi pair
 
@@ -984,17 +989,14 @@ __device__ __forceinline__ double dpp_d(double v) {
 
 // Sum of three values over each aligned group of G lanes (G a power of two
 // <= 64), every lane receiving the sums: quad permutations (xor 1, xor 2),
-// then the half-row and row mirrors, then cross-row shuffles.
+// then the half-row and row mirrors, then the cross-row lane swaps.
 __device__ __forceinline__ void group_allreduce3_q(double &x, double &y, double &z, int G) {
     if (G >= 2) { x += dpp_d<0xB1>(x); y += dpp_d<0xB1>(y); z += dpp_d<0xB1>(z); }
     if (G >= 4) { x += dpp_d<0x4E>(x); y += dpp_d<0x4E>(y); z += dpp_d<0x4E>(z); }
     if (G >= 8) { x += dpp_d<0x141>(x); y += dpp_d<0x141>(y); z += dpp_d<0x141>(z); }
     if (G >= 16) { x += dpp_d<0x140>(x); y += dpp_d<0x140>(y); z += dpp_d<0x140>(z); }
-    for (int o = 16; o < G; o <<= 1) {
-        x += __shfl_xor(x, o);
-        y += __shfl_xor(y, o);
-        z += __shfl_xor(z, o);
-    }
+    if (G >= 32) { x = xor16_sum(x); y = xor16_sum(y); z = xor16_sum(z); }
+    if (G >= 64) { x = xor32_sum(x); y = xor32_sum(y); z = xor32_sum(z); }
 }
 
 // Round-robin pairing as rr_pair, without integer division.
@@ -1092,27 +1094,22 @@ __device__ __forceinline__ void rr_pair(int kp, int t, int p, int &a, int &b) {
     }
 }
 
-// INLDS: columns of A (and V when VLDS) live in LDS.  LOGROT: V is not
-// kept here; every pair's rotation (c, s) is logged and replayed afterwards
-// on the rows of V by k_svd_replay_v (rows of V evolve independently).
-template <bool INLDS, bool VLDS, bool LOGROT>
+// The columns of A and, when wanted, of V live in LDS.
 __global__ __launch_bounds__(SVD_NT) void k_svd_jacobi(int m, int k, const double *__restrict__ A,
                                                    long lda, double *__restrict__ sig,
                                                    double *__restrict__ U, long ldu,
                                                    double *__restrict__ V, long ldv,
                                                    double log_scale, double delta, int cap,
-                                                   int *iout, double *gwork,
-                                                   double2 *__restrict__ rotlog,
-                                                   int *__restrict__ posout) {
+                                                   int *iout) {
     extern __shared__ double lds[];
     const int tid = threadIdx.x;
     const int nth = blockDim.x;  // chosen by the launcher for the problem size
     // Columns in LDS use an odd stride (in doubles) so that the 16 pairs a
     // wave touches start in distinct banks.
-    const int ldw = INLDS ? (m | 1) : m;
-    double *W = INLDS ? lds : gwork;  // m x k, ld ldw
-    double *Vw = (V && !LOGROT) ? (VLDS ? lds + (long)ldw * k : gwork + (long)m * k) : nullptr;
-    const int ldvw = VLDS ? (k | 1) : k;
+    const int ldw = m | 1;
+    double *W = lds;  // m x k, ld ldw
+    double *Vw = V ? lds + (long)ldw * k : nullptr;
+    const int ldvw = k | 1;
     __shared__ int s_rot;
     __shared__ double s_sig[1024];
     __shared__ double s_sorted[1024];
@@ -1154,8 +1151,6 @@ __global__ __launch_bounds__(SVD_NT) void k_svd_jacobi(int m, int k, const doubl
             long j = e / k, i = e - j * k;
             Vw[i + j * ldvw] = (i == s_perm[j]) ? 1.0 : 0.0;
         }
-    if (LOGROT)
-        for (int j = tid; j < k; j += nth) posout[1024 + j] = s_perm[j];
     __syncthreads();
     const int knz = s_knz;
 
@@ -1266,8 +1261,6 @@ __global__ __launch_bounds__(SVD_NT) void k_svd_jacobi(int m, int k, const doubl
                 big = rot && ga * ga > 1e-16 * (al * be);
                 }
                 if (big) big_local = 1;
-                if (LOGROT && p < P && gl == 0)
-                    rotlog[((long)sweep * (kp - 1) + t) * P + p] = make_double2(cs, sn);
                 if (rot && !fix16 && !fix32) {
                     if (full) {
 #pragma unroll
@@ -1397,7 +1390,6 @@ __global__ __launch_bounds__(SVD_NT) void k_svd_jacobi(int m, int k, const doubl
     for (int j = tid; j < k; j += nth) {
         sig[s_pos[j]] = ldexp(s_sig[j], s_exp);
         s_sorted[s_pos[j]] = s_sig[j];  // scaled by 2^-e
-        if (LOGROT) posout[j] = s_pos[j];
     }
     for (long e = tid; e < (long)m * k; e += nth) {
         long j = e / m, i = e - j * m;
@@ -1432,43 +1424,7 @@ __global__ __launch_bounds__(SVD_NT) void k_svd_jacobi(int m, int k, const doubl
         iout[0] = numrank;
         iout[1] = rho;
         iout[2] = (sweep < max_sweeps) ? sweep + 1 : max_sweeps;
-        // sweeps written to the log: the loop breaks after a rotation-free
-        // sweep (logged as identities) or stops at max_sweeps
-        if (LOGROT) iout[3] = (sweep < max_sweeps) ? sweep + 1 : max_sweeps;
-        if (LOGROT) iout[4] = knz;
     }
-}
-
-// Replays the logged Jacobi rotations on the rows of V (V starts as I):
-// one wave per row, the row kept in LDS; each round applies the P disjoint
-// pair rotations in parallel.  Row i of V ends at V[i, pos[j]] = row[j].
-__global__ __launch_bounds__(64) void k_svd_replay_v(int k, const double2 *__restrict__ rotlog,
-                                                    const int *__restrict__ nsw,
-                                                    const int *__restrict__ pos,
-                                                    double *__restrict__ V, long ldv) {
-    __shared__ double row[1024];
-    const int i = blockIdx.x, lane = threadIdx.x;
-    const int knz = nsw[1];
-    const int kp = knz + (knz & 1), P = kp / 2;
-    const int *perm = pos + 1024;
-    for (int j = lane; j < 1024; j += 64) row[j] = (j < k && perm[j] == i) ? 1.0 : 0.0;
-    __syncthreads();
-    const int sweeps = *nsw;
-    for (int sw = 0; sw < sweeps; sw++)
-        for (int t = 0; t < kp - 1; t++) {
-            for (int p = lane; p < P; p += 64) {
-                int a, b;
-                rr_pair(kp, t, p, a, b);
-                double2 cs = rotlog[((long)sw * (kp - 1) + t) * P + p];
-                if (a < knz && b < knz && cs.y != 0.0) {
-                    double x = row[a], y = row[b];
-                    row[a] = cs.x * x - cs.y * y;
-                    row[b] = cs.y * x + cs.x * y;
-                }
-            }
-            __syncthreads();
-        }
-    for (int j = lane; j < k; j += 64) V[i + (long)pos[j] * ldv] = row[j];
 }
 
 // ---- one-sided Jacobi on one wave: k <= 32 columns, m <= 64 rows ---------
@@ -1653,14 +1609,20 @@ __global__ __launch_bounds__(64) void k_svd_jacobi_wave(int m, int k, const doub
     }
 }
 
-// ---- one-sided Jacobi for more than 1024 columns -------------------------
-// The columns live in HBM and every round of the circle schedule is one
-// launch: workgroup p owns pair p of the round (the pairs of a round are
-// disjoint), forms the three dot products over the m rows, and rotates its
-// two columns of W and of V.  Same rotation rule, threshold, scaling and
-// rank decisions as the one-workgroup kernel; the host checks once per
-// sweep whether any pair was still unsettled.
+// ---- one-sided Jacobi over many workgroups ---------------------------------
+// For column counts whose rotations one CU's LDS bandwidth or size would bound
+// (the line: SVD_ONE_WG_MAX).  The columns are cut into blocks of
+// B; a launch is one round of the circle schedule over the blocks, workgroup p
+// taking its pair of blocks (2 B columns of W, and of V) into LDS and rotating
+// every pair of columns across the two blocks, one wave a pair, B steps; the
+// first round of a sweep also takes the pairs inside the blocks.  A sweep is
+// thus k / B - 1 launches, each column read and written once a launch.  Same
+// rotation rule, threshold, scaling and rank decisions as the one-workgroup
+// kernel; the host checks once per sweep whether any pair was still unsettled.
+// Columns too long for 4 of them to fit in LDS (m + k above 4800) go through
+// HBM: one launch a round of single columns, one workgroup a pair (k_lj_round).
 constexpr int LJ_NT = 256;
+constexpr int LJ_LDS_DOUBLES = 19456;  // 152 KB
 
 __device__ __forceinline__ void lj_sum3(double &x, double &y, double &z, double *red) {
     for (int o = 32; o >= 1; o >>= 1) {
@@ -1761,6 +1723,153 @@ __global__ __launch_bounds__(LJ_NT) void k_lj_round(int m, int k, int kp, int t,
             const double x = va[i], y = vb[i];
             va[i] = cs * x - sn * y;
             vb[i] = sn * x + cs * y;
+        }
+    }
+}
+
+// Round t of the circle schedule over nblk (even) blocks of B columns, G lanes
+// a pair.  NR > 0: the columns are padded with zeros to G NR rows in LDS (no
+// guards; a lane holds NR rows of its pair in registers), and between the
+// blocks' pairs column g of the first block stays in its group's registers, so
+// only the second block goes through LDS.  NR = 0: columns of any length.  The
+// rotation's scalar work (about 60 FP64 instructions, a chain of some 600
+// cycles) is done by every lane of a group: sixteen lanes a pair, four pairs a
+// wave, keeps it from filling the FP64 pipes, which a wave a pair did (192
+// columns: 326 us a sweep that way).  ldc (odd): LDS stride of a column.
+template <int B, int G, int NR>
+__global__ __launch_bounds__(B * G) void k_lj_block(int m, int k, int nblk, int t, int ldc,
+                                                    double *__restrict__ W,
+                                                    double *__restrict__ V, double tol,
+                                                    int *__restrict__ flag) {
+    extern __shared__ double lds[];
+    const int g = threadIdx.x / G, gl = threadIdx.x % G;
+    int I, J;
+    rr_pair(nblk, t, blockIdx.x, I, J);
+    // columns beyond k belong to no pair; without a second block only the
+    // pairs inside the first one are left (round 0)
+    auto gcol = [&](int c) { return c < B ? I * B + c : J * B + (c - B); };
+    if ((I * B >= k || J * B >= k) && t != 0) return;  // uniform per workgroup
+    const int voff = NR > 0 ? G * NR : m;              // V's rows follow W's
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const int c = g + h * B, gc = gcol(c);
+        double *d = lds + (long)c * ldc;
+        if (gc < k) {
+            const double *w = W + (long)gc * m;
+            for (int i = gl; i < (NR > 0 ? G * NR : m); i += G) d[i] = (i < m) ? w[i] : 0.0;
+            if (V) {
+                const double *v = V + (long)gc * k;
+                for (int i = gl; i < (NR > 0 ? G * NR : k); i += G)
+                    d[voff + i] = (i < k) ? v[i] : 0.0;
+            }
+        }
+    }
+    __syncthreads();
+    bool open = false;
+    const double tol2 = tol * tol;
+    if (NR > 0 && t != 0) {
+        constexpr int R = NR > 0 ? NR : 1;
+        double *ca = lds + (long)g * ldc + gl;
+        double x[R], v[R];
+#pragma unroll
+        for (int q = 0; q < R; q++) {
+            x[q] = ca[G * q];
+            v[q] = V ? ca[G * R + G * q] : 0.0;
+        }
+        for (int s = 0; s < B; s++) {
+            const int b = B + ((g + s) & (B - 1));
+            if (gcol(g) < k && gcol(b) < k) {  // uniform per group
+                double *cb = lds + (long)b * ldc + gl;
+                double y[R];
+#pragma unroll
+                for (int q = 0; q < R; q++) y[q] = cb[G * q];
+                double al = 0.0, be = 0.0, ga = 0.0;
+#pragma unroll
+                for (int q = 0; q < R; q++) {
+                    al += x[q] * x[q];
+                    be += y[q] * y[q];
+                    ga += x[q] * y[q];
+                }
+                group_allreduce3_q(al, be, ga, G);
+                const double g2 = ga * ga, ab = al * be;
+                if (g2 > tol2 * ab && al > 0.0 && be > 0.0) {
+                    open = open || g2 > 4.0 * tol2 * ab;
+                    double cs, sn;
+                    jacobi_cs(al, be, ga, cs, sn);
+#pragma unroll
+                    for (int q = 0; q < R; q++) {
+                        cb[G * q] = sn * x[q] + cs * y[q];
+                        x[q] = cs * x[q] - sn * y[q];
+                    }
+                    if (V) {
+#pragma unroll
+                        for (int q = 0; q < R; q++) y[q] = cb[G * R + G * q];
+#pragma unroll
+                        for (int q = 0; q < R; q++) {
+                            cb[G * R + G * q] = sn * v[q] + cs * y[q];
+                            v[q] = cs * v[q] - sn * y[q];
+                        }
+                    }
+                }
+            }
+            __syncthreads();
+        }
+#pragma unroll
+        for (int q = 0; q < R; q++) {
+            ca[G * q] = x[q];
+            if (V) ca[G * R + G * q] = v[q];
+        }
+        __syncthreads();
+    } else {
+        const int len = NR > 0 ? (V ? 2 : 1) * G * NR : m + (V ? k : 0);
+        const int steps = (t == 0) ? 2 * B - 1 : B;
+        for (int s = 0; s < steps; s++) {
+            int a, b;
+            if (t == 0) {
+                rr_pair_fast(2 * B, s, g, a, b);
+            } else {
+                a = g;
+                b = B + ((g + s) & (B - 1));
+            }
+            if (gcol(a) < k && gcol(b) < k) {  // uniform per group
+                double *ca = lds + (long)a * ldc, *cb = lds + (long)b * ldc;
+                double al = 0.0, be = 0.0, ga = 0.0;
+#pragma unroll 4
+                for (int i = gl; i < m; i += G) {
+                    const double x = ca[i], y = cb[i];
+                    al += x * x;
+                    be += y * y;
+                    ga += x * y;
+                }
+                group_allreduce3_q(al, be, ga, G);
+                const double g2 = ga * ga, ab = al * be;
+                if (g2 > tol2 * ab && al > 0.0 && be > 0.0) {
+                    open = open || g2 > 4.0 * tol2 * ab;
+                    double cs, sn;
+                    jacobi_cs(al, be, ga, cs, sn);
+#pragma unroll 4
+                    for (int i = gl; i < len; i += G) {
+                        const double x = ca[i], y = cb[i];
+                        ca[i] = cs * x - sn * y;
+                        cb[i] = sn * x + cs * y;
+                    }
+                }
+            }
+            __syncthreads();
+        }
+    }
+    if (open && gl == 0) atomicOr(flag, 1);
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const int c = g + h * B, gc = gcol(c);
+        if (gc < k) {
+            const double *d = lds + (long)c * ldc;
+            double *w = W + (long)gc * m;
+            for (int i = gl; i < m; i += G) w[i] = d[i];
+            if (V) {
+                double *v = V + (long)gc * k;
+                for (int i = gl; i < k; i += G) v[i] = d[voff + i];
+            }
         }
     }
 }
@@ -1995,7 +2104,7 @@ void allow_big_lds() {
     set_lds_attr(k_chol_fast<512, CHOL_FAST_C, true>, CHOL_LDS_DOUBLES);
     set_lds_attr(k_chol_blk<true>, CB_LDS_DOUBLES);
     set_lds_attr(k_chol_blk<false>, CB_LDS_DOUBLES);
-    set_lds_attr(k_svd_jacobi<true, true, false>, SVD_LDS_DOUBLES);
+    set_lds_attr(k_svd_jacobi, SVD_LDS_DOUBLES);
     set_lds_attr(k_svd_jacobi_wave<4, 2>, SVW_LDS_DOUBLES);
     set_lds_attr(k_svd_jacobi_wave<4, 4>, SVW_LDS_DOUBLES);
     set_lds_attr(k_svd_jacobi_wave<4, 8>, SVW_LDS_DOUBLES);
@@ -2005,11 +2114,27 @@ void allow_big_lds() {
     set_lds_attr(k_svd_jacobi_wave<8, 8>, SVW_LDS_DOUBLES);
     set_lds_attr(k_svd_jacobi_wave<16, 2>, SVW_LDS_DOUBLES);
     set_lds_attr(k_svd_jacobi_wave<16, 4>, SVW_LDS_DOUBLES);
-    set_lds_attr(k_svd_jacobi<true, false, true>, SVD_LDS_DOUBLES);
+    set_lds_attr(k_lj_block<16, 16, 8>, LJ_LDS_DOUBLES);
+    set_lds_attr(k_lj_block<16, 16, 12>, LJ_LDS_DOUBLES);
+    set_lds_attr(k_lj_block<16, 16, 16>, LJ_LDS_DOUBLES);
+    set_lds_attr(k_lj_block<8, 32, 0>, LJ_LDS_DOUBLES);
+    set_lds_attr(k_lj_block<2, 64, 0>, LJ_LDS_DOUBLES);
     done = true;
 }
 
-// Jacobi SVD of an m x k matrix with k > 1024 (outputs as ptt_hip_svd_jacobi).
+// One launch a round of block pairs (see k_lj_block).
+template <int B, int G, int NR>
+void lj_block_sweep(int m, int k, double *W, double *V, double tol, int *flag) {
+    const int ldc = (NR > 0 ? (V ? 2 : 1) * G * NR : m + (V ? k : 0)) | 1;
+    int nblk = (k + B - 1) / B;
+    nblk += nblk & 1;
+    const size_t shm = sizeof(double) * 2 * B * (size_t)ldc;
+    for (int t = 0; t < nblk - 1; t++)
+        PTT_LAUNCH("lj_block", (k_lj_block<B, G, NR>), dim3(nblk / 2), dim3(B * G), shm, m, k, nblk,
+                   t, ldc, W, V, tol, flag);
+}
+
+// Jacobi SVD of an m x k matrix over many workgroups (outputs as ptt_hip_svd_jacobi).
 // Sweeps run until one sweep leaves no pair unsettled (one flag read per
 // sweep), at most 40 as in the one-workgroup kernel.
 void svd_jacobi_large(int m, int k, const double *A, long lda, double *sig, double *U, long ldu,
@@ -2027,14 +2152,28 @@ void svd_jacobi_large(int m, int k, const double *A, long lda, double *sig, doub
     PTT_LAUNCH("lj_load", k_lj_load, dim3(stream_blocks(total, 256)), dim3(256), 0, m, k, A, lda,
                dexp, W, Vw);
     const int kp = k + (k & 1), P = kp / 2;
+    const long ldc = (m + (V ? k : 0)) | 1;  // LDS stride of a column
+    const int most = m > k ? m : k;
     const double tol = 0x1.0p-53 * (double)m;
     const int max_sweeps = 40;
     int sweep = 0;
     for (; sweep < max_sweeps; sweep++) {
         ptt_hip_zero(flag, sizeof(double));
-        for (int t = 0; t < kp - 1; t++)
-            PTT_LAUNCH("lj_round", k_lj_round, dim3(P), dim3(LJ_NT), 0, m, k, kp, t, W, Vw, tol,
-                       flag);
+        // blocks of 16 columns while two of them fit in LDS, then 8, then 2
+        if (most <= 128)
+            lj_block_sweep<16, 16, 8>(m, k, W, Vw, tol, flag);
+        else if (most <= 192)
+            lj_block_sweep<16, 16, 12>(m, k, W, Vw, tol, flag);
+        else if (most <= 256)
+            lj_block_sweep<16, 16, 16>(m, k, W, Vw, tol, flag);
+        else if (16 * ldc <= LJ_LDS_DOUBLES)
+            lj_block_sweep<8, 32, 0>(m, k, W, Vw, tol, flag);
+        else if (4 * ldc <= LJ_LDS_DOUBLES)
+            lj_block_sweep<2, 64, 0>(m, k, W, Vw, tol, flag);
+        else
+            for (int t = 0; t < kp - 1; t++)
+                PTT_LAUNCH("lj_round", k_lj_round, dim3(P), dim3(LJ_NT), 0, m, k, kp, t, W, Vw, tol,
+                           flag);
         int f = 0;
         ptt_hip_d2h(&f, flag, sizeof(int));
         if (!f) break;
@@ -2118,7 +2257,9 @@ void ptt_hip_svd_jacobi(int m, int k, double *A, long lda, double *sig, double *
     ptt_hip_init();
     allow_big_lds();
     if (m <= 0 || k <= 0) return;
-    if (k > 1024) {
+    // LDS footprint of the one-workgroup kernel's padded columns
+    const size_t lds_need = (size_t)(m | 1) * k + (V ? (size_t)(k | 1) * k : 0);
+    if (k > SVD_ONE_WG_MAX || (lds_need > (size_t)SVD_LDS_DOUBLES && !(k <= SVW_K && m <= SVW_M))) {
         svd_jacobi_large(m, k, A, lda, sig, U, ldu, V, ldv, log_scale, delta, cap, iout);
         return;
     }
@@ -2154,7 +2295,7 @@ void ptt_hip_svd_jacobi(int m, int k, double *A, long lda, double *sig, double *
         return;
     }
     // algorithmic work of a dense SVD with left vectors (Golub-Reinsch
-    // count 4 m k^2 + 8 k^3; right vectors are counted by their replay)
+    // count 4 m k^2 + 8 k^3, 9 k^3 for the right vectors)
     const double svd_flops = 4.0 * m * (double)k * k + 8.0 * (double)k * k * k;
     const double svd_bytes = 8.0 * (2.0 * m * (double)k + k);
     // threads: each Jacobi pair gets G lanes with about SVD_RV rows per lane, the
@@ -2166,37 +2307,9 @@ void ptt_hip_svd_jacobi(int m, int k, double *A, long lda, double *sig, double *
     nth = ((nth + 63) / 64) * 64;
     if (nth > SVD_NT) nth = SVD_NT;
     if (nth < 64) nth = 64;
-    const size_t kk = (size_t)(k | 1) * k;  // padded V footprint (LDS case)
-    const size_t mk = (size_t)m * k;
-    const size_t mkl = (size_t)(m | 1) * k;  // LDS footprint of the padded columns
-    if (mkl + (V ? kk : 0) <= (size_t)SVD_LDS_DOUBLES) {
-        PTT_LAUNCH_FB("svd_jacobi", svd_flops + (V ? 9.0 * k * (double)k * k : 0.0), svd_bytes,
-                   (k_svd_jacobi<true, true, false>), dim3(1), dim3(nth),
-                   (mkl + (V ? kk : 0)) * sizeof(double), m, k, A, lda, sig, U, ldu, V, ldv,
-                   log_scale, delta, cap, iout, (double *)nullptr, (double2 *)nullptr,
-                   (int *)nullptr);
-    } else if (mkl <= (size_t)SVD_LDS_DOUBLES) {
-        // columns in LDS; V (if wanted) from the rotation log
-        const int kp = k + (k & 1), P = kp / 2;
-        const size_t logn = (size_t)40 * (kp - 1) * P;
-        char *ws = (char *)ptt_hip_scratch(PTT_WS_SKETCH, logn * sizeof(double2) + 2048 * sizeof(int));
-        double2 *rotlog = (double2 *)ws;
-        int *pos = (int *)(ws + logn * sizeof(double2));
-        PTT_LAUNCH_FB("svd_jacobi", svd_flops, svd_bytes, (k_svd_jacobi<true, false, true>),
-                   dim3(1), dim3(nth),
-                   mkl * sizeof(double), m, k, A, lda, sig, U, ldu, V, ldv, log_scale, delta, cap,
-                   iout, (double *)nullptr, rotlog, pos);
-        if (V)
-            PTT_LAUNCH_FB("svd_replay_v", 9.0 * k * (double)k * k, 8.0 * k * (double)k,
-                          k_svd_replay_v, dim3(k), dim3(64), 0, k, rotlog, iout + 3,
-                       pos, V, ldv);
-    } else {
-        double *gwork = (double *)ptt_hip_scratch(PTT_WS_SKETCH, (mk + (V ? kk : 0)) * sizeof(double));
-        PTT_LAUNCH_FB("svd_jacobi", svd_flops + (V ? 9.0 * k * (double)k * k : 0.0), svd_bytes,
-                   (k_svd_jacobi<false, false, false>), dim3(1), dim3(nth), 0, m, k,
-                   A, lda, sig, U, ldu, V, ldv, log_scale, delta, cap, iout, gwork,
-                   (double2 *)nullptr, (int *)nullptr);
-    }
+    PTT_LAUNCH_FB("svd_jacobi", svd_flops + (V ? 9.0 * k * (double)k * k : 0.0), svd_bytes,
+                  k_svd_jacobi, dim3(1), dim3(nth), lds_need * sizeof(double), m, k, A, lda, sig, U,
+                  ldu, V, ldv, log_scale, delta, cap, iout);
 }
 
 void ptt_hip_svd_factors(int m, int rhomax, const int *drho, const double *U, long ldu,
