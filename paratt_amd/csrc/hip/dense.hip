@@ -20,7 +20,6 @@ using namespace ptt;
 namespace {
 
 constexpr int NT = 1024;
-constexpr int LDS_DOUBLES = 17408;  // 136 KB dynamic + static arrays <= 160 KB LDS
 // The Jacobi kernel holds 24 KB of static LDS (sorting and packing tables),
 // so its dynamic budget is smaller: 17280 doubles + 24.1 KB < 160 KB.
 constexpr int SVD_LDS_DOUBLES = 17280;
@@ -44,194 +43,187 @@ __device__ double max_sq(const double *D, int c) {
     return m;
 }
 
-template <bool INLDS>
-__global__ __launch_bounds__(NT) void k_chol_qr_factor(int c, const double *__restrict__ G,
-                                                       double shift, double tiny,
-                                                       double *__restrict__ R,
-                                                       double *__restrict__ T, int *info,
-                                                       double *dinfo, double *gwork,
-                                                       int want_kappa) {
-    extern __shared__ double lds[];
-    const int tid = threadIdx.x;
-    // INLDS: the work matrix is LDS-resident (the compiler sees the shared
-    // address space and issues ds_* instructions); else global scratch.
-    double *S = INLDS ? lds : gwork;
-    double *D = S + (long)c * c;
-    double *col = D + c;   // temp vector
-    double *dd = col + c;  // deficient flags
-    double *pv = dd + c;   // power-iteration vector (2c)
-    __shared__ int s_def;
-    __shared__ double s_red[NT / 64];
-    __shared__ double s_rjj, s_scal;
-    __shared__ int s_isdef;
+// ---- factors of more than 128 columns ----------------------------------------
+// Blocks of 128 columns: the scaled Gram (k_chol_scale) is factored block row by
+// block row, the diagonal block by k_chol_blk (with its inverse), the rest of
+// the block row as T_PP^T S and the trailing update as matrix products on the
+// matrix cores; the inverse's off-diagonal blocks are two products each.  One
+// workgroup eliminating column by column through global memory took 1680 us at
+// 192 columns.
 
-    for (int j = tid; j < c; j += NT) {
-        double g = G[j + (long)j * c];
-        D[j] = g > 0.0 ? sqrt(g) : 0.0;
+// D and its inverse (c each), S = D^-1 G D^-1 + shift I (ld c; rows and columns of a zero diagonal
+// are zero).
+__global__ void k_chol_scale(int c, const double *__restrict__ G, double shift,
+                             double *__restrict__ D, double *__restrict__ iD,
+                             double *__restrict__ S) {
+    const long total = (long)c * c;
+    for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < total;
+         e += (long)gridDim.x * blockDim.x) {
+        const int k = (int)(e / c), i = (int)(e - (long)k * c);
+        const double gi = G[i + (long)i * c], gk = G[k + (long)k * c];
+        const double di = gi > 0.0 ? sqrt(gi) : 0.0, dk = gk > 0.0 ? sqrt(gk) : 0.0;
+        double v = (di > 0.0 && dk > 0.0) ? G[e] / (di * dk) : 0.0;
+        if (i == k) {
+            D[i] = di;
+            iD[i] = di > 0.0 ? 1.0 / di : 0.0;
+            if (di > 0.0) v += shift;
+        }
+        S[e] = v;
     }
-    if (tid == 0) s_def = 0;
-    __syncthreads();
-    // G is symmetric: S(i,k) = G[i + k*c] / (D_i D_k), stored row-major.
-    for (long e = tid; e < (long)c * c; e += NT) {
-        int k = (int)(e % c), i = (int)(e / c);
-        double di = D[i], dk = D[k];
-        S[e] = (di > 0.0 && dk > 0.0) ? G[k + (long)i * c] / (di * dk) : 0.0;
+}
+
+// R = Rs D, T = D^-1 Ts in place (zeros below the diagonal), T NULL for R only.
+__global__ void k_chol_unscale(int c, const double *__restrict__ D, double *__restrict__ R,
+                               double *__restrict__ T) {
+    const long total = (long)c * c;
+    for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < total;
+         e += (long)gridDim.x * blockDim.x) {
+        const int k = (int)(e / c), i = (int)(e - (long)k * c);
+        R[e] = (i <= k) ? R[e] * D[k] : 0.0;
+        if (T) T[e] = (i <= k && D[i] > 0.0) ? T[e] / D[i] : 0.0;
     }
-    __syncthreads();
-    // lambda_max of the scaled Gram by power iteration (before it is overwritten)
+}
+
+// Deficient pivots and the condition estimates, from G, D, R and T as the
+// smaller factors' kernels report them: Gershgorin's bound, else the pivots
+// where they decide, else power iterations.  binfo[b]: deficient pivots of
+// block b.  y, z: c doubles of scratch each.  One workgroup.
+__global__ __launch_bounds__(NT) void k_chol_report(int c, const double *__restrict__ G,
+                                                    const double *__restrict__ D,
+                                                    const double *__restrict__ iD,
+                                                    const double *__restrict__ R,
+                                                    const double *__restrict__ T, int nblk,
+                                                    const int *__restrict__ binfo,
+                                                    double *__restrict__ y,
+                                                    double *__restrict__ z, int *info,
+                                                    double *dinfo, int want_kappa) {
+    __shared__ double s_red[NT / 64], s_part[NT];
+    const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
+    const int cpad = c < NT ? c : NT, parts = NT / cpad;
     auto block_sum = [&](double v) -> double {
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+        v = wave_sum(v);
         __syncthreads();
-        if ((tid & 63) == 0) s_red[tid >> 6] = v;
+        if (lane == 0) s_red[wv] = v;
         __syncthreads();
         double t = 0.0;
         for (int i = 0; i < NT / 64; i++) t += s_red[i];
         return t;
     };
-    const int PIT = want_kappa ? 10 : 0;
-    for (int i = tid; i < c; i += NT) pv[i] = 1.0 + 0.01 * (i % 7);
-    __syncthreads();
-    double lmax = 0.0;
-    for (int it = 0; it < PIT; it++) {
-        // y = S x (rows in parallel, 8 lanes per row)
-        const int row = tid >> 3, sub = tid & 7;
-        for (int i0 = 0; i0 < c; i0 += NT / 8) {
-            int i = i0 + row;
-            double acc = 0.0;
-            if (i < c)
-                for (int l = sub; l < c; l += 8) acc += S[(long)i * c + l] * pv[l];
-            acc += __shfl_xor(acc, 1);
-            acc += __shfl_xor(acc, 2);
-            acc += __shfl_xor(acc, 4);
-            if (i < c && sub == 0) pv[c + i] = acc;
+    auto block_max = [&](double v) -> double {
+        for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o));
+        __syncthreads();
+        if (lane == 0) s_red[wv] = v;
+        __syncthreads();
+        double t = 0.0;
+        for (int i = 0; i < NT / 64; i++) t = fmax(t, s_red[i]);
+        return t;
+    };
+    double dmax = 0.0, pmax = 0.0, pneg = -INFINITY;
+    for (int j = tid; j < c; j += NT) {
+        dmax = fmax(dmax, D[j] * D[j]);
+        const double r = R[j + (long)j * c] * iD[j], p = r * r;
+        if (p > 0.0) {
+            pmax = fmax(pmax, p);
+            pneg = fmax(pneg, -p);
         }
-        __syncthreads();
-        double nn = 0.0;
-        for (int i = tid; i < c; i += NT) nn += pv[c + i] * pv[c + i];
-        nn = block_sum(nn);
-        double xn = 0.0;
-        for (int i = tid; i < c; i += NT) xn += pv[i] * pv[i];
-        xn = block_sum(xn);
-        lmax = (xn > 0.0) ? sqrt(nn / xn) : 0.0;
-        double inv = nn > 0.0 ? 1.0 / sqrt(nn) : 0.0;
-        for (int i = tid; i < c; i += NT) pv[i] = pv[c + i] * inv;
-        __syncthreads();
     }
-    // Right-looking Cholesky, upper triangle, row-major.
-    for (int j = 0; j < c; j++) {
-        if (tid == 0) {
-            double p = S[(long)j * c + j] + shift;
-            int dead = !(D[j] > 0.0) || !(p > tiny);
-            s_isdef = dead;
-            s_rjj = dead ? 0.0 : sqrt(p);
-            S[(long)j * c + j] = s_rjj;
-            dd[j] = dead ? 1.0 : 0.0;
-            if (dead) s_def += 1;
-        }
+    dmax = block_max(dmax);
+    pmax = block_max(pmax);
+    {
+        for (int o = 32; o > 0; o >>= 1) pneg = fmax(pneg, __shfl_xor(pneg, o));
         __syncthreads();
-        const double rjj = s_rjj;
-        const int dead = s_isdef;
-        for (int k = j + 1 + tid; k < c; k += NT)
-            S[(long)j * c + k] = dead ? 0.0 : S[(long)j * c + k] / rjj;
+        if (lane == 0) s_red[wv] = pneg;
         __syncthreads();
-        if (!dead) {
-            const int w = c - j - 1;
-            // entries (i,k), j < i <= k: thread -> consecutive k for fixed i
-            for (long t = tid; t < (long)w * w; t += NT) {
-                int i = j + 1 + (int)(t / w), k = j + 1 + (int)(t % w);
-                if (i <= k) S[(long)i * c + k] -= S[(long)j * c + i] * S[(long)j * c + k];
+        for (int i = 0; i < NT / 64; i++) pneg = fmax(pneg, s_red[i]);
+    }
+    const double pmin = -pneg;
+    int ndef = 0;
+    for (int b = 0; b < nblk; b++) ndef += binfo[b];
+    double fr = 0.0, ft = 0.0, eoff = 0.0, lmax = 0.0, lminv = 0.0;
+    bool gersh = false, decided = false;
+    if (T) {
+        // one wave a column
+        for (int k = wv; k < c; k += NT / 64) {
+            const double dk = iD[k];
+            double rs = 0.0;
+#pragma unroll 4
+            for (int i = lane; i < c; i += 64) {
+                const double r = R[i + (long)k * c] * dk, t = T[i + (long)k * c] * D[i];
+                fr += r * r;
+                ft += t * t;
+                if (i != k) rs += fabs(G[i + (long)k * c]) * iD[i] * dk;
             }
+            eoff = fmax(eoff, wave_sum(rs));
         }
-        __syncthreads();
-    }
-    // ||Rs||_F and R = Rs * D (column-major output, zeros below).
-    double fr = 0.0;
-    for (long e = tid; e < (long)c * c; e += NT) {
-        int i = (int)(e % c), k = (int)(e / c);
-        double v = (i <= k) ? S[(long)i * c + k] : 0.0;
-        fr += v * v;
-        R[e] = v * D[k];
-    }
-    fr = block_sum(fr);
-    // In-place inverse of the upper triangle, column by column (row-major S:
-    // row i of the inverse is contiguous); 8 lanes per row share each dot.
-    for (int j = 0; j < c; j++) {
-        const bool dead = dd[j] != 0.0;
-        for (int i = tid; i < j; i += NT) col[i] = S[(long)i * c + j];
-        __syncthreads();
-        const double tjj = dead ? 0.0 : 1.0 / S[(long)j * c + j];
-        const int row = tid >> 3, sub = tid & 7;
-        for (int i0 = 0; i0 < j; i0 += NT / 8) {
-            int i = i0 + row;
-            double sacc = 0.0;
-            if (i < j && !dead)
-                for (int l = i + sub; l < j; l += 8) sacc += S[(long)i * c + l] * col[l];
-            sacc += __shfl_xor(sacc, 1);
-            sacc += __shfl_xor(sacc, 2);
-            sacc += __shfl_xor(sacc, 4);
-            if (i < j && sub == 0) S[(long)i * c + j] = dead ? 0.0 : -sacc * tjj;
+        fr = block_sum(fr);
+        ft = block_sum(ft);
+        eoff = block_max(eoff);
+        gersh = want_kappa && eoff < 0.5;
+        decided = ndef > 0 || !(pmax <= 1e12 * pmin);
+        const int PIT = (want_kappa && !gersh && !decided) ? 6 : 0;
+        for (int side = 0; side < 2; side++) {
+            for (int i = tid; i < c; i += NT) y[i] = 1.0 + 0.01 * (i % 7);
+            __syncthreads();
+            for (int it = 0; it < PIT; it++) {
+                double xn = 0.0;
+                for (int i = tid; i < c; i += NT) xn += y[i] * y[i];
+                xn = block_sum(xn);
+                const double is = xn > 0.0 ? 1.0 / sqrt(xn) : 0.0;
+                // side 0: z = S y; side 1: z = Ts^T y, then y = Ts z
+                for (int k = wv; k < c; k += NT / 64) {
+                    double acc = 0.0;
+                    if (side == 0)
+#pragma unroll 4
+                        for (int i = lane; i < c; i += 64)
+                            acc += G[i + (long)k * c] * iD[i] * y[i];
+                    else
+#pragma unroll 4
+                        for (int i = lane; i <= k; i += 64) acc += T[i + (long)k * c] * D[i] * y[i];
+                    acc = wave_sum(acc);
+                    if (lane == 0) z[k] = acc * is * (side == 0 ? iD[k] : 1.0);
+                }
+                __syncthreads();
+                if (side == 1) {
+                    // rows on consecutive lanes, the columns split over parts
+                    for (int i0 = 0; i0 < c; i0 += cpad) {
+                        const int i = i0 + tid % cpad, part = tid / cpad;
+                        double acc = 0.0;
+                        if (i < c && part < parts) {
+                            const int per = (c - i0 + parts - 1) / parts;
+                            const int k0 = i0 + part * per, k1 = min(c, k0 + per);
+#pragma unroll 8
+                            for (int k = k0; k < k1; k++) acc += T[i + (long)k * c] * z[k];
+                        }
+                        __syncthreads();
+                        s_part[tid] = acc;
+                        __syncthreads();
+                        if (part == 0 && i < c) {
+                            for (int q = 1; q < parts; q++) acc += s_part[tid + q * cpad];
+                            y[i] = acc * D[i];
+                        }
+                    }
+                } else {
+                    for (int i = tid; i < c; i += NT) y[i] = z[i];
+                }
+                __syncthreads();
+                double nn = 0.0;
+                for (int i = tid; i < c; i += NT) nn += y[i] * y[i];
+                nn = block_sum(nn);
+                (side == 0 ? lmax : lminv) = sqrt(nn);
+            }
+            __syncthreads();
         }
-        __syncthreads();
-        if (tid == 0) S[(long)j * c + j] = tjj;
-        __syncthreads();
-    }
-    double ft = 0.0;
-    for (long e = tid; e < (long)c * c; e += NT) {
-        int i = (int)(e % c), k = (int)(e / c);
-        double v = (i <= k) ? S[(long)i * c + k] : 0.0;
-        ft += v * v;
-        T[e] = (D[i] > 0.0) ? v / D[i] : 0.0;
-    }
-    ft = block_sum(ft);
-    // lambda_max(G^-1) = ||Rs^-1||_2^2 by power iteration on Ts Ts^T
-    for (int i = tid; i < c; i += NT) pv[i] = 1.0 + 0.01 * (i % 5);
-    __syncthreads();
-    double lminv = 0.0;
-    for (int it = 0; it < PIT; it++) {
-        const int row = tid >> 3, sub = tid & 7;
-        // u = Ts^T x  (u_k = sum_{i<=k} Ts(i,k) x_i)
-        for (int k0 = 0; k0 < c; k0 += NT / 8) {
-            int k = k0 + row;
-            double acc = 0.0;
-            if (k < c)
-                for (int i = sub; i <= k; i += 8) acc += S[(long)i * c + k] * pv[i];
-            acc += __shfl_xor(acc, 1);
-            acc += __shfl_xor(acc, 2);
-            acc += __shfl_xor(acc, 4);
-            if (k < c && sub == 0) col[k] = acc;
-        }
-        __syncthreads();
-        // y = Ts u  (y_i = sum_{k>=i} Ts(i,k) u_k)
-        for (int i0 = 0; i0 < c; i0 += NT / 8) {
-            int i = i0 + row;
-            double acc = 0.0;
-            if (i < c)
-                for (int k = i + sub; k < c; k += 8) acc += S[(long)i * c + k] * col[k];
-            acc += __shfl_xor(acc, 1);
-            acc += __shfl_xor(acc, 2);
-            acc += __shfl_xor(acc, 4);
-            if (i < c && sub == 0) pv[c + i] = acc;
-        }
-        __syncthreads();
-        double nn = 0.0;
-        for (int i = tid; i < c; i += NT) nn += pv[c + i] * pv[c + i];
-        nn = block_sum(nn);
-        double xn = 0.0;
-        for (int i = tid; i < c; i += NT) xn += pv[i] * pv[i];
-        xn = block_sum(xn);
-        lminv = (xn > 0.0) ? sqrt(nn / xn) : 0.0;
-        double inv = nn > 0.0 ? 1.0 / sqrt(nn) : 0.0;
-        for (int i = tid; i < c; i += NT) pv[i] = pv[c + i] * inv;
-        __syncthreads();
     }
     if (tid == 0) {
-        dinfo[0] = sqrt(fr) * sqrt(ft);      // Frobenius condition (upper bound, >= c)
-        dinfo[1] = want_kappa ? sqrt(lmax * lminv) : 0.0;  // 2-norm condition of Rs
-        dinfo[2] = (double)s_def;
-        dinfo[3] = max_sq(D, c);
-        info[0] = s_def;
+        dinfo[0] = sqrt(fr) * sqrt(ft);
+        dinfo[1] = !(T && want_kappa) ? 0.0
+                   : gersh            ? sqrt((1.0 + eoff) / (1.0 - eoff))
+                   : decided          ? (pmin > 0.0 && pmin < INFINITY ? sqrt(pmax / pmin) : 0.0)
+                                      : sqrt(lmax * lminv);
+        dinfo[2] = (double)ndef;
+        dinfo[3] = dmax;
+        info[0] = ndef;
     }
-    (void)s_scal;
 }
 
 // Low-latency variant for c <= CMAX <= 128 (the whole problem in LDS, the
@@ -242,8 +234,7 @@ __global__ __launch_bounds__(NT) void k_chol_qr_factor(int c, const double *__re
 // Rs = diag(sqrt p) L^T, so Ts = Rs^-1 = L^-T diag(1/sqrt p).  A dead pivot
 // skips its step, which leaves row and column j of Ts zero.  Ts(i,k) for
 // i < k is kept transposed in the lower triangle of S, its diagonal in tdg.
-// NTH threads (64, 256 or 512, chosen for c).  Same outputs and conventions
-// as k_chol_qr_factor.
+// NTH threads (64, 256 or 512, chosen for c).
 constexpr int CHOL_FAST_C = 128;
 constexpr int CHOL_BLK = 32;
 constexpr int CHOL_LDS_DOUBLES = 20400;  // c(c+1) + 5c + 3*32*32 = 20224 at c = 128; 159.4 KB
@@ -606,11 +597,15 @@ __device__ __forceinline__ double rcp2(double x) {
     return fma(r, e, r);
 }
 
+// With `unit` the input is already scaled (a diagonal block of a larger scaled
+// Gram, ptt_hip_chol_qr_factor beyond 128 columns): D = 1, pivots are tested as
+// they come.  ldg, ldo: leading dimensions of G and of R and T.
 template <bool WT>
-__global__ __launch_bounds__(512) void k_chol_blk(int c, const double *__restrict__ G,
+__global__ __launch_bounds__(512) void k_chol_blk(int c, const double *__restrict__ G, long ldg,
                                                   double shift, double tiny,
                                                   double *__restrict__ R, double *__restrict__ T,
-                                                  int *info, double *dinfo, int want_kappa) {
+                                                  long ldo, int *info, double *dinfo,
+                                                  int want_kappa, int unit) {
     constexpr int nth = 512;
     extern __shared__ double lds[];
     double *S = lds;                  // 128 x 129, S[i + j * CB_LD]
@@ -647,8 +642,8 @@ __global__ __launch_bounds__(512) void k_chol_blk(int c, const double *__restric
     for (int j = tid; j < 128; j += nth) {
         double dj = 0.0;
         if (j < c) {
-            const double g = G[j + (long)j * c];
-            dj = g > 0.0 ? sqrt(g) : 0.0;
+            const double g = G[j + (long)j * ldg];
+            dj = unit ? 1.0 : g > 0.0 ? sqrt(g) : 0.0;
         }
         D[j] = dj;
         iD[j] = dj > 0.0 ? 1.0 / dj : 0.0;
@@ -663,7 +658,7 @@ __global__ __launch_bounds__(512) void k_chol_blk(int c, const double *__restric
 #pragma unroll
             for (int h = 0; h < 2; h++) {
                 const int j = wv + u * (nth / 64), i = lane + 64 * h;
-                gv[u][h] = (i < c && j < c) ? G[i + (long)j * c] : 0.0;
+                gv[u][h] = (i < c && j < c) ? G[i + (long)j * ldg] : 0.0;
             }
 #pragma unroll
         for (int u = 0; u < 16; u++)
@@ -882,8 +877,8 @@ __global__ __launch_bounds__(512) void k_chol_blk(int c, const double *__restric
             }
             fr += rv * rv;
             ft += tv * tv;
-            R[i + (long)k * c] = rv * dk;
-            if (WT) T[i + (long)k * c] = tv * iD[i];
+            R[i + (long)k * ldo] = rv * dk;
+            if (WT) T[i + (long)k * ldo] = tv * iD[i];
         }
     }
     if (!WT) {
@@ -2093,7 +2088,6 @@ void set_lds_attr(KF kern, int ndoubles) {
 void allow_big_lds() {
     static bool done = false;
     if (done) return;
-    set_lds_attr(k_chol_qr_factor<true>, LDS_DOUBLES);
     set_lds_attr(k_chol_fast<64, 16, false>, CHOL_LDS_DOUBLES);
     set_lds_attr(k_chol_fast<256, 48, false>, CHOL_LDS_DOUBLES);
     set_lds_attr(k_chol_fast<256, 32, false>, CHOL_LDS_DOUBLES);
@@ -2199,7 +2193,6 @@ void ptt_hip_chol_qr_factor(int c, const double *G, double shift, double tiny, d
         const char *e = getenv("PARATT_AMD_CHOL_UNBLOCKED");
         g_chol_unblocked = (e && e[0] == '1') ? 1 : 0;
     }
-    size_t need = (size_t)c * c + 5 * (size_t)c;
     if (c <= CHOL_FAST_C) {
         const size_t fneed = (size_t)c * (c | 1) + 5 * (size_t)c + 3 * CHOL_BLK * CHOL_BLK;
         // fewer threads for small factors: the steps are barrier-bound
@@ -2229,26 +2222,53 @@ void ptt_hip_chol_qr_factor(int c, const double *G, double shift, double tiny, d
             // panels of 16 columns: two barriers per panel
             const size_t bneed = (size_t)CB_LDS_DOUBLES * sizeof(double);
             if (T)
-                PTT_LAUNCH_FB(nm, fl, by, k_chol_blk<true>, dim3(1), dim3(512), bneed, c, G, shift,
-                              tiny, R, T, info, dinfo, wk);
+                PTT_LAUNCH_FB(nm, fl, by, k_chol_blk<true>, dim3(1), dim3(512), bneed, c, G,
+                              (long)c, shift, tiny, R, T, (long)c, info, dinfo, wk, 0);
             else
                 PTT_LAUNCH_FB(nm, fl, by, k_chol_blk<false>, dim3(1), dim3(512), bneed, c, G,
-                              shift, tiny, R, T, info, dinfo, wk);
+                              (long)c, shift, tiny, R, T, (long)c, info, dinfo, wk, 0);
         }
 #undef PTT_CHOL_FAST
         return;
     }
-    // the large-factor kernel always forms the inverse
-    if (!T) T = (double *)ptt_hip_scratch(PTT_WS_TMP2, sizeof(double) * (size_t)c * c);
-    if (need <= (size_t)LDS_DOUBLES) {
-        PTT_LAUNCH("chol_qr_factor", k_chol_qr_factor<true>, dim3(1), dim3(NT),
-                   need * sizeof(double), c, G, shift, tiny, R, T, info, dinfo, (double *)nullptr,
-                   want_kappa);
-    } else {
-        double *gwork = (double *)ptt_hip_scratch(PTT_WS_SKETCH, need * sizeof(double));
-        PTT_LAUNCH("chol_qr_factor", k_chol_qr_factor<false>, dim3(1), dim3(NT), 0, c, G, shift,
-                   tiny, R, T, info, dinfo, gwork, want_kappa);
+    // blocks of 128 columns
+    const int nblk = (c + 127) / 128;
+    const size_t cc = (size_t)c * c;
+    double *ws = (double *)ptt_hip_scratch(
+        PTT_WS_SKETCH, sizeof(double) * (2 * cc + 128 * (size_t)c + 4 * (size_t)c + 4 * nblk) +
+                           sizeof(int) * (size_t)nblk);
+    double *S = ws, *Tw = S + cc, *X = Tw + cc, *D = X + 128 * (size_t)c, *iD = D + c, *y = iD + c,
+           *z = y + c;
+    double *bd = z + c;
+    int *bi = (int *)(bd + 4 * nblk);
+    double *Ti = T ? T : Tw;  // the diagonal blocks' inverses are needed either way
+    if (T && nblk > 2) ptt_hip_zero(T, sizeof(double) * cc);  // its lower blocks are operands
+    PTT_LAUNCH("chol_scale", k_chol_scale, dim3(stream_blocks((long)cc, 256)), dim3(256), 0, c, G,
+               shift, D, iD, S);
+    const size_t bneed = (size_t)CB_LDS_DOUBLES * sizeof(double);
+    for (int b = 0; b < nblk; b++) {
+        const int b0 = 128 * b, cb = c - b0 < 128 ? c - b0 : 128, rest = c - b0 - cb;
+        const size_t dg = (size_t)b0 + (size_t)b0 * c;
+        PTT_LAUNCH_FB("chol_qr_factor", 2.0 * cb * (double)cb * cb / 3.0, 24.0 * cb * (double)cb,
+                      k_chol_blk<true>, dim3(1), dim3(512), bneed, cb, S + dg, (long)c, 0.0, tiny,
+                      R + dg, Ti + dg, (long)c, bi + b, bd + 4 * b, 0, 1);
+        if (rest > 0) {
+            const size_t right = dg + (size_t)cb * c, trail = right + cb;
+            ptt_hip_dgemm('T', 'N', cb, rest, cb, 1.0, Ti + dg, c, S + right, c, 0.0, R + right, c);
+            ptt_hip_dgemm('T', 'N', rest, rest, cb, -1.0, R + right, c, R + right, c, 1.0,
+                          S + trail, c);
+        }
+        if (T && b > 0) {
+            // T[0:b0, b] = -T[0:b0, 0:b0] R[0:b0, b] T_bb
+            const size_t up = (size_t)b0 * c;
+            ptt_hip_dgemm('N', 'N', b0, cb, cb, -1.0, R + up, c, Ti + dg, c, 0.0, X, b0);
+            ptt_hip_dgemm('N', 'N', b0, cb, b0, 1.0, T, c, X, b0, 0.0, T + up, c);
+        }
     }
+    PTT_LAUNCH("chol_unscale", k_chol_unscale, dim3(stream_blocks((long)cc, 256)), dim3(256), 0, c,
+               D, R, T);
+    PTT_LAUNCH("chol_report", k_chol_report, dim3(1), dim3(NT), 0, c, G, D, iD, R, T, nblk, bi, y, z,
+               info, dinfo, want_kappa);
 }
 
 void ptt_hip_svd_jacobi(int m, int k, double *A, long lda, double *sig, double *U, long ldu,
