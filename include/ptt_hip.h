@@ -68,7 +68,7 @@ void ptt_hip_side_join(void);
  * is valid until the next call for the same slot with a larger size. */
 enum { PTT_WS_GRAM = 0, PTT_WS_SMALL, PTT_WS_TMP, PTT_WS_TMP2, PTT_WS_INT,
        PTT_WS_COEF, PTT_WS_SKETCH, PTT_WS_SMALL2, PTT_WS_RSK, PTT_WS_SIDE, PTT_WS_EIG,
-       PTT_WS_RES, PTT_WS_RSIDE, PTT_WS_ROUT0, PTT_WS_ROUT1, PTT_WS_NSLOTS };
+       PTT_WS_RES, PTT_WS_RSIDE, PTT_WS_ROUT0, PTT_WS_ROUT1, PTT_WS_TREE, PTT_WS_NSLOTS };
 void *ptt_hip_scratch(int slot, size_t bytes);
 /* Exchange the buffer of the TMP slot with a caller buffer: on return *buf
  * points at the old scratch (capacity *cap_bytes updated) and the slot owns
@@ -235,6 +235,49 @@ int ptt_hip_syev_gram_noalloc(int c, const double *G, double *sig, double *U, lo
  * = U[:, colidx] diag(sig). */
 void ptt_hip_svd_factors_perm(int m, int rho, const int *colidx, const double *U, long ldu,
                               const double *sig, double wscale, double *W, double *US);
+/* ---- low-rank bonds: Householder trees (c <= 32 columns) ----------------------
+ * The rows are cut into blocks, factored one workgroup each (level 0), their
+ * c x c factors stacked and factored in turn up to a single block (the root).
+ * F (pl->fsize doubles) and S (pl->ssize) belong to one factorisation and are
+ * read by its applications. */
+enum { PTT_TSQR_LEVELS = 6 };
+typedef struct {
+    int c, levels;
+    long rows, fsize, ssize;
+    int nblk[PTT_TSQR_LEVELS], brows[PTT_TSQR_LEVELS];
+    long lrows[PTT_TSQR_LEVELS], foff[PTT_TSQR_LEVELS], soff[PTT_TSQR_LEVELS];
+} ptt_tsqr_plan;
+/* Returns 0, or -1 when the tree would be too deep. */
+int ptt_hip_tsqr_plan(int c, long rows, ptt_tsqr_plan *pl);
+/* A (element (row, col) at row * rs + col * cs) = Q R: the reflectors overwrite
+ * A.  drho (may be NULL): the matrix has rows_per_rank * *drho rows, at most
+ * pl->rows.  R (c x c, ld c) receives the factor, divided by 2^e where its
+ * magnitude would leave FP64's safe range, e added to the device int *escale;
+ * R NULL leaves the root to ptt_hip_tsqr_svd. */
+void ptt_hip_tsqr_factor(const ptt_tsqr_plan *pl, double *A, long rs, long cs, const int *drho,
+                         long rows_per_rank, double *F, double *S, double *R, int *escale);
+/* The root of M^T = Q R (A = M, rs = c, cs = 1) and the SVD of L = R^T:
+ * singular values (32, device), info = {numerical rank, rank kept by the tail
+ * rule against delta and cap, sweeps, columns factored}, *rho = the rank kept,
+ * X = the right singular vectors of L (c x rho, ld 32), US = U Sigma (row i at
+ * i * 32), and the root's rows of Q X in W (2 * lrows[1] * 32 doubles).  A tree
+ * of one level writes alpha (Q X)^T to Y (rho x rows) instead. */
+void ptt_hip_tsqr_svd(const ptt_tsqr_plan *pl, double *A, long rs, long cs, const int *drho,
+                      long rows_per_rank, double *F, double *S, double delta, int cap,
+                      double *sig, int *info, int *rho, double *X, double *US, double *W,
+                      double *Y, double alpha);
+/* The rest of both applications of a right-to-left bond in as few launches as
+ * their trees allow: Y0 (rho x rows) = alpha0 (Q0 X)^T below the root of pl0
+ * (after ptt_hip_tsqr_svd; nothing for one level), and Y1 (rows x *p1,
+ * column-major) = alpha1 Q1 US1 for the left-to-right tree pl1 (A1 column-major;
+ * pl1 may be NULL; F1 NULL: A1 is an explicit Q and Y1 = alpha1 A1 US1).  W0,
+ * W1: as W above, per tree. */
+void ptt_hip_tsqr_finish(const ptt_tsqr_plan *pl0, const double *A0, const int *drho0,
+                         long rows_per_rank0, const double *F0, const double *S0,
+                         const int *rho0, double *W0, double *Y0, double alpha0,
+                         const ptt_tsqr_plan *pl1, const double *A1, const double *F1,
+                         const double *S1, const double *US1, const int *p1, double *W1,
+                         double *Y1, double alpha1);
 /* ---- rank-predictor network (FP32, 18 -> 64 -> 64 -> 64 -> 1, tanh-GELU) ----
  * X: nsamp x 18 row-major, Y: nsamp targets, P: ptt_hip_mlp_nparam() floats. */
 int ptt_hip_mlp_nparam(void);

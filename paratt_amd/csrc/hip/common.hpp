@@ -54,6 +54,27 @@ inline unsigned stream_blocks(long n, int threads) {
     return (unsigned)(b < 1 ? 1 : (b > cap ? cap : b));
 }
 
+// 1/x (x normal) and sqrt(x) (x > 0, normal) from the hardware approximations
+// and Newton steps: to about an ulp, in a third of the library calls' latency.
+__device__ __forceinline__ double rcp_nr(double x) {
+    double r = __builtin_amdgcn_rcp(x);
+    double e = fma(-x, r, 1.0);
+    r = fma(r, e, r);
+    e = fma(-x, r, 1.0);
+    return fma(r, e, r);
+}
+__device__ __forceinline__ double sqrt_nr(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    double e = fma(-h, g, 0.5);
+    g = fma(g, e, g);
+    h = fma(h, e, h);
+    e = fma(-g, g, x);
+    g = fma(e, h, g);
+    e = fma(-g, g, x);
+    return fma(e, h, g);
+}
+
 // ---- sums across the lanes of a wave
 // DPP move of a double inside a quad / row (dpp_ctrl CTRL); every source lane
 // used below is a valid lane of the same row.
@@ -77,6 +98,15 @@ __device__ __forceinline__ double xor16_sum(double x) {
     const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
     const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
     return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
+}
+// x of lane ^ 16
+__device__ __forceinline__ double xor16_other(double x) {
+    const int lo = __double2loint(x), hi = __double2hiint(x);
+    const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+    // one of the pair is x itself
+    const bool odd = (threadIdx.x & 16) != 0;
+    return __hiloint2double(odd ? h[0] : h[1], odd ? l[0] : l[1]);
 }
 __device__ __forceinline__ double xor32_sum(double x) {
     const int lo = __double2loint(x), hi = __double2hiint(x);

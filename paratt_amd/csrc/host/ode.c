@@ -142,6 +142,7 @@ static void round_rel_cap_role(paratt *x, double eps, int cap, int role) {
     int d = x->numDim;
     int *mr = (int *)ptt_host_malloc(sizeof(int) * (d + 1));
     for (int k = 0; k <= d; k++) mr[k] = (k == 0 || k == d) ? 1 : cap;
+    ptt_host_whole_spectra(g_learn.mode != 0 || g_learn.log_on);
     const int have = (role >= 0 && g_hist[role].valid && g_hist[role].d == d && d <= 64);
     float *feat = NULL;
     if (have && (g_learn.mode == 1 || g_learn.log_on)) {
@@ -184,6 +185,7 @@ static void round_rel_cap_role(paratt *x, double eps, int cap, int role) {
     } else {
         paratt_amd_truncate_rel(x, eps, mr);
     }
+    ptt_host_whole_spectra(0);
     if (role >= 0) {
         double spec[64 * LN_SPEC];
         paratt_amd_last_round_spectra(spec);

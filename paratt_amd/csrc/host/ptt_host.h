@@ -9,6 +9,10 @@
  * borrowed view (coreMem == NULL) the result is copied back instead, so the
  * caller's pointers never change (`count` doubles of result). */
 void ptt_host_swap_core_with_tmp(attac_tt *x, int k, long count);
+void ptt_host_swap_core_with_slot(attac_tt *x, int k, long count, int slot); /* another slot */
+/* Roundings keep every bond's whole spectrum, also below the resolution of
+ * FP64 (the rank predictor's features and training data): on = 1. */
+void ptt_host_whole_spectra(int on);
 /* Set the diagonal of an m x m device matrix to alpha. */
 void ptt_host_set_diag(double *A, int m, double alpha);
 /* Wrap raw (d, n, r, cores) arrays of the pattac* API as a borrowed TT. */

@@ -281,6 +281,11 @@ static double last_core_sumsq(attac_tt *x) {
     return ss;
 }
 
+/* Set while a left-to-right sweep may hand over to the Householder trees: a
+ * core that one Cholesky-QR pass does not orthogonalise is left as it is and
+ * the factorisation returns -1. */
+static int g_one_pass_only = 0;
+
 /* Cholesky-QR of a core viewed as len x c (trans 'T': columns, LTR) or as
  * c x len (trans 'N': rows, RTL).  On return the core holds Q (alpha
  * applied) and R (c x c upper, A = Q*R resp. M = R^T*Q) is in *Rout.
@@ -326,6 +331,7 @@ static int cholqr_core_g(attac_tt *x, int core, double *buf, char trans, long le
         /* the carried core of the left-to-right sweep, brought into range */
         if (t > 0 || buf || trans != 'T' || !rescale_if_extreme(A, len * c, o.maxdiag)) break;
     }
+    if (g_one_pass_only && !(o.deficient == 0 && o.kappa <= KAPPA_ONE_PASS)) return -1;
     if (!buf && trans == 'T' && core < 64) g_stats.kappa_ltr[core] = o.kappa;
     if (!buf && trans == 'N' && core < 64) g_stats.kappa_rtl[core] = o.kappa;
     if (one_pass) *one_pass = 0;
@@ -407,8 +413,11 @@ static void set_identity(double *dst, int m, double alpha) {
 }
 
 /* Left-to-right sweep over cores 0..d-2.  qscale[k]: alpha of core k's Q;
- * rscale[k]: alpha applied when R_k multiplies core k+1. */
-static void ltr_sweep(attac_tt *x, const double *qscale, const double *rscale) {
+ * rscale[k]: alpha applied when R_k multiplies core k+1.  With hand_over the
+ * sweep stops before the first core after core 0 that needs more than one
+ * Cholesky-QR pass.  Returns the cores left orthogonal (d - 1 if all). */
+static int ltr_sweep_until(attac_tt *x, const double *qscale, const double *rscale,
+                           int hand_over) {
     int d = x->numDim;
     int *r = x->ttRank, *n = x->dim;
     for (int i = 0; i < d - 1; i++) {
@@ -429,7 +438,14 @@ static void ltr_sweep(attac_tt *x, const double *qscale, const double *rscale) {
         }
         step_ws w = get_ws(c);
         const double *R = NULL;
+        g_one_pass_only = hand_over && i > 0;
         int passes = cholqr_core(x, i, NULL, 'T', m, c, qscale[i], &w, &R, 0, NULL, NULL);
+        g_one_pass_only = 0;
+        if (passes < 0) {
+            side_flush();
+            ptt_hip_side_join();
+            return i;
+        }
         if (i < 64) g_stats.ltr_cholqr_passes[i] = passes;
         /* core i+1 (c x wcols) <- rscale * R * core i+1 */
         if (c <= 128) {
@@ -444,6 +460,11 @@ static void ltr_sweep(attac_tt *x, const double *qscale, const double *rscale) {
     }
     side_flush();
     ptt_hip_side_join(); /* every Q formed on the side stream is in place */
+    return d - 1;
+}
+
+static void ltr_sweep(attac_tt *x, const double *qscale, const double *rscale) {
+    (void)ltr_sweep_until(x, qscale, rscale, 0);
 }
 
 /* Reference tail rule (pattac.c:468-481) on a descending list: the loop
@@ -959,6 +980,156 @@ static void fill_scales(const attac_tt *x, double *inv, double *sq) {
     }
 }
 
+/* ---- low-rank trains ---------------------------------------------------------
+ * Trains whose bond ranks are all at most TREE_RANK are rounded by Householder
+ * trees (tsqr.hip) with every rank decided and kept on the device: a fixed
+ * sequence of launches, one host read between the sweeps (the norm sets the
+ * tolerance) and one at the end (ranks and singular values).  The left-to-right
+ * sweep keeps each core's reflectors in place instead of forming Q; the
+ * right-to-left sweep applies them to U Sigma of the bond before.  Accuracy is
+ * that of an orthogonal factorisation at every bond, as on the LQ route.
+ * The lines: above 32 columns a block of 512 rows no longer fits a workgroup's
+ * registers.  From 17 to 32 the trees (255 us a bond at 22 columns, n = 83; 350
+ * at 32, n = 32) lose to the Gram route on well-conditioned trains (211, 266
+ * us), which take one Cholesky-QR pass and no Jacobi sweeps, and win on
+ * ill-conditioned ones (some 600 us a bond there: three to four passes a
+ * factorisation): such a train starts on the Cholesky-QR sweep and changes over
+ * at the first core after core 0 that one pass does not orthogonalise. */
+#define TREE_RANK_ALWAYS 16
+#define TREE_RANK 32
+#define TREE_ROWS 65536
+static int g_whole_spectra = 0;
+void ptt_host_whole_spectra(int on) { g_whole_spectra = on; }
+
+/* 0: not by trees; 1: by trees; 2: by trees once a core is ill-conditioned. */
+static int tree_route(const attac_tt *x) {
+    const int d = x->numDim;
+    int route = 1;
+    if (d < 2 || g_leaf32 || g_pred || g_whole_spectra) return 0;
+    for (int k = 0; k < d; k++) {
+        const int r0 = x->ttRank[k], r1 = x->ttRank[k + 1];
+        if (r0 < 1 || r1 < 1 || (k > 0 && r0 > TREE_RANK)) return 0;
+        if (k > 0 && r0 > TREE_RANK_ALWAYS) route = 2;
+        if ((long)r0 * x->dim[k] > TREE_ROWS || (long)r1 * x->dim[k] > TREE_ROWS) return 0;
+    }
+    return route;
+}
+
+typedef struct {
+    double sig[32];
+    int info[4];
+} bond_record;
+
+/* from: the first core to factor; the cores before it are orthogonal, and the
+ * train holds 2^-g_escale times the input. */
+static double tree_round(attac_tt *x, const int *maxr, double tol, int tol_is_rel,
+                         const double *rscale, const double *nscale, int from) {
+    const int escale = g_escale;
+    const int d = x->numDim;
+    int *r = x->ttRank;
+    const int *n = x->dim;
+    ptt_tsqr_plan *pl = (ptt_tsqr_plan *)ptt_host_malloc(sizeof(ptt_tsqr_plan) * 2 * (size_t)d);
+    ptt_tsqr_plan *pr = pl + d; /* right-to-left trees, by core */
+    int *kept = (int *)ptt_host_malloc(sizeof(int) * (size_t)(d + 1)); /* largest rank left */
+    for (int k = 0; k <= d; k++) kept[k] = (k > 0 && k < d && maxr[k] < r[k]) ? maxr[k] : r[k];
+    for (int k = 0; k <= d; k++)
+        if (kept[k] < 1) kept[k] = 1;
+    /* one arena: the left-to-right trees' F and S per core, one right-to-left
+     * tree's, two hand-down buffers each, the small matrices, the records */
+    size_t fs = 0, rf = 0, rs = 0, w0 = 0, w1 = 0;
+    size_t *off = (size_t *)ptt_host_malloc(sizeof(size_t) * 2 * (size_t)d);
+    for (int i = 0; i < d; i++) {
+        if (i < d - 1) {
+            (void)ptt_hip_tsqr_plan(r[i + 1], (long)r[i] * n[i], &pl[i]);
+            off[2 * i] = fs;
+            off[2 * i + 1] = fs + (size_t)pl[i].fsize;
+            if (i >= from) { /* before it: explicit Qs, level 0's blocks only */
+                fs += (size_t)pl[i].fsize + (size_t)pl[i].ssize;
+                if (pl[i].levels > 1 && (size_t)pl[i].lrows[1] > w1) w1 = (size_t)pl[i].lrows[1];
+            }
+        }
+        if (i > 0) {
+            (void)ptt_hip_tsqr_plan(r[i], (long)n[i] * kept[i + 1], &pr[i]);
+            if ((size_t)pr[i].fsize > rf) rf = (size_t)pr[i].fsize;
+            if ((size_t)pr[i].ssize > rs) rs = (size_t)pr[i].ssize;
+            if (pr[i].levels > 1 && (size_t)pr[i].lrows[1] > w0) w0 = (size_t)pr[i].lrows[1];
+        }
+    }
+    const size_t rec = sizeof(bond_record) / sizeof(double);
+    double *ws = (double *)ptt_hip_scratch(
+        PTT_WS_TREE, sizeof(double) * (fs + rf + rs + 64 * (w0 + w1) + 3 * 1024 +
+                                       (rec + 1) * (size_t)d));
+    double *F0 = ws + fs, *S0 = F0 + rf, *W0 = S0 + rs, *W1 = W0 + 64 * w0;
+    double *R = W1 + 64 * w1, *X = R + 1024, *US = X + 1024, *records = US + 1024;
+    int *rho = (int *)(records + rec * (size_t)d); /* device ranks, by bond */
+    /* norm and exponent come back in one read */
+    double *dss = (double *)ptt_hip_scratch(PTT_WS_INT, sizeof(int) * 64) + 24;
+    ptt_hip_zero(dss, 2 * sizeof(double));
+    for (int i = from; i < d - 1; i++) {
+        const int c = r[i + 1];
+        const long m = (long)r[i] * n[i], wcols = (long)n[i + 1] * r[i + 2];
+        ptt_hip_tsqr_factor(&pl[i], x->coreList[i], 1, m, NULL, 0, ws + off[2 * i],
+                            ws + off[2 * i + 1], R, (int *)(dss + 1));
+        ptt_hip_dgemm('N', 'N', c, (int)wcols, c, rscale[i], R, c, x->coreList[i + 1], c, 0.0,
+                      x->coreList[i + 1], c);
+        if (i < 64) g_stats.ltr_cholqr_passes[i] = 0;
+    }
+    const int rl = r[d - 1];
+    ptt_hip_sumsq(rl, n[d - 1] * r[d], x->coreList[d - 1], rl, dss);
+    double back[2];
+    ptt_hip_d2h(back, dss, sizeof back);
+    double ss = back[0];
+    memcpy(&g_escale, &back[1], sizeof(int));
+    g_escale += escale;
+    if (!(ss >= MAG_LO && ss <= MAG_HI)) ss = last_core_sumsq(x);
+    const double nrm_s = sqrt(ss);
+    const double abs_tol = tol_is_rel ? tol * nrm_s : ldexp(tol, -g_escale);
+    const double delta = abs_tol / sqrt(d - 1.0);
+    for (int i = d - 1; i > 0; i--) {
+        const int c = r[i];
+        const long wmax = (long)n[i] * kept[i + 1], m1 = (long)r[i - 1] * n[i - 1];
+        const int *drho = (i == d - 1) ? NULL : rho + i + 1;
+        double *sig = records + rec * (size_t)i;
+        double *M = x->coreList[i], *A1 = x->coreList[i - 1];
+        double *Y0 = (double *)ptt_hip_scratch(PTT_WS_TMP, sizeof(double) * (size_t)kept[i] * wmax);
+        double *Y1 = (double *)ptt_hip_scratch(PTT_WS_TMP2, sizeof(double) * (size_t)m1 * kept[i]);
+        ptt_hip_tsqr_factor(&pr[i], M, c, 1, drho, n[i], F0, S0, NULL, NULL);
+        ptt_hip_tsqr_svd(&pr[i], M, c, 1, drho, n[i], F0, S0, delta, maxr[i], sig,
+                         (int *)(sig + 32), rho + i, X, US, W0, Y0, nscale[i]);
+        ptt_hip_tsqr_finish(&pr[i], M, drho, n[i], F0, S0, rho + i, W0, Y0, nscale[i], &pl[i - 1],
+                            A1, i - 1 < from ? NULL : ws + off[2 * (i - 1)],
+                            ws + off[2 * (i - 1) + 1], US, rho + i, W1, Y1, i == 1 ? nscale[0] : 1.0);
+        ptt_host_swap_core_with_slot(x, i, (long)kept[i] * wmax, PTT_WS_TMP);
+        ptt_host_swap_core_with_slot(x, i - 1, m1 * kept[i], PTT_WS_TMP2);
+    }
+    bond_record *h = (bond_record *)ptt_host_malloc(sizeof(bond_record) * (size_t)d);
+    ptt_hip_d2h(h + 1, records + rec, sizeof(bond_record) * (size_t)(d - 1));
+    for (int i = 1; i < d; i++) {
+        const int k = h[i].info[1];
+        if (i < 64) {
+            const double *sv = h[i].sig;
+            g_stats.numrank[i] = h[i].info[0];
+            g_stats.svd_sweeps[i] = h[i].info[2];
+            g_stats.rtl_cholqr_passes[i] = 0;
+            g_stats.kappa_rtl[i] = sv[k - 1] > 0.0 ? sv[0] / sv[k - 1] : 0.0;
+            for (int q = 0; q < 4; q++) {
+                const int j = k - 1 + q;
+                g_stats.sig[i][q] = j < 32 ? sv[j] : 0.0;
+            }
+            for (int q = 0; q < 16; q++) {
+                const int j = k - 13 + q;
+                g_spec[i][q] = (j >= 0 && j < 32) ? sv[j] : 0.0;
+            }
+            g_spec[i][16] = sv[0];
+            g_spec[i][17] = k;
+            g_spec[i][18] = r[i];
+        }
+        r[i] = k;
+    }
+    free(h); free(off); free(kept); free(pl);
+    return nrm_s;
+}
+
 /* Shared driver: returns ||x||_n from the sweep (last core's Frobenius norm
  * in the scaled space). */
 static double round_impl_g(attac_tt *x, const int *maxRank, double tol, int tol_is_rel,
@@ -985,13 +1156,19 @@ static double round_impl_g(attac_tt *x, const int *maxRank, double tol, int tol_
     double nrm = 0.0;
     if (d >= 2) {
         g_escale = 0;
-        ltr_sweep(x, qs, rs);
-        /* norm in the scaled space: last core after the sweep (the train
-         * holds 2^-g_escale times the input from here to the end) */
-        const double ss = last_core_sumsq(x);
-        const double nrm_s = sqrt(ss);
-        const double abs_tol = tol_is_rel ? tol * nrm_s : ldexp(tol, -g_escale);
-        rtl_sweep(x, mr, abs_tol, sq);
+        double nrm_s;
+        const int route = tree_route(x);
+        const int done = route == 1 ? 0 : ltr_sweep_until(x, qs, rs, route == 2);
+        if (route == 1 || done < d - 1) {
+            nrm_s = tree_round(x, mr, tol, tol_is_rel, rs, sq, done);
+        } else {
+            /* norm in the scaled space: last core after the sweep (the train
+             * holds 2^-g_escale times the input from here to the end) */
+            const double ss = last_core_sumsq(x);
+            nrm_s = sqrt(ss);
+            const double abs_tol = tol_is_rel ? tol * nrm_s : ldexp(tol, -g_escale);
+            rtl_sweep(x, mr, abs_tol, sq);
+        }
         if (g_escale != 0) {
             /* core 0 carries the train's magnitude after the sweep */
             ptt_hip_scale(x->coreList[0], (long)x->ttRank[0] * x->dim[0] * x->ttRank[1],
@@ -1030,9 +1207,27 @@ void paratt_amd_truncate_rel(paratt *x_ptt, double eps_rel, int *maxRank) {
 
 void paratt_amd_truncate_rel_sketch(paratt *x_ptt, double eps_rel, int *maxRank,
                                     const int *pred_rank) {
+    /* refused predictions leave the plain rounding's result: a train that it
+     * takes through the trees is kept until one step has been accepted */
+    attac_tt *x = x_ptt->x, *keep = NULL;
+    const int d = x->numDim;
+    int *mr = (int *)ptt_host_malloc(sizeof(int) * (size_t)(d + 1));
+    memcpy(mr, maxRank, sizeof(int) * (size_t)(d + 1));
+    if (tree_route(x)) {
+        keep = alloc_tt(d, x->dim, x->ttRank);
+        copy_rank_change_tt(keep, x);
+    }
     g_pred = pred_rank;
-    round_impl(x_ptt->x, maxRank, eps_rel, 1);
+    round_impl(x, mr, eps_rel, 1);
     g_pred = NULL;
+    if (keep && g_sketch_counts[1] == 0) {
+        const int tried = g_sketch_counts[0];
+        copy_rank_change_tt(x, keep);
+        round_impl(x, mr, eps_rel, 1);
+        g_sketch_counts[0] = tried;
+    }
+    if (keep) free_tt(keep);
+    free(mr);
 }
 
 void pattacTruncate(MPI_Comm comm, const int d, int *distrib_dim_mat, int *rx, double **x,

@@ -140,18 +140,22 @@ void ptt_host_reserve_train(attac_tt *x, const long *count) {
         }
 }
 
-void ptt_host_swap_core_with_tmp(attac_tt *x, int k, long count) {
+void ptt_host_swap_core_with_slot(attac_tt *x, int k, long count, int slot) {
     if (x->coreMem == NULL) {
         /* borrowed view: copy the result back into the caller's buffer
          * (rounding never outgrows the input core) */
-        double *tmp = (double *)ptt_hip_scratch(PTT_WS_TMP, 8);
+        double *tmp = (double *)ptt_hip_scratch(slot, 8);
         ptt_hip_d2d(x->coreList[k], tmp, sizeof(double) * (size_t)count);
         return;
     }
     size_t cap = (size_t)x->coreMem[k] * sizeof(double);
-    ptt_hip_swap_tmp(PTT_WS_TMP, &x->coreList[k], &cap);
+    ptt_hip_swap_tmp(slot, &x->coreList[k], &cap);
     size_t el = cap / sizeof(double);
     x->coreMem[k] = (int)(el > 2147483647UL ? 2147483647UL : el);
+}
+
+void ptt_host_swap_core_with_tmp(attac_tt *x, int k, long count) {
+    ptt_host_swap_core_with_slot(x, k, count, PTT_WS_TMP);
 }
 
 void ptt_host_set_diag(double *A, int m, double alpha) { ptt_hip_set_diag(A, m, m, alpha); }
