@@ -199,6 +199,13 @@ void ptt_hip_chol_qr_factor(int c, const double *G, double shift, double tiny,
 void ptt_hip_svd_jacobi(int m, int k, double *A, long lda, double *sig,
                         double *U, long ldu, double *V, long ldv,
                         double log_scale, double delta, int cap, int *iout);
+/* Singular values (k, descending) and right singular vectors (V, k x k, ldv;
+ * columns of zero singular values are zero) of L = R^T, R upper triangular k x k
+ * (ldr), k <= 128; X: k x k scratch.  Content below u times the largest column
+ * is dropped.  iout = {numerical rank, tail-rule rank (against delta and cap),
+ * sweeps} as in ptt_hip_svd_jacobi; iout needs 5 ints. */
+void ptt_hip_svd_right(int k, const double *R, long ldr, double *X, double *sig, double *V,
+                       long ldv, double delta, int cap, int *iout);
 /* From U (m x k, ldu) and sig: W (rho x m, ld rho) = diag(1/sig) U_rho^T
  * scaled by wscale, and US (m x rho, ld m) = U_rho diag(sig).
  * rho is read from device *drho, or is rhomax when drho is NULL.  Either

@@ -61,6 +61,10 @@ static double g_spec[64][SPEC_W];
 
 void paratt_amd_last_round_spectra(double *out) { memcpy(out, g_spec, sizeof g_spec); }
 
+/* Every bond's whole spectrum is wanted (ptt_host_whole_spectra). */
+static int g_whole_spectra = 0;
+void ptt_host_whole_spectra(int on) { g_whole_spectra = on; }
+
 /* The leading singular values of the current bond as the step brought them
  * to the host for its decisions (g_hsig_n = 0: not brought), reused by the
  * statistics and the spectrum record instead of another round trip. */
@@ -482,7 +486,9 @@ static int tail_rule(const double *sig, int nsig, double tail0, double delta) {
 }
 
 /* Robust right-to-left step: explicit LQ by (shifted) Cholesky-QR, SVD of
- * L with right vectors, new core = V_rho^T Q.  The rows of M are first put
+ * L, new core = V_rho^T Q.  Up to 128 rows the SVD pivots L's columns itself and
+ * gives the right vectors alone: U Sigma = L V.  Beyond (and where the whole
+ * spectrum is wanted, noise included) the rows of M are first put
  * in order of decreasing norm (the Gram's diagonal), so that the columns of
  * L come by decreasing norm: Drmac and Veselic's diagonal pivoting (SIAM J.
  * Matrix Anal. Appl. 29, 2008), applied statically as on the Gram route,
@@ -496,7 +502,8 @@ static int rtl_step_robust(attac_tt *x, int i, const int *maxr, double delta,
     long w = (long)n[i] * r[i + 1];
     const double *R = NULL, *T1 = NULL;
     int one_pass = 0;
-    const int sorted = rows >= 8 && rows <= 1024;
+    const int right = rows <= 128 && !g_whole_spectra;
+    const int sorted = !right && rows >= 8 && rows <= 1024;
     int *perm = (int *)ws->W; /* W is free on this route */
     if (sorted) {
         double *M = x->coreList[i];
@@ -508,9 +515,14 @@ static int rtl_step_robust(attac_tt *x, int i, const int *maxr, double delta,
     }
     int passes = cholqr_core_g(x, i, NULL, 'N', w, rows, 1.0, ws, &R, 0, &one_pass, &T1, sorted);
     *passes_out = passes;
-    ptt_hip_transpose(rows, rows, R, rows, ws->L, rows, 1.0);
-    ptt_hip_svd_jacobi(rows, rows, ws->L, rows, ws->sig, ws->U, rows, ws->V, rows, 0.0, delta,
-                       maxr[i], ws->iinfo + 1);
+    if (right) {
+        ptt_hip_svd_right(rows, R, rows, ws->U, ws->sig, ws->V, rows, delta, maxr[i],
+                          ws->iinfo + 1);
+    } else {
+        ptt_hip_transpose(rows, rows, R, rows, ws->L, rows, 1.0);
+        ptt_hip_svd_jacobi(rows, rows, ws->L, rows, ws->sig, ws->U, rows, ws->V, rows, 0.0, delta,
+                           maxr[i], ws->iinfo + 1);
+    }
     /* sigma, factor info and SVD info are contiguous: one transfer */
     const size_t nb = sizeof(double) * ((size_t)rows + 8) + sizeof(int) * 8;
     double *hb = (double *)ptt_host_malloc(nb);
@@ -522,12 +534,12 @@ static int rtl_step_robust(attac_tt *x, int i, const int *maxr, double delta,
     int rho = io[1];
     if (i < 64) { g_stats.svd_sweeps[i] = io[2]; g_stats.numrank[i] = io[0]; }
     double *tmp = (double *)ptt_hip_scratch(PTT_WS_TMP, sizeof(double) * (size_t)rho * w);
-    if (sorted) {
-        ptt_hip_svd_factors(rows, rho, ws->iinfo + 2, ws->U, rows, ws->sig, 1.0, NULL, ws->L);
-        ptt_hip_unpermute_rows(rows, rho, perm, ws->L, rows, ws->US, rows);
-    } else {
-        ptt_hip_svd_factors(rows, rho, ws->iinfo + 2, ws->U, rows, ws->sig, 1.0, NULL, ws->US);
-    }
+    double *us = sorted ? ws->L : ws->US;
+    if (right)
+        ptt_hip_dgemm('T', 'N', rows, rho, rows, 1.0, R, rows, ws->V, rows, 0.0, us, rows);
+    else
+        ptt_hip_svd_factors(rows, rho, ws->iinfo + 2, ws->U, rows, ws->sig, 1.0, NULL, us);
+    if (sorted) ptt_hip_unpermute_rows(rows, rho, perm, us, rows, ws->US, rows);
     ptt_hip_dgemm('T', 'N', rho, (int)w, rows, nscale[i], ws->V, rows, x->coreList[i], rows, 0.0,
                   tmp, rho);
     ptt_host_swap_core_with_tmp(x, i, (long)rho * w);
@@ -998,9 +1010,6 @@ static void fill_scales(const attac_tt *x, double *inv, double *sq) {
 #define TREE_RANK_ALWAYS 16
 #define TREE_RANK 32
 #define TREE_ROWS 65536
-static int g_whole_spectra = 0;
-void ptt_host_whole_spectra(int on) { g_whole_spectra = on; }
-
 /* 0: not by trees; 1: by trees; 2: by trees once a core is ill-conditioned. */
 static int tree_route(const attac_tt *x) {
     const int d = x->numDim;
