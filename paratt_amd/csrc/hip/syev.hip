@@ -9,9 +9,9 @@
 //   1. k_sytrd: Householder tridiagonalisation G = Q T Q^T, one workgroup,
 //      G held in registers (two lanes per row), one reflector per step with
 //      two workgroup barriers;
-//   2. k_stedc: Cuppen's divide and conquer on T (split into 1 x 1 blocks,
-//      merged bottom-up by rank-one updates), with the deflation rules of
-//      Dongarra and Sorensen, the secular-equation iteration of Li's "middle
+//   2. k_dc_leaf, k_dc_roots, k_dc_vecs, k_dc_top: Cuppen's divide and conquer
+//      on T (split into 2 x 2 blocks, merged bottom-up by rank-one updates), over
+//      several workgroups, with the deflation rules of Dongarra and Sorensen, the secular-equation iteration of Li's "middle
 //      way" (SIAM J. Sci. Comput. 1994, as in LAPACK's dlaed4) from the
 //      nearer pole, and the eigenvectors of Gu and Eisenstat (SIAM J. Matrix
 //      Anal. Appl. 16, 1995): z is recomputed from the computed roots, which
@@ -54,12 +54,14 @@ __device__ __forceinline__ double oct_prod(double x) {
     x *= dppd<0x141>(x);
     return x;
 }
-// Sum / product over aligned groups of L = 1, 2, 4 or 8 lanes.
+// Sum over aligned groups of L = 2, 4, ..., 32 lanes, product of 2, 4 or 8.
 template <int L>
 __device__ __forceinline__ double grp_sum(double x) {
     if constexpr (L == 2) x += dppd<0xB1>(x);
     if constexpr (L == 4) x = quad_sum(x);
-    if constexpr (L == 8) x = oct_sum(x);
+    if constexpr (L >= 8) x = oct_sum(x);
+    if constexpr (L >= 16) x += dppd<0x140>(x);
+    if constexpr (L == 32) x = xor16_sum(x);
     return x;
 }
 template <int L>
@@ -73,18 +75,9 @@ __device__ __forceinline__ double wave_max(double x) {
     for (int o = 32; o > 0; o >>= 1) x = fmax(x, __shfl_xor(x, o));
     return x;
 }
-// 1/x from the hardware reciprocal and two Newton steps (a few ulp; x != 0).
-__device__ __forceinline__ double rcp_nr(double x) {
-    double r = __builtin_amdgcn_rcp(x);
-    double e = fma(-x, r, 1.0);
-    r = fma(r, e, r);
-    e = fma(-x, r, 1.0);
-    return fma(r, e, r);
-}
-__device__ __forceinline__ double uniform_d(double x) {
-    const int lo = __builtin_amdgcn_readfirstlane(__double2loint(x));
-    const int hi = __builtin_amdgcn_readfirstlane(__double2hiint(x));
-    return __hiloint2double(hi, lo);
+// sqrt(x) for x >= 0 to a few ulp; 0 below 2^-900 (x not far above 1 otherwise).
+__device__ __forceinline__ double sqrt_pos(double x) {
+    return x > 0x1.0p-900 ? sqrt_nr(x) : 0.0;
 }
 
 // Workgroup barrier that orders LDS traffic only: outstanding global stores
@@ -379,18 +372,25 @@ __global__ __launch_bounds__(NMAX * 4 + 64) void k_sytrd(int n, const double *__
 // at m = lo + s/2 with coupling beta = e[m-1]:
 //   T = diag(T1 - |beta| e_last e_last^T, T2 - |beta| e_1 e_1^T) + |beta| v v^T,
 //   v = [e_last; sign(beta) e_1],
-// so the 1 x 1 leaves start from d_i - |e_{i-1}| - |e_i|.  The eigenvectors of
-// the blocks live in the block-diagonal Z (global, n x n, ld n); the
-// eigenvalues in sD.  At a merge z = [last row of Z1; sign * first row of
-// Z2] / sqrt(2) and rho = 2 |beta|.
+// so a leaf's d_i loses the |e| of the couplings that were cut beside it.  The eigenvectors of
+// the blocks live in the block-diagonal Z (n x n, ld n).  At a merge z =
+// [last row of Z1; sign * first row of Z2] / sqrt(2) and rho = 2 |beta|.
+//
+// The merges up to 32 rows run in k_dc_leaf, a workgroup per 32 rows with its Z
+// in LDS; each merge beyond takes two launches, k_dc_roots and k_dc_vecs, a
+// workgroup per 16 columns: what a merge decides once (order, deflation, the
+// vector zhat) every workgroup repeats, the roots and the eigenvectors, where
+// the work is, are divided.  The last merge (`top`) always takes this form.
+// All merges in one workgroup of 1024 threads, with Z in memory, were bound by
+// the FP64 instructions of one CU: 178 us at n = 128, 95 at 59, 62 at 32; this
+// form takes 98, 65 and 44 (with the gaps between its launches).
 //
 // Deflation (one wave per block): entries with rho |z| <= tol are deflated;
 // consecutive remaining entries whose poles are closer than the tolerance
 // allows (|t c s| <= tol for the rotation that zeroes one z) are combined by
-// that rotation.  When no such pair exists -- the common case -- the
-// non-deflated list is formed by ballots; otherwise one lane walks the block
-// in order.  Secular-equation roots: eight lanes per root.  Lower merges stage
-// the block's columns in LDS and form Z[:, nd] * U in registers.
+// that rotation.  The pairs are found by all lanes at once; one lane visits those
+// and, after each rotation, the entry that follows (a walk over every entry, with
+// the same outcome, took 10 us at 128 of them); the lists are formed by ballots.
 //
 // The top merge stops after the rank-one eigenvector matrix and leaves Z
 // as the lower merges left it: column c of Um (n x n, ld n) is the update's
@@ -398,71 +398,361 @@ __global__ __launch_bounds__(NMAX * 4 + 64) void k_sytrd(int n, const double *__
 // its rows in the order of Z's columns, and the top merge's deflating
 // rotations of Z's column pairs are applied to Um's rows instead (last
 // first), so U = (Q Z) Um.  Also written: sigma (descending, scaled back),
-// colidx (descending rank -> U column), numrank, rho, and colmap (U column
-// c's pole: Z column colmap[c]).
-//
-// part 0 runs every merge; part 1 the merges below the top one, then saves
-// the poles and the iteration count in dsave (n + 1 doubles) and exits;
-// part 2 the top merge and the decisions from that state.  Between the two
-// launches Z is final, so the back transformation Q Z can run beside part 2.
-//
-// Threads: NT = 8 NMAX.  Dynamic LDS: NMAX * NMAX doubles (the lower merges'
-// eigenvector matrices in the first half, the staged columns in the second;
-// the top merge's Um).
-template <int NMAX>
-__global__ __launch_bounds__(8 * NMAX) void k_stedc(
-    int n, const double *__restrict__ dd, const double *__restrict__ ee,
-    const int *__restrict__ eexp, double *__restrict__ Z, double *__restrict__ Um,
-    int *__restrict__ colmap, int *__restrict__ colidx, double *__restrict__ sig,
-    int *__restrict__ iout, double *__restrict__ dinfo, double delta, int cap, double budget,
-    int part, double *__restrict__ dsave) {
-    constexpr int NT = 8 * NMAX;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    extern __shared__ __align__(16) double lds[];
-    double *ums = lds;                            // NMAX * NMAX / 2
-    double *zs = lds + (NMAX * NMAX) / 2;         // NMAX * NMAX / 2
-    __shared__ double sD[NMAX], sz[NMAX], sdl[NMAX], szl[NMAX], stau[NMAX], szh[NMAX],
-        sinv[NMAX], rc[NMAX], rs[NMAX], srho[NMAX], slam[NMAX];
-    __shared__ int sperm[NMAX], snd[NMAX], sorg[NMAX], ra[NMAX], rb[NMAX], sKn[NMAX],
-        sNrot[NMAX], sflag[NMAX], spos[NMAX], scm[NMAX];
-    __shared__ int s_iters;
+// colidx (descending rank -> U column) and numrank, rho.  Z is final before the
+// top merge, so the back transformation Q Z runs beside it.
 
-    if (part == 2) {
-        // the state part 1 left: poles, iteration count; Z in place
-        for (int i = tid; i < n; i += NT) sD[i] = dsave[i];
-        if (tid == 0) s_iters = (int)dsave[n];
-    } else {
-        if (tid == 0) s_iters = 0;
-        for (int i = tid; i < n; i += NT) {
-            double di = dd[i];
-            if (i > 0) di -= fabs(ee[i - 1]);
-            if (i + 1 < n) di -= fabs(ee[i]);
-            sD[i] = di;
-        }
-        for (int j = tid / NMAX; j < n; j += NT / NMAX)
-            for (int i = tid % NMAX; i < n; i += NMAX) Z[i + (long)j * n] = (i == j) ? 1.0 : 0.0;
+// Deflation of one block by GL lanes (gl: lane in the group, which starts at
+// lane gbase of the wave); K entries at the sorted positions sperm[0 .. K).  With
+// TWO a lane takes two positions (gl, gl + 64).  Lists snd, sdl, szl and rotations
+// ra, rb, rc, rs; Kn and nrot as lane 0 has them.
+template <bool TWO>
+__device__ __forceinline__ void deflate(int GL, int gl, int gbase, int K, double rho,
+                                        const int *sperm, double *sz, double *sD, int *snd,
+                                        double *sdl, double *szl, int *ra, int *rb, double *rc,
+                                        double *rs, int &Kn_out, int &nrot_out) {
+    const unsigned long long gmask = (GL == 64) ? ~0ULL : (((1ULL << GL) - 1) << gbase);
+    const int q0 = gl, q1 = gl + 64;
+    const int j0 = (q0 < K) ? sperm[q0] : -1;
+    const int j1 = (TWO && q1 < K) ? sperm[q1] : -1;
+    const double z0 = j0 >= 0 ? sz[j0] : 0.0, z1 = j1 >= 0 ? sz[j1] : 0.0;
+    const double d0 = j0 >= 0 ? sD[j0] : 0.0, d1 = j1 >= 0 ? sD[j1] : 0.0;
+    double dmax = fmax(fabs(d0), fabs(d1)), zmax = fmax(fabs(z0), fabs(z1));
+    for (int o = 1; o < GL; o <<= 1) {
+        dmax = fmax(dmax, __shfl_xor(dmax, o, GL));
+        zmax = fmax(zmax, __shfl_xor(zmax, o, GL));
     }
-    __syncthreads();
+    const double tol = 8.0 * EPSU * fmax(dmax, zmax);
+    const bool k0 = j0 >= 0 && !(rho * fabs(z0) <= tol);
+    const bool k1 = j1 >= 0 && !(rho * fabs(z1) <= tol);
+    // kept positions of the group, bit = sorted position
+    const unsigned long long m0 = (__ballot(k0) & gmask) >> gbase;
+    const unsigned long long m1 = (__ballot(k1) & gmask) >> gbase;
+    const unsigned long long below = (gl == 0) ? 0ULL : ((~0ULL) >> (64 - gl));
+    bool close0 = false, close1 = false;
+    if (k0) {
+        const unsigned long long mm = m0 & below;
+        if (mm) {
+            const int jp = sperm[63 - __clzll(mm)];
+            const double zp = sz[jp], t = d0 - sD[jp];
+            close0 = fabs(t * z0 * zp) <= tol * (z0 * z0 + zp * zp);
+        }
+    }
+    if (k1) {
+        const unsigned long long mm = m1 & below;
+        const int p = mm ? 64 + 63 - __clzll(mm) : (m0 ? 63 - __clzll(m0) : -1);
+        if (p >= 0) {
+            const int jp = sperm[p];
+            const double zp = sz[jp], t = d1 - sD[jp];
+            close1 = fabs(t * z1 * zp) <= tol * (z1 * z1 + zp * zp);
+        }
+    }
+    const unsigned long long f0 = (__ballot(close0) & gmask) >> gbase;
+    const unsigned long long f1 = (__ballot(close1) & gmask) >> gbase;
+    unsigned long long r0 = 0, r1 = 0;  // entries rotated away
+    int nrot = 0;
+    if (f0 | f1) {
+        if (gl == 0) {
+            auto next = [](unsigned long long a, unsigned long long b, int q) {
+                const unsigned long long x = q < 63 ? a & (~0ULL << (q + 1)) : 0ULL;
+                if (x) return __ffsll((long long)x) - 1;
+                const unsigned long long y = q < 63 ? b : q < 127 ? b & (~0ULL << (q - 63)) : 0ULL;
+                return y ? 63 + __ffsll((long long)y) : -1;
+            };
+            auto before = [](unsigned long long a, unsigned long long b, int q) {
+                const unsigned long long y = q > 64 ? b & (~0ULL >> (128 - q)) : 0ULL;
+                if (y) return 127 - __clzll((long long)y);
+                const unsigned long long x = q >= 64 ? a : a & ~(~0ULL << q);
+                return x ? 63 - __clzll((long long)x) : -1;
+            };
+            int q = next(f0, f1, -1), p = before(m0, m1, q);
+            while (q >= 0) {
+                const int j = sperm[q], prev = sperm[p];
+                const double zj = sz[j], dj = sD[j], zp = sz[prev], dp = sD[prev];
+                const double t = dj - dp, t2 = zj * zj + zp * zp;
+                // |t c s| <= tol with c = zj/tau, s = -zp/tau, tau^2 = t2
+                if (fabs(t * zj * zp) <= tol * t2) {
+                    const double ta = sqrt(t2);
+                    const double c = zj / ta, sn = -zp / ta;
+                    sz[prev] = 0.0;
+                    sD[prev] = dp * c * c + dj * sn * sn;
+                    sz[j] = ta;
+                    sD[j] = dp * sn * sn + dj * c * c;
+                    ra[nrot] = prev;
+                    rb[nrot] = j;
+                    rc[nrot] = c;
+                    rs[nrot] = sn;
+                    nrot++;
+                    if (p < 64) r0 |= 1ULL << p;
+                    else r1 |= 1ULL << (p - 64);
+                    // the combined entry against the next one
+                    p = q;
+                    q = next(m0, m1, q);
+                } else {
+                    q = next(f0, f1, q);
+                    if (q >= 0) p = before(m0, m1, q);
+                }
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        r0 = __shfl(r0, 0, GL);
+        r1 = __shfl(r1, 0, GL);
+    }
+    const unsigned long long n0 = m0 & ~r0, n1 = m1 & ~r1;
+    const int c0 = __popcll(n0);
+    if ((n0 >> gl) & 1) {
+        const int pos = __popcll(n0 & below);
+        snd[pos] = j0;
+        sdl[pos] = sD[j0];
+        szl[pos] = sz[j0];
+    }
+    if (TWO && ((n1 >> gl) & 1)) {
+        const int pos = c0 + __popcll(n1 & below);
+        snd[pos] = j1;
+        sdl[pos] = sD[j1];
+        szl[pos] = sz[j1];
+    }
+    Kn_out = c0 + __popcll(n1);
+    nrot_out = nrot;
+}
 
-    bool top_done = false;
-    int s0 = 2;
-    if (part == 2)
-        while (s0 < n) s0 *= 2;
-    for (int s = s0; s / 2 < n; s *= 2) {
-        const bool top = (s >= n);
-        if (part == 1 && top) break;
-        const int ls = __builtin_ctz(s);  // all index arithmetic by shifts
-        const int nblk = (n + s - 1) >> ls;
-        // A: z and the ascending order of the eigenvalues of each block, the
-        // rank of entry j counted by eight lanes (ties by index)
+// Secular equation 1/rho + sum_j zl_j^2 / (dl_j - lambda) = 0: root i of Kn, in
+// (dl_i, dl_{i+1}) (the last one in (dl_K-1, dl_K-1 + rho |z|^2)), as tau from
+// the nearer pole org, by L lanes (lane sub of them).  Two poles: the root of the
+// quadratic, no iteration.  Bound by an iteration's chain, so a lane keeps its M
+// poles and weights in registers (padded with weight 0 at 1e300) and runs
+// straight-line code: no branch on a root's position, one reciprocal and one
+// square root a step.
+template <int L, int M>
+__device__ __forceinline__ void secular_root(int i, int Kn, int sub, double rho,
+                                             const double *dl, const double *zl, int &org,
+                                             double &tau, int &it) {
+    it = 0;
+    if (Kn == 1) {
+        org = 0;
+        tau = rho * zl[0] * zl[0];
+        return;
+    }
+    if (Kn == 2) {
+        // the roots of the quadratic, each from its nearer pole
+        const double rinv = 1.0 / rho, gap = dl[1] - dl[0];
+        const double z02 = zl[0] * zl[0], z12 = zl[1] * zl[1];
+        if (i == 0) {
+            // the sign of the secular function at the midpoint picks the nearer pole
+            if (rinv + 2.0 * (z12 - z02) / gap >= 0.0) {
+                // tau in (0, gap/2]: rinv tau^2 - a tau + b = 0
+                // (discriminant as a sum of non-negative terms)
+                const double rg = rinv * gap, a = rg + z02 + z12, bq = z02 * gap;
+                const double dm = rg - z02;
+                org = 0;
+                tau = 2.0 * bq / (a + sqrt(dm * dm + z12 * (z12 + 2.0 * (rg + z02))));
+            } else {
+                // tau in (-gap/2, 0) from the upper pole: rinv tau^2 + a tau - b = 0
+                const double a = rinv * gap - z02 - z12, bq = z12 * gap;
+                org = 1;
+                tau = (a < 0.0) ? 2.0 * bq / (a - sqrt(fabs(a * a + 4.0 * bq * rinv)))
+                                : -(a + sqrt(fabs(a * a + 4.0 * bq * rinv))) / (2.0 * rinv);
+            }
+        } else {
+            // tau > 0 beyond the upper pole: rinv tau^2 - A tau - z1^2 gap = 0
+            const double A = z02 + z12 - rinv * gap;
+            const double Dq = sqrt(A * A + 4.0 * rinv * z12 * gap);
+            org = 1;
+            tau = (A >= 0.0) ? (A + Dq) / (2.0 * rinv) : 2.0 * z12 * gap / (Dq - A);
+        }
+        return;
+    }
+    const double rinv = rcp_nr(rho);
+    const bool last = i == Kn - 1;
+    const int i1 = last ? i : i + 1;
+    const double di = dl[i], di1 = dl[i1];
+    const double zi2 = zl[i] * zl[i], zi12 = zl[i1] * zl[i1];
+    const double gap = di1 - di, mid = 0.5 * gap;
+    // this lane's poles (from pole i) and weights, the latter apart for the
+    // poles up to i (psi) and beyond (phi)
+    double dj[M], zp[M], zq[M];
+    double zz = 0.0, wm = 0.0;
+#pragma unroll
+    for (int m = 0; m < M; m++) {
+        const int j = sub + m * L;
+        const bool in = j < Kn;
+        const double z = in ? zl[in ? j : 0] : 0.0;
+        const double z2 = z * z;
+        dj[m] = in ? dl[in ? j : 0] - di : 1e300;
+        zp[m] = j <= i ? z2 : 0.0;
+        zq[m] = j <= i ? 0.0 : z2;
+        zz += z2;
+        // w at the midpoint (the last root has none)
+        wm = fma(z2, rcp_nr(last ? 1.0 : dj[m] - mid), wm);
+    }
+    zz = grp_sum<L>(zz);
+    wm = grp_sum<L>(wm) + rinv;
+    double tlo, thi;
+    org = i;
+    if (last) {
+        tlo = 0.0;
+        thi = rho * zz * (1.0 + 8.0 * EPSU) + 0x1.0p-1000;
+        tau = 0.5 * thi;
+    } else {
+        // the quadratic through the poles i and i+1 with the rest of w at the
+        // midpoint (initial guess of LAPACK's dlaed4)
+        const bool up = !(wm >= 0.0);  // nearer to pole i+1
+        const double c0 = wm + (zi2 - zi12) * rcp_nr(mid);
+        if (up) org = i1;
+        tlo = up ? -(gap - mid) : 0.0;
+        thi = up ? 0.0 : mid;
+        // lower pole: c0 t^2 - a t + bq = 0; upper: c0 t^2 + a t - bq = 0
+        const double a = c0 * gap + (up ? -(zi2 + zi12) : zi2 + zi12);
+        const double bq = (up ? zi12 : zi2) * gap;
+        const double sq = sqrt_pos(fabs(fma(a, a, (up ? 4.0 : -4.0) * bq * c0)));
+        const bool div = up ? a < 0.0 : a > 0.0;  // divide by a +- sq
+        const double num = div ? 2.0 * bq : (up ? -(a + sq) : a - sq);
+        const double den = div ? (up ? a - sq : a + sq) : 2.0 * c0;
+        const double t0 = num * rcp_nr(den);
+        tau = (t0 > tlo && t0 < thi) ? t0 : 0.5 * (tlo + thi);
+    }
+    // poles from the origin: dl - dl[org] (differences of the stored poles, as
+    // where the roots are used)
+    const double dorg = dl[org];
+#pragma unroll
+    for (int m = 0; m < M; m++) {
+        const int j = sub + m * L;
+        if (j < Kn) dj[m] = dl[j] - dorg;
+    }
+    const double ei = di - dorg, ei1 = di1 - dorg;
+    for (it = 0; it < 100; it++) {
+        double psi = 0.0, dpsi = 0.0, phi = 0.0, dphi = 0.0;
+#pragma unroll
+        for (int m = 0; m < M; m++) {
+            const double r = rcp_nr(dj[m] - tau);
+            const double tp = zp[m] * r, tq = zq[m] * r;
+            psi += tp;
+            phi += tq;
+            dpsi = fma(tp, r, dpsi);
+            dphi = fma(tq, r, dphi);
+        }
+        psi = grp_sum<L>(psi);
+        dpsi = grp_sum<L>(dpsi);
+        phi = grp_sum<L>(phi);
+        dphi = grp_sum<L>(dphi);
+        const double w = rinv + psi + phi;
+        if (w == 0.0) break;
+        if (w < 0.0) tlo = tau;
+        else thi = tau;
+        // rounding bound of w: LAPACK's dlaed4 adds the running partial sums, at
+        // most Kn times the sum of |terms|
+        const double errm =
+            (8.0 + Kn) * (phi - psi) + 2.0 * rinv + 3.0 * fabs(tau) * (dpsi + dphi);
+        if (fabs(w) <= EPSU * errm) break;
+        // the step's quotient by the hardware reciprocal and the square root by
+        // its estimate, with Newton steps: the step only steers the iteration,
+        // whose stopping test is on w, and a step outside the bracket (or not a
+        // number) falls back to bisection below
+        const double Di = ei - tau, Di1 = ei1 - tau;
+        const double c = w - Di * dpsi - Di1 * dphi;
+        const double a = (Di + Di1) * w - Di * Di1 * (dpsi + dphi);
+        const double bq = Di * Di1 * w;
+        const double sq = sqrt_pos(fabs(fma(a, a, -4.0 * bq * c)));
+        const bool neg = a <= 0.0;
+        double num = neg ? a - sq : 2.0 * bq, den = neg ? 2.0 * c : a + sq;
+        if (last) {  // the last pole's own term and a constant: Di + Di^2 dpsi / den
+            den = w - Di * dpsi;
+            num = den > 0.0 ? Di * w : NAN;
+        } else if (c == 0.0) {
+            num = bq;
+            den = a;
+        }
+        double eta = num * rcp_nr(den);
+        if (w * eta >= 0.0) eta = -w * rcp_nr(dpsi + dphi);
+        double tn = tau + eta;
+        if (!(tn > tlo && tn < thi)) tn = 0.5 * (tlo + thi);
+        if (tn == tau) break;
+        tau = tn;
+    }
+}
+
+// Gu-Eisenstat z from the computed roots, entry q by L lanes:
+// zhat_q^2 = (lambda_K-1 - d_q)/rho * prod_{i<q} (lambda_i - d_q)/(d_i - d_q)
+//            * prod_{q<=i<K-1} (lambda_i - d_q)/(d_{i+1} - d_q),
+// every factor in (0, 1) except the first (dorg: the roots' origins, lambda_i =
+// dorg_i + tau_i).
+template <int L>
+__device__ __forceinline__ double zhat_entry(int q, int Kn, int sub, double rho, const double *dl,
+                                             const double *dorg, const double *tau, double zq) {
+    const double dq = dl[q];
+    double prod = 1.0;
+#pragma unroll 4
+    for (int i = sub; i < Kn; i += L) {
+        const double num = (dorg[i] - dq) + tau[i];
+        const double dd = dl[i + (i >= q && i + 1 < Kn)] - dq;
+        prod *= num * rcp_nr(i + 1 == Kn ? rho : dd);
+    }
+    prod = grp_prod<L>(prod);
+    return copysign(sqrt(fmax(prod, 0.0)), zq);
+}
+
+// What k_dc_roots leaves for k_dc_vecs: per block of a level (index lo + .) the
+// non-deflated poles, weights, roots and deflating rotations, in block-local
+// column numbers; kn < 0: the block was not merged.
+struct DcState {
+    double *dl, *zl, *tau, *dorg, *rc, *rs, *rho;
+    int *snd, *ra, *rb, *kn, *nrot, *iters;
+};
+
+// The merges of four to smax <= 32 rows, workgroup b on rows and columns 32 b ...
+// Z's columns are written whole (zero outside the block).
+constexpr int DCL = 32, DCP = 33;
+__global__ __launch_bounds__(256) void k_dc_leaf(int n, const double *__restrict__ dd,
+                                                 const double *__restrict__ ee,
+                                                 double *__restrict__ Z, double *__restrict__ lam,
+                                                 int smax, int *iters) {
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int b0 = DCL * blockIdx.x, nb = min(DCL, n - b0);
+    __shared__ double Zs[DCL * DCP], ums[DCL * DCP];  // Z[r + DCP j]; U[q][i] at q DCP + i
+    __shared__ double sD[DCL], sz[DCL], sdl[DCL], szl[DCL], stau[DCL], sdo[DCL], szh[DCL], sinv[DCL],
+        rc[DCL], rs[DCL], srho[DCL];
+    __shared__ int sperm[DCL], snd[DCL], ra[DCL], rb[DCL], sKn[DCL], sNrot[DCL];
+    __shared__ int s_iters;
+    if (tid == 0) s_iters = 0;
+    for (int e = tid; e < DCL * DCL; e += 256) Zs[(e & 31) + DCP * (e >> 5)] = (e & 31) == (e >> 5);
+    lds_sync();
+    // Leaves of two rows (of one if even those are left to the top merge), torn
+    // off their neighbours: the 2 x 2 blocks by their Jacobi rotation.
+    if (tid < DCL && b0 + tid < n) {
+        const int i = b0 + tid;
+        const bool two = smax >= 2, pair = two && (tid ^ 1) < nb;
+        auto leaf_d = [&](int q) {
+            double x = dd[q];
+            if (q > 0 && !(two && (q & 1))) x -= fabs(ee[q - 1]);
+            if (q + 1 < n && !(two && !(q & 1))) x -= fabs(ee[q]);
+            return x;
+        };
+        const double x = leaf_d(i);
+        sD[tid] = x;
+        if (pair && ee[i & ~1] != 0.0) {
+            const double y = leaf_d(i ^ 1), off = ee[i & ~1];
+            const double a = (i & 1) ? y : x, b = (i & 1) ? x : y;
+            const double th = (b - a) / (2.0 * off);
+            const double t = copysign(1.0 / (fabs(th) + sqrt(1.0 + th * th)), th);
+            const double c = 1.0 / sqrt(1.0 + t * t), sn = t * c;
+            // columns (c, -s) for a - t e and (s, c) for b + t e
+            sD[tid] = (i & 1) ? b + t * off : a - t * off;
+            Zs[(tid & ~1) + DCP * tid] = (i & 1) ? sn : c;
+            Zs[(tid | 1) + DCP * tid] = (i & 1) ? c : -sn;
+        }
+    }
+    lds_sync();
+    for (int s = 4; s <= smax && s / 2 < nb; s *= 2) {
+        const int ls = __builtin_ctz(s);
+        const int nblk = (nb + s - 1) >> ls;
+        // z and the ascending order of the eigenvalues of each block, the rank
+        // of entry j counted by eight lanes (ties by index)
         {
             const int j = tid >> 3, sub = tid & 7;
-            const int b = j >> ls, lo = b << ls, hi = min(lo + s, n), m = lo + s / 2;
-            if (j < n && m < hi) {
+            const int lo = (j >> ls) << ls, hi = min(lo + s, nb), m = lo + s / 2;
+            if (j < nb && m < hi) {
                 if (sub == 0) {
-                    const double bt = ee[m - 1];
-                    const double sg = (bt >= 0.0) ? 1.0 : -1.0;
-                    sz[j] = (j < m ? Z[(m - 1) + (long)j * n] : sg * Z[m + (long)j * n]) * M_SQRT1_2;
+                    const double sg = (ee[b0 + m - 1] >= 0.0) ? 1.0 : -1.0;
+                    sz[j] = (j < m ? Zs[(m - 1) + DCP * j] : sg * Zs[m + DCP * j]) * M_SQRT1_2;
                 }
                 const double dj = sD[j];
                 int pos = 0;
@@ -474,569 +764,428 @@ __global__ __launch_bounds__(8 * NMAX) void k_stedc(
                 if (sub == 0) sperm[lo + pos] = j;
             }
         }
-        __syncthreads();
-        // B: deflation, a group of GL = min(s, 64) lanes per block (each lane
-        // one or two sorted positions)
+        lds_sync();
         {
-            const int GL = s < 64 ? s : 64;
-            const int gl = tid & (GL - 1);
-            const int gbase = lane - gl;
-            const unsigned long long gmask = (GL == 64) ? ~0ULL : (((1ULL << GL) - 1) << gbase);
-            const int lgl = __builtin_ctz(GL);
-            for (int b = tid >> lgl; b < nblk; b += NT >> lgl) {
-                const int lo = b << ls, hi = min(lo + s, n), m = lo + s / 2, K = hi - lo;
-                if (m >= hi) {
-                    if (gl == 0) sKn[b] = -1;
-                    continue;
+            const int b = tid >> ls, gl = tid & (s - 1), lo = b << ls;
+            if (b < nblk) {
+                const int hi = min(lo + s, nb), m = lo + s / 2;
+                int Kn = -1, nrot = 0;
+                double rho = 0.0;
+                if (m < hi) {
+                    rho = 2.0 * fabs(ee[b0 + m - 1]);
+                    Kn = 0;
+                    if (rho != 0.0)
+                        deflate<false>(s, gl, lane - gl, hi - lo, rho, sperm + lo, sz, sD,
+                                       snd + lo, sdl + lo, szl + lo, ra + lo, rb + lo, rc + lo,
+                                       rs + lo, Kn, nrot);
                 }
-                const double rho = 2.0 * fabs(ee[m - 1]);
-                if (rho == 0.0) {
-                    if (gl == 0) {
-                        srho[b] = rho;
-                        sKn[b] = 0;
-                        sNrot[b] = 0;
-                    }
-                    continue;
-                }
-                // sorted positions q0 = gl, q1 = gl + 64 (only when s = 128)
-                const int q0 = gl, q1 = gl + 64;
-                const int j0 = (q0 < K) ? sperm[lo + q0] : -1;
-                const int j1 = (s > 64 && q1 < K) ? sperm[lo + q1] : -1;
-                const double z0 = j0 >= 0 ? sz[j0] : 0.0, z1 = j1 >= 0 ? sz[j1] : 0.0;
-                const double d0 = j0 >= 0 ? sD[j0] : 0.0, d1 = j1 >= 0 ? sD[j1] : 0.0;
-                double dmax = fmax(fabs(d0), fabs(d1)), zmax = fmax(fabs(z0), fabs(z1));
-                for (int o = 1; o < GL; o <<= 1) {
-                    dmax = fmax(dmax, __shfl_xor(dmax, o, GL));
-                    zmax = fmax(zmax, __shfl_xor(zmax, o, GL));
-                }
-                const double tol = 8.0 * EPSU * fmax(dmax, zmax);
-                const bool k0 = j0 >= 0 && !(rho * fabs(z0) <= tol);
-                const bool k1 = j1 >= 0 && !(rho * fabs(z1) <= tol);
-                // kept positions of the group, bit = sorted position
-                const unsigned long long m0 = (__ballot(k0) & gmask) >> gbase;
-                const unsigned long long m1 = (__ballot(k1) & gmask) >> gbase;
-                const unsigned long long below = (gl == 0) ? 0ULL : ((~0ULL) >> (64 - gl));
-                bool close = false;
-                if (k0) {
-                    const unsigned long long mm = m0 & below;
-                    if (mm) {
-                        const int jp = sperm[lo + 63 - __clzll(mm)];
-                        const double zp = sz[jp], t = d0 - sD[jp];
-                        close = fabs(t * z0 * zp) <= tol * (z0 * z0 + zp * zp);
-                    }
-                }
-                if (k1) {
-                    const unsigned long long mm = m1 & below;
-                    const int p = mm ? 64 + 63 - __clzll(mm) : (m0 ? 63 - __clzll(m0) : -1);
-                    if (p >= 0) {
-                        const int jp = sperm[lo + p];
-                        const double zp = sz[jp], t = d1 - sD[jp];
-                        close = close || (fabs(t * z1 * zp) <= tol * (z1 * z1 + zp * zp));
-                    }
-                }
-                if ((__ballot(close) & gmask) == 0ULL) {
-                    const int c0 = __popcll(m0);
-                    if (k0) {
-                        const int pos = __popcll(m0 & below);
-                        snd[lo + pos] = j0;
-                        sdl[lo + pos] = d0;
-                        szl[lo + pos] = z0;
-                    }
-                    if (k1) {
-                        const int pos = c0 + __popcll(m1 & below);
-                        snd[lo + pos] = j1;
-                        sdl[lo + pos] = d1;
-                        szl[lo + pos] = z1;
-                    }
-                    if (gl == 0) {
-                        srho[b] = rho;
-                        sKn[b] = c0 + __popcll(m1);
-                        sNrot[b] = 0;
-                    }
-                } else if (gl == 0) {
-                    // one lane walks the sorted entries; the pending entry's
-                    // (z, d) are carried in registers and the next entry is
-                    // loaded while the current one is decided (entries not
-                    // reached yet are never written, so the early loads hold)
-                    int Kn = 0, nrot = 0, prev = -1;
-                    double zp = 0.0, dp = 0.0;
-                    int jn = sperm[lo];
-                    double zn = sz[jn], dn = sD[jn];
-                    for (int qq = lo; qq < hi; qq++) {
-                        const int j = jn;
-                        const double zj = zn, dj = dn;
-                        if (qq + 1 < hi) {
-                            jn = sperm[qq + 1];
-                            zn = sz[jn];
-                            dn = sD[jn];
-                        }
-                        if (rho * fabs(zj) <= tol) continue;
-                        if (prev < 0) {
-                            prev = j;
-                            zp = zj;
-                            dp = dj;
-                            continue;
-                        }
-                        const double t = dj - dp;
-                        const double t2 = zj * zj + zp * zp;
-                        // |t c s| <= tol with c = zj/tau, s = -zp/tau, tau^2 = t2
-                        if (fabs(t * zj * zp) <= tol * t2) {
-                            const double ta = sqrt(t2);
-                            const double c = zj / ta, sn = -zp / ta;
-                            sz[prev] = 0.0;
-                            sD[prev] = dp * c * c + dj * sn * sn;
-                            ra[lo + nrot] = prev;
-                            rb[lo + nrot] = j;
-                            rc[lo + nrot] = c;
-                            rs[lo + nrot] = sn;
-                            nrot++;
-                            prev = j;
-                            zp = ta;
-                            dp = dp * sn * sn + dj * c * c;
-                        } else {
-                            sz[prev] = zp;
-                            sD[prev] = dp;
-                            snd[lo + Kn] = prev;
-                            sdl[lo + Kn] = dp;
-                            szl[lo + Kn] = zp;
-                            Kn++;
-                            prev = j;
-                            zp = zj;
-                            dp = dj;
-                        }
-                    }
-                    if (prev >= 0) {
-                        sz[prev] = zp;
-                        sD[prev] = dp;
-                        snd[lo + Kn] = prev;
-                        sdl[lo + Kn] = dp;
-                        szl[lo + Kn] = zp;
-                        Kn++;
-                    }
+                if (gl == 0) {
                     srho[b] = rho;
                     sKn[b] = Kn;
                     sNrot[b] = nrot;
                 }
             }
         }
-        __syncthreads();
-        // C: the deflating rotations on the rows of Z (column pairs, in
-        // order); the top merge's go to its Um instead
-        for (int rr = tid; rr < n && !top; rr += NT) {
-            const int b = rr >> ls, lo = b << ls;
-            if (sKn[b] < 0) continue;
-            const int nrot = sNrot[b];
+        lds_sync();
+        // the deflating rotations on the rows of Z (column pairs, in order)
+        if (tid < nb) {
+            const int b = tid >> ls, lo = b << ls;
+            const int nrot = sKn[b] < 0 ? 0 : sNrot[b];
             for (int t = 0; t < nrot; t++) {
-                const long ia = rr + (long)ra[lo + t] * n, ib = rr + (long)rb[lo + t] * n;
-                const double qa = Z[ia], qb = Z[ib], c = rc[lo + t], sn = rs[lo + t];
-                Z[ia] = c * qa + sn * qb;
-                Z[ib] = c * qb - sn * qa;
+                const int ia = tid + DCP * ra[lo + t], ib = tid + DCP * rb[lo + t];
+                const double qa = Zs[ia], qb = Zs[ib], c = rc[lo + t], sn = rs[lo + t];
+                Zs[ia] = c * qa + sn * qb;
+                Zs[ib] = c * qb - sn * qa;
             }
         }
-        // D: secular equation 1/rho + sum_j zl_j^2 / (dl_j - lambda) = 0 for
-        // the root in (dl_i, dl_{i+1}) (the last one in (dl_K-1, dl_K-1 + rho
-        // |z|^2)), L lanes per root (L = 1..8 by block size), from the nearer pole;
-        // two poles: the root of the quadratic, no iteration
-        auto secular = [&](auto Ltag) {
-            constexpr int L = decltype(Ltag)::value;
+        auto roots = [&](auto Ltag, auto Mtag) {
+            constexpr int L = decltype(Ltag)::value, M = decltype(Mtag)::value;
             const int ri = tid / L, sub = tid & (L - 1);
-            int b = 0, lo = 0, i = 0, Kn = 0;
-            if (ri < n) {
-                b = ri >> ls;
-                lo = b << ls;
-                i = ri - lo;
-                Kn = sKn[b];
-            }
-            if (Kn > 0 && i < Kn) {
-                const double rho = srho[b];
-                const double *dl = sdl + lo, *zl = szl + lo;
-                int org;
+            const int b = ri >> ls, lo = b << ls, i = ri - lo;
+            const int Kn = ri < nb ? sKn[b] : 0;
+            if (i < Kn) {
+                int org, it;
                 double tau;
-                int it = 0;
-                if (Kn == 1) {
-                    org = 0;
-                    tau = rho * zl[0] * zl[0];
-                } else if (Kn == 2) {
-                    // the roots of the quadratic, each from its nearer pole
-                    const double rinv = 1.0 / rho, gap = dl[1] - dl[0];
-                    const double z02 = zl[0] * zl[0], z12 = zl[1] * zl[1];
-                    if (i == 0) {
-                        // the sign of the secular function at the midpoint
-                        // picks the nearer pole
-                        if (rinv + 2.0 * (z12 - z02) / gap >= 0.0) {
-                            // tau in (0, gap/2]: rinv tau^2 - a tau + b = 0
-                            // (discriminant as a sum of non-negative terms)
-                            const double rg = rinv * gap, a = rg + z02 + z12, bq = z02 * gap;
-                            const double dm = rg - z02;
-                            org = 0;
-                            tau = 2.0 * bq / (a + sqrt(dm * dm + z12 * (z12 + 2.0 * (rg + z02))));
-                        } else {
-                            // tau in (-gap/2, 0) from the upper pole: rinv tau^2 + a tau - b = 0
-                            const double a = rinv * gap - z02 - z12, bq = z12 * gap;
-                            org = 1;
-                            tau = (a < 0.0) ? 2.0 * bq / (a - sqrt(fabs(a * a + 4.0 * bq * rinv)))
-                                            : -(a + sqrt(fabs(a * a + 4.0 * bq * rinv))) / (2.0 * rinv);
-                        }
-                    } else {
-                        // tau > 0 beyond the upper pole: rinv tau^2 - A tau - z1^2 gap = 0
-                        const double A = z02 + z12 - rinv * gap;
-                        const double Dq = sqrt(A * A + 4.0 * rinv * z12 * gap);
-                        org = 1;
-                        tau = (A >= 0.0) ? (A + Dq) / (2.0 * rinv) : 2.0 * z12 * gap / (Dq - A);
-                    }
-                } else {
-                    const double rinv = 1.0 / rho;
-                    double tlo, thi;
-                    if (i < Kn - 1) {
-                        const double gap = dl[i + 1] - dl[i];
-                        const double mid = 0.5 * gap;
-                        // w at the midpoint, and the part of it from the poles
-                        // other than i, i+1 (initial guess of LAPACK's dlaed4)
-                        double w = 0.0;
-                        for (int j = sub; j < Kn; j += L)
-                            w = fma(zl[j] * zl[j], rcp_nr((dl[j] - dl[i]) - mid), w);
-                        w = grp_sum<L>(w) + rinv;
-                        const double zi2 = zl[i] * zl[i], zi12 = zl[i + 1] * zl[i + 1];
-                        const double c0 = w - zi2 / (-mid) - zi12 / (gap - mid);
-                        double t0;
-                        if (w >= 0.0) {
-                            org = i;
-                            tlo = 0.0;
-                            thi = mid;
-                            const double a = c0 * gap + zi2 + zi12, bq = zi2 * gap;
-                            if (c0 == 0.0) t0 = bq / a;
-                            else if (a <= 0.0) t0 = (a - sqrt(fabs(a * a - 4.0 * bq * c0))) / (2.0 * c0);
-                            else t0 = 2.0 * bq / (a + sqrt(fabs(a * a - 4.0 * bq * c0)));
-                        } else {
-                            org = i + 1;
-                            tlo = -(gap - mid);
-                            thi = 0.0;
-                            // c0 t^2 + a t - bq = 0, the root in (-mid, 0)
-                            const double a = c0 * gap - zi2 - zi12, bq = zi12 * gap;
-                            if (c0 == 0.0) t0 = bq / a;
-                            else if (a < 0.0) t0 = 2.0 * bq / (a - sqrt(fabs(a * a + 4.0 * bq * c0)));
-                            else t0 = -(a + sqrt(fabs(a * a + 4.0 * bq * c0))) / (2.0 * c0);
-                        }
-                        tau = (t0 > tlo && t0 < thi) ? t0 : 0.5 * (tlo + thi);
-                    } else {
-                        double zz = 0.0;
-                        for (int j = sub; j < Kn; j += L) zz = fma(zl[j], zl[j], zz);
-                        zz = grp_sum<L>(zz);
-                        org = i;
-                        tlo = 0.0;
-                        thi = rho * zz * (1.0 + 8.0 * EPSU) + 0x1.0p-1000;
-                        tau = 0.5 * thi;
-                    }
-                    const double dorg = dl[org];
-                    for (it = 0; it < 100; it++) {
-                        // poles up to i (psi) and beyond (phi), split by lane
-                        double psi = 0.0, dpsi = 0.0, phi = 0.0, dphi = 0.0;
-                        double psi2 = 0.0, dpsi2 = 0.0, phi2 = 0.0, dphi2 = 0.0;
-                        int j = sub;
-                        for (; j + L <= i; j += 2 * L) {
-                            const double t = zl[j] * rcp_nr((dl[j] - dorg) - tau);
-                            const double t2 = zl[j + L] * rcp_nr((dl[j + L] - dorg) - tau);
-                            psi = fma(zl[j], t, psi);
-                            dpsi = fma(t, t, dpsi);
-                            psi2 = fma(zl[j + L], t2, psi2);
-                            dpsi2 = fma(t2, t2, dpsi2);
-                        }
-                        for (; j <= i; j += L) {
-                            const double t = zl[j] * rcp_nr((dl[j] - dorg) - tau);
-                            psi = fma(zl[j], t, psi);
-                            dpsi = fma(t, t, dpsi);
-                        }
-                        for (; j + L < Kn; j += 2 * L) {
-                            const double t = zl[j] * rcp_nr((dl[j] - dorg) - tau);
-                            const double t2 = zl[j + L] * rcp_nr((dl[j + L] - dorg) - tau);
-                            phi = fma(zl[j], t, phi);
-                            dphi = fma(t, t, dphi);
-                            phi2 = fma(zl[j + L], t2, phi2);
-                            dphi2 = fma(t2, t2, dphi2);
-                        }
-                        for (; j < Kn; j += L) {
-                            const double t = zl[j] * rcp_nr((dl[j] - dorg) - tau);
-                            phi = fma(zl[j], t, phi);
-                            dphi = fma(t, t, dphi);
-                        }
-                        psi += psi2;
-                        dpsi += dpsi2;
-                        phi += phi2;
-                        dphi += dphi2;
-                        psi = grp_sum<L>(psi);
-                        dpsi = grp_sum<L>(dpsi);
-                        phi = grp_sum<L>(phi);
-                        dphi = grp_sum<L>(dphi);
-                        const double w = rinv + psi + phi;
-                        if (w == 0.0) break;
-                        if (w < 0.0) tlo = tau;
-                        else thi = tau;
-                        // rounding bound of w: LAPACK's dlaed4 adds the running
-                        // partial sums, at most Kn times the sum of |terms|
-                        const double errm = (8.0 + Kn) * (phi - psi) + 2.0 * rinv +
-                                            3.0 * fabs(tau) * (dpsi + dphi);
-                        if (fabs(w) <= EPSU * errm) break;
-                        // the step's quotients by the hardware reciprocal (a
-                        // few ulp): the step only steers the iteration, whose
-                        // stopping test is on w, and a step outside the
-                        // bracket falls back to bisection below
-                        double eta;
-                        if (i < Kn - 1) {
-                            const double Di = (dl[i] - dorg) - tau, Di1 = (dl[i + 1] - dorg) - tau;
-                            const double c = w - Di * dpsi - Di1 * dphi;
-                            const double a = (Di + Di1) * w - Di * Di1 * (dpsi + dphi);
-                            const double bq = Di * Di1 * w;
-                            if (c == 0.0)
-                                eta = (a != 0.0) ? bq * rcp_nr(a) : 0.5 * (tlo + thi) - tau;
-                            else if (a <= 0.0)
-                                eta = (a - sqrt(fabs(a * a - 4.0 * bq * c))) * rcp_nr(2.0 * c);
-                            else
-                                eta = 2.0 * bq * rcp_nr(a + sqrt(fabs(a * a - 4.0 * bq * c)));
-                        } else {
-                            const double Dl = (dl[i] - dorg) - tau;
-                            const double den = w - Dl * dpsi;
-                            eta = (den > 0.0) ? Dl + Dl * Dl * dpsi * rcp_nr(den)
-                                              : 0.5 * (tlo + thi) - tau;
-                        }
-                        if (w * eta >= 0.0) eta = -w * rcp_nr(dpsi + dphi);
-                        double tn = tau + eta;
-                        if (!(tn > tlo && tn < thi)) tn = 0.5 * (tlo + thi);
-                        if (tn == tau) break;
-                        tau = tn;
-                    }
-                }
+                secular_root<L, M>(i, Kn, sub, srho[b], sdl + lo, szl + lo, org, tau, it);
                 if (sub == 0) {
-                    sorg[lo + i] = org;
+                    sdo[lo + i] = sdl[lo + org];
                     stau[lo + i] = tau;
                     if (it > 0) atomicMax(&s_iters, it);
                 }
             }
         };
+        if (s == 4) roots(std::integral_constant<int, 4>{}, std::integral_constant<int, 1>{});
+        else if (s == 8) roots(std::integral_constant<int, 8>{}, std::integral_constant<int, 1>{});
+        else if (s == 16) roots(std::integral_constant<int, 8>{}, std::integral_constant<int, 2>{});
+        else roots(std::integral_constant<int, 8>{}, std::integral_constant<int, 4>{});
+        lds_sync();
         {
-            const int L = s >= 8 ? 8 : (s == 4 ? 4 : 1);
-            if (L == 8) secular(std::integral_constant<int, 8>{});
-            else if (L == 4) secular(std::integral_constant<int, 4>{});
-            else if (L == 2) secular(std::integral_constant<int, 2>{});
-            else secular(std::integral_constant<int, 1>{});
+            const int jq = tid >> 3, sub = tid & 7, b = jq >> ls, lo = b << ls, q = jq - lo;
+            const int Kn = jq < nb ? sKn[b] : 0;
+            if (q < Kn) {
+                const double z = zhat_entry<8>(q, Kn, sub, srho[b], sdl + lo, sdo + lo, stau + lo,
+                                               szl[jq]);
+                if (sub == 0) szh[jq] = z;
+            }
         }
-        __syncthreads();
-        // E: Gu-Eisenstat z from the computed roots, L lanes per entry:
-        // zhat_q^2 = (lambda_K-1 - d_q)/rho * prod_{i<q} (lambda_i - d_q)/(d_i - d_q)
-        //            * prod_{q<=i<K-1} (lambda_i - d_q)/(d_{i+1} - d_q),
-        // every factor in (0, 1) except the first
-        auto zhat = [&](auto Ltag) {
-            constexpr int L = decltype(Ltag)::value;
-            const int jq = tid / L, sub = tid & (L - 1);
-            int lo = 0, q = 0, Kn = 0;
-            if (jq < n) {
-                const int b = jq >> ls;
-                lo = b << ls;
-                q = jq - lo;
-                Kn = sKn[b];
-            }
-            if (Kn > 0 && q < Kn) {
-                const double *dl = sdl + lo;
-                const double dq = dl[q];
-                double prod = 1.0;
-                for (int i = sub; i < Kn; i += L) {
-                    const double num = (dl[sorg[lo + i]] - dq) + stau[lo + i];
-                    const double den = (i == Kn - 1) ? srho[jq >> ls] : (i < q ? dl[i] - dq : dl[i + 1] - dq);
-                    prod *= num * rcp_nr(den);
-                }
-                prod = grp_prod<L>(prod);
-                if (sub == 0) szh[lo + q] = copysign(sqrt(fmax(prod, 0.0)), szl[lo + q]);
-            }
-        };
+        lds_sync();
+        // eigenvectors of the rank-one updates, and their norms
+        for (int t = tid; t < nblk << (2 * ls); t += 256) {
+            const int jq = t >> ls, i = t & (s - 1), b = jq >> ls, lo = b << ls, q = jq - lo;
+            const int Kn = sKn[b];
+            if (q < Kn && i < Kn)
+                ums[jq * DCP + i] =
+                    szh[jq] * rcp_nr((sdl[jq] - sdo[lo + i]) - stau[lo + i]);
+        }
+        lds_sync();
         {
-            const int L = s >= 8 ? 8 : (s == 4 ? 4 : 1);
-            if (L == 8) zhat(std::integral_constant<int, 8>{});
-            else if (L == 4) zhat(std::integral_constant<int, 4>{});
-            else if (L == 2) zhat(std::integral_constant<int, 2>{});
-            else zhat(std::integral_constant<int, 1>{});
+            const int ci = tid >> 3, sub = tid & 7, b = ci >> ls, lo = b << ls, i = ci - lo;
+            const int Kn = ci < nb ? sKn[b] : 0;
+            if (i < Kn) {
+                double ss = 0.0;
+                for (int q = sub; q < Kn; q += 8) {
+                    const double u = ums[(lo + q) * DCP + i];
+                    ss = fma(u, u, ss);
+                }
+                ss = oct_sum(ss);
+                if (sub == 0) sinv[ci] = 1.0 / sqrt(ss);
+            }
         }
-        __syncthreads();
-        if (!top) {
-            // F: eigenvector matrix of each rank-one update, column i of
-            // block b at ums[lo*s + i + q*s] (i fastest: one row of U per q)
-            for (int t = tid; t < nblk << (2 * ls); t += NT) {
-                const int b = t >> (2 * ls);
-                const int rem = t & ((1 << (2 * ls)) - 1);
-                const int q = rem >> ls, i = rem & (s - 1);
-                const int lo = b << ls, Kn = sKn[b];
-                if (Kn <= 0 || q >= Kn || i >= Kn) continue;
-                const double *dl = sdl + lo;
-                ums[lo * s + i + q * s] =
-                    szh[lo + q] * rcp_nr((dl[q] - dl[sorg[lo + i]]) - stau[lo + i]);
+        lds_sync();
+        // Z[:, snd_i] = Z[:, snd] u_i over the block's rows, read by every thread
+        // before any writes.  Blocks of 16 and 32: 16 x 16 tiles on the matrix
+        // cores, issued as (U^T)(Z^T) so that a tile's lanes hold 16 consecutive
+        // rows of one column; smaller blocks: a thread an entry.
+        if (s >= 16) {
+            const int lt = ls - 4, tiles = nblk << (2 * lt);
+            const int b = wv >> (2 * lt), rem = wv & ((1 << (2 * lt)) - 1);
+            const int rb0 = (rem >> lt) * 16, cb = (rem & ((1 << lt) - 1)) * 16;
+            const int lo = b << ls, Kn = wv < tiles ? sKn[b] : 0;
+            f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+            for (int k0 = 0; k0 < Kn; k0 += 4) {
+                const int q = k0 + (lane >> 4);
+                const bool kin = q < Kn;
+                const int qi = kin ? q : 0;
+                const double ua = kin && cb + (lane & 15) < Kn
+                                      ? ums[(lo + qi) * DCP + cb + (lane & 15)] : 0.0;
+                const double zb = kin ? Zs[lo + rb0 + (lane & 15) + DCP * snd[lo + qi]] : 0.0;
+                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(ua, zb, acc, 0, 0, 0);
             }
-            // stage the non-deflated columns of each block: zs[lo*s + r + q*s]
-            {
-                const int tot = nblk << (2 * ls);
-                for (int t0 = tid; t0 < tot; t0 += 4 * NT) {
-                    double v[4];
-                    int dst[4];
+            lds_sync();
 #pragma unroll
-                    for (int u = 0; u < 4; u++) {
-                        const int t = t0 + u * NT;
-                        v[u] = 0.0;
-                        dst[u] = -1;
-                        if (t >= tot) continue;
-                        const int b = t >> (2 * ls);
-                        const int rem = t & ((1 << (2 * ls)) - 1);
-                        const int q = rem >> ls, rl = rem & (s - 1);
-                        const int lo = b << ls, hi = min(lo + s, n), Kn = sKn[b];
-                        if (Kn <= 0 || q >= Kn || lo + rl >= hi) continue;
-                        v[u] = Z[lo + rl + (long)snd[lo + q] * n];
-                        dst[u] = t;
-                    }
-#pragma unroll
-                    for (int u = 0; u < 4; u++)
-                        if (dst[u] >= 0) zs[dst[u]] = v[u];
-                }
+            for (int v = 0; v < 4; v++) {
+                const int col = cb + (lane >> 4) + 4 * v;
+                if (col < Kn)
+                    Zs[lo + rb0 + (lane & 15) + DCP * snd[lo + col]] = acc[v] * sinv[lo + col];
             }
-            __syncthreads();
-            // G: column norms of the update's eigenvectors, eight lanes per column
-            {
-                const int ci = tid >> 3, sub = tid & 7;
-                int lo = 0, i = 0, Kn = 0, b = 0;
-                if (ci < n) {
-                    b = ci >> ls;
-                    lo = b << ls;
-                    i = ci - lo;
-                    Kn = sKn[b];
-                }
-                if (Kn > 0 && i < Kn) {
-                    const double *u = ums + lo * s + i;
-                    double ss = 0.0;
-                    for (int q = sub; q < Kn; q += 8) ss = fma(u[q * s], u[q * s], ss);
-                    ss = oct_sum(ss);
-                    if (sub == 0) sinv[lo + i] = 1.0 / sqrt(ss);
-                }
-            }
-            __syncthreads();
-            // H: Z[:, nd_i] = (staged columns) * u_i * sinv_i over the block's
-            // rows.  Blocks of 16 and more: 16 x 16 output tiles on the FP64
-            // matrix cores, issued as (U^T)(ZS^T) so that a tile's lanes hold 16
-            // consecutive rows of one column (128-byte stores); a wave per tile,
-            // the k steps beyond Kn zeroed in both operands.  Smaller blocks: a
-            // thread per (block, group of 16 columns, row), rows fastest.
-            if (s >= 16) {
-                const int lt = ls - 4;
-                const int tiles = nblk << (2 * lt);
-                for (int t = wv; t < tiles; t += NT / 64) {
-                    const int b = t >> (2 * lt), rem = t & ((1 << (2 * lt)) - 1);
-                    const int rb = (rem >> lt) * 16, cb = (rem & ((1 << lt) - 1)) * 16;
-                    const int lo = b << ls, hi = min(lo + s, n), Kn = sKn[b];
-                    if (Kn <= 0 || cb >= Kn || lo + rb >= hi) continue;
-                    f64x4 acc = {0.0, 0.0, 0.0, 0.0};
-                    const double *ub = ums + lo * s + cb + (lane & 15);
-                    const double *zb = zs + lo * s + rb + (lane & 15);
-                    for (int k0 = 0; k0 < Kn; k0 += 4) {
-                        const int q = k0 + (lane >> 4);
-                        const bool kin = q < Kn;
-                        const double ua = kin ? ub[q * s] : 0.0;  // U[q][cb + l%16]
-                        const double zb2 = kin ? zb[q * s] : 0.0;  // ZS[rb + l%16][q]
-                        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(ua, zb2, acc, 0, 0, 0);
-                    }
-#pragma unroll
-                    for (int v = 0; v < 4; v++) {
-                        const int col = cb + (lane >> 4) + 4 * v, row = lo + rb + (lane & 15);
-                        if (col < Kn && row < hi)
-                            Z[row + (long)snd[lo + col] * n] = acc[v] * sinv[lo + col];
-                    }
-                }
-            } else
-            {
-                const int lcg = (ls > 4) ? ls - 4 : 0;  // column groups of 16: s/16 of them
-                const int tot = nblk << (lcg + ls);
-                for (int t = tid; t < tot; t += NT) {
-                    const int rl = t & (s - 1);
-                    const int bc = t >> ls;
-                    const int cg = bc & ((1 << lcg) - 1), b = bc >> lcg;
-                    const int lo = b << ls, hi = min(lo + s, n), Kn = sKn[b];
-                    const int i0 = cg * 16;
-                    if (Kn <= 0 || i0 >= Kn || lo + rl >= hi) continue;
-                    const int nc = min(16, Kn - i0);
-                    double acc[16];
-#pragma unroll
-                    for (int c = 0; c < 16; c++) acc[c] = 0.0;
-                    const double *zb = zs + lo * s + rl;
-                    const double *ub = ums + lo * s + i0;
-                    for (int q = 0; q < Kn; q++) {
-                        const double zv = zb[q * s];
-                        // 16-byte aligned: lo * s, q * s and i0 are even
-                        const double2 *uq = reinterpret_cast<const double2 *>(ub + q * s);
-#pragma unroll
-                        for (int c = 0; c < 8; c++) {
-                            const double2 u2 = uq[c];
-                            acc[2 * c] = fma(zv, u2.x, acc[2 * c]);
-                            acc[2 * c + 1] = fma(zv, u2.y, acc[2 * c + 1]);
-                        }
-                    }
-#pragma unroll
-                    for (int c = 0; c < 16; c++)
-                        if (c < nc)
-                            Z[lo + rl + (long)snd[lo + i0 + c] * n] = acc[c] * sinv[lo + i0 + c];
-                }
-            }
-            for (int t = tid; t < n; t += NT) {
-                const int b = t >> ls, lo = b << ls, i = t - lo, Kn = sKn[b];
-                if (Kn <= 0 || i >= Kn) continue;
-                sD[snd[lo + i]] = sdl[lo + sorg[lo + i]] + stau[lo + i];
-            }
-            __syncthreads();
         } else {
-            // top merge: column order (non-deflated first), eigenvalues per
-            // column, and the padded, normalised eigenvector matrix of the update
-            const int Kn = sKn[0] > 0 ? sKn[0] : 0;
-            for (int j = tid; j < n; j += NT) sflag[j] = 0;
-            __syncthreads();
-            for (int q = tid; q < Kn; q += NT) sflag[snd[q]] = 1;
-            __syncthreads();
-            // column c's pole: Z column scm[c]; Z column j's column: spos[j]
-            for (int j = tid; j < n; j += NT) {
-                if (sflag[j]) continue;
-                int pos = Kn;
-                for (int q = 0; q < j; q++) pos += !sflag[q];
-                colmap[pos] = j;
-                scm[pos] = j;
-                spos[j] = pos;
-                slam[pos] = sD[j];
+            const int r = tid & 31, i = tid >> 5, b = r >> ls, lo = b << ls;
+            const int Kn = r < nb ? sKn[b] : 0;
+            double acc = 0.0;
+            if (i < Kn)
+                for (int q = 0; q < Kn; q++)
+                    acc = fma(Zs[r + DCP * snd[lo + q]], ums[(lo + q) * DCP + i], acc);
+            lds_sync();
+            if (i < Kn) Zs[r + DCP * snd[lo + i]] = acc * sinv[lo + i];
+        }
+        if (tid < nb) {
+            const int b = tid >> ls, lo = b << ls, i = tid - lo;
+            if (i < sKn[b]) sD[snd[tid]] = sdo[tid] + stau[tid];
+        }
+        lds_sync();
+    }
+    for (int j = tid >> 5; j < nb; j += 8)
+        for (int r = tid & 31; r < n; r += 32)
+            Z[r + (long)(b0 + j) * n] = (r >= b0 && r < b0 + nb) ? Zs[r - b0 + DCP * j] : 0.0;
+    if (tid < nb) lam[b0 + tid] = sD[tid];
+    if (tid == 0) {
+        iters[blockIdx.x] = s_iters;
+        if (blockIdx.x == 0) iters[4] = 0;
+    }
+}
+
+// One merge of blocks of s <= S rows, first half: workgroup g of a block's
+// ceil(s/16) finds roots 16 g .. 16 g + 15, L lanes a root; the block's
+// first also leaves the deflation's outcome.
+template <int S, int L>
+__global__ __launch_bounds__(16 * L) void k_dc_roots(int n, int s, const double *__restrict__ ee,
+                                                  const double *__restrict__ Z,
+                                                  const double *__restrict__ lam_in,
+                                                  double *__restrict__ lam_out, DcState st) {
+    const int tid = threadIdx.x;
+    const int gpb = (s + 15) >> 4, b = blockIdx.x / gpb, g = blockIdx.x - b * gpb;
+    const int lo = b * s, hi = min(lo + s, n), m = lo + s / 2, K = hi - lo;
+    __shared__ double sD[S], sz[S], sdl[S], szl[S], rc[S], rs[S];
+    __shared__ int sperm[S], snd[S], ra[S], rb[S], sflag[S];
+    __shared__ int s_kn, s_nrot;
+    if (m >= hi) {  // nothing to merge with
+        if (g == 0) {
+            if (tid < K) lam_out[lo + tid] = lam_in[lo + tid];
+            if (tid == 0) {
+                st.kn[b] = -1;
+                st.nrot[b] = 0;
             }
-            for (int q = tid; q < Kn; q += NT) {
-                colmap[q] = snd[q];
-                scm[q] = snd[q];
-                spos[snd[q]] = q;
-                slam[q] = sdl[sorg[q]] + stau[q];
+        }
+        return;
+    }
+    const double bt = ee[m - 1], rho = 2.0 * fabs(bt);
+    if (tid < K) {
+        const int j = lo + tid;
+        sD[tid] = lam_in[j];
+        sz[tid] = (j < m ? Z[(m - 1) + (long)j * n]
+                         : (bt >= 0.0 ? 1.0 : -1.0) * Z[m + (long)j * n]) * M_SQRT1_2;
+        sflag[tid] = 0;
+    }
+    __syncthreads();
+    {
+        constexpr int LP = 16 * L / S > 8 ? 8 : 16 * L / S;
+        const int j = tid / LP, sub = tid & (LP - 1);
+        if (j < K) {
+            const double dj = sD[j];
+            int pos = 0;
+#pragma unroll 8
+            for (int q = sub; q < K; q += LP) {
+                const double dq = sD[q];
+                pos += (dq < dj) || (dq == dj && q < j);
             }
-            __syncthreads();
-            // Um in LDS (ld n), row r = Z column r
-            double *um = lds;
-            {
-                const int i = tid >> 3, sub = tid & 7;
-                if (i < Kn) {
-                    const double li = sdl[sorg[i]], ti = stau[i];
-                    double ss = 0.0;
-                    for (int q = sub; q < Kn; q += 8) {
-                        const double u = szh[q] * rcp_nr((sdl[q] - li) - ti);
-                        ss = fma(u, u, ss);
-                    }
-                    ss = oct_sum(ss);
-                    const double iv = 1.0 / sqrt(ss);
-                    for (int r = sub; r < n; r += 8) {
-                        const int q = spos[r];
-                        um[r + i * n] = (q < Kn) ? szh[q] * rcp_nr((sdl[q] - li) - ti) * iv : 0.0;
-                    }
-                } else if (i < n) {
-                    const int j = scm[i];
-                    for (int r = sub; r < n; r += 8) um[r + i * n] = (r == j) ? 1.0 : 0.0;
+            pos = (int)grp_sum<LP>((double)pos);
+            if (sub == 0) sperm[pos] = j;
+        }
+    }
+    __syncthreads();
+    if (tid < 64) {
+        int Kn = 0, nrot = 0;
+        if (rho != 0.0)
+            deflate<(S > 64)>(64, tid, 0, K, rho, sperm, sz, sD, snd, sdl, szl, ra, rb, rc, rs, Kn,
+                              nrot);
+        if (tid == 0) {
+            s_kn = Kn;
+            s_nrot = nrot;
+        }
+    }
+    __syncthreads();
+    const int Kn = s_kn;
+    const int i = 16 * g + tid / L, sub = tid & (L - 1);
+    if (i < Kn) {
+        int org, it;
+        double tau;
+        secular_root<L, S / L>(i, Kn, sub, rho, sdl, szl, org, tau, it);
+        if (sub == 0) {
+            st.dorg[lo + i] = sdl[org];
+            st.tau[lo + i] = tau;
+            lam_out[lo + snd[i]] = sdl[org] + tau;
+            if (it > 0) atomicMax(st.iters + 4, it);
+        }
+    }
+    if (g != 0) return;
+    if (tid < Kn) sflag[snd[tid]] = 1;
+    __syncthreads();
+    if (tid < K && !sflag[tid]) lam_out[lo + tid] = sD[tid];
+    if (tid < Kn) {
+        st.dl[lo + tid] = sdl[tid];
+        st.zl[lo + tid] = szl[tid];
+        st.snd[lo + tid] = snd[tid];
+    }
+    if (tid < s_nrot) {
+        st.ra[lo + tid] = ra[tid];
+        st.rb[lo + tid] = rb[tid];
+        st.rc[lo + tid] = rc[tid];
+        st.rs[lo + tid] = rs[tid];
+    }
+    if (tid == 0) {
+        st.rho[b] = rho;
+        st.kn[b] = Kn;
+        st.nrot[b] = s_nrot;
+    }
+}
+
+// Second half, of a merge below the top: workgroup g of a block forms the new
+// columns of Z at roots 16 g .. 16 g + 15 and copies the deflated ones among the
+// block's columns 16 g .. 16 g + 15, from Zin into Zout (whole columns, zero
+// outside the block).
+template <int S>
+__global__ __launch_bounds__(256) void k_dc_vecs(int n, int s, const double *__restrict__ Zin,
+                                                 double *__restrict__ Zout, DcState st) {
+    static_assert(S == 64, "a wave per 16 rows of the block");
+    constexpr int LD = S + 1;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int gpb = (s + 15) >> 4, b = blockIdx.x / gpb, g = blockIdx.x - b * gpb;
+    const int lo = b * s, hi = min(lo + s, n), K = hi - lo;
+    __shared__ double Zs[S * LD];      // Zs[r + LD j]
+    __shared__ double us[S * 17];      // U[q][c] of the 16 own columns
+    __shared__ double sdl[S], szl[S], stau[S], sdo[S], szh[S], sinv[16], rc[S], rs[S];
+    __shared__ int snd[S], sflag[S], ra[S], rb[S];
+    const int Kn = max(st.kn[b], 0), nrot = Kn > 0 || st.kn[b] == 0 ? st.nrot[b] : 0;
+    const double rho = Kn > 0 ? st.rho[b] : 0.0;
+    {
+        double z[S / 4];
+#pragma unroll
+        for (int t = 0; t < S / 4; t++) {
+            const int j = wv + 4 * t;
+            z[t] = (lane < K && j < K) ? Zin[lo + lane + (long)(lo + j) * n] : 0.0;
+        }
+#pragma unroll
+        for (int t = 0; t < S / 4; t++) Zs[lane + LD * (wv + 4 * t)] = z[t];
+    }
+    if (tid < S) sflag[tid] = 0;
+    if (tid < Kn) {
+        sdl[tid] = st.dl[lo + tid];
+        szl[tid] = st.zl[lo + tid];
+        stau[tid] = st.tau[lo + tid];
+        snd[tid] = st.snd[lo + tid];
+        sdo[tid] = st.dorg[lo + tid];
+    }
+    if (tid < nrot) {
+        ra[tid] = st.ra[lo + tid];
+        rb[tid] = st.rb[lo + tid];
+        rc[tid] = st.rc[lo + tid];
+        rs[tid] = st.rs[lo + tid];
+    }
+    __syncthreads();
+    if (tid < Kn) sflag[snd[tid]] = 1;
+    if (tid >= 128 && tid < 128 + K) {  // the deflating rotations, a thread a row
+        const int r = tid - 128;
+        for (int t = 0; t < nrot; t++) {
+            const int ia = r + LD * ra[t], ib = r + LD * rb[t];
+            const double qa = Zs[ia], qb = Zs[ib], c = rc[t], sn = rs[t];
+            Zs[ia] = c * qa + sn * qb;
+            Zs[ib] = c * qb - sn * qa;
+        }
+    }
+    {
+        const int q = tid >> 2, sub = tid & 3;
+        if (q < Kn) {
+            const double z = zhat_entry<4>(q, Kn, sub, rho, sdl, sdo, stau, szl[q]);
+            if (sub == 0) szh[q] = z;
+        }
+    }
+    __syncthreads();
+    for (int e = tid; e < S * 16; e += 256) {
+        const int q = e >> 4, c = e & 15, i = 16 * g + c;
+        us[q * 17 + c] = (q < Kn && i < Kn)
+                             ? szh[q] * rcp_nr((sdl[q] - sdo[i]) - stau[i]) : 0.0;
+    }
+    __syncthreads();
+    {
+        const int c = tid >> 4, sub = tid & 15;
+        double ss = 0.0;
+#pragma unroll
+        for (int m = 0; m < S / 16; m++) {
+            const double u = us[(sub + 16 * m) * 17 + c];
+            ss = fma(u, u, ss);
+        }
+        ss = grp_sum<16>(ss);
+        if (sub == 0) sinv[c] = 16 * g + c < Kn ? 1.0 / sqrt(ss) : 0.0;
+    }
+    __syncthreads();
+    f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+    for (int k0 = 0; k0 < Kn; k0 += 4) {
+        const int q = k0 + (lane >> 4);
+        const bool kin = q < Kn;
+        const double ua = us[q * 17 + (lane & 15)];  // zero beyond Kn
+        const double zb = kin ? Zs[16 * wv + (lane & 15) + LD * snd[kin ? q : 0]] : 0.0;
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(ua, zb, acc, 0, 0, 0);
+    }
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const int c = (lane >> 4) + 4 * v, i = 16 * g + c, r = 16 * wv + (lane & 15);
+        if (i < Kn && r < K) Zout[lo + r + (long)(lo + snd[i]) * n] = acc[v] * sinv[c];
+    }
+    // deflated columns, and the zeros outside the block of every column written
+    for (int c = wv; c < 16; c += 4) {
+        const int i = 16 * g + c;
+        if (i < K && !sflag[i] && lane < K) Zout[lo + lane + (long)(lo + i) * n] = Zs[lane + LD * i];
+        for (int r = lane; r < n; r += 64)
+            if (r < lo || r >= hi) {
+                if (i < Kn) Zout[r + (long)(lo + snd[i]) * n] = 0.0;
+                if (i < K && !sflag[i]) Zout[r + (long)(lo + i) * n] = 0.0;
+            }
+    }
+}
+
+// Second half, of the top merge: workgroup g < ceil(n/16) forms columns 16 g ..
+// of Um; the last one orders the eigenvalues (lam, by Z column) and decides.
+template <int S>
+__global__ __launch_bounds__(256) void k_dc_top(int n, DcState st, const double *__restrict__ lam,
+                                                const int *__restrict__ eexp,
+                                                double *__restrict__ Um, int *__restrict__ colidx,
+                                                double *__restrict__ sig, int *__restrict__ iout,
+                                                double *__restrict__ dinfo, double delta, int cap,
+                                                double budget) {
+    constexpr int LD = S + 1;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int g = blockIdx.x;
+    __shared__ double um[16 * LD];  // own columns, um[r + LD c]
+    __shared__ double sdl[S], szl[S], stau[S], sdo[S], szh[S], slam[S], rc[S], rs[S];
+    __shared__ int snd[S], sflag[S], spos[S], scm[S], ra[S], rb[S];
+    const int Kn = max(st.kn[0], 0), nrot = st.nrot[0];
+    if (tid < n) sflag[tid] = 0;
+    if (tid < Kn) {
+        sdl[tid] = st.dl[tid];
+        szl[tid] = st.zl[tid];
+        stau[tid] = st.tau[tid];
+        snd[tid] = st.snd[tid];
+        sdo[tid] = st.dorg[tid];
+    }
+    if (tid < nrot) {
+        ra[tid] = st.ra[tid];
+        rb[tid] = st.rb[tid];
+        rc[tid] = st.rc[tid];
+        rs[tid] = st.rs[tid];
+    }
+    __syncthreads();
+    if (tid < Kn) {
+        sflag[snd[tid]] = 1;
+        scm[tid] = snd[tid];
+        spos[snd[tid]] = tid;
+    }
+    __syncthreads();
+    // column c's pole: Z column scm[c]; Z column j's column: spos[j]
+    if (tid < n && !sflag[tid]) {
+        int pos = Kn;
+#pragma unroll 8
+        for (int q = 0; q < tid; q++) pos += !sflag[q];
+        scm[pos] = tid;
+        spos[tid] = pos;
+    }
+    if (g + 1 < (int)gridDim.x) {
+        const double rho = Kn > 0 ? st.rho[0] : 0.0;
+        constexpr int LP = 256 / S > 8 ? 8 : 256 / S;
+        const int q = tid / LP, sub = tid & (LP - 1);
+        if (q < Kn) {
+            const double z = zhat_entry<LP>(q, Kn, sub, rho, sdl, sdo, stau, szl[q]);
+            if (sub == 0) szh[q] = z;
+        }
+        __syncthreads();
+        {
+            const int c = tid >> 4, sb = tid & 15, i = 16 * g + c;
+            if (i < Kn) {
+                const double li = sdo[i], ti = stau[i];
+                double u[S / 16 > 0 ? S / 16 : 1];
+                double ss = 0.0;
+#pragma unroll
+                for (int m = 0; m < S / 16; m++) {
+                    const int r = sb + 16 * m;
+                    const int p = r < n ? spos[r] : S;
+                    u[m] = p < Kn ? szh[p] * rcp_nr((sdl[p] - li) - ti) : 0.0;
+                    ss = fma(u[m], u[m], ss);
                 }
+                ss = grp_sum<16>(ss);
+                const double iv = 1.0 / sqrt(ss);
+#pragma unroll
+                for (int m = 0; m < S / 16; m++) um[sb + 16 * m + LD * c] = u[m] * iv;
+            } else if (i < n) {
+                const int j = scm[i];
+#pragma unroll
+                for (int m = 0; m < S / 16; m++) um[sb + 16 * m + LD * c] = (sb + 16 * m == j) ? 1.0 : 0.0;
             }
-            __syncthreads();
-            // Z G_0 ... G_{k-1} Um = Z (G_0 (... (G_{k-1} Um))): each rotation
-            // of Z's columns (a, b) acts on Um's rows a and b, last first
-            const int nrot = sNrot[0];
-            for (int i = tid; i < n && nrot > 0; i += NT) {
-                double *col = um + i * n;
+        }
+        __syncthreads();
+        // Z G_0 ... G_{k-1} Um = Z (G_0 (... (G_{k-1} Um))): each rotation
+        // of Z's columns (a, b) acts on Um's rows a and b, last first
+        if (nrot > 0) {
+            if (tid < 16 && 16 * g + tid < n) {
+                double *col = um + LD * tid;
                 for (int t = nrot - 1; t >= 0; t--) {
                     const int a = ra[t], b = rb[t];
                     const double c = rc[t], sn = rs[t];
@@ -1046,41 +1195,29 @@ __global__ __launch_bounds__(8 * NMAX) void k_stedc(
                 }
             }
             __syncthreads();
-            for (int e = tid; e < n * n; e += NT) Um[e] = um[e];
-            top_done = true;
-            __syncthreads();
-            break;
         }
-    }
-    if (part == 1) {
-        // the poles after the lower merges and their iteration count
-        __syncthreads();
-        for (int i = tid; i < n; i += NT) dsave[i] = sD[i];
-        if (tid == 0) dsave[n] = (double)s_iters;
+        for (int c = wv; c < 16; c += 4)
+            for (int r = lane; r < n; r += 64)
+                if (16 * g + c < n) Um[r + (long)(16 * g + c) * n] = um[r + LD * c];
         return;
     }
-    if (!top_done) {
-        // n == 1: no merge at all
-        for (int j = tid; j < n; j += NT) {
-            colmap[j] = j;
-            slam[j] = sD[j];
-            Um[j + (long)j * n] = 1.0;
-        }
-        __syncthreads();
-    }
+    __syncthreads();
     // final order (descending), dropped tail, numerical rank, tail rule
-    __shared__ int s_keep;
+    if (tid < n) slam[tid] = lam[scm[tid]];
+    __syncthreads();
     {
-        // rank of column c in descending order, eight lanes per column
-        const int c = tid >> 3, sub = tid & 7;
+        // rank of column c in descending order
+        constexpr int LP = 256 / S > 8 ? 8 : 256 / S;
+        const int c = tid / LP, sub = tid & (LP - 1);
         if (c < n) {
             const double lc = slam[c];
             int pos = 0;
-            for (int q = sub; q < n; q += 8) {
+#pragma unroll 8
+            for (int q = sub; q < n; q += LP) {
                 const double lq = slam[q];
                 pos += (lq > lc) || (lq == lc && q < c);
             }
-            pos = (int)oct_sum((double)pos);
+            pos = (int)grp_sum<LP>((double)pos);
             if (sub == 0) {
                 colidx[pos] = c;
                 sdl[pos] = lc;  // sdl reused: eigenvalues in descending order (scaled)
@@ -1100,17 +1237,18 @@ __global__ __launch_bounds__(8 * NMAX) void k_stedc(
     //    the tail T(q) over [q, numrank) shrinking as q grows.
     // The suffix sums are wave scans; the least q of each rule is the first
     // set bit of a ballot.
+    __shared__ int s_keep;
     if (wv == 0) {
         const bool in0 = lane < n, in1 = lane + 64 < n;
-        const double h0 = in0 ? fmax(sdl[lane], 0.0) : 0.0;
-        const double h1 = in1 ? fmax(sdl[lane + 64 < NMAX ? lane + 64 : 0], 0.0) : 0.0;
+        const double h0 = in0 ? fmax(sdl[lane < S ? lane : 0], 0.0) : 0.0;
+        const double h1 = in1 ? fmax(sdl[lane + 64 < S ? lane + 64 : 0], 0.0) : 0.0;
         const double lmax = readlane_d(h0, 0);
         const double lim = budget * lmax;
         const double S1 = suffix_sum(h1);
         const double S0 = suffix_sum(h0) + readlane_d(S1, 0);
-        const unsigned long long b0 = __ballot(in0 && S0 <= lim && h0 < lmax);
-        const unsigned long long b1 = __ballot(in1 && S1 <= lim && h1 < lmax);
-        const int keep = b0 ? __ffsll((long long)b0) - 1 : (b1 ? 63 + __ffsll((long long)b1) : n);
+        const unsigned long long k0 = __ballot(in0 && S0 <= lim && h0 < lmax);
+        const unsigned long long k1 = __ballot(in1 && S1 <= lim && h1 < lmax);
+        const int keep = k0 ? __ffsll((long long)k0) - 1 : (k1 ? 63 + __ffsll((long long)k1) : n);
         const double cum = (keep >= n) ? 0.0 : (keep < 64 ? readlane_d(S0, keep) : readlane_d(S1, keep - 64));
         const double thr2 = (double)n * EPSU * EPSU * lmax;  // (sqrt(n) u sigma_0)^2
         int numrank = 0;
@@ -1128,16 +1266,18 @@ __global__ __launch_bounds__(8 * NMAX) void k_stedc(
         if (rho > cap) rho = cap;
         if (rho < 1) rho = 1;
         if (lane == 0) {
+            int it = st.iters[4];
+            for (int q = 0; 32 * q < n; q++) it = max(it, st.iters[q]);
             iout[0] = numrank;
             iout[1] = rho;
-            iout[2] = s_iters;
+            iout[2] = it;
             dinfo[5] = ldexp(cum, es);
             s_keep = keep;
         }
     }
     __syncthreads();
     const int keep = s_keep;
-    for (int q = tid; q < n; q += NT) sig[q] = (q < keep) ? ldexp(sqrt(fmax(sdl[q], 0.0)), es / 2) : 0.0;
+    if (tid < n) sig[tid] = (tid < keep) ? ldexp(sqrt(fmax(sdl[tid], 0.0)), es / 2) : 0.0;
 }
 
 // ---- 3. back transformation -----------------------------------------------
@@ -1233,65 +1373,90 @@ void launch_ormtr(int c, const double *Vh, const double *tau, const double *Z, d
                   dim3(256), ((size_t)c * c + c) * sizeof(double), c, Vh, tau, Z, W);
 }
 
-// Tridiagonalisation, divide and conquer and back transformation, W = Q Z.
-// With the side stream on, the back transformation runs there beside the
-// top merge (the merges below it leave Z final); the main stream waits for
-// it before returning.
-template <int NMAX>
-void launch_syev(int c, const double *G, double *Vh, double *tau, double *d, double *e, int *ex,
-                 double *Z, double *Um, double *W, int *colmap, int *colidx, double *sig,
-                 int *iout, double *dinfo, double delta, int cap, double budget, double *dsave) {
-    static bool attr = false;
-    if (!attr) {
-        HIPCHECK(hipFuncSetAttribute((const void *)k_stedc<NMAX>,
-                                     hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     NMAX * NMAX * (int)sizeof(double)));
-        attr = true;
-    }
-    ormtr_attr();
-    const double cc = (double)c;
-    const size_t shm = (size_t)NMAX * NMAX * sizeof(double);
-    PTT_LAUNCH_FB("syev_sytrd", 4.0 * cc * cc * cc / 3.0, 8.0 * cc * cc * 2.0, k_sytrd<NMAX>,
-                  dim3(1), dim3(4 * NMAX + 64), 0, c, G, (long)c, Vh, tau, d, e, ex, dinfo);
-    if (!ptt_hip_side_enabled()) {
-        PTT_LAUNCH_FB("syev_stedc", 2.0 * cc * cc * cc / 3.0, 8.0 * cc * cc * 3.0, k_stedc<NMAX>,
-                      dim3(1), dim3(8 * NMAX), shm, c, d, e, ex, Z, Um, colmap, colidx, sig, iout,
-                      dinfo, delta, cap, budget, 0, dsave);
-        launch_ormtr(c, Vh, tau, Z, W);
-        return;
-    }
-    PTT_LAUNCH_FB("syev_stedc", cc * cc * cc / 3.0, 8.0 * cc * cc * 2.0, k_stedc<NMAX>, dim3(1),
-                  dim3(8 * NMAX), shm, c, d, e, ex, Z, Um, colmap, colidx, sig, iout, dinfo,
-                  delta, cap, budget, 1, dsave);
-    ptt_hip_side_begin();
-    launch_ormtr(c, Vh, tau, Z, W);
-    ptt_hip_side_end(0);
-    PTT_LAUNCH_FB("syev_stedc_top", cc * cc * cc / 3.0, 8.0 * cc * cc * 2.0, k_stedc<NMAX>,
-                  dim3(1), dim3(8 * NMAX), shm, c, d, e, ex, Z, Um, colmap, colidx, sig, iout,
-                  dinfo, delta, cap, budget, 2, dsave);
-    ptt_hip_side_wait(0);
+// Workspace of one eigen-decomposition of order c: reflectors, Z twice (a merge
+// below the top reads one and writes the other), the top update's matrix and the
+// back-transformed vectors (c x c each), then tau, d, e, the poles twice and the
+// state between a merge's launches.
+constexpr size_t syev_ws_doubles(size_t c) { return 5 * c * c + 13 * c + 64; }
+
+// Top merge and decisions (n <= S).
+template <int S>
+void launch_top(int n, int s, const double *e, const double *Z, const double *lam, double *lam2,
+                const DcState &st, const int *ex, double *Um, int *colidx, double *sig, int *iout,
+                double *dinfo, double delta, int cap, double budget) {
+    constexpr int L = S > 64 ? 32 : 16;
+    const double nn = (double)n;
+    PTT_LAUNCH_FB("syev_roots", 60.0 * nn * nn, 8.0 * 4.0 * nn, (k_dc_roots<S, L>),
+                  dim3(cdiv(s, 16)), dim3(16 * L), 0, n, s, e, Z, lam, lam2, st);
+    PTT_LAUNCH_FB("syev_top", 10.0 * nn * nn, 8.0 * nn * nn, k_dc_top<S>, dim3(cdiv(n, 16) + 1),
+                  dim3(256), 0, n, st, lam2, ex, Um, colidx, sig, iout, dinfo, delta, cap, budget);
 }
 
-// Workspace of one eigen-decomposition of order c: reflectors, divide and
-// conquer vectors, the top update's matrix, the back-transformed vectors
-// (c x c each), then tau, d, e, two int vectors and the c + 1 doubles that
-// pass the divide and conquer's state to its top merge.
-constexpr size_t syev_ws_doubles(size_t c) { return 4 * c * c + 8 * c + 8; }
-
+// Tridiagonalisation, divide and conquer, back transformation W = Q Z, and
+// U = W Um.  With the side stream on, the back transformation runs there beside
+// the top merge (the merges below it leave Z final); the main stream waits for
+// it before the product.
 void syev_run(int c, const double *G, double *sig, double *U, long ldu, int *colidx, int *iout,
               double *dinfo, double delta, int cap, double budget, double *ws) {
     const size_t cc = (size_t)c * c;
-    double *Vh = ws, *Z = Vh + cc, *Um = Z + cc, *W = Um + cc;
-    double *tau = W + cc, *d = tau + c, *e = d + c;
-    int *colmap = (int *)(e + c);
-    int *ex = colmap + c;
-    double *dsave = (double *)(colmap + 2 * (size_t)c);  // c + 1 doubles
+    double *Vh = ws, *Z = Vh + cc, *Z2 = Z + cc, *Um = Z2 + cc, *W = Um + cc;
+    double *tau = W + cc, *d = tau + c, *e = d + c, *lam = e + c, *lam2 = lam + c;
+    DcState st;
+    st.dl = lam2 + c;
+    st.zl = st.dl + c;
+    st.tau = st.zl + c;
+    st.dorg = st.tau + c;
+    st.rc = st.dorg + c;
+    st.rs = st.rc + c;
+    st.rho = st.rs + c;  // up to 4 blocks
+    st.snd = (int *)(st.rho + 4);
+    st.ra = st.snd + c;
+    st.rb = st.ra + c;
+    st.kn = st.rb + c;
+    st.nrot = st.kn + 4;
+    st.iters = st.nrot + 4;  // one per leaf workgroup (4), then the larger merges'
+    int *ex = st.iters + 8;
+    ormtr_attr();
+    const double n = (double)c;
     if (c <= 64)
-        launch_syev<64>(c, G, Vh, tau, d, e, ex, Z, Um, W, colmap, colidx, sig, iout, dinfo,
-                        delta, cap, budget, dsave);
+        PTT_LAUNCH_FB("syev_sytrd", 4.0 * n * n * n / 3.0, 8.0 * n * n * 2.0, k_sytrd<64>, dim3(1),
+                      dim3(4 * 64 + 64), 0, c, G, (long)c, Vh, tau, d, e, ex, dinfo);
     else
-        launch_syev<128>(c, G, Vh, tau, d, e, ex, Z, Um, W, colmap, colidx, sig, iout, dinfo,
-                         delta, cap, budget, dsave);
+        PTT_LAUNCH_FB("syev_sytrd", 4.0 * n * n * n / 3.0, 8.0 * n * n * 2.0, k_sytrd<128>, dim3(1),
+                      dim3(4 * 128 + 64), 0, c, G, (long)c, Vh, tau, d, e, ex, dinfo);
+    int top = 2;
+    while (top < c) top *= 2;
+    PTT_LAUNCH_FB("syev_leaf", 2.0 * 32.0 * 32.0 * n, 8.0 * n * n, k_dc_leaf, dim3(cdiv(c, DCL)),
+                  dim3(256), 0, c, d, e, Z, lam, top / 2 < DCL ? top / 2 : DCL, st.iters);
+    if (top == 128) {  // the two blocks of 64
+        PTT_LAUNCH_FB("syev_roots", 60.0 * 64.0 * n, 8.0 * 4.0 * n, (k_dc_roots<64, 16>), dim3(2 * 4),
+                      dim3(256), 0, c, 64, e, Z, lam, lam2, st);
+        PTT_LAUNCH_FB("syev_vecs", 2.0 * 64.0 * 64.0 * n, 8.0 * 2.0 * n * n, k_dc_vecs<64>,
+                      dim3(2 * 4), dim3(256), 0, c, 64, Z, Z2, st);
+        double *t = Z;
+        Z = Z2;
+        Z2 = t;
+        t = lam;
+        lam = lam2;
+        lam2 = t;
+    }
+    const bool side = ptt_hip_side_enabled();
+    if (side) {
+        ptt_hip_side_begin();
+        launch_ormtr(c, Vh, tau, Z, W);
+        ptt_hip_side_end(0);
+    }
+    if (top == 128)
+        launch_top<128>(c, top, e, Z, lam, lam2, st, ex, Um, colidx, sig, iout, dinfo, delta, cap,
+                        budget);
+    else if (top == 64)
+        launch_top<64>(c, top, e, Z, lam, lam2, st, ex, Um, colidx, sig, iout, dinfo, delta, cap,
+                       budget);
+    else
+        launch_top<32>(c, top, e, Z, lam, lam2, st, ex, Um, colidx, sig, iout, dinfo, delta, cap,
+                       budget);
+    if (side) ptt_hip_side_wait(0);
+    else launch_ormtr(c, Vh, tau, Z, W);
     ptt_hip_dgemm('N', 'N', c, c, c, 1.0, W, c, Um, c, 0.0, U, ldu);
 }
 
