@@ -124,5 +124,41 @@ __device__ __forceinline__ double wave_sum(double x) {
     x = xor16_sum(x);
     return xor32_sum(x);
 }
+// Value of lane N of each row of 16 lanes, on all of them.
+template <int N>
+__device__ __forceinline__ double row_bcast(double v) {
+    return __longlong_as_double(
+        __builtin_amdgcn_update_dpp(0LL, __double_as_longlong(v), 0x150 + N, 0xF, 0xF, true));
+}
+__device__ __forceinline__ double row16_sum(double x) {
+    x = quad_sum(x);
+    x += dppd<0x141>(x);
+    return x + dppd<0x140>(x);
+}
+// Largest over the 64 lanes of a wave, the way of wave_sum.
+__device__ __forceinline__ double wave_max(double x) {
+    x = fmax(x, dppd<0xB1>(x));
+    x = fmax(x, dppd<0x4E>(x));
+    x = fmax(x, dppd<0x141>(x));
+    x = fmax(x, dppd<0x140>(x));
+    {
+        const int lo = __double2loint(x), hi = __double2hiint(x);
+        const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+        const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+        x = fmax(__hiloint2double(h[0], l[0]), __hiloint2double(h[1], l[1]));
+    }
+    const int lo = __double2loint(x), hi = __double2hiint(x);
+    const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+    return fmax(__hiloint2double(h[0], l[0]), __hiloint2double(h[1], l[1]));
+}
+
+// Workgroup barrier that orders LDS traffic only: outstanding global stores
+// do not hold the barrier.
+__device__ __forceinline__ void lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
 
 }  // namespace ptt

@@ -31,18 +31,6 @@ constexpr int SVD_ONE_WG_MAX = 56;
 constexpr int SVD_NT = 1024;  // Jacobi SVD workgroup: at most 16 waves, four per SIMD
 constexpr int SVD_RV = 8;     // rows per lane held in registers by a Jacobi pair
 
-// Work matrix S is stored ROW-major in LDS (S[i*c + k] = entry (i,k)) so the
-// pivot row read by every thread in the trailing update is contiguous and
-// each thread's own entries are consecutive across lanes: no bank conflicts.
-// Largest D_j^2 (the Gram's largest diagonal entry, as the factor saw it):
-// reported in dinfo[3] so that callers can tell a Gram whose entries left
-// FP64's range (squares of core entries below ~2^-450 or above 2^450).
-__device__ double max_sq(const double *D, int c) {
-    double m = 0.0;
-    for (int j = 0; j < c; j++) m = fmax(m, D[j] * D[j]);
-    return m;
-}
-
 // ---- factors of more than 128 columns ----------------------------------------
 // Blocks of 128 columns: the scaled Gram (k_chol_scale) is factored block row by
 // block row, the diagonal block by k_chol_blk (with its inverse), the rest of
@@ -226,714 +214,449 @@ __global__ __launch_bounds__(NT) void k_chol_report(int c, const double *__restr
     }
 }
 
-// Low-latency variant for c <= CMAX <= 128 (the whole problem in LDS, the
-// trailing matrix of the elimination in registers, one barrier per
-// elimination step).  With WT the elimination also carries the identity
-// ([S | I] -> [U | L^-1], S = L U, U = diag(p) L^T), which gives the inverse
-// of the scaled factor without a separate triangular inversion:
-// Rs = diag(sqrt p) L^T, so Ts = Rs^-1 = L^-T diag(1/sqrt p).  A dead pivot
-// skips its step, which leaves row and column j of Ts zero.  Ts(i,k) for
-// i < k is kept transposed in the lower triangle of S, its diagonal in tdg.
-// NTH threads (64, 256 or 512, chosen for c).
-constexpr int CHOL_FAST_C = 128;
-constexpr int CHOL_BLK = 32;
-constexpr int CHOL_LDS_DOUBLES = 20400;  // c(c+1) + 5c + 3*32*32 = 20224 at c = 128; 159.4 KB
-
-template <int NTH, int CMAX, bool WT>
-__global__ __launch_bounds__(NTH) void k_chol_fast(int c, const double *__restrict__ G,
-                                                   double shift, double tiny,
-                                                   double *__restrict__ R, double *__restrict__ T,
-                                                   int *info, double *dinfo, int want_kappa) {
-    extern __shared__ double lds[];
-    const int tid = threadIdx.x;
-    constexpr int nth = NTH;
-    // c x c row-major with an odd row stride: column-wise walks (stride ldS)
-    // fall in distinct LDS banks
-    const int ldS = c | 1;
-    double *S = lds;
-    double *D = S + (long)c * ldS;  // Jacobi scaling
-    double *tdg = D + c;          // raw pivots, then the diagonal of Ts
-    double *dd = tdg + c;         // deficient flags
-    double *pv = dd + c;          // power-iteration vectors (2c)
-    double *Y = pv + 2 * c;       // 3 blocks of 32 x 32 (blocked inverse)
-    __shared__ int s_def;
-    __shared__ double s_red[2 * (NT / 64)];
-
-    auto block_sum2 = [&](double &a, double &b) {
-        for (int o = 32; o > 0; o >>= 1) {
-            a += __shfl_xor(a, o);
-            b += __shfl_xor(b, o);
-        }
-        __syncthreads();
-        if ((tid & 63) == 0) {
-            s_red[2 * (tid >> 6)] = a;
-            s_red[2 * (tid >> 6) + 1] = b;
-        }
-        __syncthreads();
-        a = 0.0;
-        b = 0.0;
-        for (int i = 0; i < nth / 64; i++) {
-            a += s_red[2 * i];
-            b += s_red[2 * i + 1];
-        }
-    };
-
-    for (int j = tid; j < c; j += nth) {
-        double g = G[j + (long)j * c];
-        D[j] = g > 0.0 ? sqrt(g) : 0.0;
-    }
-    // half-wave hw of 32 lanes (lane hl); H half-waves in the workgroup
-    constexpr int H = NTH / 32;
-    const int hw = tid >> 5, hl = tid & 31;
-    __syncthreads();
-    for (int i = hw; i < c; i += H) {
-        const double di = D[i];
-        for (int k = hl; k < c; k += 32) {
-            const double dk = D[k];
-            S[i * ldS + k] = (di > 0.0 && dk > 0.0) ? G[k + (long)i * c] / (di * dk) : 0.0;
-        }
-    }
-    // start vector of the power iterations, unit length
-    double nrm0 = 0.0;
-    for (int i = 0; i < c; i++) nrm0 += (1.0 + 0.01 * (i % 7)) * (1.0 + 0.01 * (i % 7));
-    nrm0 = 1.0 / sqrt(nrm0);
-    for (int i = tid; i < c; i += nth) pv[i] = (1.0 + 0.01 * (i % 7)) * nrm0;
-    // S and pv are read across threads from here on
-    __syncthreads();
-    // Gershgorin certificate: the scaled Gram is I + E; if ||E||_inf = e <
-    // 1/2 then kappa_2(Gram) <= (1+e)/(1-e) and the power iterations are
-    // skipped (the bound is reported instead of the estimate).
-    double eoff = 0.0, dummy0 = 0.0;
-    const int row8 = tid >> 3, sub8 = tid & 7;
-    if (want_kappa) {
-        // row sums of the symmetric S, 8 lanes per row
-        for (int i0 = 0; i0 < c; i0 += nth / 8) {
-            const int i = i0 + row8;
-            double rs = 0.0;
-            if (i < c)
-                for (int l = sub8; l < c; l += 8)
-                    if (l != i) rs += fabs(S[(long)i * ldS + l]);
-            rs += __shfl_xor(rs, 1);
-            rs += __shfl_xor(rs, 2);
-            rs += __shfl_xor(rs, 4);
-            eoff = fmax(eoff, rs);
-        }
-        for (int o = 32; o > 0; o >>= 1) eoff = fmax(eoff, __shfl_xor(eoff, o));
-        __syncthreads();
-        if ((tid & 63) == 0) s_red[tid >> 6] = eoff;
-        __syncthreads();
-        eoff = 0.0;
-        for (int i = 0; i < nth / 64; i++) eoff = fmax(eoff, s_red[i]);
-        __syncthreads();
-    }
-    (void)dummy0;
-    const bool gersh = want_kappa && eoff < 0.5;
-    // The power iterations run after the factorisation, and only when its
-    // pivots leave the answer open: kappa_2 of the scaled Gram is at least
-    // max pivot / min pivot (each pivot lies between lambda_min and
-    // lambda_max), so a dead pivot or a pivot ratio above 1e12 already
-    // decides for the shifted factorisation (condition of the factor > 1e6).
-    double lmax = 0.0;
-    auto power_max = [&](int PIT) {
-    for (int it = 0; it < PIT; it++) {
-        // y = S x with x of unit length: lambda ~ ||y||
-        for (int i0 = 0; i0 < c; i0 += nth / 8) {
-            int i = i0 + row8;
-            double acc = 0.0;
-            if (i < c)
-                for (int l = sub8; l < c; l += 8) acc += S[(long)i * ldS + l] * pv[l];
-            acc += __shfl_xor(acc, 1);
-            acc += __shfl_xor(acc, 2);
-            acc += __shfl_xor(acc, 4);
-            if (i < c && sub8 == 0) pv[c + i] = acc;
-        }
-        __syncthreads();
-        double nn = 0.0, dummy = 0.0;
-        for (int i = tid; i < c; i += nth) nn += pv[c + i] * pv[c + i];
-        block_sum2(nn, dummy);
-        lmax = sqrt(nn);
-        double inv = nn > 0.0 ? 1.0 / lmax : 0.0;
-        for (int i = tid; i < c; i += nth) pv[i] = pv[c + i] * inv;
-        __syncthreads();
-    }
-    };
-    // Cholesky, upper triangle.  Thread (hw, hl) holds S[hw + H s][hl + 32 t]
-    // in registers; at step j the half-wave owning row j publishes it through
-    // a double-buffered LDS row (one barrier per step: the buffer written at
-    // step j + 2 was last read before the barrier of step j + 1).  Rows are
-    // scaled by 1/sqrt(pivot) once all pivots are known.
-    constexpr int SN = (CMAX + H - 1) / H, TN = (CMAX + 31) / 32, RB = 32 * TN;
-    constexpr int NP = WT ? 2 : 1;  // row parts published per step
-    static_assert(H * SN <= RB && 2 * NP * RB <= 3 * CHOL_BLK * CHOL_BLK, "row buffer layout");
-    double a[SN][TN];
-    double e[WT ? SN : 1][WT ? TN : 1];  // rows of L^-1 (identity at the start)
-    if (WT) {
-#pragma unroll
-        for (int s2 = 0; s2 < SN; s2++)
-#pragma unroll
-            for (int t = 0; t < TN; t++) e[s2][t] = (hw + H * s2 == hl + 32 * t) ? 1.0 : 0.0;
-    }
-#pragma unroll
-    for (int s2 = 0; s2 < SN; s2++)
-#pragma unroll
-        for (int t = 0; t < TN; t++) {
-            const int i = hw + H * s2, k = hl + 32 * t;
-            a[s2][t] = (i < c && k < c) ? S[(long)i * ldS + k] : 0.0;
-        }
-    // Y is free until the outputs: two rows of NP * RB doubles.  Every read of a
-    // step is issued at once (indices < RB, values outside the active
-    // triangle are masked), and the deficiency count is kept in a register
-    // (the pivot test is uniform across the workgroup).
-    double *rowbuf = Y;
-    int ndef = 0;
-    for (int j = 0; j < c; j++) {
-        double *rb = rowbuf + (j & 1) * NP * RB;
-        if (hw == j % H) {
-            const int sj = j / H;
-#pragma unroll
-            for (int s2 = 0; s2 < SN; s2++)
-                if (s2 == sj) {
-#pragma unroll
-                    for (int t = 0; t < TN; t++) {
-                        rb[hl + 32 * t] = a[s2][t];
-                        if (WT) rb[RB + hl + 32 * t] = e[WT ? s2 : 0][WT ? t : 0];
-                    }
-                }
-        }
-        __syncthreads();
-        const double pj = rb[j], dj = D[j];
-        double rk[TN], ri[SN], re[TN];
-#pragma unroll
-        for (int t = 0; t < TN; t++) {
-            rk[t] = rb[hl + 32 * t];
-            re[t] = WT ? rb[RB + hl + 32 * t] : 0.0;
-        }
-#pragma unroll
-        for (int s2 = 0; s2 < SN; s2++) ri[s2] = rb[hw + H * s2];
-        const double p = pj + shift;
-        const bool dead = !(dj > 0.0) || !(p > tiny);
-        ndef += dead ? 1 : 0;
-        if (tid == 0) {
-            tdg[j] = dead ? 0.0 : p;
-            dd[j] = dead ? 1.0 : 0.0;
-        }
-        if (!dead) {
-            // Only rows below j change (their multiplier is zero otherwise).
-            // Columns are not masked: entries left of the diagonal or beyond
-            // c never feed the upper triangle, the published row holds finite
-            // values everywhere (zeros beyond c), and row j of L^-1 is
-            // exactly zero beyond column j.
-            // Register blocks with nothing to do are skipped on uniform
-            // tests: row blocks whose rows are all <= j, column blocks of U
-            // entirely at or left of column j, and column blocks of L^-1
-            // entirely right of column j.
-            const double ip = 1.0 / p;
-#pragma unroll
-            for (int s2 = 0; s2 < SN; s2++) {
-                if (H * s2 + H - 1 <= j) continue;
-                const int i = hw + H * s2;
-                const double sji = (i > j) ? ri[s2] * ip : 0.0;
-#pragma unroll
-                for (int t = 0; t < TN; t++) {
-                    if (32 * t + 31 > j) a[s2][t] = a[s2][t] - sji * rk[t];
-                    if (WT && 32 * t <= j)
-                        e[WT ? s2 : 0][WT ? t : 0] = e[WT ? s2 : 0][WT ? t : 0] - sji * re[t];
-                }
-            }
-        }
-    }
-    if (tid == 0) s_def = ndef;
-    __syncthreads();  // every pivot is in tdg
-    double pmax = 0.0, pmin = INFINITY;
-    for (int j = 0; j < c; j++) {
-        const double pj = tdg[j];
-        if (pj > 0.0) {
-            pmax = fmax(pmax, pj);
-            pmin = fmin(pmin, pj);
-        }
-    }
-    const bool decided = (ndef > 0) || !(pmax <= 1e12 * pmin);
-    const int PIT = (want_kappa && !gersh && !decided && WT) ? 6 : 0;
-    power_max(PIT);  // S still holds the scaled Gram (the factor is in registers)
-#pragma unroll
-    for (int s2 = 0; s2 < SN; s2++)
-#pragma unroll
-        for (int t = 0; t < TN; t++) {
-            const int i = hw + H * s2, k = hl + 32 * t;
-            if (i < c && k >= i && k < c) {
-                const double pq = tdg[i];
-                const double rqq = pq > 0.0 ? sqrt(pq) : 0.0;
-                const double iq = pq > 0.0 ? 1.0 / rqq : 0.0;
-                S[(long)i * ldS + k] = (k == i) ? rqq : a[s2][t] * iq;
-            }
-            if (WT && i < c && k < i) {
-                // Ts(k, i) = L^-1(i, k) / sqrt(p_i), stored at S[i * ldS + k]
-                const double pq = tdg[i];
-                const double iq = pq > 0.0 ? 1.0 / sqrt(pq) : 0.0;
-                S[(long)i * ldS + k] = e[WT ? s2 : 0][WT ? t : 0] * iq;
-            }
-        }
-    __syncthreads();
-    if (!WT) {
-        // factor only: R = Rs * D, no inverse and no condition estimate
-        for (int k = hw; k < c; k += H) {
-            const double dk = D[k];
-            for (int i = hl; i < c; i += 32) R[i + (long)k * c] = (i <= k) ? S[i * ldS + k] * dk : 0.0;
-        }
-        if (tid == 0) {
-            dinfo[0] = 0.0;
-            dinfo[1] = 0.0;
-            dinfo[2] = (double)s_def;
-            dinfo[3] = max_sq(D, c);
-        dinfo[3] = max_sq(D, c);
-            info[0] = s_def;
-        }
-        return;
-    }
-    // diagonal of Ts (dead rows and columns are zero)
-    for (int j = tid; j < c; j += nth) tdg[j] = (dd[j] != 0.0) ? 0.0 : 1.0 / S[(long)j * ldS + j];
-    __syncthreads();
-    auto tget = [&](int i, int k) -> double {  // Ts(i,k), i <= k
-        return (i == k) ? tdg[i] : S[(long)k * ldS + i];
-    };
-    // outputs and Frobenius norms
-    double fr = 0.0, ft = 0.0;
-    for (int k = hw; k < c; k += H) {
-        const double dk = D[k];
-        for (int i = hl; i < c; i += 32) {
-            const double rv = (i <= k) ? S[i * ldS + k] : 0.0;
-            const double tv = (i <= k) ? tget(i, k) : 0.0;
-            fr += rv * rv;
-            ft += tv * tv;
-            R[i + (long)k * c] = rv * dk;
-            T[i + (long)k * c] = (D[i] > 0.0) ? tv / D[i] : 0.0;
-        }
-    }
-    block_sum2(fr, ft);
-    // lambda_max(Ts Ts^T) by power iteration
-    for (int i = tid; i < c; i += nth) pv[i] = (1.0 + 0.01 * (i % 7)) * nrm0;
-    __syncthreads();
-    double lminv = 0.0;
-    for (int it = 0; it < PIT; it++) {
-        for (int k0 = 0; k0 < c; k0 += nth / 8) {  // u = Ts^T x
-            int k = k0 + row8;
-            double acc = 0.0;
-            if (k < c)
-                for (int i = sub8; i <= k; i += 8) acc += tget(i, k) * pv[i];
-            acc += __shfl_xor(acc, 1);
-            acc += __shfl_xor(acc, 2);
-            acc += __shfl_xor(acc, 4);
-            if (k < c && sub8 == 0) pv[c + k] = acc;
-        }
-        __syncthreads();
-        for (int i0 = 0; i0 < c; i0 += nth / 8) {  // y = Ts u  (into Y scratch)
-            int i = i0 + row8;
-            double acc = 0.0;
-            if (i < c)
-                for (int k = i + sub8; k < c; k += 8) acc += tget(i, k) * pv[c + k];
-            acc += __shfl_xor(acc, 1);
-            acc += __shfl_xor(acc, 2);
-            acc += __shfl_xor(acc, 4);
-            if (i < c && sub8 == 0) Y[i] = acc;
-        }
-        __syncthreads();
-        double nn = 0.0, dummy = 0.0;
-        for (int i = tid; i < c; i += nth) nn += Y[i] * Y[i];
-        block_sum2(nn, dummy);
-        lminv = sqrt(nn);
-        double inv = nn > 0.0 ? 1.0 / lminv : 0.0;
-        for (int i = tid; i < c; i += nth) pv[i] = Y[i] * inv;
-        __syncthreads();
-    }
-    if (tid == 0) {
-        dinfo[0] = sqrt(fr) * sqrt(ft);
-        // 2-norm condition of Rs = sqrt(kappa_2 of the scaled Gram)
-        dinfo[1] = !want_kappa ? 0.0
-                   : gersh     ? sqrt((1.0 + eoff) / (1.0 - eoff))
-                   : decided   ? ((pmin > 0.0 && pmin < INFINITY) ? sqrt(pmax / pmin) : 0.0)
-                               : sqrt(lmax * lminv);
-        dinfo[2] = (double)s_def;
-        dinfo[3] = max_sq(D, c);
-        info[0] = s_def;
-    }
-}
-
-// ---- blocked Cholesky of a scaled Gram, c <= 128 ---------------------------
-// Same contract as k_chol_fast (scaled Gram S = D^-1 G D^-1 with unit
-// diagonal, shifted pivots, dead pivots skipped, R = Rs D and T = D^-1 Ts,
-// Frobenius and 2-norm condition estimates), organised in panels of 16
-// columns so that the workgroup meets two barriers per panel instead of one
-// per column:
-//   1. wave 0 factors the panel (rows 16P.., 16 columns; two rows per lane)
-//      in LDL^T form: a step needs the pivot, one reciprocal and a rank-one
-//      update of the panel's later columns, whose multipliers come from the
-//      diagonal block's column j, broadcast through 16 LDS slots inside the
-//      wave (no workgroup barrier); the columns are then scaled by
-//      1/sqrt(pivot) into L;
-//   2. the eight waves update the trailing lower triangle by 16 x 16 tiles,
-//      A22 -= L21 L21^T, on the FP64 matrix cores (four 16x16x4 steps a tile).
-// With the inverse wanted, X = L^-1 follows by blocks: each diagonal block is
-// inverted by forward substitution (one lane per column), then wave J forms
-// block column J down the rows, X_IJ = -X_II sum_{K<I} L_IK X_KJ, on the
-// matrix cores; Ts = X^T is kept in the upper triangle of S (the diagonal
-// blocks separately).  S lives in LDS column-major with an odd stride.
-constexpr int CB_LD = 129;
-constexpr int CB_XS = 16 * 17;  // one diagonal block of X, row-major, stride 17
-constexpr int CB_LDS_DOUBLES = 128 * CB_LD + 8 * CB_XS + 6 * 128;  // 19584: 153 KB
+// ---- Cholesky of a scaled Gram, c <= 128, on one workgroup ------------------
+// Scaled Gram S = D^-1 G D^-1 with unit diagonal, shifted pivots, dead pivots
+// skipped, R = Rs D and T = D^-1 Ts, Frobenius and 2-norm condition estimates.
+// Bound by its serial chain (a pivot, a reciprocal, an update, c times over), so
+// everything else is kept off that chain.  NB blocks of 16 columns, a wave each:
+//   1. panel P is factored in LDL^T form by the wave (or two) whose lanes hold
+//      its rows, one row a lane.  Each of them keeps the diagonal block as well,
+//      once in every 16 lanes, so that the pivot and the multipliers come by a
+//      DPP row broadcast: a step has no LDS access and no barrier (through LDS it
+//      took about twice as long).  The columns are scaled by 1/sqrt(pivot) after
+//      the panel, the roots taken by one lane each;
+//   2. A22 -= L21 L21^T by 16 x 16 tiles on the FP64 matrix cores, the next
+//      panel's column of tiles first; the other tiles and the inverse of the
+//      diagonal block run beside the next panel's factorisation.
+//   3. with the inverse wanted, row I of X = L^-1, X_IJ = -X_II sum_{K<I} L_IK
+// X_KJ, on the matrix cores, beside the panel after next; the last two rows
+// after the factorisation.  Ts = X^T is kept in the upper triangle of S (the
+// diagonal blocks separately).  R's rows are written beside the panels too.  S lives in LDS
+// column-major with an odd stride.  The power iterations hold their matrix in
+// registers, 4 rows x NB columns a thread, with one barrier a product.
+// Measured (us, well conditioned / with the iterations; before: column by column
+// with a workgroup barrier a column up to 48, panels through LDS beyond):
+// c = 16: 15 / 31 -> 7 / 12, 32: 20 / 35 -> 12 / 18, 48: 37 / 60 -> 16 / 23,
+// 64: 47 / 70 -> 20 / 27, 128: 96 / 146 -> 39 / 52, of which the panels are 24.
+template <int NB>
+struct chol_geom {
+    static constexpr int N = 16 * NB;            // padded order
+    static constexpr int LD = N + 1;
+    static constexpr int XS = 16 * 17;           // one diagonal block of X, row-major, stride 17
+    static constexpr int LDS_DOUBLES = N * LD + NB * XS + 6 * N;  // 153 KB at NB = 8
+};
 
 typedef double f64x4_t __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ double lane_d(double v, int l) {
-    const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
-    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
-    return __hiloint2double(hi, lo);
+// One panel in registers: dg the diagonal block's row lane % 16, pw the lane's
+// own row, psel the pivot of row lane % 16.  (Forming the next reciprocal between
+// a step's updates made no difference: the updates' issue bounds a step.)
+template <int J, int M>
+__device__ __forceinline__ void chol_update(double (&dg)[16], double (&pw)[16], double w0,
+                                            double w1) {
+    if constexpr (M < 16) {
+        const double um = row_bcast<M>(dg[J]);
+        dg[M] = fma(-w0, um, dg[M]);
+        pw[M] = fma(-w1, um, pw[M]);
+        // formed here, not sunk to its use
+        __asm__ __volatile__("" : "+v"(dg[M]), "+v"(pw[M]));
+        chol_update<J, M + 1>(dg, pw, w0, w1);
+    }
 }
-// 1/x from the hardware reciprocal and two Newton steps (x != 0)
-__device__ __forceinline__ double rcp2(double x) {
-    double r = __builtin_amdgcn_rcp(x);
-    double e = fma(-x, r, 1.0);
-    r = fma(r, e, r);
-    e = fma(-x, r, 1.0);
-    return fma(r, e, r);
+template <int J>
+__device__ __forceinline__ void chol_steps(double (&dg)[16], double (&pw)[16], int r,
+                                           unsigned alive, double shift, double tiny,
+                                           double &psel) {
+    if constexpr (J < 16) {
+        const double p = row_bcast<J>(dg[J]) + shift;
+        const bool live = ((alive >> J) & 1u) && p > tiny;
+        const double ip = live ? rcp_nr(p) : 0.0;
+        if (r == J) psel = live ? p : 0.0;
+        // multipliers (unscaled column / pivot) of the rows below row J
+        const double w0 = r > J ? dg[J] * ip : 0.0, w1 = pw[J] * ip;
+        chol_update<J, J + 1>(dg, pw, w0, w1);
+        chol_steps<J + 1>(dg, pw, r, alive, shift, tiny, psel);
+    }
+}
+template <int M>
+__device__ __forceinline__ void chol_scale_cols(double (&dg)[16], double (&pw)[16], double isq) {
+    if constexpr (M < 16) {
+        const double f = row_bcast<M>(isq);
+        dg[M] *= f;
+        pw[M] *= f;
+        chol_scale_cols<M + 1>(dg, pw, isq);
+    }
+}
+// Inverse of a 16 x 16 lower triangle by columns: lane r of 16 holds row r of it
+// in l and column r of the inverse in x; idg the reciprocal of row r's diagonal.
+template <int K, int I>
+__device__ __forceinline__ void tri_update(const double (&l)[16], double (&x)[16]) {
+    if constexpr (I < 16) {
+        x[I] = fma(-row_bcast<I>(l[K]), x[K], x[I]);
+        __asm__ __volatile__("" : "+v"(x[I]));
+        tri_update<K, I + 1>(l, x);
+    }
+}
+template <int K>
+__device__ __forceinline__ void tri_inverse(const double (&l)[16], double (&x)[16], double idg) {
+    if constexpr (K < 16) {
+        x[K] *= row_bcast<K>(idg);
+        tri_update<K, K + 1>(l, x);
+        tri_inverse<K + 1>(l, x, idg);
+    }
+}
+
+// Tile t of a lower triangle of tiles, row by row.
+__device__ __forceinline__ void tri_tile(int t, int &I, int &J) {
+    I = 0;
+    while ((I + 1) * (I + 2) / 2 <= t) I++;
+    J = t - I * (I + 1) / 2;
 }
 
 // With `unit` the input is already scaled (a diagonal block of a larger scaled
 // Gram, ptt_hip_chol_qr_factor beyond 128 columns): D = 1, pivots are tested as
 // they come.  ldg, ldo: leading dimensions of G and of R and T.
-template <bool WT>
-__global__ __launch_bounds__(512) void k_chol_blk(int c, const double *__restrict__ G, long ldg,
-                                                  double shift, double tiny,
-                                                  double *__restrict__ R, double *__restrict__ T,
-                                                  long ldo, int *info, double *dinfo,
-                                                  int want_kappa, int unit) {
-    constexpr int nth = 512;
+template <int NB, bool WT>
+__global__ __launch_bounds__(64 * NB) void k_chol_blk(int c, const double *__restrict__ G, long ldg,
+                                                      double shift, double tiny,
+                                                      double *__restrict__ R,
+                                                      double *__restrict__ T, long ldo, int *info,
+                                                      double *dinfo, int want_kappa, int unit) {
+    using geom = chol_geom<NB>;
+    constexpr int N = geom::N, LD = geom::LD, XS = geom::XS;
     extern __shared__ double lds[];
-    double *S = lds;                  // 128 x 129, S[i + j * CB_LD]
-    double *Xd = S + 128 * CB_LD;     // diagonal blocks of X = L^-1
-    double *D = Xd + 8 * CB_XS;       // Jacobi scaling
-    double *tdg = D + 128;            // pivots (0 when dead)
-    double *idg = tdg + 128;          // 1 / sqrt(pivot) (0 when dead)
-    double *iD = idg + 128;           // 1 / D (0 where D is)
-    double *pv = iD + 128;            // power-iteration vectors (2 x 128)
-    __shared__ int s_def;
-    __shared__ double s_red[2 * (nth / 64)];
-    __shared__ double ub[16];  // column of the panel's diagonal block
+    double *S = lds;            // N x N, S[i + j * LD]
+    double *Xd = S + N * LD;    // diagonal blocks of X = L^-1
+    double *D = Xd + NB * XS;   // Jacobi scaling
+    double *iD = D + N;         // 1 / D (0 where D is)
+    double *tdg = iD + N;       // pivots (0 when dead)
+    double *idg = tdg + N;      // 1 / sqrt(pivot) (0 when dead)
+    double *pv = idg + N;       // power-iteration vectors (2 x N)
+    __shared__ double s_red[2 * NB];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int li = lane & 15, lg = lane >> 4;
+    // row ti, columns tj, tj + 4, ... of the copies in and out
+    const int ti = tid % N, tj = tid / N;
+    const int npn = (c + 15) >> 4;
 
-    auto block_sum2 = [&](double &a, double &b) {
-        for (int o = 32; o > 0; o >>= 1) {
-            a += __shfl_xor(a, o);
-            b += __shfl_xor(b, o);
+    // S = D^-1 G D^-1 from the lower tiles of G, all loads of a thread in flight
+    // at once (one CU's loads of 128 KB took a tenth of the whole)
+    double eoff = 0.0, dmax = 0.0;
+    {
+        // wave w's tiles: the pairs (w, w + u mod NB), each pair once
+        constexpr int PER = NB / 2 + 1;
+        auto tile = [&](int u, int &I, int &J) {
+            const int o = wv + u < NB ? wv + u : wv + u - NB;
+            I = o > wv ? o : wv;
+            J = o > wv ? wv : o;
+            return 2 * u < NB || wv < NB / 2 || u == 0;
+        };
+        double gv[PER][4];
+#pragma unroll
+        for (int u = 0; u < PER; u++) {
+            int I, J;
+            const bool mine = tile(u, I, J);
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int i = 16 * I + li, j = 16 * J + 4 * q + lg;
+                gv[u][q] = (mine && i < c && j < c) ? G[i + (long)j * ldg] : 0.0;
+            }
+        }
+        if (tid < N) {
+            double dj = 0.0;
+            if (tid < c) {
+                const double g = G[tid + (long)tid * ldg];
+                dj = unit ? 1.0 : g > 0.0 ? sqrt(g) : 0.0;
+            }
+            D[tid] = dj;
+            iD[tid] = dj > 0.0 ? 1.0 / dj : 0.0;
+            tdg[tid] = 0.0;
+            idg[tid] = 0.0;
+            pv[tid] = tid < c ? 1.0 + 0.01 * (tid % 7) : 0.0;
         }
         __syncthreads();
-        if (lane == 0) {
-            s_red[2 * wv] = a;
-            s_red[2 * wv + 1] = b;
+#pragma unroll
+        for (int u = 0; u < PER; u++) {
+            int I, J;
+            if (tile(u, I, J)) {
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const int i = 16 * I + li, j = 16 * J + 4 * q + lg;
+                    const double s = gv[u][q] * iD[i] * iD[j];
+                    S[i + j * LD] = s;
+                    if (I != J) S[j + i * LD] = s;
+                }
+            }
         }
-        __syncthreads();
-        a = 0.0;
-        b = 0.0;
-        for (int i = 0; i < nth / 64; i++) {
-            a += s_red[2 * i];
-            b += s_red[2 * i + 1];
+    }
+    __syncthreads();
+    if (want_kappa) {
+        // row sums of |S - I|, a quarter of the columns a thread
+        double rs = 0.0;
+#pragma unroll 8
+        for (int u = 0; u < 4 * NB; u++) {
+            const int j = tj + 4 * u;
+            rs += j != ti ? fabs(S[ti + j * LD]) : 0.0;
+        }
+        Xd[tj * N + ti] = rs;  // free until the inverse
+        lds_sync();
+        for (int i = lane; i < N; i += 64)
+            eoff = fmax(eoff, (Xd[i] + Xd[N + i]) + (Xd[2 * N + i] + Xd[3 * N + i]));
+    }
+    for (int i = lane; i < N; i += 64) dmax = fmax(dmax, D[i] * D[i]);
+    // Gershgorin certificate: S = I + E with ||E||_inf = e < 1/2 has kappa_2 <=
+    // (1+e)/(1-e), and the power iterations are skipped
+    eoff = wave_max(eoff);
+    dmax = wave_max(dmax);
+    const bool gersh = want_kappa && eoff < 0.5;
+    // y = M x for the N x N matrix whose rows 16 wv + 4 lg + v, columns li + 16 q
+    // a thread holds in m
+    auto matvec = [&](const double (&m)[4][NB], const double *x, double *y) {
+        double xv[NB], s[4];
+#pragma unroll
+        for (int q = 0; q < NB; q++) xv[q] = x[li + 16 * q];
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            s[v] = 0.0;
+#pragma unroll
+            for (int q = 0; q < NB; q++) s[v] = fma(m[v][q], xv[q], s[v]);
+            s[v] = row16_sum(s[v]);
+        }
+        if (li < 4) y[16 * wv + 4 * lg + li] = li == 0 ? s[0] : li == 1 ? s[1] : li == 2 ? s[2] : s[3];
+        lds_sync();
+    };
+    auto norm2 = [&](const double *x) {
+        double s = 0.0;
+        for (int i = lane; i < N; i += 64) s = fma(x[i], x[i], s);
+        return wave_sum(s);
+    };
+    constexpr int PIT = 6;
+    double lmax = 0.0, lminv = 0.0;
+    if (WT && want_kappa && !gersh) {
+        // lambda_max(S) <= c: six products need no scaling in between
+        double m[4][NB];
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+#pragma unroll
+            for (int q = 0; q < NB; q++) m[v][q] = S[(li + 16 * q) + (16 * wv + 4 * lg + v) * LD];
+        for (int it = 0; it < PIT; it++) matvec(m, pv + (it & 1) * N, pv + (~it & 1) * N);
+        lmax = sqrt(norm2(pv) / norm2(pv + N));  // PIT is even: the last product is in pv
+    }
+    lds_sync();
+
+    // A tile (I, J) of the trailing matrix less L_IP L_JP^T
+    auto update_tile = [&](int I, int J, int P) {
+        const int bi = 16 * I, bj = 16 * J;
+        f64x4_t acc;
+#pragma unroll
+        for (int v = 0; v < 4; v++) acc[v] = S[(bi + lg + 4 * v) + (bj + li) * LD];
+#pragma unroll
+        for (int kk = 0; kk < 4; kk++) {
+            const int kc = 16 * P + 4 * kk + lg;
+            const double a = -S[(bi + li) + kc * LD];
+            const double b = S[(bj + li) + kc * LD];
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
+        }
+#pragma unroll
+        for (int v = 0; v < 4; v++) S[(bi + lg + 4 * v) + (bj + li) * LD] = acc[v];
+    };
+    auto invert_diag = [&](int B) {
+        double l[16], x[16];
+#pragma unroll
+        for (int k = 0; k < 16; k++) {
+            l[k] = S[(16 * B + li) + (16 * B + k) * LD];
+            x[k] = k == li ? 1.0 : 0.0;
+        }
+        tri_inverse<0>(l, x, idg[16 * B + li]);
+        if (lane < 16) {
+#pragma unroll
+            for (int i = 0; i < 16; i++) Xd[B * XS + i * 17 + li] = x[i];
         }
     };
 
-    for (int j = tid; j < 128; j += nth) {
-        double dj = 0.0;
-        if (j < c) {
-            const double g = G[j + (long)j * ldg];
-            dj = unit ? 1.0 : g > 0.0 ? sqrt(g) : 0.0;
-        }
-        D[j] = dj;
-        iD[j] = dj > 0.0 ? 1.0 / dj : 0.0;
-    }
-    __syncthreads();
-    // S = D^-1 G D^-1: thread (wave, lane) fills rows lane, lane + 64 of
-    // columns wave, wave + 8, ..., all 32 of its loads in flight at once
-    {
-        double gv[16][2];
-#pragma unroll
-        for (int u = 0; u < 16; u++)
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const int j = wv + u * (nth / 64), i = lane + 64 * h;
-                gv[u][h] = (i < c && j < c) ? G[i + (long)j * ldg] : 0.0;
-            }
-#pragma unroll
-        for (int u = 0; u < 16; u++)
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const int j = wv + u * (nth / 64), i = lane + 64 * h;
-                S[i + j * CB_LD] = gv[u][h] * iD[i] * iD[j];
-            }
-    }
-    double nrm0 = 0.0;
-    for (int i = 0; i < c; i++) nrm0 += (1.0 + 0.01 * (i % 7)) * (1.0 + 0.01 * (i % 7));
-    nrm0 = 1.0 / sqrt(nrm0);
-    for (int i = tid; i < c; i += nth) pv[i] = (1.0 + 0.01 * (i % 7)) * nrm0;
-    __syncthreads();
-    // Gershgorin certificate (kappa_2 <= (1+e)/(1-e) when e = ||S - I||_inf
-    // < 1/2), else power iterations on S
-    double eoff = 0.0;
-    const int row8 = tid >> 3, sub8 = tid & 7;
-    if (want_kappa) {
-        // off-diagonal absolute row sums (= column sums, S symmetric): thread
-        // (i, part) sums a quarter of column i, consecutive i on consecutive
-        // lanes (conflict-free LDS reads)
-        const int i = tid & 127, part = tid >> 7;
-        double rs = 0.0;
-        if (i < c) {
-#pragma unroll 8
-            for (int l = part; l < 128; l += 4)
-                rs += (l != i) ? fabs(S[i + l * CB_LD]) : 0.0;
-        }
-        pv[128 + i] = 0.0;
-        __syncthreads();
-        if (part == 0) pv[128 + i] = rs;
-        __syncthreads();
-        if (part == 1) pv[128 + i] += rs;
-        __syncthreads();
-        if (part == 2) pv[128 + i] += rs;
-        __syncthreads();
-        if (part == 3) pv[128 + i] += rs;
-        __syncthreads();
-        double e = (tid < 128) ? pv[128 + tid] : 0.0;
-        for (int o = 32; o > 0; o >>= 1) e = fmax(e, __shfl_xor(e, o));
-        if (lane == 0) s_red[wv] = e;
-        __syncthreads();
-        for (int w = 0; w < nth / 64; w++) eoff = fmax(eoff, s_red[w]);
-        __syncthreads();
-    }
-    const bool gersh = want_kappa && eoff < 0.5;
-    const int PIT = (want_kappa && !gersh) ? 6 : 0;
-    double lmax = 0.0;
-    for (int it = 0; it < PIT; it++) {
-        for (int i0 = 0; i0 < c; i0 += nth / 8) {
-            const int i = i0 + row8;
-            double acc = 0.0;
-            if (i < c)
-                for (int l = sub8; l < c; l += 8) acc += S[i + l * CB_LD] * pv[l];
-            acc += __shfl_xor(acc, 1);
-            acc += __shfl_xor(acc, 2);
-            acc += __shfl_xor(acc, 4);
-            if (i < c && sub8 == 0) pv[128 + i] = acc;
-        }
-        __syncthreads();
-        double nn = 0.0, dummy = 0.0;
-        for (int i = tid; i < c; i += nth) nn += pv[128 + i] * pv[128 + i];
-        block_sum2(nn, dummy);
-        lmax = sqrt(nn);
-        const double inv = nn > 0.0 ? 1.0 / lmax : 0.0;
-        for (int i = tid; i < c; i += nth) pv[i] = pv[128 + i] * inv;
-        __syncthreads();
-    }
-
-    // ---- factorization, panel by panel
-    const int npn = (c + 15) >> 4;
-    int ndef = 0;
-    for (int P = 0; P < npn; P++) {
-        const int rb0 = 16 * P;
-        if (wv == 0) {
-            double pa[2][16];
-#pragma unroll
-            for (int s2 = 0; s2 < 2; s2++)
-#pragma unroll
-                for (int m = 0; m < 16; m++) {
-                    const int r = rb0 + lane + 64 * s2;
-                    pa[s2][m] = (r < 128) ? S[r + (rb0 + m) * CB_LD] : 0.0;
-                }
-#pragma unroll
-            for (int j = 0; j < 16; j++) {
-                const int cj = rb0 + j;
-                // column j of the diagonal block (rows rb0 .. rb0+15, unscaled)
-                // through 16 LDS slots: the pivot and the multipliers of the
-                // later columns land in every lane's registers in one round
-                // trip (a wave's LDS accesses complete in order)
-                if (lane < 16) ub[lane] = pa[0][j];
-                const double p = ub[j] + shift;
-                const bool live = (cj < c) && (D[cj] > 0.0) && (p > tiny);
-                ndef += (cj < c && !live) ? 1 : 0;
-                if (lane == 0) tdg[cj] = live ? p : 0.0;
-                const double ip = live ? rcp2(p) : 0.0;
-                // multipliers of the rows below row cj (unscaled column / pivot)
-                const double w0 = (lane > j) ? pa[0][j] * ip : 0.0;
-                const double w1 = pa[1][j] * ip;
-#pragma unroll
-                for (int m = j + 1; m < 16; m++) {
-                    const double um = ub[m];
-                    pa[0][m] = fma(-w0, um, pa[0][m]);
-                    pa[1][m] = fma(-w1, um, pa[1][m]);
-                }
-                // the step's products are formed here, not sunk to their use
-#pragma unroll
-                for (int m = j + 1; m < 16; m++) {
-                    __asm__ __volatile__("" : "+v"(pa[0][m]));
-                    __asm__ __volatile__("" : "+v"(pa[1][m]));
-                }
-            }
-            // L = unscaled column / sqrt(pivot), sqrt(pivot) on the diagonal
-#pragma unroll
-            for (int m = 0; m < 16; m++) {
-                const int cm = rb0 + m;
-                const double pm = tdg[cm];
-                const double sq = pm > 0.0 ? sqrt(pm) : 0.0;
-                const double isq = pm > 0.0 ? 1.0 / sq : 0.0;
-                if (lane == 0) idg[cm] = isq;
-#pragma unroll
-                for (int s2 = 0; s2 < 2; s2++) {
-                    const int r = rb0 + lane + 64 * s2;
-                    if (r < 128 && r >= cm) S[r + cm * CB_LD] = (r == cm) ? sq : pa[s2][m] * isq;
-                }
-            }
-        }
-        __syncthreads();
-        // trailing update of the lower tiles (I >= J) below the panel
-        const int nb = npn - (P + 1);
-        const int ntile = nb * (nb + 1) / 2;
-        for (int t = wv; t < ntile; t += nth / 64) {
-            int I = 0;
-            while ((I + 1) * (I + 2) / 2 <= t) I++;
-            const int J = t - I * (I + 1) / 2;
-            const int bi = 16 * (P + 1 + I), bj = 16 * (P + 1 + J);
-            f64x4_t acc;
-#pragma unroll
-            for (int v = 0; v < 4; v++) acc[v] = S[(bi + (lane >> 4) + 4 * v) + (bj + (lane & 15)) * CB_LD];
+    // X_IJ, J < I, stored transposed: Ts[16J + j][16I + i] = X_IJ[i][j]
+    auto x_tile = [&](int I, int J) {
+        f64x4_t acc = {0.0, 0.0, 0.0, 0.0};
+        for (int K = J; K < I; K++) {
 #pragma unroll
             for (int kk = 0; kk < 4; kk++) {
-                const int kc = rb0 + 4 * kk + (lane >> 4);
-                const double a = -S[(bi + (lane & 15)) + kc * CB_LD];
-                const double b = S[(bj + (lane & 15)) + kc * CB_LD];
+                const int k = 4 * kk + lg;
+                const double a = S[(16 * I + li) + (16 * K + k) * LD];
+                const double b =
+                    (K == J) ? Xd[J * XS + k * 17 + li] : S[(16 * J + li) + (16 * K + k) * LD];
                 acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
             }
-#pragma unroll
-            for (int v = 0; v < 4; v++) S[(bi + (lane >> 4) + 4 * v) + (bj + (lane & 15)) * CB_LD] = acc[v];
         }
-        __syncthreads();
-    }
-    if (tid == 0) s_def = ndef;
-
-    if (WT) {
-        // diagonal blocks of X = L^-1: lane l < 16 of wave B forms column l
-        for (int B = wv; B < npn; B += nth / 64) {
-            if (lane < 16) {
-                const int b0 = 16 * B;
-                double x[16];
+        // X_IJ = -X_II acc: register kk of acc is the B operand of step kk
+        f64x4_t x = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-                for (int i = 0; i < 16; i++) {
-                    double acc = (i == lane) ? 1.0 : 0.0;
-#pragma unroll
-                    for (int k = 0; k < i; k++) acc = fma(-S[(b0 + i) + (b0 + k) * CB_LD], x[k], acc);
-                    x[i] = acc * idg[b0 + i];
-                    __builtin_amdgcn_sched_barrier(0);  // a row's loads stay with the row
-                }
-#pragma unroll
-                for (int i = 0; i < 16; i++) Xd[B * CB_XS + i * 17 + lane] = x[i];
-            }
+        for (int kk = 0; kk < 4; kk++) {
+            const double a = -Xd[I * XS + li * 17 + 4 * kk + lg];
+            x = __builtin_amdgcn_mfma_f64_16x16x4f64(a, acc[kk], x, 0, 0, 0);
         }
-        __syncthreads();
-        // block column J of X (wave J), stored transposed: Ts[16J + j][16I + i] = X_IJ[i][j]
-        for (int J = wv; J < npn; J += nth / 64) {
-            for (int I = J + 1; I < npn; I++) {
-                f64x4_t acc = {0.0, 0.0, 0.0, 0.0};
-                for (int K = J; K < I; K++) {
 #pragma unroll
-                    for (int kk = 0; kk < 4; kk++) {
-                        const int k = 4 * kk + (lane >> 4);
-                        const double a = S[(16 * I + (lane & 15)) + (16 * K + k) * CB_LD];
-                        const double b = (K == J) ? Xd[J * CB_XS + k * 17 + (lane & 15)]
-                                                  : S[(16 * J + (lane & 15)) + (16 * K + k) * CB_LD];
-                        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
-                    }
-                }
-                // X_IJ = -X_II acc: register kk of acc is the B operand of step kk
-                f64x4_t x = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-                for (int kk = 0; kk < 4; kk++) {
-                    const double a = -Xd[I * CB_XS + (lane & 15) * 17 + 4 * kk + (lane >> 4)];
-                    x = __builtin_amdgcn_mfma_f64_16x16x4f64(a, acc[kk], x, 0, 0, 0);
-                }
-#pragma unroll
-                for (int v = 0; v < 4; v++)
-                    S[(16 * J + (lane & 15)) + (16 * I + (lane >> 4) + 4 * v) * CB_LD] = x[v];
-            }
-        }
-    }
-    __syncthreads();
-    // Ts(i, k), i <= k
-    auto tget = [&](int i, int k) -> double {
-        if (i == k) return idg[i];
-        if ((i >> 4) == (k >> 4)) return Xd[(i >> 4) * CB_XS + (k & 15) * 17 + (i & 15)];
-        return S[i + k * CB_LD];
+        for (int v = 0; v < 4; v++) S[(16 * J + li) + (16 * I + lg + 4 * v) * LD] = x[v];
     };
     double fr = 0.0, ft = 0.0;
-    for (int k = wv; k < c; k += nth / 64) {
-        const double dk = D[k];
-        for (int i = lane; i < c; i += 64) {
-            double rv = 0.0, tv = 0.0;
-            if (i <= k) {
-                rv = S[k + i * CB_LD];
-                if (WT) tv = tget(i, k);
+    // rows of R (and the zeros of T left of them) of block B, by wave w of nw
+    auto put_rows = [&](int B, int w, int nw) {
+        const int i = 16 * B + li;
+        for (int k = 4 * w + lg; k < c; k += 4 * nw) {
+            const double rv = k >= i ? S[k + i * LD] : 0.0;
+            if (i < c) {
+                fr = fma(rv, rv, fr);
+                R[i + (long)k * ldo] = rv * D[k];
+                if (WT && k < 16 * B) T[i + (long)k * ldo] = 0.0;
             }
-            fr += rv * rv;
-            ft += tv * tv;
-            R[i + (long)k * ldo] = rv * dk;
-            if (WT) T[i + (long)k * ldo] = tv * iD[i];
+        }
+    };
+
+    // ---- factorization, panel by panel
+    for (int P = 0; P < npn; P++) {
+        const int rb0 = 16 * P;
+        // waves that hold the rows below the panel's diagonal block
+        const int fw = 16 * (npn - P - 1) > 64 ? 2 : 1;
+        double dg[16], pw[16];
+        double sq = 0.0;
+        if (wv < fw) {
+            const int r = rb0 + 16 + 64 * wv + lane;
+#pragma unroll
+            for (int m = 0; m < 16; m++) {
+                dg[m] = S[(rb0 + li) + (rb0 + m) * LD];
+                pw[m] = r < N ? S[r + (rb0 + m) * LD] : 0.0;
+            }
+            double psel = 0.0;
+            const unsigned alive = (unsigned)__ballot(rb0 + li < c && D[rb0 + li] > 0.0);
+            chol_steps<0>(dg, pw, li, alive, shift, tiny, psel);
+            sq = psel > 0.0 ? sqrt_nr(psel) : 0.0;
+            const double isq = psel > 0.0 ? rcp_nr(sq) : 0.0;
+            chol_scale_cols<0>(dg, pw, isq);
+            if (wv == 0 && lane < 16) {
+                tdg[rb0 + li] = psel;
+                idg[rb0 + li] = isq;
+            }
+            if (r < N) {
+#pragma unroll
+                for (int m = 0; m < 16; m++) S[r + (rb0 + m) * LD] = pw[m];
+            }
+        } else if (P > 0) {
+            // beside it: the rest of the previous panel's update, its diagonal
+            // block's inverse, the row of X above it, and its rows of R
+            const int nb = npn - (P + 1), nt = nb * (nb + 1) / 2;
+            const int w = wv - fw, nw = NB - fw;
+            for (int t = w; t < nt; t += nw) {
+                int I, J;
+                tri_tile(t, I, J);
+                update_tile(P + 1 + I, P + 1 + J, P - 1);
+            }
+            if (WT) {
+                if (w == nw - 1) invert_diag(P - 1);
+                for (int J = w; J < P - 2; J += nw) x_tile(P - 2, J);
+            }
+            put_rows(P - 1, w, nw);
+        }
+        lds_sync();
+        // the diagonal block of L: every wave that factored has read S's
+        if (wv == 0 && lane < 16) {
+#pragma unroll
+            for (int m = 0; m < 16; m++)
+                if (m <= li) S[(rb0 + li) + (rb0 + m) * LD] = m == li ? sq : dg[m];
+        }
+        for (int I = P + 1 + wv; I < npn; I += NB) update_tile(I, P + 1, P);
+        lds_sync();
+    }
+    double pmax = 0.0, pmin = INFINITY;
+    int ndef = 0;
+    for (int i0 = 0; i0 < N; i0 += 64) {
+        const double p = (i0 + lane < c) ? tdg[i0 + lane] : 0.0;
+        pmax = fmax(pmax, p);
+        if (p > 0.0) pmin = fmin(pmin, p);
+        ndef += __popcll(__ballot(i0 + lane < c && !(p > 0.0)));
+    }
+    pmax = wave_max(pmax);
+    pmin = -wave_max(-pmin);
+
+    put_rows(npn - 1, wv, NB);
+    if (WT) {
+        if (wv == NB - 1) invert_diag(npn - 1);
+        for (int J = wv; J < npn - 2; J += NB) x_tile(npn - 2, J);
+        lds_sync();
+        for (int J = wv; J < npn - 1; J += NB) x_tile(npn - 1, J);
+        lds_sync();
+    }
+    // Ts(i, k), 0 below the diagonal
+    auto tget = [&](int i, int k) -> double {
+        const int ib = i >> 4, kb = k >> 4;
+        const double off = S[i + k * LD], dia = Xd[ib * XS + (k & 15) * 17 + (i & 15)];
+        // a block beyond c has no diagonal block
+        return ib < kb ? off : (ib == kb && i <= k && k < c) ? dia : 0.0;
+    };
+    if (WT) {
+        // the upper tiles of T (put_rows wrote the zeros of the others)
+        for (int t = wv; t < npn * (npn + 1) / 2; t += NB) {
+            int I, J;
+            tri_tile(t, I, J);
+            const int i = 16 * J + li;
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int k = 16 * I + 4 * q + lg;
+                const double tv = tget(i, k);
+                if (i < c && k < c) {
+                    ft = fma(tv, tv, ft);
+                    T[i + (long)k * ldo] = tv * iD[i];
+                }
+            }
         }
     }
-    if (!WT) {
-        if (tid == 0) {
-            dinfo[0] = 0.0;
-            dinfo[1] = 0.0;
-            dinfo[2] = (double)s_def;
-            dinfo[3] = max_sq(D, c);
-        dinfo[3] = max_sq(D, c);
-            info[0] = s_def;
+    const bool decided = ndef > 0 || !(pmax <= 1e12 * pmin);
+    if (WT) {
+        fr = wave_sum(fr);
+        ft = wave_sum(ft);
+        if (lane == 0) {
+            s_red[2 * wv] = fr;
+            s_red[2 * wv + 1] = ft;
         }
-        return;
-    }
-    block_sum2(fr, ft);
-    // lambda_max(Ts Ts^T) by power iteration
-    for (int i = tid; i < c; i += nth) pv[i] = (1.0 + 0.01 * (i % 7)) * nrm0;
-    __syncthreads();
-    double lminv = 0.0;
-    for (int it = 0; it < PIT; it++) {
-        for (int k0 = 0; k0 < c; k0 += nth / 8) {  // u = Ts^T x
-            const int k = k0 + row8;
-            double acc = 0.0;
-            if (k < c)
-                for (int i = sub8; i <= k; i += 8) acc += tget(i, k) * pv[i];
-            acc += __shfl_xor(acc, 1);
-            acc += __shfl_xor(acc, 2);
-            acc += __shfl_xor(acc, 4);
-            if (k < c && sub8 == 0) pv[128 + k] = acc;
+        if (tid < N) pv[tid] = tid < c ? 1.0 + 0.01 * (tid % 7) : 0.0;
+        lds_sync();
+        fr = 0.0;
+        ft = 0.0;
+        for (int w = 0; w < NB; w++) {
+            fr += s_red[2 * w];
+            ft += s_red[2 * w + 1];
         }
-        __syncthreads();
-        for (int i0 = 0; i0 < c; i0 += nth / 8) {  // y = Ts u (into tdg, free now)
-            const int i = i0 + row8;
-            double acc = 0.0;
-            if (i < c)
-                for (int k = i + sub8; k < c; k += 8) acc += tget(i, k) * pv[128 + k];
-            acc += __shfl_xor(acc, 1);
-            acc += __shfl_xor(acc, 2);
-            acc += __shfl_xor(acc, 4);
-            if (i < c && sub8 == 0) tdg[i] = acc;
+        if (want_kappa && !gersh && !decided) {
+            // lambda_max(Ts Ts^T) <= ft = ||Ts||_F^2, divided out of every product.
+            // (kappa_2 of S is at least the ratio of two pivots, each of which lies
+            // between lambda_min and lambda_max: beyond 1e12, or with a dead pivot,
+            // it is known to be too large without the iterations.)
+            const double ift = 1.0 / ft;
+            double m[4][NB], mt[4][NB];
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+#pragma unroll
+                for (int q = 0; q < NB; q++) {
+                    const int r = 16 * wv + 4 * lg + v, k = li + 16 * q;
+                    m[v][q] = tget(r, k);
+                    mt[v][q] = tget(k, r) * ift;
+                }
+            double prev = 1.0;
+            for (int it = 0; it < PIT; it++) {
+                if (it == PIT - 1) prev = norm2(pv);
+                matvec(mt, pv, pv + N);
+                matvec(m, pv + N, pv);
+            }
+            lminv = ft * sqrt(norm2(pv) / prev);
         }
-        __syncthreads();
-        double nn = 0.0, dummy = 0.0;
-        for (int i = tid; i < c; i += nth) nn += tdg[i] * tdg[i];
-        block_sum2(nn, dummy);
-        lminv = sqrt(nn);
-        const double inv = nn > 0.0 ? 1.0 / lminv : 0.0;
-        for (int i = tid; i < c; i += nth) pv[i] = tdg[i] * inv;
-        __syncthreads();
     }
     if (tid == 0) {
-        dinfo[0] = sqrt(fr) * sqrt(ft);
-        dinfo[1] = !want_kappa ? 0.0 : gersh ? sqrt((1.0 + eoff) / (1.0 - eoff)) : sqrt(lmax * lminv);
-        dinfo[2] = (double)s_def;
-        dinfo[3] = max_sq(D, c);
-        info[0] = s_def;
+        dinfo[0] = WT ? sqrt(fr) * sqrt(ft) : 0.0;
+        dinfo[1] = !(WT && want_kappa) ? 0.0
+                   : gersh             ? sqrt((1.0 + eoff) / (1.0 - eoff))
+                   : decided           ? (pmax > 0.0 && pmin < INFINITY ? sqrt(pmax / pmin) : 0.0)
+                                       : sqrt(lmax * lminv);
+        dinfo[2] = (double)ndef;
+        dinfo[3] = dmax;
+        info[0] = ndef;
     }
 }
 
@@ -2071,8 +1794,6 @@ __global__ void k_permute_rows(int m, int n, const int *__restrict__ perm,
     }
 }
 
-// 1: the column-by-column kernel for 48 < c <= 128 (PARATT_AMD_CHOL_UNBLOCKED=1)
-int g_chol_unblocked = -1;
 // 0: small SVDs on the one-workgroup kernel too (PARATT_AMD_SVD_NO_WAVE=1)
 int g_svd_wave = [] {
     const char *e = getenv("PARATT_AMD_SVD_NO_WAVE");
@@ -2088,16 +1809,8 @@ void set_lds_attr(KF kern, int ndoubles) {
 void allow_big_lds() {
     static bool done = false;
     if (done) return;
-    set_lds_attr(k_chol_fast<64, 16, false>, CHOL_LDS_DOUBLES);
-    set_lds_attr(k_chol_fast<256, 48, false>, CHOL_LDS_DOUBLES);
-    set_lds_attr(k_chol_fast<256, 32, false>, CHOL_LDS_DOUBLES);
-    set_lds_attr(k_chol_fast<256, 32, true>, CHOL_LDS_DOUBLES);
-    set_lds_attr(k_chol_fast<512, CHOL_FAST_C, false>, CHOL_LDS_DOUBLES);
-    set_lds_attr(k_chol_fast<64, 16, true>, CHOL_LDS_DOUBLES);
-    set_lds_attr(k_chol_fast<256, 48, true>, CHOL_LDS_DOUBLES);
-    set_lds_attr(k_chol_fast<512, CHOL_FAST_C, true>, CHOL_LDS_DOUBLES);
-    set_lds_attr(k_chol_blk<true>, CB_LDS_DOUBLES);
-    set_lds_attr(k_chol_blk<false>, CB_LDS_DOUBLES);
+    set_lds_attr(k_chol_blk<8, true>, chol_geom<8>::LDS_DOUBLES);
+    set_lds_attr(k_chol_blk<8, false>, chol_geom<8>::LDS_DOUBLES);
     set_lds_attr(k_svd_jacobi, SVD_LDS_DOUBLES);
     set_lds_attr(k_svd_jacobi_wave<4, 2>, SVW_LDS_DOUBLES);
     set_lds_attr(k_svd_jacobi_wave<4, 4>, SVW_LDS_DOUBLES);
@@ -2114,6 +1827,20 @@ void allow_big_lds() {
     set_lds_attr(k_lj_block<8, 32, 0>, LJ_LDS_DOUBLES);
     set_lds_attr(k_lj_block<2, 64, 0>, LJ_LDS_DOUBLES);
     done = true;
+}
+
+// k_chol_blk with NB blocks of 16 columns, with the inverse when T is given.
+template <int NB>
+void launch_chol(const char *nm, double fl, double by, int c, const double *G, long ldg,
+                 double shift, double tiny, double *R, double *T, long ldo, int *info,
+                 double *dinfo, int want_kappa, int unit) {
+    const size_t need = chol_geom<NB>::LDS_DOUBLES * sizeof(double);
+    if (T)
+        PTT_LAUNCH_FB(nm, fl, by, (k_chol_blk<NB, true>), dim3(1), dim3(64 * NB), need, c, G, ldg,
+                      shift, tiny, R, T, ldo, info, dinfo, want_kappa, unit);
+    else
+        PTT_LAUNCH_FB(nm, fl, by, (k_chol_blk<NB, false>), dim3(1), dim3(64 * NB), need, c, G, ldg,
+                      shift, tiny, R, T, ldo, info, dinfo, want_kappa, unit);
 }
 
 // One launch a round of block pairs (see k_lj_block).
@@ -2189,46 +1916,22 @@ void ptt_hip_chol_qr_factor(int c, const double *G, double shift, double tiny, d
                             double *T, int *info, double *dinfo, int want_kappa) {
     ptt_hip_init();
     allow_big_lds();
-    if (g_chol_unblocked < 0) {
-        const char *e = getenv("PARATT_AMD_CHOL_UNBLOCKED");
-        g_chol_unblocked = (e && e[0] == '1') ? 1 : 0;
-    }
-    if (c <= CHOL_FAST_C) {
-        const size_t fneed = (size_t)c * (c | 1) + 5 * (size_t)c + 3 * CHOL_BLK * CHOL_BLK;
-        // fewer threads for small factors: the steps are barrier-bound
+    if (c <= 128) {
         const char *nm = T ? "chol_qr_factor" : "chol_factor_only";
         const double fl = 2.0 * c * (double)c * c / 3.0, by = 8.0 * 3.0 * c * (double)c;
         const int wk = T ? want_kappa : 0;
-#define PTT_CHOL_FAST(NTH_, CMAX_)                                                         \
-    do {                                                                                    \
-        if (T)                                                                              \
-            PTT_LAUNCH_FB(nm, fl, by, (k_chol_fast<NTH_, CMAX_, true>), dim3(1), dim3(NTH_),  \
-                          fneed * sizeof(double), c, G, shift, tiny, R, T, info, dinfo, wk);  \
-        else                                                                                \
-            PTT_LAUNCH_FB(nm, fl, by, (k_chol_fast<NTH_, CMAX_, false>), dim3(1), dim3(NTH_), \
-                          fneed * sizeof(double), c, G, shift, tiny, R, T, info, dinfo, wk);  \
-    } while (0)
-        if (c <= 16) {
-            PTT_CHOL_FAST(64, 16);
-        } else if (c <= 32) {
-            // register blocks sized for 32 columns: a 48-column layout would
-            // spend three quarters of its updates on rows and columns beyond c
-            PTT_CHOL_FAST(256, 32);
-        } else if (c <= 48) {
-            PTT_CHOL_FAST(256, 48);
-        } else if (g_chol_unblocked) {
-            PTT_CHOL_FAST(512, CHOL_FAST_C);
-        } else {
-            // panels of 16 columns: two barriers per panel
-            const size_t bneed = (size_t)CB_LDS_DOUBLES * sizeof(double);
-            if (T)
-                PTT_LAUNCH_FB(nm, fl, by, k_chol_blk<true>, dim3(1), dim3(512), bneed, c, G,
-                              (long)c, shift, tiny, R, T, (long)c, info, dinfo, wk, 0);
-            else
-                PTT_LAUNCH_FB(nm, fl, by, k_chol_blk<false>, dim3(1), dim3(512), bneed, c, G,
-                              (long)c, shift, tiny, R, T, (long)c, info, dinfo, wk, 0);
-        }
-#undef PTT_CHOL_FAST
+        // the fewest waves whose blocks hold c columns; beyond four blocks all eight
+        // waves, whose spare ones take part in the tile products
+        if (c <= 16)
+            launch_chol<1>(nm, fl, by, c, G, c, shift, tiny, R, T, c, info, dinfo, wk, 0);
+        else if (c <= 32)
+            launch_chol<2>(nm, fl, by, c, G, c, shift, tiny, R, T, c, info, dinfo, wk, 0);
+        else if (c <= 48)
+            launch_chol<3>(nm, fl, by, c, G, c, shift, tiny, R, T, c, info, dinfo, wk, 0);
+        else if (c <= 64)
+            launch_chol<4>(nm, fl, by, c, G, c, shift, tiny, R, T, c, info, dinfo, wk, 0);
+        else
+            launch_chol<8>(nm, fl, by, c, G, c, shift, tiny, R, T, c, info, dinfo, wk, 0);
         return;
     }
     // blocks of 128 columns
@@ -2245,13 +1948,11 @@ void ptt_hip_chol_qr_factor(int c, const double *G, double shift, double tiny, d
     if (T && nblk > 2) ptt_hip_zero(T, sizeof(double) * cc);  // its lower blocks are operands
     PTT_LAUNCH("chol_scale", k_chol_scale, dim3(stream_blocks((long)cc, 256)), dim3(256), 0, c, G,
                shift, D, iD, S);
-    const size_t bneed = (size_t)CB_LDS_DOUBLES * sizeof(double);
     for (int b = 0; b < nblk; b++) {
         const int b0 = 128 * b, cb = c - b0 < 128 ? c - b0 : 128, rest = c - b0 - cb;
         const size_t dg = (size_t)b0 + (size_t)b0 * c;
-        PTT_LAUNCH_FB("chol_qr_factor", 2.0 * cb * (double)cb * cb / 3.0, 24.0 * cb * (double)cb,
-                      k_chol_blk<true>, dim3(1), dim3(512), bneed, cb, S + dg, (long)c, 0.0, tiny,
-                      R + dg, Ti + dg, (long)c, bi + b, bd + 4 * b, 0, 1);
+        launch_chol<8>("chol_qr_factor", 2.0 * cb * (double)cb * cb / 3.0, 24.0 * cb * (double)cb, cb,
+                       S + dg, c, 0.0, tiny, R + dg, Ti + dg, c, bi + b, bd + 4 * b, 0, 1);
         if (rest > 0) {
             const size_t right = dg + (size_t)cb * c, trail = right + cb;
             ptt_hip_dgemm('T', 'N', cb, rest, cb, 1.0, Ti + dg, c, S + right, c, 0.0, R + right, c);

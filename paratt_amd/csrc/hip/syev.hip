@@ -71,21 +71,9 @@ __device__ __forceinline__ double grp_prod(double x) {
     if constexpr (L == 8) x = oct_prod(x);
     return x;
 }
-__device__ __forceinline__ double wave_max(double x) {
-    for (int o = 32; o > 0; o >>= 1) x = fmax(x, __shfl_xor(x, o));
-    return x;
-}
 // sqrt(x) for x >= 0 to a few ulp; 0 below 2^-900 (x not far above 1 otherwise).
 __device__ __forceinline__ double sqrt_pos(double x) {
     return x > 0x1.0p-900 ? sqrt_nr(x) : 0.0;
-}
-
-// Workgroup barrier that orders LDS traffic only: outstanding global stores
-// (the reflectors written as they are formed) do not hold the barrier.
-__device__ __forceinline__ void lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 // Inclusive suffix sum over the 64 lanes of a wave: x_lane + ... + x_63.

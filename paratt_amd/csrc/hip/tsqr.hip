@@ -34,18 +34,6 @@ constexpr int TQ_NT = 256;  // threads of a block's workgroup
 constexpr int TQ_C = 32;    // columns at most; also ld of F and X
 constexpr int TQ_LD = 33;   // LDS stride of small matrices
 
-// Value of lane N of each row of 16 lanes, on all of them.
-template <int N>
-__device__ __forceinline__ double row_bcast(double v) {
-    return __longlong_as_double(
-        __builtin_amdgcn_update_dpp(0LL, __double_as_longlong(v), 0x150 + N, 0xF, 0xF, true));
-}
-__device__ __forceinline__ double row16_sum(double x) {
-    x = quad_sum(x);
-    x += dppd<0x141>(x);
-    return x + dppd<0x140>(x);
-}
-
 // Layout of a block: a row of 16 lanes holds one part's rows, part + 16 s for
 // s < RP; lane li of it columns li + 16 k, k < NC.  The pivot column's rows thus
 // reach every column by a lane broadcast inside the 16-lane row (one
