@@ -151,6 +151,11 @@ void ptt_hip_sumsq(int m, int n, const double *A, long lda, double *out);
 void ptt_hip_dgemm(char ta, char tb, int M, int N, int K, double alpha,
                    const double *A, long lda, const double *B, long ldb,
                    double beta, double *C, long ldc);
+/* One mode of an inner product: out (rx1 x ry1) = s sum_j X_j^T a Y_j over the n
+ * mode indices of the cores x (rx0 x n x rx1) and y (ry0 x n x ry1), a rx0 x ry0.
+ * out may be a.  Returns 0, having done nothing, beyond ranks of 64. */
+int ptt_hip_dot_mode(int n, int rx0, int rx1, int ry0, int ry1, const double *a, const double *x,
+                     const double *y, double s, double *out);
 /* Gram matrices with a split over the long dimension:
  * trans 'T': G (c x c) = A^T A for A (m x c, lda);
  * trans 'N': G (c x c) = A A^T for A (c x w, lda). */
