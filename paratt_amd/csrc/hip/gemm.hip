@@ -512,7 +512,12 @@ void launch_skinny(int side, int M, int N, int K, double alpha, const double *A,
     skinny_lds_attr();
     const int big = side == 1 ? N : M, small = side == 1 ? M : N;
     const unsigned tiles = cdiv(big, SK_T);
-    const dim3 grid(tiles < 256 ? tiles : 256);
+    // A workgroup takes a CU's registers.  On the side stream some CUs are left to
+    // the main stream: its one-workgroup factorisation and the copy that reports it
+    // to the host otherwise wait until the whole product is done.  No more rounds of
+    // tiles than that costs.
+    const unsigned cus = g_launch == g_stream ? 256u : 248u;
+    const dim3 grid(tiles < cus ? tiles : cdiv(tiles, cdiv(tiles, cus)));
     // one ticket counter per stream (the side stream's products may run
     // beside the main stream's)
     static unsigned *tickets = nullptr;

@@ -36,7 +36,7 @@ namespace {
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
 constexpr double EPSU = 0x1.0p-53;
-constexpr int EIG_NMAX = 128;
+constexpr int EIG_NMAX = 192;
 
 __device__ __forceinline__ double quad_prod(double x) {
     x *= dppd<0xB1>(x);
@@ -130,15 +130,26 @@ __device__ __forceinline__ double readlane_d(double v, int l) {
 }
 __device__ __forceinline__ double sel(bool c, double x, double y) { return c ? x : y; }
 
+// Tile rows a row wave holds: two beyond 128 rows (row wave I: I and I + NB / 2),
+// so that the workgroup keeps 256 registers a lane.
 template <int NMAX>
-__global__ __launch_bounds__(NMAX * 4 + 64) void k_sytrd(int n, const double *__restrict__ G,
+struct sytrd_geom {
+    static constexpr int NB = NMAX / 16, TR = NMAX > 128 ? 2 : 1, NWR = NB / TR;
+    static constexpr int E = (NMAX + 63) / 64;  // entries of a row a lane of the reflector wave
+    static constexpr int NT = 64 * NWR + 64;
+};
+
+template <int NMAX>
+__global__ __launch_bounds__(sytrd_geom<NMAX>::NT) void k_sytrd(int n, const double *__restrict__ G,
                                                          long ldg, double *__restrict__ Vh,
                                                          double *__restrict__ tau_out,
                                                          double *__restrict__ d_out,
                                                          double *__restrict__ e_out,
                                                          int *__restrict__ eexp,
                                                          double *__restrict__ dinfo) {
-    constexpr int NB = NMAX / 16, NTM = 64 * NB, NT = NTM + 64, NW = NT / 64;
+    using geom = sytrd_geom<NMAX>;
+    constexpr int NB = geom::NB, TR = geom::TR, NWR = geom::NWR, E = geom::E;
+    constexpr int NTM = 64 * NWR, NT = NTM + 64, NW = NT / 64;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const bool star = (tid >= NTM);  // the reflector wave
     const int I = wv, ga = lane >> 4, gj = lane & 15;
@@ -150,20 +161,22 @@ __global__ __launch_bounds__(NMAX * 4 + 64) void k_sytrd(int n, const double *__
     __shared__ double s_max[NW], s_tr[NW];
     __shared__ int s_e;
 
-    double g[NB][4];
+    double g[TR][NB][4];
     double amax = 0.0, tr = 0.0;
 #pragma unroll
-    for (int J = 0; J < NB; J++)
+    for (int t = 0; t < TR; t++)
 #pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const int row = 16 * I + ga + 4 * v, col = 16 * J + gj;
-            double x = 0.0;
-            if (!star && row < n && col < n)
-                x = (row <= col) ? G[row + (long)col * ldg] : G[col + (long)row * ldg];
-            g[J][v] = x;
-            amax = fmax(amax, fabs(x));
-            if (row == col) tr += x;
-        }
+        for (int J = 0; J < NB; J++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int row = 16 * (I + NWR * t) + ga + 4 * v, col = 16 * J + gj;
+                double x = 0.0;
+                if (!star && row < n && col < n)
+                    x = (row <= col) ? G[row + (long)col * ldg] : G[col + (long)row * ldg];
+                g[t][J][v] = x;
+                amax = fmax(amax, fabs(x));
+                if (row == col) tr += x;
+            }
     amax = wave_max(amax);
     tr = wave_sum(tr);
     if (lane == 0) {
@@ -185,35 +198,43 @@ __global__ __launch_bounds__(NMAX * 4 + 64) void k_sytrd(int n, const double *__
     __syncthreads();
     const int es = s_e;
 #pragma unroll
-    for (int J = 0; J < NB; J++)
+    for (int t = 0; t < TR; t++)
 #pragma unroll
-        for (int v = 0; v < 4; v++) g[J][v] = ldexp(g[J][v], -es);
+        for (int J = 0; J < NB; J++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) g[t][J][v] = ldexp(g[t][J][v], -es);
 
-    // Row i of this wave's tile row into rowb[slot] (called by the whole
+    // Row i of this wave's tile row t into rowb[slot] (called by the whole
     // wave; i wave-uniform, held by the lanes with a = i % 4 in register
     // v = (i % 16) / 4).
     auto copy_row = [&](int i, int slot) {
         const int v = (i & 15) >> 2;
-        if (ga == (i & 3)) {
-            // g[J][v] by a 0/1 mask (exact: one term is nonzero), so every
-            // register index stays constant and g stays in registers
-            const double m0 = (v == 0) ? 1.0 : 0.0, m1 = (v == 1) ? 1.0 : 0.0;
-            const double m2 = (v == 2) ? 1.0 : 0.0, m3 = (v == 3) ? 1.0 : 0.0;
 #pragma unroll
-            for (int J = 0; J < NB; J++)
-                rowb[slot][16 * J + gj] =
-                    fma(g[J][3], m3, fma(g[J][2], m2, fma(g[J][1], m1, g[J][0] * m0)));
-        }
+        for (int t = 0; t < TR; t++)
+            if (I + NWR * t == i >> 4 && ga == (i & 3)) {
+                // g[t][J][v] by a 0/1 mask (exact: one term is nonzero), so every
+                // register index stays constant and g stays in registers
+                const double m0 = (v == 0) ? 1.0 : 0.0, m1 = (v == 1) ? 1.0 : 0.0;
+                const double m2 = (v == 2) ? 1.0 : 0.0, m3 = (v == 3) ? 1.0 : 0.0;
+#pragma unroll
+                for (int J = 0; J < NB; J++)
+                    rowb[slot][16 * J + gj] = fma(
+                        g[t][J][3], m3, fma(g[t][J][2], m2, fma(g[t][J][1], m1, g[t][J][0] * m0)));
+            }
     };
-    // The reflector wave turns row p (entries a0 = row[lane], a1 =
-    // row[lane + 64]) into the reflector for step p, from column p below the
-    // diagonal: v into vb[slot], tau, d_p, e_p = beta (the row waves copy v
-    // to Vh at the start of step p).
+    // The reflector wave turns row p (entries a[u] = row[lane + 64 u]) into the
+    // reflector for step p, from column p below the diagonal: v into vb[slot],
+    // tau, d_p, e_p = beta (the row waves copy v to Vh at the start of step p).
     // x0 = row[p+1] and dp = row[p] arrive as wave-uniform values (formed by
     // every lane with the owner lane's arithmetic, so no lane reads).
-    auto reflector = [&](int p, int slot, double a0, double a1, double x0, double dp) {
-        const int i0 = lane, i1 = lane + 64;
-        double s2 = (i0 >= p + 2 ? a0 * a0 : 0.0) + (i1 >= p + 2 && i1 < NMAX ? a1 * a1 : 0.0);
+    auto reflector = [&](int p, int slot, const double(&a)[E], double x0, double dp) {
+        double s2 = 0.0;
+#pragma unroll
+        for (int u = 0; u < E; u++) {
+            const int i = lane + 64 * u;
+            const double x = (i >= p + 2 && i < NMAX) ? a[u] : 0.0;
+            s2 = fma(x, x, s2);
+        }
         s2 = wave_sum(s2);
         double beta, tk, scl;
         if (s2 == 0.0) {
@@ -225,10 +246,12 @@ __global__ __launch_bounds__(NMAX * 4 + 64) void k_sytrd(int n, const double *__
             tk = (beta - x0) * rcp_nr(beta);
             scl = rcp_nr(x0 - beta);
         }
-        const double w0 = (i0 == p + 1) ? 1.0 : (i0 > p + 1 ? a0 * scl : 0.0);
-        const double w1 = (i1 == p + 1) ? 1.0 : (i1 > p + 1 ? a1 * scl : 0.0);
-        if (i0 < NMAX) vb[slot][i0] = w0;
-        if (i1 < NMAX) vb[slot][i1] = w1;
+#pragma unroll
+        for (int u = 0; u < E; u++) {
+            const int i = lane + 64 * u;
+            const double w = (i == p + 1) ? 1.0 : (i > p + 1 ? a[u] * scl : 0.0);
+            if (i < NMAX) vb[slot][i] = w;
+        }
         if (lane == 0) {
             tkb[slot] = tk;
             sd[p] = dp;
@@ -236,10 +259,11 @@ __global__ __launch_bounds__(NMAX * 4 + 64) void k_sytrd(int n, const double *__
             st[p] = tk;
         }
     };
-    // entries of an LDS row vector at columns lane and lane + 64
-    auto lrow = [&](const double *v, double &x0, double &x1) {
-        x0 = v[lane];
-        x1 = (lane + 64 < NMAX) ? v[lane + 64 < NMAX ? lane + 64 : 0] : 0.0;
+    // entries of an LDS row vector at columns lane + 64 u
+    auto lrow = [&](const double *v, double(&x)[E]) {
+#pragma unroll
+        for (int u = 0; u < E; u++)
+            x[u] = (lane + 64 * u < NMAX) ? v[lane + 64 * u < NMAX ? lane + 64 * u : 0] : 0.0;
     };
 
     if (!star && I == 0) {
@@ -248,9 +272,9 @@ __global__ __launch_bounds__(NMAX * 4 + 64) void k_sytrd(int n, const double *__
     }
     lds_sync();
     if (star) {
-        double a0, a1;
-        lrow(rowb[1], a0, a1);
-        reflector(0, 0, a0, a1, rowb[1][1 < NMAX ? 1 : 0], rowb[1][0]);
+        double a[E];
+        lrow(rowb[1], a);
+        reflector(0, 0, a, rowb[1][1 < NMAX ? 1 : 0], rowb[1][0]);
     }
     lds_sync();
 
@@ -259,40 +283,55 @@ __global__ __launch_bounds__(NMAX * 4 + 64) void k_sytrd(int n, const double *__
         const double tk = tkb[k & 1];
         if (!star) {
             for (int i = tid; i < n; i += NTM) Vh[i + (long)k * n] = vk[i];
-            const bool act = (16 * I + 15 > k);
+            const bool act = (16 * (I + NWR * (TR - 1)) + 15 > k);
             if (tk != 0.0) {
-                double vJ[NB];
+                // two tile rows leave no registers for v and p: they are read where
+                // they are used
+                constexpr bool HOLD = TR == 1;
+                double vJ[HOLD ? NB : 1], dot = 0.0;
                 if (act) {
-                    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+                    double acc[TR][4];
+#pragma unroll
+                    for (int t = 0; t < TR; t++)
+#pragma unroll
+                        for (int v = 0; v < 4; v++) acc[t][v] = 0.0;
 #pragma unroll
                     for (int J = 0; J < NB; J++) {
-                        vJ[J] = vk[16 * J + gj];
+                        const double vj = vk[16 * J + gj];
+                        if (HOLD) vJ[HOLD ? J : 0] = vj;
 #pragma unroll
-                        for (int v = 0; v < 4; v++) acc[v] = fma(g[J][v], vJ[J], acc[v]);
+                        for (int t = 0; t < TR; t++)
+#pragma unroll
+                            for (int v = 0; v < 4; v++) acc[t][v] = fma(g[t][J][v], vj, acc[t][v]);
                     }
-                    // reduce-scatter over the 16 lanes of the row: lane j
-                    // ends with the sum for v = 2 (j / 8 % 2) + (j / 4 % 2)
-                    const bool h8 = (gj & 8) != 0, h4 = (gj & 4) != 0;
-                    const double k0 = sel(h8, acc[2], acc[0]), k1 = sel(h8, acc[3], acc[1]);
-                    const double s0 = sel(h8, acc[0], acc[2]), s1 = sel(h8, acc[1], acc[3]);
-                    const double u0 = k0 + dppd<0x128>(s0);  // row_ror:8
-                    const double u1 = k1 + dppd<0x128>(s1);
-                    const double kk2 = sel(h4, u1, u0), ss2 = sel(h4, u0, u1);
-                    double x = kk2 + dppd<0x141>(ss2);  // half-row mirror: 4-lane groups swap
-                    x = quad_sum(x);
-                    if ((gj & 3) == 0) {
-                        const int vi = 2 * (int)h8 + (int)h4;
-                        pp[16 * I + ga + 4 * vi] = tk * x;
+#pragma unroll
+                    for (int t = 0; t < TR; t++) {
+                        // reduce-scatter over the 16 lanes of the row: lane j
+                        // ends with the sum for v = 2 (j / 8 % 2) + (j / 4 % 2)
+                        const bool h8 = (gj & 8) != 0, h4 = (gj & 4) != 0;
+                        const double k0 = sel(h8, acc[t][2], acc[t][0]);
+                        const double k1 = sel(h8, acc[t][3], acc[t][1]);
+                        const double s0 = sel(h8, acc[t][0], acc[t][2]);
+                        const double s1 = sel(h8, acc[t][1], acc[t][3]);
+                        const double u0 = k0 + dppd<0x128>(s0);  // row_ror:8
+                        const double u1 = k1 + dppd<0x128>(s1);
+                        const double kk2 = sel(h4, u1, u0), ss2 = sel(h4, u0, u1);
+                        double x = kk2 + dppd<0x141>(ss2);  // half-row mirror: 4-lane groups swap
+                        x = quad_sum(x);
+                        if ((gj & 3) == 0) {
+                            const int vi = 2 * (int)h8 + (int)h4;
+                            pp[16 * (I + NWR * t) + ga + 4 * vi] = tk * x;
+                        }
                     }
                 }
                 lds_sync();
                 if (act) {
-                    double pJ[NB];
-                    double dot = 0.0;
+                    double pJ[HOLD ? NB : 1];
 #pragma unroll
                     for (int J = 0; J < NB; J++) {
-                        pJ[J] = pp[16 * J + gj];
-                        dot = fma(pJ[J], vJ[J], dot);
+                        const double pj = pp[16 * J + gj];
+                        if (HOLD) pJ[HOLD ? J : 0] = pj;
+                        dot = fma(pj, HOLD ? vJ[HOLD ? J : 0] : vk[16 * J + gj], dot);
                     }
                     // p^T v over the 16 columns j of the row (each DPP row
                     // forms the same sum)
@@ -300,48 +339,60 @@ __global__ __launch_bounds__(NMAX * 4 + 64) void k_sytrd(int n, const double *__
                     dot += dppd<0x141>(dot);
                     dot += dppd<0x140>(dot);
                     const double kk = 0.5 * tk * dot;
-                    double vr[4], wr[4];
 #pragma unroll
-                    for (int v = 0; v < 4; v++) {
-                        const int row = 16 * I + ga + 4 * v;
-                        vr[v] = vk[row];
-                        wr[v] = pp[row] - 2.0 * kk * vr[v];
+                    for (int t = 0; t < TR; t++) {
+                        double vr[4], wr[4];
+#pragma unroll
+                        for (int v = 0; v < 4; v++) {
+                            const int row = 16 * (I + NWR * t) + ga + 4 * v;
+                            vr[v] = vk[row];
+                            wr[v] = pp[row] - 2.0 * kk * vr[v];
+                        }
+#pragma unroll
+                        for (int J = 0; J < NB; J++) {
+                            const double pj = HOLD ? pJ[HOLD ? J : 0] : pp[16 * J + gj];
+                            const double vj = HOLD ? vJ[HOLD ? J : 0] : vk[16 * J + gj];
+#pragma unroll
+                            for (int v = 0; v < 4; v++)
+                                g[t][J][v] = fma(-vr[v], pj, fma(-vj, wr[v], g[t][J][v]));
+                        }
+                        if (!HOLD) __asm__ __volatile__("" ::: "memory");
                     }
-#pragma unroll
-                    for (int J = 0; J < NB; J++)
-#pragma unroll
-                        for (int v = 0; v < 4; v++)
-                            g[J][v] = fma(-vr[v], pJ[J], fma(-vJ[J], wr[v], g[J][v]));
                 }
             }
             // row k+2 (now updated through step k) for the reflector wave
-            if (I == (k + 2) >> 4) copy_row(k + 2, (k + 1) & 1);
+            copy_row(k + 2, (k + 1) & 1);
         } else {
             // row k+1, updated through step k-1 (copied before the last barrier),
             // and its entries k+1 (the diagonal) and k+2 as uniform values
             const int k1 = k + 1, k2 = (k + 2 < NMAX) ? k + 2 : k + 1;
             const double *rk = rowb[k & 1];
-            double a0, a1;
-            lrow(rk, a0, a1);
+            double a[E];
+            lrow(rk, a);
             double dp = rk[k1];
             double x0 = (k + 2 < NMAX) ? rk[k2] : 0.0;
             if (tk != 0.0) {
-                double v0, v1;
-                lrow(vk, v0, v1);
+                double v[E];
+                lrow(vk, v);
                 const double vx = vk[k2];
                 lds_sync();
-                double p0, p1;
-                lrow(pp, p0, p1);
+                double p[E];
+                lrow(pp, p);
                 const double pk = pp[k1], px = pp[k2];
-                const double kk = 0.5 * tk * wave_sum(fma(p0, v0, p1 * v1));
+                // fma from zero: a bare product could be contracted into the first
+                // addition across lanes, whose result would then differ by lane
+                double pv = 0.0;
+#pragma unroll
+                for (int u = E - 1; u >= 0; u--) pv = fma(p[u], v[u], pv);
+                const double kk = 0.5 * tk * wave_sum(pv);
                 const double w = pk - 2.0 * kk;  // v_{k+1} = 1
-                a0 = fma(-1.0, p0, fma(-v0, w, a0));
-                a1 = fma(-1.0, p1, fma(-v1, w, a1));
+#pragma unroll
+                for (int u = 0; u < E; u++) a[u] = fma(-1.0, p[u], fma(-v[u], w, a[u]));
                 // the owner lanes' arithmetic for entries k+1 and k+2
                 dp = fma(-1.0, pk, fma(-1.0, w, dp));
                 if (k + 2 < NMAX) x0 = fma(-1.0, px, fma(-vx, w, x0));
             }
-            reflector(k1, k1 & 1, a0, a1, x0, dp);
+            reflector(k1, k1 & 1, a, x0, dp);
         }
         lds_sync();
     }
@@ -390,69 +441,82 @@ __global__ __launch_bounds__(NMAX * 4 + 64) void k_sytrd(int n, const double *__
 // top merge, so the back transformation Q Z runs beside it.
 
 // Deflation of one block by GL lanes (gl: lane in the group, which starts at
-// lane gbase of the wave); K entries at the sorted positions sperm[0 .. K).  With
-// TWO a lane takes two positions (gl, gl + 64).  Lists snd, sdl, szl and rotations
+// lane gbase of the wave); K entries at the sorted positions sperm[0 .. K).  A
+// lane takes the positions gl + 64 w, w < NW.  Lists snd, sdl, szl and rotations
 // ra, rb, rc, rs; Kn and nrot as lane 0 has them.
-template <bool TWO>
+template <int NW>
 __device__ __forceinline__ void deflate(int GL, int gl, int gbase, int K, double rho,
                                         const int *sperm, double *sz, double *sD, int *snd,
                                         double *sdl, double *szl, int *ra, int *rb, double *rc,
                                         double *rs, int &Kn_out, int &nrot_out) {
-    const unsigned long long gmask = (GL == 64) ? ~0ULL : (((1ULL << GL) - 1) << gbase);
-    const int q0 = gl, q1 = gl + 64;
-    const int j0 = (q0 < K) ? sperm[q0] : -1;
-    const int j1 = (TWO && q1 < K) ? sperm[q1] : -1;
-    const double z0 = j0 >= 0 ? sz[j0] : 0.0, z1 = j1 >= 0 ? sz[j1] : 0.0;
-    const double d0 = j0 >= 0 ? sD[j0] : 0.0, d1 = j1 >= 0 ? sD[j1] : 0.0;
-    double dmax = fmax(fabs(d0), fabs(d1)), zmax = fmax(fabs(z0), fabs(z1));
+    typedef unsigned long long u64;
+    const u64 gmask = (GL == 64) ? ~0ULL : (((1ULL << GL) - 1) << gbase);
+    const u64 below = (gl == 0) ? 0ULL : ((~0ULL) >> (64 - gl));
+    int jw[NW];
+    double zw[NW], dw[NW], dmax = 0.0, zmax = 0.0;
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+        const int q = gl + 64 * w;
+        jw[w] = (q < K) ? sperm[q] : -1;
+        zw[w] = jw[w] >= 0 ? sz[jw[w]] : 0.0;
+        dw[w] = jw[w] >= 0 ? sD[jw[w]] : 0.0;
+        dmax = fmax(dmax, fabs(dw[w]));
+        zmax = fmax(zmax, fabs(zw[w]));
+    }
     for (int o = 1; o < GL; o <<= 1) {
         dmax = fmax(dmax, __shfl_xor(dmax, o, GL));
         zmax = fmax(zmax, __shfl_xor(zmax, o, GL));
     }
     const double tol = 8.0 * EPSU * fmax(dmax, zmax);
-    const bool k0 = j0 >= 0 && !(rho * fabs(z0) <= tol);
-    const bool k1 = j1 >= 0 && !(rho * fabs(z1) <= tol);
-    // kept positions of the group, bit = sorted position
-    const unsigned long long m0 = (__ballot(k0) & gmask) >> gbase;
-    const unsigned long long m1 = (__ballot(k1) & gmask) >> gbase;
-    const unsigned long long below = (gl == 0) ? 0ULL : ((~0ULL) >> (64 - gl));
-    bool close0 = false, close1 = false;
-    if (k0) {
-        const unsigned long long mm = m0 & below;
-        if (mm) {
-            const int jp = sperm[63 - __clzll(mm)];
-            const double zp = sz[jp], t = d0 - sD[jp];
-            close0 = fabs(t * z0 * zp) <= tol * (z0 * z0 + zp * zp);
-        }
+    // kept positions of the group, bit = sorted position; the position kept
+    // before q, and the first one of a mask after q (-1: none)
+    u64 m[NW], f[NW], r[NW];
+    bool keep[NW];
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+        keep[w] = jw[w] >= 0 && !(rho * fabs(zw[w]) <= tol);
+        m[w] = (__ballot(keep[w]) & gmask) >> gbase;
+        r[w] = 0;
     }
-    if (k1) {
-        const unsigned long long mm = m1 & below;
-        const int p = mm ? 64 + 63 - __clzll(mm) : (m0 ? 63 - __clzll(m0) : -1);
-        if (p >= 0) {
-            const int jp = sperm[p];
-            const double zp = sz[jp], t = d1 - sD[jp];
-            close1 = fabs(t * z1 * zp) <= tol * (z1 * z1 + zp * zp);
+    auto before = [&](int q) {
+        int p = -1;
+#pragma unroll
+        for (int w = 0; w < NW; w++) {
+            const int l = q - 64 * w;  // bits below l
+            const u64 x = l >= 64 ? m[w] : l > 0 ? m[w] & (~0ULL >> (64 - l)) : 0ULL;
+            if (x) p = 64 * w + 63 - __clzll((long long)x);
         }
+        return p;
+    };
+    auto next = [&](const u64(&a)[NW], int q) {
+        int p = -1;
+#pragma unroll
+        for (int w = NW - 1; w >= 0; w--) {
+            const int l = q + 1 - 64 * w;  // bits from l
+            const u64 x = l <= 0 ? a[w] : l < 64 ? a[w] & (~0ULL << l) : 0ULL;
+            if (x) p = 64 * w + __ffsll((long long)x) - 1;
+        }
+        return p;
+    };
+    u64 any = 0;
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+        bool close = false;
+        if (keep[w]) {
+            const int p = before(gl + 64 * w);
+            if (p >= 0) {
+                const int jp = sperm[p];
+                const double zp = sz[jp], t = dw[w] - sD[jp];
+                close = fabs(t * zw[w] * zp) <= tol * (zw[w] * zw[w] + zp * zp);
+            }
+        }
+        f[w] = (__ballot(close) & gmask) >> gbase;
+        any |= f[w];
     }
-    const unsigned long long f0 = (__ballot(close0) & gmask) >> gbase;
-    const unsigned long long f1 = (__ballot(close1) & gmask) >> gbase;
-    unsigned long long r0 = 0, r1 = 0;  // entries rotated away
     int nrot = 0;
-    if (f0 | f1) {
+    if (any) {
         if (gl == 0) {
-            auto next = [](unsigned long long a, unsigned long long b, int q) {
-                const unsigned long long x = q < 63 ? a & (~0ULL << (q + 1)) : 0ULL;
-                if (x) return __ffsll((long long)x) - 1;
-                const unsigned long long y = q < 63 ? b : q < 127 ? b & (~0ULL << (q - 63)) : 0ULL;
-                return y ? 63 + __ffsll((long long)y) : -1;
-            };
-            auto before = [](unsigned long long a, unsigned long long b, int q) {
-                const unsigned long long y = q > 64 ? b & (~0ULL >> (128 - q)) : 0ULL;
-                if (y) return 127 - __clzll((long long)y);
-                const unsigned long long x = q >= 64 ? a : a & ~(~0ULL << q);
-                return x ? 63 - __clzll((long long)x) : -1;
-            };
-            int q = next(f0, f1, -1), p = before(m0, m1, q);
+            int q = next(f, -1), p = before(q);
             while (q >= 0) {
                 const int j = sperm[q], prev = sperm[p];
                 const double zj = sz[j], dj = sD[j], zp = sz[prev], dp = sD[prev];
@@ -470,36 +534,35 @@ __device__ __forceinline__ void deflate(int GL, int gl, int gbase, int K, double
                     rc[nrot] = c;
                     rs[nrot] = sn;
                     nrot++;
-                    if (p < 64) r0 |= 1ULL << p;
-                    else r1 |= 1ULL << (p - 64);
+#pragma unroll
+                    for (int w = 0; w < NW; w++)
+                        if (p >> 6 == w) r[w] |= 1ULL << (p & 63);
                     // the combined entry against the next one
                     p = q;
-                    q = next(m0, m1, q);
+                    q = next(m, q);
                 } else {
-                    q = next(f0, f1, q);
-                    if (q >= 0) p = before(m0, m1, q);
+                    q = next(f, q);
+                    if (q >= 0) p = before(q);
                 }
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        r0 = __shfl(r0, 0, GL);
-        r1 = __shfl(r1, 0, GL);
+#pragma unroll
+        for (int w = 0; w < NW; w++) r[w] = __shfl(r[w], 0, GL);
     }
-    const unsigned long long n0 = m0 & ~r0, n1 = m1 & ~r1;
-    const int c0 = __popcll(n0);
-    if ((n0 >> gl) & 1) {
-        const int pos = __popcll(n0 & below);
-        snd[pos] = j0;
-        sdl[pos] = sD[j0];
-        szl[pos] = sz[j0];
+    int c0 = 0;
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+        const u64 nw = m[w] & ~r[w];
+        if ((nw >> gl) & 1) {
+            const int pos = c0 + __popcll(nw & below);
+            snd[pos] = jw[w];
+            sdl[pos] = sD[jw[w]];
+            szl[pos] = sz[jw[w]];
+        }
+        c0 += __popcll(nw);
     }
-    if (TWO && ((n1 >> gl) & 1)) {
-        const int pos = c0 + __popcll(n1 & below);
-        snd[pos] = j1;
-        sdl[pos] = sD[j1];
-        szl[pos] = sz[j1];
-    }
-    Kn_out = c0 + __popcll(n1);
+    Kn_out = c0;
     nrot_out = nrot;
 }
 
@@ -763,7 +826,7 @@ __global__ __launch_bounds__(256) void k_dc_leaf(int n, const double *__restrict
                     rho = 2.0 * fabs(ee[b0 + m - 1]);
                     Kn = 0;
                     if (rho != 0.0)
-                        deflate<false>(s, gl, lane - gl, hi - lo, rho, sperm + lo, sz, sD,
+                        deflate<1>(s, gl, lane - gl, hi - lo, rho, sperm + lo, sz, sD,
                                        snd + lo, sdl + lo, szl + lo, ra + lo, rb + lo, rc + lo,
                                        rs + lo, Kn, nrot);
                 }
@@ -888,7 +951,7 @@ __global__ __launch_bounds__(256) void k_dc_leaf(int n, const double *__restrict
     if (tid < nb) lam[b0 + tid] = sD[tid];
     if (tid == 0) {
         iters[blockIdx.x] = s_iters;
-        if (blockIdx.x == 0) iters[4] = 0;
+        if (blockIdx.x == 0) iters[8] = 0;
     }
 }
 
@@ -944,7 +1007,7 @@ __global__ __launch_bounds__(16 * L) void k_dc_roots(int n, int s, const double 
     if (tid < 64) {
         int Kn = 0, nrot = 0;
         if (rho != 0.0)
-            deflate<(S > 64)>(64, tid, 0, K, rho, sperm, sz, sD, snd, sdl, szl, ra, rb, rc, rs, Kn,
+            deflate<(S + 63) / 64>(64, tid, 0, K, rho, sperm, sz, sD, snd, sdl, szl, ra, rb, rc, rs, Kn,
                               nrot);
         if (tid == 0) {
             s_kn = Kn;
@@ -962,7 +1025,7 @@ __global__ __launch_bounds__(16 * L) void k_dc_roots(int n, int s, const double 
             st.dorg[lo + i] = sdl[org];
             st.tau[lo + i] = tau;
             lam_out[lo + snd[i]] = sdl[org] + tau;
-            if (it > 0) atomicMax(st.iters + 4, it);
+            if (it > 0) atomicMax(st.iters + 8, it);
         }
     }
     if (g != 0) return;
@@ -990,17 +1053,18 @@ __global__ __launch_bounds__(16 * L) void k_dc_roots(int n, int s, const double 
 // Second half, of a merge below the top: workgroup g of a block forms the new
 // columns of Z at roots 16 g .. 16 g + 15 and copies the deflated ones among the
 // block's columns 16 g .. 16 g + 15, from Zin into Zout (whole columns, zero
-// outside the block).
+// outside the block).  A workgroup takes 64 rows of the block's.
 template <int S>
 __global__ __launch_bounds__(256) void k_dc_vecs(int n, int s, const double *__restrict__ Zin,
                                                  double *__restrict__ Zout, DcState st) {
-    static_assert(S == 64, "a wave per 16 rows of the block");
-    constexpr int LD = S + 1;
+    constexpr int LD = 65, NCH = S / 64;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int gpb = (s + 15) >> 4, b = blockIdx.x / gpb, g = blockIdx.x - b * gpb;
+    const int gpb = (s + 15) >> 4, r0 = 64 * (blockIdx.x % NCH), bg = blockIdx.x / NCH;
+    const int b = bg / gpb, g = bg - b * gpb;
     const int lo = b * s, hi = min(lo + s, n), K = hi - lo;
-    __shared__ double Zs[S * LD];      // Zs[r + LD j]
-    __shared__ double us[S * 17];      // U[q][c] of the 16 own columns
+    extern __shared__ double vlds[];
+    double *Zs = vlds;          // Zs[r - r0 + LD j]
+    double *us = Zs + S * LD;   // U[q][c] of the 16 own columns
     __shared__ double sdl[S], szl[S], stau[S], sdo[S], szh[S], sinv[16], rc[S], rs[S];
     __shared__ int snd[S], sflag[S], ra[S], rb[S];
     const int Kn = max(st.kn[b], 0), nrot = Kn > 0 || st.kn[b] == 0 ? st.nrot[b] : 0;
@@ -1010,7 +1074,7 @@ __global__ __launch_bounds__(256) void k_dc_vecs(int n, int s, const double *__r
 #pragma unroll
         for (int t = 0; t < S / 4; t++) {
             const int j = wv + 4 * t;
-            z[t] = (lane < K && j < K) ? Zin[lo + lane + (long)(lo + j) * n] : 0.0;
+            z[t] = (r0 + lane < K && j < K) ? Zin[lo + r0 + lane + (long)(lo + j) * n] : 0.0;
         }
 #pragma unroll
         for (int t = 0; t < S / 4; t++) Zs[lane + LD * (wv + 4 * t)] = z[t];
@@ -1031,8 +1095,8 @@ __global__ __launch_bounds__(256) void k_dc_vecs(int n, int s, const double *__r
     }
     __syncthreads();
     if (tid < Kn) sflag[snd[tid]] = 1;
-    if (tid >= 128 && tid < 128 + K) {  // the deflating rotations, a thread a row
-        const int r = tid - 128;
+    if (tid >= 192) {  // the deflating rotations, a thread a row
+        const int r = tid - 192;
         for (int t = 0; t < nrot; t++) {
             const int ia = r + LD * ra[t], ib = r + LD * rb[t];
             const double qa = Zs[ia], qb = Zs[ib], c = rc[t], sn = rs[t];
@@ -1041,9 +1105,10 @@ __global__ __launch_bounds__(256) void k_dc_vecs(int n, int s, const double *__r
         }
     }
     {
-        const int q = tid >> 2, sub = tid & 3;
+        constexpr int LP = 256 / S;
+        const int q = tid / LP, sub = tid & (LP - 1);
         if (q < Kn) {
-            const double z = zhat_entry<4>(q, Kn, sub, rho, sdl, sdo, stau, szl[q]);
+            const double z = zhat_entry<LP>(q, Kn, sub, rho, sdl, sdo, stau, szl[q]);
             if (sub == 0) szh[q] = z;
         }
     }
@@ -1076,13 +1141,15 @@ __global__ __launch_bounds__(256) void k_dc_vecs(int n, int s, const double *__r
     }
 #pragma unroll
     for (int v = 0; v < 4; v++) {
-        const int c = (lane >> 4) + 4 * v, i = 16 * g + c, r = 16 * wv + (lane & 15);
+        const int c = (lane >> 4) + 4 * v, i = 16 * g + c, r = r0 + 16 * wv + (lane & 15);
         if (i < Kn && r < K) Zout[lo + r + (long)(lo + snd[i]) * n] = acc[v] * sinv[c];
     }
     // deflated columns, and the zeros outside the block of every column written
     for (int c = wv; c < 16; c += 4) {
         const int i = 16 * g + c;
-        if (i < K && !sflag[i] && lane < K) Zout[lo + lane + (long)(lo + i) * n] = Zs[lane + LD * i];
+        if (i < K && !sflag[i] && r0 + lane < K)
+            Zout[lo + r0 + lane + (long)(lo + i) * n] = Zs[lane + LD * i];
+        if (r0 != 0) continue;
         for (int r = lane; r < n; r += 64)
             if (r < lo || r >= hi) {
                 if (i < Kn) Zout[r + (long)(lo + snd[i]) * n] = 0.0;
@@ -1214,7 +1281,7 @@ __global__ __launch_bounds__(256) void k_dc_top(int n, DcState st, const double 
     }
     __syncthreads();
     const int es = *eexp;
-    // Wave 0 holds the descending values two per lane and decides:
+    // Wave 0 holds the descending values lane + 64 w and decides:
     //  - the smallest eigenvalues are dropped while their running sum stays
     //    within lim = budget * lmax: the suffix sums S(q) and the values grow
     //    as q falls, so the dropped set is {q >= keep} with keep the least q
@@ -1227,34 +1294,56 @@ __global__ __launch_bounds__(256) void k_dc_top(int n, DcState st, const double 
     // set bit of a ballot.
     __shared__ int s_keep;
     if (wv == 0) {
-        const bool in0 = lane < n, in1 = lane + 64 < n;
-        const double h0 = in0 ? fmax(sdl[lane < S ? lane : 0], 0.0) : 0.0;
-        const double h1 = in1 ? fmax(sdl[lane + 64 < S ? lane + 64 : 0], 0.0) : 0.0;
-        const double lmax = readlane_d(h0, 0);
+        constexpr int NW = (S + 63) / 64;
+        double h[NW], suf[NW];
+#pragma unroll
+        for (int w = 0; w < NW; w++)
+            h[w] = lane + 64 * w < n ? fmax(sdl[lane + 64 * w < S ? lane + 64 * w : 0], 0.0) : 0.0;
+        const double lmax = readlane_d(h[0], 0);
         const double lim = budget * lmax;
-        const double S1 = suffix_sum(h1);
-        const double S0 = suffix_sum(h0) + readlane_d(S1, 0);
-        const unsigned long long k0 = __ballot(in0 && S0 <= lim && h0 < lmax);
-        const unsigned long long k1 = __ballot(in1 && S1 <= lim && h1 < lmax);
-        const int keep = k0 ? __ffsll((long long)k0) - 1 : (k1 ? 63 + __ffsll((long long)k1) : n);
-        const double cum = (keep >= n) ? 0.0 : (keep < 64 ? readlane_d(S0, keep) : readlane_d(S1, keep - 64));
+        // suffix sums of x over all words, into suf
+        auto suffix = [&](const double(&x)[NW]) {
+            double rest = 0.0;
+#pragma unroll
+            for (int w = NW - 1; w >= 0; w--) {
+                suf[w] = w == NW - 1 ? suffix_sum(x[w]) : suffix_sum(x[w]) + rest;
+                rest = readlane_d(suf[w], 0);
+            }
+        };
+        suffix(h);
+        int keep = n;
+        double cum = 0.0;
+#pragma unroll
+        for (int w = NW - 1; w >= 0; w--) {
+            const unsigned long long k =
+                __ballot(lane + 64 * w < n && suf[w] <= lim && h[w] < lmax);
+            if (k) {
+                keep = 64 * w + __ffsll((long long)k) - 1;
+                cum = readlane_d(suf[w], keep & 63);
+            }
+        }
         const double thr2 = (double)n * EPSU * EPSU * lmax;  // (sqrt(n) u sigma_0)^2
         int numrank = 0;
         if (lmax > 0.0)
-            numrank = __popcll(__ballot(lane < keep && h0 > thr2)) +
-                      __popcll(__ballot(lane + 64 < keep && h1 > thr2));
+#pragma unroll
+            for (int w = 0; w < NW; w++)
+                numrank += __popcll(__ballot(lane + 64 * w < keep && h[w] > thr2));
         const double dl2 =
             (delta > 0.0) ? exp(2.0 * (log(delta) - (es / 2) * 0.6931471805599453)) : -1.0;
-        const double T1 = suffix_sum(lane + 64 < numrank ? h1 : 0.0);
-        const double T0 = suffix_sum(lane < numrank ? h0 : 0.0) + readlane_d(T1, 0);
-        const unsigned long long c0 = __ballot(lane < numrank && T0 < dl2);
-        const unsigned long long c1 = __ballot(lane + 64 < numrank && T1 < dl2);
-        int rho = c0 ? __ffsll((long long)c0) - 1 : (c1 ? 63 + __ffsll((long long)c1) : numrank);
+#pragma unroll
+        for (int w = 0; w < NW; w++) h[w] = lane + 64 * w < numrank ? h[w] : 0.0;
+        suffix(h);
+        int rho = numrank;
+#pragma unroll
+        for (int w = NW - 1; w >= 0; w--) {
+            const unsigned long long k = __ballot(lane + 64 * w < numrank && suf[w] < dl2);
+            if (k) rho = 64 * w + __ffsll((long long)k) - 1;
+        }
         if (rho > n) rho = n;
         if (rho > cap) rho = cap;
         if (rho < 1) rho = 1;
         if (lane == 0) {
-            int it = st.iters[4];
+            int it = st.iters[8];
             for (int q = 0; 32 * q < n; q++) it = max(it, st.iters[q]);
             iout[0] = numrank;
             iout[1] = rho;
@@ -1271,63 +1360,70 @@ __global__ __launch_bounds__(256) void k_dc_top(int n, DcState st, const double 
 // ---- 3. back transformation -----------------------------------------------
 // W = H_0 H_1 ... H_{n-3} Z, the reflectors applied last first.  Sixteen lanes (one DPP row) own a column, each holding the rows
 // l, l+16, ..., so a reflector's dot product reduces inside the row; a
-// workgroup of four waves owns 16 columns and stages the reflectors in LDS.
-constexpr int ORM_RPL = EIG_NMAX / 16;  // rows per lane
-__global__ __launch_bounds__(256) void k_ormtr(int n, const double *__restrict__ Vh,
+// workgroup of four waves owns 16 columns and stages the reflectors in LDS, `ch`
+// at a time (all of them up to 128 rows).
+template <int RPL>  // rows per lane
+__global__ __launch_bounds__(256) void k_ormtr(int n, int ch, const double *__restrict__ Vh,
                                                const double *__restrict__ tau,
                                                const double *__restrict__ Z,
                                                double *__restrict__ W) {
-    extern __shared__ double vs[];  // n x n reflectors, then n taus
+    extern __shared__ double vs[];  // ch x n reflectors, then n taus
     const int tid = threadIdx.x;
-    const long nn = (long)n * n;
-    for (long e0 = tid; e0 < nn; e0 += 4 * 256) {
-        double v[4];
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const long e = e0 + (long)u * 256;
-            v[u] = (e < nn) ? Vh[e] : 0.0;
-        }
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const long e = e0 + (long)u * 256;
-            if (e < nn) vs[e] = v[u];
-        }
-    }
-    for (int i = tid; i < n; i += 256) vs[nn + i] = tau[i];
-    __syncthreads();
     const int l = tid & 15;
     const int c = blockIdx.x * 16 + (tid >> 4);
     const bool live = c < n;  // rows of 16 lanes: uniform per DPP row
     const double *zc = Z + (long)(live ? c : 0) * n;
-    double x[ORM_RPL];
+    double x[RPL];
 #pragma unroll
-    for (int m = 0; m < ORM_RPL; m++) {
+    for (int m = 0; m < RPL; m++) {
         const int i = l + 16 * m;
         x[m] = (live && i < n) ? zc[i] : 0.0;
     }
-    for (int k = n - 3; k >= 0; k--) {
-        const double tk = vs[nn + k];
-        if (tk == 0.0) continue;
-        const double *v = vs + (long)k * n;
-        double vr[ORM_RPL];
-        double d0 = 0.0, d1 = 0.0;
+    double *ts = vs + (long)ch * n;
+    for (int i = tid; i < n; i += 256) ts[i] = tau[i];
+    for (int k1 = n; k1 > 0; k1 -= ch) {  // reflectors kb .. k1 - 1
+        const int kb = k1 > ch ? k1 - ch : 0;
+        const long cnt = (long)(k1 - kb) * n;
+        const double *src = Vh + (long)kb * n;
+        if (k1 < n) __syncthreads();
+        for (long e0 = tid; e0 < cnt; e0 += 4 * 256) {
+            double v[4];
 #pragma unroll
-        for (int m = 0; m < ORM_RPL; m++) {
-            const int i = l + 16 * m;
-            vr[m] = (i < n) ? v[i] : 0.0;
-            if (m & 1) d1 = fma(vr[m], x[m], d1);
-            else d0 = fma(vr[m], x[m], d0);
+            for (int u = 0; u < 4; u++) {
+                const long e = e0 + (long)u * 256;
+                v[u] = (e < cnt) ? src[e] : 0.0;
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const long e = e0 + (long)u * 256;
+                if (e < cnt) vs[e] = v[u];
+            }
         }
-        double dt = quad_sum(d0 + d1);
-        dt += dppd<0x141>(dt);
-        dt += dppd<0x140>(dt);
-        dt *= tk;
+        __syncthreads();
+        for (int k = min(k1 - 1, n - 3); k >= kb; k--) {
+            const double tk = ts[k];
+            if (tk == 0.0) continue;
+            const double *v = vs + (long)(k - kb) * n;
+            double vr[RPL];
+            double d0 = 0.0, d1 = 0.0;
 #pragma unroll
-        for (int m = 0; m < ORM_RPL; m++) x[m] = fma(-dt, vr[m], x[m]);
+            for (int m = 0; m < RPL; m++) {
+                const int i = l + 16 * m;
+                vr[m] = (i < n) ? v[i] : 0.0;
+                if (m & 1) d1 = fma(vr[m], x[m], d1);
+                else d0 = fma(vr[m], x[m], d0);
+            }
+            double dt = quad_sum(d0 + d1);
+            dt += dppd<0x141>(dt);
+            dt += dppd<0x140>(dt);
+            dt *= tk;
+#pragma unroll
+            for (int m = 0; m < RPL; m++) x[m] = fma(-dt, vr[m], x[m]);
+        }
     }
     if (live)
 #pragma unroll
-        for (int m = 0; m < ORM_RPL; m++) {
+        for (int m = 0; m < RPL; m++) {
             const int i = l + 16 * m;
             if (i < n) W[i + (long)c * n] = x[m];
         }
@@ -1347,18 +1443,31 @@ __global__ void k_svd_factors_perm(int m, int rho, const int *__restrict__ colid
     }
 }
 
-void ormtr_attr() {
+constexpr int ORM_LDS_DOUBLES = 128 * 128 + 256;
+
+void syev_attr() {
     static bool done = false;
     if (done) return;
-    HIPCHECK(hipFuncSetAttribute((const void *)k_ormtr, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                 (EIG_NMAX * EIG_NMAX + EIG_NMAX) * (int)sizeof(double)));
+    auto set = [](const void *f, int doubles) {
+        HIPCHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     doubles * (int)sizeof(double)));
+    };
+    set((const void *)k_ormtr<8>, ORM_LDS_DOUBLES);
+    set((const void *)k_ormtr<12>, ORM_LDS_DOUBLES);
+    set((const void *)k_dc_vecs<128>, 128 * (65 + 17));
     done = true;
 }
 
 void launch_ormtr(int c, const double *Vh, const double *tau, const double *Z, double *W) {
     const double cc = (double)c * c;
-    PTT_LAUNCH_FB("syev_ormtr", 4.0 * cc * c, 8.0 * 3.0 * cc, k_ormtr, dim3(cdiv(c, 16)),
-                  dim3(256), ((size_t)c * c + c) * sizeof(double), c, Vh, tau, Z, W);
+    const int ch = c * c + c <= ORM_LDS_DOUBLES ? c : (ORM_LDS_DOUBLES - c) / c;
+    const size_t shm = ((size_t)ch * c + c) * sizeof(double);
+    if (c <= 128)
+        PTT_LAUNCH_FB("syev_ormtr", 4.0 * cc * c, 8.0 * 3.0 * cc, k_ormtr<8>, dim3(cdiv(c, 16)),
+                      dim3(256), shm, c, ch, Vh, tau, Z, W);
+    else
+        PTT_LAUNCH_FB("syev_ormtr", 4.0 * cc * c, 8.0 * 3.0 * cc, k_ormtr<12>, dim3(cdiv(c, 16)),
+                      dim3(256), shm, c, ch, Vh, tau, Z, W);
 }
 
 // Workspace of one eigen-decomposition of order c: reflectors, Z twice (a merge
@@ -1402,31 +1511,45 @@ void syev_run(int c, const double *G, double *sig, double *U, long ldu, int *col
     st.rb = st.ra + c;
     st.kn = st.rb + c;
     st.nrot = st.kn + 4;
-    st.iters = st.nrot + 4;  // one per leaf workgroup (4), then the larger merges'
-    int *ex = st.iters + 8;
-    ormtr_attr();
+    st.iters = st.nrot + 4;  // one per leaf workgroup (up to 8), then the larger merges'
+    int *ex = st.iters + 10;
+    syev_attr();
     const double n = (double)c;
     if (c <= 64)
         PTT_LAUNCH_FB("syev_sytrd", 4.0 * n * n * n / 3.0, 8.0 * n * n * 2.0, k_sytrd<64>, dim3(1),
                       dim3(4 * 64 + 64), 0, c, G, (long)c, Vh, tau, d, e, ex, dinfo);
-    else
+    else if (c <= 128)
         PTT_LAUNCH_FB("syev_sytrd", 4.0 * n * n * n / 3.0, 8.0 * n * n * 2.0, k_sytrd<128>, dim3(1),
                       dim3(4 * 128 + 64), 0, c, G, (long)c, Vh, tau, d, e, ex, dinfo);
+    else
+        PTT_LAUNCH_FB("syev_sytrd", 4.0 * n * n * n / 3.0, 8.0 * n * n * 2.0, k_sytrd<192>, dim3(1),
+                      dim3(2 * 192 + 64), 0, c, G, (long)c, Vh, tau, d, e, ex, dinfo);
     int top = 2;
     while (top < c) top *= 2;
     PTT_LAUNCH_FB("syev_leaf", 2.0 * 32.0 * 32.0 * n, 8.0 * n * n, k_dc_leaf, dim3(cdiv(c, DCL)),
                   dim3(256), 0, c, d, e, Z, lam, top / 2 < DCL ? top / 2 : DCL, st.iters);
-    if (top == 128) {  // the two blocks of 64
-        PTT_LAUNCH_FB("syev_roots", 60.0 * 64.0 * n, 8.0 * 4.0 * n, (k_dc_roots<64, 16>), dim3(2 * 4),
-                      dim3(256), 0, c, 64, e, Z, lam, lam2, st);
+    auto swap = [](double *&a, double *&b) {
+        double *t = a;
+        a = b;
+        b = t;
+    };
+    if (top >= 128) {  // blocks of 64
+        const int nb = (int)cdiv(c, 64);
+        PTT_LAUNCH_FB("syev_roots", 60.0 * 64.0 * n, 8.0 * 4.0 * n, (k_dc_roots<64, 16>),
+                      dim3(nb * 4), dim3(256), 0, c, 64, e, Z, lam, lam2, st);
         PTT_LAUNCH_FB("syev_vecs", 2.0 * 64.0 * 64.0 * n, 8.0 * 2.0 * n * n, k_dc_vecs<64>,
-                      dim3(2 * 4), dim3(256), 0, c, 64, Z, Z2, st);
-        double *t = Z;
-        Z = Z2;
-        Z2 = t;
-        t = lam;
-        lam = lam2;
-        lam2 = t;
+                      dim3(nb * 4), dim3(256), 64 * (65 + 17) * sizeof(double), c, 64, Z, Z2, st);
+        swap(Z, Z2);
+        swap(lam, lam2);
+    }
+    if (top == 256) {  // blocks of 128 (the second may hold no more than 64 rows)
+        PTT_LAUNCH_FB("syev_roots", 60.0 * 128.0 * n, 8.0 * 4.0 * n, (k_dc_roots<128, 32>),
+                      dim3(2 * 8), dim3(512), 0, c, 128, e, Z, lam, lam2, st);
+        PTT_LAUNCH_FB("syev_vecs", 2.0 * 128.0 * 128.0 * n, 8.0 * 2.0 * n * n, k_dc_vecs<128>,
+                      dim3(2 * 8 * 2), dim3(256), 128 * (65 + 17) * sizeof(double), c, 128, Z, Z2,
+                      st);
+        swap(Z, Z2);
+        swap(lam, lam2);
     }
     const bool side = ptt_hip_side_enabled();
     if (side) {
@@ -1434,7 +1557,10 @@ void syev_run(int c, const double *G, double *sig, double *U, long ldu, int *col
         launch_ormtr(c, Vh, tau, Z, W);
         ptt_hip_side_end(0);
     }
-    if (top == 128)
+    if (top == 256)
+        launch_top<EIG_NMAX>(c, top, e, Z, lam, lam2, st, ex, Um, colidx, sig, iout, dinfo, delta,
+                             cap, budget);
+    else if (top == 128)
         launch_top<128>(c, top, e, Z, lam, lam2, st, ex, Um, colidx, sig, iout, dinfo, delta, cap,
                         budget);
     else if (top == 64)
@@ -1451,7 +1577,7 @@ void syev_run(int c, const double *G, double *sig, double *U, long ldu, int *col
 // Fixed workspace of the entry point that allocates nothing: one copy per
 // GPU, held until the process ends.  Host code reaches it only through the
 // device address from hipGetSymbolAddress (the name is a host stand-in).
-constexpr int NOALLOC_CMAX = EIG_NMAX;
+constexpr int NOALLOC_CMAX = 128;
 __device__ __align__(256) double scratch[syev_ws_doubles(NOALLOC_CMAX)];
 constexpr int NOALLOC_MAXDEV = 64;
 double *g_scratch_dev[NOALLOC_MAXDEV] = {nullptr};

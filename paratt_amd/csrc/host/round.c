@@ -627,7 +627,7 @@ static int rtl_step_fast(attac_tt *x, int i, const int *maxr, double delta,
     if (rows > 1024) return -1;
     ptt_hip_gram('N', rows, w, M, rows, ws->G);
     rside_flush(); /* the previous bond's new core beside this bond's eigensolver */
-    const int eig = (rows <= 128) && gram_use_eig();
+    const int eig = (rows <= 192) && gram_use_eig();
     int *cidx = (int *)ws->Rtmp;
     if (eig) {
         /* G = U diag(sig^2) U^T; eigenvalues below the Gram's own rounding
@@ -664,7 +664,7 @@ static int rtl_step_fast(attac_tt *x, int i, const int *maxr, double delta,
     const unsigned long long tk = ptt_hip_d2h_begin(ws->sig, nb);
     const int spec = eig ? (maxr[i] < rows ? maxr[i] : rows) : 0;
     /* the new core may go to the side stream (decided once sigma is read) */
-    const int side_ok = spec > 0 && x->coreMem != NULL && ptt_hip_side_enabled() &&
+    const int side_ok = spec > 0 && rows <= 128 && x->coreMem != NULL && ptt_hip_side_enabled() &&
                         (double)spec * rows * (double)w >= 0x1.0p28;
     const int sp = g_rside_parity;
     double *Wspec = ws->W;
