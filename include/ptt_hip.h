@@ -211,6 +211,10 @@ void ptt_hip_svd_jacobi(int m, int k, double *A, long lda, double *sig,
  * sweeps} as in ptt_hip_svd_jacobi; iout needs 5 ints. */
 void ptt_hip_svd_right(int k, const double *R, long ldr, double *X, double *sig, double *V,
                        long ldv, double delta, int cap, int *iout);
+/* The same for k <= 192 from approximate left singular vectors U (k x k, ldu,
+ * orthogonal, any order; may be V): nothing is dropped. */
+void ptt_hip_svd_right_from(int k, const double *R, long ldr, const double *U, long ldu, double *X,
+                            double *sig, double *V, long ldv, double delta, int cap, int *iout);
 /* From U (m x k, ldu) and sig: W (rho x m, ld rho) = diag(1/sig) U_rho^T
  * scaled by wscale, and US (m x rho, ld m) = U_rho diag(sig).
  * rho is read from device *drho, or is rhomax when drho is NULL.  Either

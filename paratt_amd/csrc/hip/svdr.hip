@@ -28,6 +28,7 @@ using namespace ptt;
 namespace {
 
 constexpr int SR_K = 128;
+constexpr int SR_KMAX = 192;  // started from approximate vectors
 constexpr int RJ_NT = 512;  // Jacobi
 
 // Column q of L is row q of R.  Lane li of a 16-lane row holds columns li + 16
@@ -315,6 +316,34 @@ __device__ int right_sweeps(double *X, int ld, int r, int k, double *nrm, int *f
     return sweep < 40 ? sweep + 1 : 40;
 }
 
+// X (k x k, k <= 64) to entries of order one by an exact power of two; all of its
+// columns count.  One workgroup.
+__global__ __launch_bounds__(256) void k_right_start(int k, double *__restrict__ X,
+                                                     int *__restrict__ nform) {
+    __shared__ double red[4];
+    double x[16], m = 0.0;
+#pragma unroll
+    for (int t = 0; t < 16; t++) {
+        const int e = threadIdx.x + 256 * t;
+        x[t] = e < k * k ? X[e] : 0.0;
+        m = fmax(m, fabs(x[t]));
+    }
+    m = wave_max(m);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    m = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
+    const int ex = (m > 0.0 && m < INFINITY) ? ilogb(m) : 0;
+#pragma unroll
+    for (int t = 0; t < 16; t++) {
+        const int e = threadIdx.x + 256 * t;
+        if (e < k * k) X[e] = ldexp(x[t], -ex);
+    }
+    if (threadIdx.x == 0) {
+        nform[0] = k;
+        nform[1] = ex;
+    }
+}
+
 // r <= 64 columns; KR: rows of a column in LDS (k rounded up to 64 or 128).
 template <int KR>
 __global__ __launch_bounds__(RJ_NT) void k_right_jacobi(int k, const double *__restrict__ Xg,
@@ -389,6 +418,28 @@ __global__ __launch_bounds__(RJ_NT) void k_right_jacobi(int k, const double *__r
     }
 }
 
+// k_right_jacobi on the nform[0] <= 64 columns of X.
+void right_jacobi(int k, const double *X, const int *nform, double *sig, double *V, long ldv,
+                  double delta, int cap, int *iout) {
+    static bool attr = false;
+    if (!attr) {
+        auto set = [](const void *f, int rows) {
+            HIPCHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                         64 * (rows + 1) * (int)sizeof(double)));
+        };
+        set((const void *)k_right_jacobi<64>, 64);
+        set((const void *)k_right_jacobi<128>, 128);
+        attr = true;
+    }
+    const double jf = 12.0 * k * (double)k * k, jb = 16.0 * k * (double)k;
+#define PTT_RJ(KR)                                                                          \
+    PTT_LAUNCH_FB("svd_right_jacobi", jf, jb, k_right_jacobi<KR>, dim3(1), dim3(RJ_NT),        \
+                  64 * (KR + 1) * sizeof(double), k, X, nform, sig, V, ldv, delta, cap, iout)
+    if (k <= 64) PTT_RJ(64);
+    else PTT_RJ(128);
+#undef PTT_RJ
+}
+
 }  // namespace
 
 extern "C" {
@@ -402,16 +453,6 @@ void ptt_hip_svd_right(int k, const double *R, long ldr, double *X, double *sig,
     if (k < 1 || k > SR_K) {
         fprintf(stderr, "ptt_hip_svd_right: k = %d out of range\n", k);
         exit(1);
-    }
-    static bool attr = false;
-    if (!attr) {
-        auto set = [](const void *f, int rows) {
-            HIPCHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         64 * (rows + 1) * (int)sizeof(double)));
-        };
-        set((const void *)k_right_jacobi<64>, 64);
-        set((const void *)k_right_jacobi<128>, 128);
-        attr = true;
     }
     int *nform = iout + 3;
     const double fl = 4.0 / 3.0 * k * (double)k * k;
@@ -437,13 +478,27 @@ void ptt_hip_svd_right(int k, const double *R, long ldr, double *X, double *sig,
             return;
         }
     }
-    const double jf = 12.0 * k * (double)k * k, jb = 16.0 * k * (double)k;
-#define PTT_RJ(KR)                                                                          \
-    PTT_LAUNCH_FB("svd_right_jacobi", jf, jb, k_right_jacobi<KR>, dim3(1), dim3(RJ_NT),        \
-                  64 * (KR + 1) * sizeof(double), k, X, nform, sig, V, ldv, delta, cap, iout)
-    if (k <= 64) PTT_RJ(64);
-    else PTT_RJ(128);
-#undef PTT_RJ
+    right_jacobi(k, X, nform, sig, V, ldv, delta, cap, iout);
+}
+
+// The rotations start from U, orthogonal up to rounding, whose columns approximate
+// L's left singular vectors: the columns of X = R U are then nearly orthogonal
+// already (R U = V Sigma for the exact ones), two or three sweeps instead of six to
+// ten, and no pivoted QR.
+void ptt_hip_svd_right_from(int k, const double *R, long ldr, const double *U, long ldu, double *X,
+                            double *sig, double *V, long ldv, double delta, int cap, int *iout) {
+    ptt_hip_init();
+    if (k < 1 || k > SR_KMAX) {
+        fprintf(stderr, "ptt_hip_svd_right_from: k = %d out of range\n", k);
+        exit(1);
+    }
+    ptt_hip_dgemm('N', 'N', k, k, k, 1.0, R, ldr, U, ldu, 0.0, X, k);
+    if (k > 64) {
+        ptt_hip_svd_jacobi(k, k, X, k, sig, V, ldv, nullptr, 0, 0.0, delta, cap, iout);
+        return;
+    }
+    PTT_LAUNCH("svd_right_start", k_right_start, dim3(1), dim3(256), 0, k, X, iout + 3);
+    right_jacobi(k, X, iout + 3, sig, V, ldv, delta, cap, iout);
 }
 
 }  // extern "C"

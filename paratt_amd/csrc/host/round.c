@@ -494,15 +494,19 @@ static int tail_rule(const double *sig, int nsig, double tail0, double delta) {
  * Matrix Anal. Appl. 29, 2008), applied statically as on the Gram route,
  * which cuts the Jacobi sweeps on graded bonds.  With P M = L Q and L =
  * U Sigma V^T, M = (P^T U) Sigma (V^T Q): the new core is unchanged and only
- * the rows of U Sigma are put back. */
+ * the rows of U Sigma are put back.
+ * warm: the Gram route has just refused the bond and left its Gram in ws->G and
+ * its vectors U in ws->V, which resolve every direction: the Jacobi starts from
+ * R U, at any number of rows the Gram route takes. */
 static int rtl_step_robust(attac_tt *x, int i, const int *maxr, double delta,
-                           const double *nscale, step_ws *ws, int *passes_out) {
+                           const double *nscale, step_ws *ws, int *passes_out, int warm) {
     int *r = x->ttRank, *n = x->dim;
     int rows = r[i];
     long w = (long)n[i] * r[i + 1];
     const double *R = NULL, *T1 = NULL;
     int one_pass = 0;
-    const int right = rows <= 128 && !g_whole_spectra;
+    if (g_whole_spectra) warm = 0;
+    const int right = (rows <= 128 || warm) && !g_whole_spectra;
     const int sorted = !right && rows >= 8 && rows <= 1024;
     int *perm = (int *)ws->W; /* W is free on this route */
     if (sorted) {
@@ -513,9 +517,13 @@ static int rtl_step_robust(attac_tt *x, int i, const int *maxr, double delta,
         ptt_hip_permute_rows(rows, (int)w, perm, M, rows, t2, rows);
         ptt_hip_d2d(M, t2, sizeof(double) * (size_t)rows * w);
     }
-    int passes = cholqr_core_g(x, i, NULL, 'N', w, rows, 1.0, ws, &R, 0, &one_pass, &T1, sorted);
+    int passes = cholqr_core_g(x, i, NULL, 'N', w, rows, 1.0, ws, &R, 0, &one_pass, &T1,
+                               sorted || warm);
     *passes_out = passes;
-    if (right) {
+    if (warm) {
+        ptt_hip_svd_right_from(rows, R, rows, ws->V, rows, ws->U, ws->sig, ws->V, rows, delta,
+                               maxr[i], ws->iinfo + 1);
+    } else if (right) {
         ptt_hip_svd_right(rows, R, rows, ws->U, ws->sig, ws->V, rows, delta, maxr[i],
                           ws->iinfo + 1);
     } else {
@@ -553,7 +561,8 @@ static int rtl_step_robust(attac_tt *x, int i, const int *maxr, double delta,
  * itself, so the tail rule is decided exactly as with an orthogonal LQ;
  * the residual is skipped when the trace alone shows that the cap binds.
  * Returns rho, or a negative value when the step must be redone by the
- * robust path (the core is left unchanged in that case). */
+ * robust path (the core is left unchanged in that case; -3: ws->G and ws->V
+ * hold its Gram and vectors that resolve every direction). */
 /* Accuracy of the Gram route against an orthogonal (LQ) factorization for a
  * cut after rho of the rows singular values sig (descending): the Gram's
  * rounding, ~ rows*u*s0^2, turns the kept subspace by about
@@ -688,6 +697,8 @@ static int rtl_step_fast(attac_tt *x, int i, const int *maxr, double delta,
     const int *io = (const int *)(hb + rows + 8) + 1;
     int numrank = io[0];
     if (i < 64) { g_stats.svd_sweeps[i] = io[2]; g_stats.numrank[i] = numrank; }
+    /* refused: -3 when the vectors in ws->V resolve every direction */
+    const int refused = (eig && numrank == rows) ? -3 : -2;
     int cap = maxr[i] < rows ? maxr[i] : rows;
     int rho0 = cap < numrank ? cap : numrank;
     if (rho0 < 1) rho0 = 1;
@@ -707,7 +718,7 @@ static int rtl_step_fast(attac_tt *x, int i, const int *maxr, double delta,
     if (side_ok && rho0 == spec && cut_at_cap) {
         if (!gram_route_accurate(sig, rows, rho0, hb[rows + 5])) {
             free(hb);
-            return -2;
+            return refused;
         }
         g_rside_parity ^= 1;
         double *B = (double *)ptt_hip_scratch(PTT_WS_ROUT0 + sp,
@@ -791,7 +802,7 @@ static int rtl_step_fast(attac_tt *x, int i, const int *maxr, double delta,
     if (trust) trust = gram_route_accurate(sig, rows, rho, hb[rows + 5]);
     if (!trust) {
         free(hb);
-        return -2;
+        return refused;
     }
     if (rho < rho0) {
         /* keep the first rho rows of the new core and the first rho columns of U Sigma */
@@ -934,8 +945,9 @@ static void rtl_sweep(attac_tt *x, const int *maxr, double abs_tol, const double
             if (i < 64) g_spec[i][19] = (sk > 0) ? 1.0 : 0.0;
             prev_robust = (rho < 0);
             if (rho < 0) {
+                const int warm = (rho == -3);
                 int passes = 0;
-                rho = rtl_step_robust(x, i, maxr, delta, nscale, &ws, &passes);
+                rho = rtl_step_robust(x, i, maxr, delta, nscale, &ws, &passes, warm);
                 if (i < 64) g_stats.rtl_cholqr_passes[i] = 10 + passes;
                 /* a well-conditioned bond lets the next one try the Gram route */
                 if (i < 64 && g_stats.kappa_rtl[i] <= 1.0e2) prev_robust = 0;
