@@ -72,6 +72,9 @@ __global__ void k_chol_unscale(int c, const double *__restrict__ D, double *__re
     }
 }
 
+// Orders up to which k_chol_report iterates from registers: 16 waves of 12 rows.
+constexpr int CR_REG = 192;
+
 // Deficient pivots and the condition estimates, from G, D, R and T as the
 // smaller factors' kernels report them: Gershgorin's bound, else the pivots
 // where they decide, else power iterations.  binfo[b]: deficient pivots of
@@ -86,6 +89,7 @@ __global__ __launch_bounds__(NT) void k_chol_report(int c, const double *__restr
                                                     double *__restrict__ z, int *info,
                                                     double *dinfo, int want_kappa) {
     __shared__ double s_red[NT / 64], s_part[NT];
+    __shared__ double s_x[CR_REG], s_y[CR_REG], s_q[NT / 64][CR_REG];
     const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
     const int cpad = c < NT ? c : NT, parts = NT / cpad;
     auto block_sum = [&](double v) -> double {
@@ -149,7 +153,85 @@ __global__ __launch_bounds__(NT) void k_chol_report(int c, const double *__restr
         gersh = want_kappa && eoff < 0.5;
         decided = ndef > 0 || !(pmax <= 1e12 * pmin);
         const int PIT = (want_kappa && !gersh && !decided) ? 6 : 0;
-        for (int side = 0; side < 2; side++) {
+        if (PIT > 0 && c <= CR_REG) {
+            // the matrix in registers, rows 12 wv + 3 lg + v, columns li + 16 q; S
+            // first, then Ts^T (beyond this order every product reads it from
+            // memory: 246 us at 192 columns)
+            const int li = lane & 15, lg = lane >> 4, r0 = 12 * wv + 3 * lg;
+            double m[3][12];
+            auto load = [&](const double *__restrict__ A, const double *__restrict__ cs,
+                            const double *__restrict__ rs) {
+#pragma unroll
+                for (int v = 0; v < 3; v++)
+#pragma unroll
+                    for (int q = 0; q < 12; q++) {
+                        const int r = r0 + v, k = li + 16 * q;
+                        m[v][q] = (r < c && k < c)
+                                      ? A[k + (long)r * c] * cs[k] * (rs ? rs[r] : 1.0) : 0.0;
+                    }
+            };
+            // y = m x, by rows
+            auto rows = [&](const double *x, double *y) {
+                double t[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+                for (int q = 0; q < 12; q++) {
+                    const double xq = x[li + 16 * q];
+#pragma unroll
+                    for (int v = 0; v < 3; v++) t[v] = fma(m[v][q], xq, t[v]);
+                }
+#pragma unroll
+                for (int v = 0; v < 3; v++) t[v] = row16_sum(t[v]);
+                if (li < 3) y[r0 + li] = li == 0 ? t[0] : li == 1 ? t[1] : t[2];
+                __syncthreads();
+            };
+            // y = f m^T x, by columns
+            auto cols = [&](const double *x, double *y, double f) {
+                const double x0 = x[r0], x1 = x[r0 + 1], x2 = x[r0 + 2];
+#pragma unroll
+                for (int q = 0; q < 12; q++) {
+                    double t = fma(m[2][q], x2, fma(m[1][q], x1, fma(m[0][q], x0, 0.0)));
+                    t = xor32_sum(xor16_sum(t));
+                    if (lane < 16) s_q[wv][lane + 16 * q] = t;
+                }
+                __syncthreads();
+                if (tid < CR_REG) {
+                    double t = 0.0;
+#pragma unroll
+                    for (int w = 0; w < NT / 64; w++) t += s_q[w][tid];
+                    y[tid] = f * t;
+                }
+                __syncthreads();
+            };
+            auto norm2 = [&](const double *x) {
+                double t = 0.0;
+                for (int i = lane; i < CR_REG; i += 64) t = fma(x[i], x[i], t);
+                return wave_sum(t);
+            };
+            auto start = [&]() {
+                if (tid < CR_REG) s_x[tid] = tid < c ? 1.0 + 0.01 * (tid % 7) : 0.0;
+                __syncthreads();
+            };
+            // lambda_max(S) <= c: no scaling between the products
+            load(G, iD, iD);
+            start();
+            for (int it = 0; it < PIT; it += 2) {
+                rows(s_x, s_y);
+                rows(s_y, s_x);
+            }
+            lmax = sqrt(norm2(s_x) / norm2(s_y));
+            __syncthreads();
+            // lambda_max(Ts Ts^T) <= ft, divided out of every product
+            load(T, D, nullptr);
+            start();
+            double prev = 1.0;
+            for (int it = 0; it < PIT; it++) {
+                if (it == PIT - 1) prev = norm2(s_x);
+                rows(s_x, s_y);
+                cols(s_y, s_x, 1.0 / ft);
+            }
+            lminv = ft * sqrt(norm2(s_x) / prev);
+        }
+        for (int side = 0; side < 2 && c > CR_REG; side++) {
             for (int i = tid; i < c; i += NT) y[i] = 1.0 + 0.01 * (i % 7);
             __syncthreads();
             for (int it = 0; it < PIT; it++) {

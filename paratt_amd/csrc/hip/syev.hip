@@ -303,6 +303,7 @@ __global__ __launch_bounds__(sytrd_geom<NMAX>::NT) void k_sytrd(int n, const dou
                         for (int t = 0; t < TR; t++)
 #pragma unroll
                             for (int v = 0; v < 4; v++) acc[t][v] = fma(g[t][J][v], vj, acc[t][v]);
+                        if (!HOLD && J % 3 == 2) __asm__ __volatile__("" ::: "memory");
                     }
 #pragma unroll
                     for (int t = 0; t < TR; t++) {
@@ -332,6 +333,7 @@ __global__ __launch_bounds__(sytrd_geom<NMAX>::NT) void k_sytrd(int n, const dou
                         const double pj = pp[16 * J + gj];
                         if (HOLD) pJ[HOLD ? J : 0] = pj;
                         dot = fma(pj, HOLD ? vJ[HOLD ? J : 0] : vk[16 * J + gj], dot);
+                        if (!HOLD && J % 3 == 2) __asm__ __volatile__("" ::: "memory");
                     }
                     // p^T v over the 16 columns j of the row (each DPP row
                     // forms the same sum)
@@ -355,8 +357,9 @@ __global__ __launch_bounds__(sytrd_geom<NMAX>::NT) void k_sytrd(int n, const dou
 #pragma unroll
                             for (int v = 0; v < 4; v++)
                                 g[t][J][v] = fma(-vr[v], pj, fma(-vj, wr[v], g[t][J][v]));
+                            // (limits how many reads are hoisted)
+                            if (!HOLD && J % 3 == 2) __asm__ __volatile__("" ::: "memory");
                         }
-                        if (!HOLD) __asm__ __volatile__("" ::: "memory");
                     }
                 }
             }

@@ -485,6 +485,10 @@ static int tail_rule(const double *sig, int nsig, double tail0, double delta) {
     return rho;
 }
 
+/* Columns beyond which the SVD of a bond with more rows than columns starts from the
+ * eigenvectors of the small Gram. */
+#define TALL_WARM_MIN 32
+
 /* Robust right-to-left step: explicit LQ by (shifted) Cholesky-QR, SVD of
  * L, new core = V_rho^T Q.  Up to 128 rows the SVD pivots L's columns itself and
  * gives the right vectors alone: U Sigma = L V.  Beyond (and where the whole
@@ -916,8 +920,22 @@ static void rtl_sweep(attac_tt *x, const int *maxr, double abs_tol, const double
             /* L has only w columns: SVD of the core itself (M = L*Q with Q = I_w) */
             int k = (int)w;
             ws = get_ws(rows > k ? rows : k);
-            ptt_hip_svd_jacobi(rows, k, x->coreList[i], rows, ws.sig, ws.U, rows, ws.V, k, 0.0,
-                               delta, cap, ws.iinfo + 1);
+            if (k > TALL_WARM_MIN && k <= 192 && !g_whole_spectra && gram_use_eig()) {
+                /* The rotations start from M V0, V0 the eigenvectors of M^T M: its
+                 * columns are nearly orthogonal (any orthogonal V0 gives the same
+                 * result in more sweeps), and V = V0 times what they accumulate. */
+                ptt_hip_gram('T', k, rows, x->coreList[i], rows, ws.G);
+                ptt_hip_syev_gram(k, ws.G, ws.sig, ws.T1, k, (int *)ws.Rtmp, ws.iinfo + 1,
+                                  ws.dinfo, 0.0, k, 0.0);
+                ptt_hip_dgemm('N', 'N', rows, k, k, 1.0, x->coreList[i], rows, ws.T1, k, 0.0, ws.L,
+                              rows);
+                ptt_hip_svd_jacobi(rows, k, ws.L, rows, ws.sig, ws.U, rows, ws.T2, k, 0.0, delta,
+                                   cap, ws.iinfo + 1);
+                ptt_hip_dgemm('N', 'N', k, k, k, 1.0, ws.T1, k, ws.T2, k, 0.0, ws.V, k);
+            } else {
+                ptt_hip_svd_jacobi(rows, k, x->coreList[i], rows, ws.sig, ws.U, rows, ws.V, k, 0.0,
+                                   delta, cap, ws.iinfo + 1);
+            }
             int io[3];
             ptt_hip_d2h(io, ws.iinfo + 1, sizeof(int) * 3);
             g_hsig_n = 0;
