@@ -68,7 +68,8 @@ void ptt_hip_side_join(void);
  * is valid until the next call for the same slot with a larger size. */
 enum { PTT_WS_GRAM = 0, PTT_WS_SMALL, PTT_WS_TMP, PTT_WS_TMP2, PTT_WS_INT,
        PTT_WS_COEF, PTT_WS_SKETCH, PTT_WS_SMALL2, PTT_WS_RSK, PTT_WS_SIDE, PTT_WS_EIG,
-       PTT_WS_RES, PTT_WS_RSIDE, PTT_WS_ROUT0, PTT_WS_ROUT1, PTT_WS_TREE, PTT_WS_NSLOTS };
+       PTT_WS_RES, PTT_WS_RSIDE, PTT_WS_ROUT0, PTT_WS_ROUT1, PTT_WS_TREE, PTT_WS_QFACT,
+       PTT_WS_NSLOTS };
 void *ptt_hip_scratch(int slot, size_t bytes);
 /* Exchange the buffer of the TMP slot with a caller buffer: on return *buf
  * points at the old scratch (capacity *cap_bytes updated) and the slot owns

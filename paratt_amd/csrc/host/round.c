@@ -290,6 +290,25 @@ static double last_core_sumsq(attac_tt *x) {
  * the factorisation returns -1. */
 static int g_one_pass_only = 0;
 
+/* Condition of the last factor up to which Q may be left unformed (below). */
+#define KAPPA_UNFORMED 4.0
+
+/* Set during a rounding: where core k's last factor T goes (c x c, NULL beyond 128
+ * columns), and whether core k holds A with Q = qalpha A T left unformed.  The
+ * right-to-left sweep multiplies core k by U Sigma of the bond after it, so A (T U
+ * Sigma) takes one core-sized product instead of two: the last pass of a
+ * factorisation left a write and a read of every core (95 us at 131072 x 128,
+ * beside the main stream but on the same HBM and matrix cores) for a c x c by c x
+ * rho product.  Both orders round to u times the condition of T, but not with the same
+ * constant: at conditions up to 30 the cores of a rounding at n = 301, 59 columns were
+ * 1.4 times as far from LAPACK's (2.8e-12 against 2.0e-12), so only a T of condition
+ * at most KAPPA_UNFORMED is left. */
+typedef struct {
+    double *t, alpha;
+    int unformed;
+} q_factor;
+static q_factor *g_qf = NULL;
+
 /* Cholesky-QR of a core viewed as len x c (trans 'T': columns, LTR) or as
  * c x len (trans 'N': rows, RTL).  On return the core holds Q (alpha
  * applied) and R (c x c upper, A = Q*R resp. M = R^T*Q) is in *Rout.
@@ -316,12 +335,13 @@ static int cholqr_core_g(attac_tt *x, int core, double *buf, char trans, long le
      * orthogonality (mixed-precision CholeskyQR2: Yamazaki, Tomov and
      * Dongarra, SIAM J. Sci. Comput. 37, 2015). */
     const int leaf32 = g_leaf32 && trans == 'T' && !buf && c <= 128;
+    q_factor *qf = (trans == 'T' && !buf && g_qf && g_qf[core].t) ? &g_qf[core] : NULL;
     /* a one-pass bond's Q may go to the side stream: T is then factored
      * straight into a side buffer */
-    const int side_q = trans == 'T' && !buf && c <= 128 && len * c >= (1L << 22) &&
+    const int side_q = trans == 'T' && !buf && !qf && c <= 128 && len * c >= (1L << 22) &&
                        ptt_hip_side_enabled();
     int side_p = 0;
-    double *T1 = side_q ? side_tbuf(&side_p) : w->T1;
+    double *T1 = qf ? qf->t : side_q ? side_tbuf(&side_p) : w->T1;
     chol_out o;
     for (int t = 0; t < 2; t++) {
         if (t == 0 && gram_ready)
@@ -349,7 +369,10 @@ static int cholqr_core_g(attac_tt *x, int core, double *buf, char trans, long le
         }
         /* small products gain less from the overlap than the copy of T and
          * the stream events cost */
-        if (side_q)
+        if (qf && o.kappa <= KAPPA_UNFORMED) {
+            qf->alpha = qalpha;
+            qf->unformed = 1;
+        } else if (side_q)
             apply_right_side(x, core, len, c, T1, side_p, qalpha);
         else if (trans == 'T')
             apply_right(x, core, buf, len, c, T1, qalpha);
@@ -388,7 +411,7 @@ static int cholqr_core_g(attac_tt *x, int core, double *buf, char trans, long le
         A = buf ? buf : x->coreList[core];
         ptt_hip_gram(trans, c, len, A, trans == 'T' ? len : c, w->G);
         double *Rp = (passes % 2 == 0) ? w->R2 : w->R3;
-        double *Tp = (passes % 2 == 0) ? w->T2 : w->T3;
+        double *Tp = qf ? qf->t : (passes % 2 == 0) ? w->T2 : w->T3;
         chol_out q = run_chol(c, w->G, 0.0, Rp, Tp, w);
         if (q.deficient != 0 || q.kappa > KAPPA_TWO_PASS) {
             launch_chol_shifted(c, w->G, shift, Rp, Tp, w);
@@ -398,7 +421,10 @@ static int cholqr_core_g(attac_tt *x, int core, double *buf, char trans, long le
         }
         if (passes >= CHOLQR_MAX_PASSES) need = 0;
         const double a = (need == 0) ? qalpha : 1.0;
-        if (trans == 'T') apply_right(x, core, buf, len, c, Tp, a);
+        if (qf && need == 0 && q.deficient == 0 && q.kappa <= KAPPA_UNFORMED) {
+            qf->alpha = qalpha;
+            qf->unformed = 1;
+        } else if (trans == 'T') apply_right(x, core, buf, len, c, Tp, a);
         else apply_left_t(x, core, buf, c, len, Tp, a);
         /* Racc <- Rp * Racc, into the buffer Racc does not occupy */
         double *out = spare[si];
@@ -997,6 +1023,12 @@ static void rtl_sweep(attac_tt *x, const int *maxr, double abs_tol, const double
             g_spec[i][18] = rows;
         }
         /* core i-1 (m1 x rows) <- left_alpha * core i-1 * U_rho Sigma_rho */
+        if (g_qf && g_qf[i - 1].unformed) {
+            ptt_hip_dgemm('N', 'N', rows, rho, rows, g_qf[i - 1].alpha, g_qf[i - 1].t, rows, ws.US,
+                          rows, 0.0, ws.U, rows);
+            ws.US = ws.U;
+            g_qf[i - 1].unformed = 0;
+        }
         if (rho <= 128) {
             ptt_hip_dgemm('N', 'N', (int)m1, rho, rows, left_alpha, x->coreList[i - 1], m1, ws.US,
                           rows, 0.0, x->coreList[i - 1], m1);
@@ -1197,6 +1229,25 @@ static double round_impl_g(attac_tt *x, const int *maxRank, double tol, int tol_
         g_escale = 0;
         double nrm_s;
         const int route = tree_route(x);
+        q_factor *qf = NULL;
+        if (route == 0) {
+            /* (a train that may change over to the trees needs its Qs) */
+            size_t need = 0;
+            qf = (q_factor *)calloc((size_t)d, sizeof *qf);
+            if (!qf) {
+                fprintf(stderr, "%s:Line %d %s::out of memory\n", __FILE__, __LINE__, __func__);
+                exit(1);
+            }
+            for (int k = 0; k + 1 < d; k++)
+                if (x->ttRank[k + 1] <= 128) need += (size_t)x->ttRank[k + 1] * x->ttRank[k + 1];
+            double *t = need ? (double *)ptt_hip_scratch(PTT_WS_QFACT, sizeof(double) * need) : NULL;
+            for (int k = 0; k + 1 < d; k++)
+                if (x->ttRank[k + 1] <= 128) {
+                    qf[k].t = t;
+                    t += (size_t)x->ttRank[k + 1] * x->ttRank[k + 1];
+                }
+            g_qf = qf;
+        }
         const int done = route == 1 ? 0 : ltr_sweep_until(x, qs, rs, route == 2);
         if (route == 1 || done < d - 1) {
             nrm_s = tree_round(x, mr, tol, tol_is_rel, rs, sq, done);
@@ -1208,6 +1259,8 @@ static double round_impl_g(attac_tt *x, const int *maxRank, double tol, int tol_
             const double abs_tol = tol_is_rel ? tol * nrm_s : ldexp(tol, -g_escale);
             rtl_sweep(x, mr, abs_tol, sq);
         }
+        g_qf = NULL;
+        free(qf);
         if (g_escale != 0) {
             /* core 0 carries the train's magnitude after the sweep */
             ptt_hip_scale(x->coreList[0], (long)x->ttRank[0] * x->dim[0] * x->ttRank[1],
