@@ -224,7 +224,7 @@ void ptt_hip_svd_factors(int m, int rhomax, const int *drho, const double *U,
                          long ldu, const double *sig, double wscale, double *W,
                          double *US);
 /* Eigen-decomposition of a symmetric positive semi-definite c x c Gram G
- * (ld c, c <= 128): Householder tridiagonalisation, divide and conquer,
+ * (ld c, c <= 192): Householder tridiagonalisation, divide and conquer,
  * back transformation.  sig[q] = sqrt(lambda_q) in descending order; the
  * eigenvector of sig[q] is column colidx[q] (device ints) of U (c x c, ldu).
  * The smallest eigenvalues whose sum is at most budget * lambda_max are set

@@ -1,5 +1,5 @@
 // syev.hip -- eigen-decomposition of a symmetric positive semi-definite
-// Gram matrix (c <= 128) for the Gram route of the right-to-left truncation
+// Gram matrix (c <= 192) for the Gram route of the right-to-left truncation
 // step: G = U diag(sigma^2) U^T.
 //
 // The step needs the left singular vectors and values of a bond matrix M
@@ -7,12 +7,13 @@
 // G performs about 8 sweeps x 127 rounds of pair rotations (~100 MFLOP at
 // c = 128) on one CU; this solver does ~7 MFLOP:
 //   1. k_sytrd: Householder tridiagonalisation G = Q T Q^T, one workgroup,
-//      G held in registers (two lanes per row), one reflector per step with
-//      two workgroup barriers;
+//      G held in registers (16 x 16 tiles), one reflector per step with two
+//      workgroup barriers;
 //   2. k_dc_leaf, k_dc_roots, k_dc_vecs, k_dc_top: Cuppen's divide and conquer
 //      on T (split into 2 x 2 blocks, merged bottom-up by rank-one updates), over
-//      several workgroups, with the deflation rules of Dongarra and Sorensen, the secular-equation iteration of Li's "middle
-//      way" (SIAM J. Sci. Comput. 1994, as in LAPACK's dlaed4) from the
+//      several workgroups, with the deflation rules of Dongarra and Sorensen,
+//      the secular-equation iteration of Li's "middle way" (SIAM J. Sci.
+//      Comput. 1994, as in LAPACK's dlaed4) from the
 //      nearer pole, and the eigenvectors of Gu and Eisenstat (SIAM J. Matrix
 //      Anal. Appl. 16, 1995): z is recomputed from the computed roots, which
 //      makes the vectors numerically orthogonal without reorthogonalisation;
@@ -95,8 +96,8 @@ __device__ __forceinline__ int even_exp(double a) {
 }
 
 // ---- 1. tridiagonalisation ------------------------------------------------
-// Register tiles: G is cut into 16 x 16 tiles; row wave I (NB = NMAX/16 of
-// them) holds tile row I.  Lane l (a = l/16, j = l%16) holds rows
+// Register tiles: G is cut into 16 x 16 tiles; row wave I holds tile row I (NB =
+// NMAX/16 of them), beyond 128 rows tile rows I and I + NB/2.  Lane l (a = l/16, j = l%16) holds rows
 // 16I + a + 4v (v = 0..3) of column 16J + j of every tile J: g[J][v].
 // Entries beyond n are zero and stay zero.  A lane thus needs only the NB
 // entries of v (and of p) at its columns and four at its rows, which keeps
@@ -123,6 +124,12 @@ __device__ __forceinline__ int even_exp(double a) {
 // columns of Vh (n x n, ld n; rows <= k zero, v_{k+1} = 1), the exponent of
 // the power-of-two scaling, max |G| (dinfo[6]) and the trace of G (dinfo[7]).
 // Only the upper triangle of G is read.
+//
+// Bound by the chain of a step (about 1 us: the product's lane sums, two barriers,
+// the reflector wave's two reductions and its root); at 192 rows also by the row
+// waves' FP64 issue (288 multiply-adds a lane a step).  Measured: 26 us at 32 rows,
+// 43 at 59, 124 at 128, 395 at 192 (734 when v and p were held in registers, which
+// spilled).  A raised priority of the reflector wave made no difference.
 __device__ __forceinline__ double readlane_d(double v, int l) {
     const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
     const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
@@ -425,7 +432,8 @@ __global__ __launch_bounds__(sytrd_geom<NMAX>::NT) void k_sytrd(int n, const dou
 // the work is, are divided.  The last merge (`top`) always takes this form.
 // All merges in one workgroup of 1024 threads, with Z in memory, were bound by
 // the FP64 instructions of one CU: 178 us at n = 128, 95 at 59, 62 at 32; this
-// form takes 98, 65 and 44 (with the gaps between its launches).
+// form takes 98, 65 and 44 (with the gaps between its launches).  Half of the leaf
+// kernel's time is its roots: 1500 cycles an iteration, 4 to 8 iterations a level.
 //
 // Deflation (one wave per block): entries with rho |z| <= tol are deflated;
 // consecutive remaining entries whose poles are closer than the tolerance
