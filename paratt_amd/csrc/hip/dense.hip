@@ -318,8 +318,8 @@ __global__ __launch_bounds__(NT) void k_chol_report(int c, const double *__restr
 // registers, 4 rows x NB columns a thread, with one barrier a product.
 // Measured (us, well conditioned / with the iterations; before: column by column
 // with a workgroup barrier a column up to 48, panels through LDS beyond):
-// c = 16: 15 / 31 -> 7 / 12, 32: 20 / 35 -> 12 / 18, 48: 37 / 60 -> 16 / 23,
-// 64: 47 / 70 -> 20 / 27, 128: 96 / 146 -> 39 / 52, of which the panels are 24.
+// c = 16: 15 / 31 -> 7 / 10, 32: 20 / 35 -> 12 / 17, 48: 37 / 60 -> 16 / 21,
+// 64: 47 / 70 -> 20 / 26, 128: 96 / 146 -> 39 / 49, of which the panels are 24.
 template <int NB>
 struct chol_geom {
     static constexpr int N = 16 * NB;            // padded order
@@ -502,9 +502,16 @@ __global__ __launch_bounds__(64 * NB) void k_chol_blk(int c, const double *__res
             s[v] = 0.0;
 #pragma unroll
             for (int q = 0; q < NB; q++) s[v] = fma(m[v][q], xv[q], s[v]);
-            s[v] = row16_sum(s[v]);
         }
-        if (li < 4) y[16 * wv + 4 * lg + li] = li == 0 ? s[0] : li == 1 ? s[1] : li == 2 ? s[2] : s[3];
+        // the four rows' sums over the 16 lanes at once: lane li ends with row
+        // 2 (li / 8 % 2) + (li / 4 % 2) (four sums by turns: 32
+        // columns 18.1 us instead of 16.7)
+        const bool h8 = (li & 8) != 0, h4 = (li & 4) != 0;
+        const double u0 = (h8 ? s[2] : s[0]) + dppd<0x128>(h8 ? s[0] : s[2]);  // row_ror:8
+        const double u1 = (h8 ? s[3] : s[1]) + dppd<0x128>(h8 ? s[1] : s[3]);
+        // half-row mirror: the 4-lane groups swap
+        const double t = quad_sum((h4 ? u1 : u0) + dppd<0x141>(h4 ? u0 : u1));
+        if ((li & 3) == 0) y[16 * wv + 4 * lg + 2 * (int)h8 + (int)h4] = t;
         lds_sync();
     };
     auto norm2 = [&](const double *x) {

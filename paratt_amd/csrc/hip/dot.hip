@@ -17,8 +17,10 @@
 // X_j is loaded beside the first product, Y_{j+1} beside the second.
 // Measured (us a mode, with the sum over workgroups): n = 1024, ranks 64: 33 (two
 // tiled products and a reduction over the splits of K, which this replaces: 60),
-// 48: 19, 40: 24, 32: 11, 16: 7; n = 300, ranks 64: 22.  Two thirds of the floor
-// are left at 64: a mode index waits for its loads with two waves a SIMD.
+// 48: 19, 40: 24, 32: 11, 16: 7; n = 300, ranks 64: 22.  At 64 a mode index costs
+// 6.1 us a CU against 5.0 at the 53 TFLOP/s that the matrix cores hold under such a
+// load, and a mode some 6 us for a's operands and the sums.  Loading a product and a
+// half ahead (35 us) and handing the indices out round robin (34) gave nothing.
 #include "common.hpp"
 
 using namespace ptt;
