@@ -1230,8 +1230,7 @@ static double round_impl_g(attac_tt *x, const int *maxRank, double tol, int tol_
         double nrm_s;
         const int route = tree_route(x);
         q_factor *qf = NULL;
-        if (route == 0) {
-            /* (a train that may change over to the trees needs its Qs) */
+        if (route != 1) {
             size_t need = 0;
             qf = (q_factor *)calloc((size_t)d, sizeof *qf);
             if (!qf) {
@@ -1250,6 +1249,11 @@ static double round_impl_g(attac_tt *x, const int *maxRank, double tol, int tol_
         }
         const int done = route == 1 ? 0 : ltr_sweep_until(x, qs, rs, route == 2);
         if (route == 1 || done < d - 1) {
+            /* a train that changes over to the trees needs its Qs */
+            for (int k = 0; k < done; k++)
+                if (qf && qf[k].unformed)
+                    apply_right(x, k, NULL, (long)x->ttRank[k] * x->dim[k], x->ttRank[k + 1],
+                                qf[k].t, qf[k].alpha);
             nrm_s = tree_round(x, mr, tol, tol_is_rel, rs, sq, done);
         } else {
             /* norm in the scaled space: last core after the sweep (the train
