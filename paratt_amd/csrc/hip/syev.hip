@@ -273,6 +273,10 @@ __global__ __launch_bounds__(sytrd_geom<NMAX>::NT) void k_sytrd(int n, const dou
             x[u] = (lane + 64 * u < NMAX) ? v[lane + 64 * u < NMAX ? lane + 64 * u : 0] : 0.0;
     };
 
+    // p starts as zero: a wave whose rows stop mattering before the first reflector
+    // (leading zero or diagonal rows) never writes its entries, which later steps
+    // multiply by v = 0
+    for (int i = tid; i < NMAX; i += NT) pp[i] = 0.0;
     if (!star && I == 0) {
         copy_row(0, 1);
         copy_row(1, 0);
