@@ -232,7 +232,8 @@ void ptt_hip_svd_factors(int m, int rhomax, const int *drho, const double *U,
  * sqrt(c) eps sig_0), iout[1] = the reference's tail-rule rank against
  * delta, capped by min(c, cap), floor 1 (pattac.c:468-481), iout[2] = most
  * secular-equation iterations of one root; dinfo[6] = max |G_ij|,
- * dinfo[7] = trace(G). */
+ * dinfo[7] = trace(G).  With a NaN or an infinity in G's upper triangle every
+ * sig is NaN and the numerical rank 0. */
 void ptt_hip_syev_gram(int c, const double *G, double *sig, double *U, long ldu, int *colidx,
                        int *iout, double *dinfo, double delta, int cap, double budget);
 /* ptt_hip_syev_gram without any allocation: same kernels, same results, the

@@ -25,6 +25,9 @@
 // (bond matrices of deep trains reach 1e-60 and below); sigma is scaled back.
 // Eigenvectors of the Gram carry the Gram's rounding (~ c u ||G||), as the
 // Cholesky route does; callers decide whether that resolution suffices.
+// A Gram with an entry that is not finite is taken as zero and its sigma come out
+// as NaN: the orders and lists of the divide and conquer are permutations only of
+// values that compare, and index memory.
 #include "common.hpp"
 
 #include <cmath>
@@ -38,6 +41,7 @@ typedef double f64x4 __attribute__((ext_vector_type(4)));
 
 constexpr double EPSU = 0x1.0p-53;
 constexpr int EIG_NMAX = 192;
+constexpr int EIG_NONFINITE = 0x7fffffff;  // in place of the scaling's exponent
 
 __device__ __forceinline__ double quad_prod(double x) {
     x *= dppd<0xB1>(x);
@@ -122,7 +126,8 @@ __device__ __forceinline__ int even_exp(double a) {
 //
 // Outputs: d (diagonal), e (off-diagonal), tau, the reflectors in the
 // columns of Vh (n x n, ld n; rows <= k zero, v_{k+1} = 1), the exponent of
-// the power-of-two scaling, max |G| (dinfo[6]) and the trace of G (dinfo[7]).
+// the power-of-two scaling (EIG_NONFINITE: an entry of G is not finite), max |G|
+// (dinfo[6], infinite then) and the trace of G (dinfo[7]).
 // Only the upper triangle of G is read.
 //
 // Bound by the chain of a step (about 1 us: the product's lane sums, two barriers,
@@ -181,7 +186,7 @@ __global__ __launch_bounds__(sytrd_geom<NMAX>::NT) void k_sytrd(int n, const dou
                 if (!star && row < n && col < n)
                     x = (row <= col) ? G[row + (long)col * ldg] : G[col + (long)row * ldg];
                 g[t][J][v] = x;
-                amax = fmax(amax, fabs(x));
+                amax = fmax(amax, fabs(x) < INFINITY ? fabs(x) : INFINITY);
                 if (row == col) tr += x;
             }
     amax = wave_max(amax);
@@ -200,6 +205,7 @@ __global__ __launch_bounds__(sytrd_geom<NMAX>::NT) void k_sytrd(int n, const dou
         s_e = even_exp(m);
         dinfo[6] = m;
         dinfo[7] = t;
+        if (!(m < INFINITY)) s_e = EIG_NONFINITE;
         *eexp = s_e;
     }
     __syncthreads();
@@ -209,7 +215,8 @@ __global__ __launch_bounds__(sytrd_geom<NMAX>::NT) void k_sytrd(int n, const dou
 #pragma unroll
         for (int J = 0; J < NB; J++)
 #pragma unroll
-            for (int v = 0; v < 4; v++) g[t][J][v] = ldexp(g[t][J][v], -es);
+            for (int v = 0; v < 4; v++)
+                g[t][J][v] = es == EIG_NONFINITE ? 0.0 : ldexp(g[t][J][v], -es);
 
     // Row i of this wave's tile row t into rowb[slot] (called by the whole
     // wave; i wave-uniform, held by the lanes with a = i % 4 in register
@@ -1295,7 +1302,8 @@ __global__ __launch_bounds__(256) void k_dc_top(int n, DcState st, const double 
         }
     }
     __syncthreads();
-    const int es = *eexp;
+    const bool finite = *eexp != EIG_NONFINITE;
+    const int es = finite ? *eexp : 0;
     // Wave 0 holds the descending values lane + 64 w and decides:
     //  - the smallest eigenvalues are dropped while their running sum stays
     //    within lim = budget * lmax: the suffix sums S(q) and the values grow
@@ -1369,7 +1377,8 @@ __global__ __launch_bounds__(256) void k_dc_top(int n, DcState st, const double 
     }
     __syncthreads();
     const int keep = s_keep;
-    if (tid < n) sig[tid] = (tid < keep) ? ldexp(sqrt(fmax(sdl[tid], 0.0)), es / 2) : 0.0;
+    if (tid < n)
+        sig[tid] = !finite ? NAN : (tid < keep) ? ldexp(sqrt(fmax(sdl[tid], 0.0)), es / 2) : 0.0;
 }
 
 // ---- 3. back transformation -----------------------------------------------
