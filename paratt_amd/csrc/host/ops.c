@@ -178,25 +178,37 @@ static double inner_sweep(int d, const int *n, const int *rx, double *const *x, 
     }
     for (int i = 0; i < d; i++) nmax = n[i] > nmax ? n[i] : nmax;
     double *a = (double *)ptt_hip_scratch(PTT_WS_SKETCH, sizeof(double) * (size_t)rmax * rmax);
-    /* a = x0^T y0 (rx1 x ry1), K = rx0*n0 */
-    ptt_hip_dgemm('T', 'N', rx[1], ry[1], rx[0] * n[0], s[0], x[0], (long)rx[0] * n[0], y[0],
-                  (long)ry[0] * n[0], 0.0, a, rx[1]);
-    for (int i = 1; i < d; i++) {
-        if (ptt_hip_dot_mode(n[i], rx[i], rx[i + 1], ry[i], ry[i + 1], a, x[i], y[i], s[i], a))
-            continue;
-        /* ranks beyond that kernel's */
-        double *b =
-            (double *)ptt_hip_scratch(PTT_WS_TMP2, sizeof(double) * (size_t)rmax * rmax * nmax);
-        long nry = (long)n[i] * ry[i + 1];
-        /* b = a * y_i : (rx_i x ry_i) * (ry_i x n*ry_{i+1}) */
-        ptt_hip_dgemm('N', 'N', rx[i], (int)nry, ry[i], 1.0, a, rx[i], y[i], ry[i], 0.0, b, rx[i]);
-        /* a = x_i^T b : (rx_i*n x rx_{i+1})^T (rx_i*n x ry_{i+1}) */
-        long rxn = (long)rx[i] * n[i];
-        ptt_hip_dgemm('T', 'N', rx[i + 1], ry[i + 1], (int)rxn, s[i], x[i], rxn, b, rxn, 0.0, a,
-                      rx[i + 1]);
-    }
     double v = 0.0;
-    ptt_hip_d2h(&v, a, sizeof(double));
+    /* general: by two products a mode, for ranks beyond the one-mode kernel's and
+     * once more where the result is not a number.  That kernel pads ranks to blocks
+     * of 16 with zeros, and zero times an infinity of y is not; masking the padded
+     * rows there costs every inner product up to 3% (n = 1024, ranks 60: 45 -> 46.5
+     * us a mode). */
+    for (int general = 0; general < 2; general++) {
+        int padded = 0;
+        /* a = x0^T y0 (rx1 x ry1), K = rx0*n0 */
+        ptt_hip_dgemm('T', 'N', rx[1], ry[1], rx[0] * n[0], s[0], x[0], (long)rx[0] * n[0], y[0],
+                      (long)ry[0] * n[0], 0.0, a, rx[1]);
+        for (int i = 1; i < d; i++) {
+            if (!general && ptt_hip_dot_mode(n[i], rx[i], rx[i + 1], ry[i], ry[i + 1], a, x[i],
+                                             y[i], s[i], a)) {
+                padded = 1;
+                continue;
+            }
+            double *b =
+                (double *)ptt_hip_scratch(PTT_WS_TMP2, sizeof(double) * (size_t)rmax * rmax * nmax);
+            long nry = (long)n[i] * ry[i + 1];
+            /* b = a * y_i : (rx_i x ry_i) * (ry_i x n*ry_{i+1}) */
+            ptt_hip_dgemm('N', 'N', rx[i], (int)nry, ry[i], 1.0, a, rx[i], y[i], ry[i], 0.0, b,
+                          rx[i]);
+            /* a = x_i^T b : (rx_i*n x rx_{i+1})^T (rx_i*n x ry_{i+1}) */
+            long rxn = (long)rx[i] * n[i];
+            ptt_hip_dgemm('T', 'N', rx[i + 1], ry[i + 1], (int)rxn, s[i], x[i], rxn, b, rxn, 0.0,
+                          a, rx[i + 1]);
+        }
+        ptt_hip_d2h(&v, a, sizeof(double));
+        if (!padded || v == v) break;
+    }
     return v;
 }
 

@@ -51,3 +51,16 @@ def test_rounding(n, r, bad, core):
     P.truncate(dz, tol, z.r)
     out = to_host(dz)
     assert out.r == good.r and O.rel_diff(out, good) < 1e-11
+
+
+@pytest.mark.parametrize("r", [3, 16, 17, 40, 48, 64, 70])
+@pytest.mark.parametrize("where", ["x", "y"])
+@pytest.mark.parametrize("core", [1, 2])
+def test_inner_product_of_positive_trains_with_an_infinity(r, where, core):
+    """Every other term is positive: the sum is infinite and not NaN."""
+    rng = np.random.default_rng(r)
+    n, ranks = [20, 70, 33, 9], [1, r, max(1, r - 2), r, 1]
+    t = {q: O.HostTT(n, ranks, [rng.random(ranks[k] * n[k] * ranks[k + 1]) + 0.1
+                                for k in range(4)]) for q in "xy"}
+    t[where].cores[core][-7] = np.inf
+    assert P.dotprod(P.DevTT.from_host(t["x"]), P.DevTT.from_host(t["y"])) == np.inf
