@@ -152,7 +152,10 @@ __global__ __launch_bounds__(NT) void k_chol_report(int c, const double *__restr
         eoff = block_max(eoff);
         gersh = want_kappa && eoff < 0.5;
         decided = ndef > 0 || !(pmax <= 1e12 * pmin);
-        const int PIT = (want_kappa && !gersh && !decided) ? 6 : 0;
+        // Ten products a side: the estimate comes from below and sets the number of
+        // passes, one up to 30 (130 columns of condition 34 read 29.0 after six products,
+        // 30.7 after ten).  192 columns: 76 us with six, 88 with ten.
+        const int PIT = (want_kappa && !gersh && !decided) ? 10 : 0;
         if (PIT > 0 && c <= CR_REG) {
             // the matrix in registers, rows 12 wv + 3 lg + v, columns li + 16 q; S
             // first, then Ts^T (beyond this order every product reads it from
@@ -207,13 +210,13 @@ __global__ __launch_bounds__(NT) void k_chol_report(int c, const double *__restr
                 for (int i = lane; i < CR_REG; i += 64) t = fma(x[i], x[i], t);
                 return wave_sum(t);
             };
-            auto start = [&]() {
-                if (tid < CR_REG) s_x[tid] = tid < c ? 1.0 + 0.01 * (tid % 7) : 0.0;
+            auto start = [&](int period) {
+                if (tid < CR_REG) s_x[tid] = tid < c ? 1.0 + 0.01 * (tid % period) : 0.0;
                 __syncthreads();
             };
             // lambda_max(S) <= c: no scaling between the products
             load(G, iD, iD);
-            start();
+            start(7);
             for (int it = 0; it < PIT; it += 2) {
                 rows(s_x, s_y);
                 rows(s_y, s_x);
@@ -222,7 +225,7 @@ __global__ __launch_bounds__(NT) void k_chol_report(int c, const double *__restr
             __syncthreads();
             // lambda_max(Ts Ts^T) <= ft, divided out of every product
             load(T, D, nullptr);
-            start();
+            start(5);
             double prev = 1.0;
             for (int it = 0; it < PIT; it++) {
                 if (it == PIT - 1) prev = norm2(s_x);
@@ -232,7 +235,7 @@ __global__ __launch_bounds__(NT) void k_chol_report(int c, const double *__restr
             lminv = ft * sqrt(norm2(s_x) / prev);
         }
         for (int side = 0; side < 2 && c > CR_REG; side++) {
-            for (int i = tid; i < c; i += NT) y[i] = 1.0 + 0.01 * (i % 7);
+            for (int i = tid; i < c; i += NT) y[i] = 1.0 + 0.01 * (i % (side == 0 ? 7 : 5));
             __syncthreads();
             for (int it = 0; it < PIT; it++) {
                 double xn = 0.0;
