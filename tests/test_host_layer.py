@@ -1,0 +1,55 @@
+"""What the C host layer queues and allocates, on a CPU: its sources compiled
+against host_stub.c, which stands in for the kernels without computing anything."""
+import ctypes as C
+import os
+import subprocess
+
+import pytest
+
+import paratt_amd as P
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HOST = os.path.join(ROOT, "paratt_amd", "csrc", "host")
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("host") / "host.so")
+    subprocess.run(["gcc", "-std=c99", "-O1", "-fPIC", "-shared", "-DPARATT_AMD_NO_MPI",
+                    "-I" + os.path.join(ROOT, "include"), "-I" + HOST,
+                    os.path.join(ROOT, "tests", "host_stub.c"), os.path.join(HOST, "round.c"),
+                    os.path.join(HOST, "tt.c"), "-o", so, "-lm"], check=True, timeout=120)
+    L = C.CDLL(so)
+    PP, IP = C.POINTER(P.Paratt), C.POINTER(C.c_int)
+    L.alloc_ptt.restype = PP
+    L.free_ptt.argtypes = [PP]
+    L.paratt_amd_truncate_rel.argtypes = [PP, C.c_double, IP]
+    return L
+
+
+def _ints(v):
+    return (C.c_int * len(v))(*v)
+
+
+def _count(L, name):
+    return C.c_long.in_dll(L, name).value
+
+
+def _set_condition(L, kappa, deficient=0):
+    C.c_double.in_dll(L, "stub_kappa").value = kappa
+    C.c_int.in_dll(L, "stub_deficient").value = deficient
+
+
+@pytest.mark.parametrize("kappa,side,main", [(1.5, 0, 0), (4.0, 0, 0), (4.1, 2, 1), (30.0, 2, 1)])
+def test_formed_q_of_a_rounding_goes_to_the_side_stream(lib, kappa, side, main):
+    """One-pass bonds: left unformed up to a condition of 4; beyond it the products of
+    cores of at least 4M elements (the middle two) run on the side stream."""
+    n, r = [300] * 4, [1, 128, 128, 128, 1]
+    x = lib.alloc_ptt(4, _ints(n), _ints(r))
+    _set_condition(lib, kappa)
+    lib.stub_reset()
+    lib.paratt_amd_truncate_rel(x, 1e-8, _ints([1, 64, 64, 64, 1]))
+    assert list(x.contents.x.contents.ttRank[:5]) == [1, 64, 64, 64, 1]
+    got = (_count(lib, "stub_side_inplace"), _count(lib, "stub_main_inplace"))
+    lib.free_ptt(x)
+    assert got == (side, main)
