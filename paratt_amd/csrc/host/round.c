@@ -292,6 +292,8 @@ static double last_core_sumsq(attac_tt *x) {
  * core that one Cholesky-QR pass does not orthogonalise is left as it is and
  * the factorisation returns -1. */
 static int g_one_pass_only = 0;
+/* The last left-to-right sweep met a core (after core 0) of more than one pass. */
+static int g_sweep_multi = 0;
 
 /* Condition of the last factor up to which Q may be left unformed (below). */
 #define KAPPA_UNFORMED 4.0
@@ -453,6 +455,7 @@ static int ltr_sweep_until(attac_tt *x, const double *qscale, const double *rsca
                            int hand_over) {
     int d = x->numDim;
     int *r = x->ttRank, *n = x->dim;
+    g_sweep_multi = 0;
     for (int i = 0; i < d - 1; i++) {
         long m = (long)r[i] * n[i];
         int c = r[i + 1];
@@ -480,6 +483,7 @@ static int ltr_sweep_until(attac_tt *x, const double *qscale, const double *rsca
             return i;
         }
         if (i < 64) g_stats.ltr_cholqr_passes[i] = passes;
+        if (i > 0 && passes > 1) g_sweep_multi = 1;
         /* core i+1 (c x wcols) <- rscale * R * core i+1 */
         if (c <= 128) {
             ptt_hip_dgemm('N', 'N', c, (int)wcols, c, rscale[i], R, c, x->coreList[i + 1], c, 0.0,
@@ -925,6 +929,13 @@ static int rtl_step_sketch(attac_tt *x, int i, const int *maxr, double delta,
     return rho;
 }
 
+/* Columns of the sketch that pred allows for bond i of rows x w; 0: none. */
+static int sketch_columns(const int *pred, int i, int rows, long w) {
+    if (i >= 64 || pred[i] <= 0 || pred[i] > 128 - SKETCH_OVERSAMPLE) return 0;
+    const int l = pred[i] + SKETCH_OVERSAMPLE;
+    return (2 * l <= rows && (long)l <= w) ? l : 0;
+}
+
 /* Right-to-left truncation (pattac.c:297-522) of a left-orthogonal TT whose
  * cores carry the reference's scaled magnitudes; tol is absolute in that
  * scaled space.  nscale[k] = sqrt(n_k) is applied to each finished core. */
@@ -976,13 +987,11 @@ static void rtl_sweep(attac_tt *x, const int *maxr, double abs_tol, const double
         } else {
             ws = get_ws(rows);
             int sk = -1;
-            if (g_pred && i < 64 && g_pred[i] > 0) {
-                const int l = g_pred[i] + SKETCH_OVERSAMPLE;
-                if (l <= 128 && 2 * l <= rows && (long)l <= w) {
-                    g_sketch_counts[0]++;
-                    sk = rtl_step_sketch(x, i, maxr, delta, nscale, &ws, l);
-                    if (sk > 0) g_sketch_counts[1]++;
-                }
+            const int l = g_pred ? sketch_columns(g_pred, i, rows, w) : 0;
+            if (l > 0) {
+                g_sketch_counts[0]++;
+                sk = rtl_step_sketch(x, i, maxr, delta, nscale, &ws, l);
+                if (sk > 0) g_sketch_counts[1]++;
             }
             /* Bond spectra change slowly along the train: once the Gram
              * route was rejected at the right neighbour, go straight to the
@@ -1306,10 +1315,21 @@ void paratt_amd_truncate_rel(paratt *x_ptt, double eps_rel, int *maxRank) {
 
 void paratt_amd_truncate_rel_sketch(paratt *x_ptt, double eps_rel, int *maxRank,
                                     const int *pred_rank) {
-    /* refused predictions leave the plain rounding's result: a train that it
-     * takes through the trees is kept until one step has been accepted */
     attac_tt *x = x_ptt->x, *keep = NULL;
     const int d = x->numDim;
+    /* No bond is large enough for a sketch of its prediction (ranks only fall on
+     * the way): the plain rounding, decided before anything is queued. */
+    int any = 0;
+    for (int i = 1; pred_rank && i < d; i++)
+        any = any || sketch_columns(pred_rank, i, x->ttRank[i],
+                                    (long)x->dim[i] * x->ttRank[i + 1]) > 0;
+    if (!any) {
+        round_impl(x, maxRank, eps_rel, 1);
+        return;
+    }
+    /* Refused predictions leave the plain rounding's result.  A train that it would
+     * hand over to the trees (17 to 32 columns and a core of more than one pass;
+     * smaller ones take no sketch) is kept until a step has been accepted. */
     int *mr = (int *)ptt_host_malloc(sizeof(int) * (size_t)(d + 1));
     memcpy(mr, maxRank, sizeof(int) * (size_t)(d + 1));
     if (tree_route(x)) {
@@ -1319,7 +1339,7 @@ void paratt_amd_truncate_rel_sketch(paratt *x_ptt, double eps_rel, int *maxRank,
     g_pred = pred_rank;
     round_impl(x, mr, eps_rel, 1);
     g_pred = NULL;
-    if (keep && g_sketch_counts[1] == 0) {
+    if (keep && g_sketch_counts[1] == 0 && g_sweep_multi) {
         const int tried = g_sketch_counts[0];
         copy_rank_change_tt(x, keep);
         round_impl(x, mr, eps_rel, 1);

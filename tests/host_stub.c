@@ -15,13 +15,14 @@ double stub_kappa = 1.5;
 int stub_deficient = 0;
 long stub_side_inplace; /* in-place products queued on the side stream (Q = A T) */
 long stub_main_inplace; /* the same on the main stream, c x c from the right */
-long stub_chol, stub_tree_factors, stub_syncs;
+long stub_chol, stub_tree_factors, stub_eigen, stub_mallocs;
 size_t stub_live, stub_peak;
 
 static int on_side;
 
 void stub_reset(void) {
-    stub_side_inplace = stub_main_inplace = stub_chol = stub_tree_factors = stub_syncs = 0;
+    stub_side_inplace = stub_main_inplace = 0;
+    stub_chol = stub_tree_factors = stub_eigen = stub_mallocs = 0;
     stub_peak = stub_live;
 }
 
@@ -30,6 +31,7 @@ void *ptt_hip_malloc(size_t bytes) {
     size_t *p = (size_t *)calloc(1, bytes + 64);
     if (!p) abort();
     p[0] = bytes;
+    stub_mallocs++;
     stub_live += bytes;
     if (stub_live > stub_peak) stub_peak = stub_live;
     return p + 8;
@@ -42,7 +44,6 @@ void ptt_hip_free(void *p) {
 }
 void ptt_hip_free_many(int count, void *const *p) {
     for (int i = 0; i < count; i++) ptt_hip_free(p[i]);
-    if (count > 0) stub_syncs++;
 }
 static struct {
     void *p;
@@ -119,6 +120,7 @@ static void flat(int k, int cap, double *sig, int *iout) {
 void ptt_hip_syev_gram(int c, const double *G, double *sig, double *U, long ldu, int *ci, int *iout,
                        double *dinfo, double delta, int cap, double budget) {
     (void)G; (void)U; (void)ldu; (void)ci; (void)delta; (void)budget;
+    stub_eigen++;
     flat(c, cap, sig, iout);
     dinfo[5] = 0.0;
     dinfo[6] = 1.0;

@@ -24,6 +24,8 @@ def lib(tmp_path_factory):
     L.alloc_ptt.restype = PP
     L.free_ptt.argtypes = [PP]
     L.paratt_amd_truncate_rel.argtypes = [PP, C.c_double, IP]
+    L.paratt_amd_truncate_rel_sketch.argtypes = [PP, C.c_double, IP, IP]
+    L.paratt_amd_last_sketch_counts.argtypes = [IP]
     return L
 
 
@@ -53,3 +55,52 @@ def test_formed_q_of_a_rounding_goes_to_the_side_stream(lib, kappa, side, main):
     got = (_count(lib, "stub_side_inplace"), _count(lib, "stub_main_inplace"))
     lib.free_ptt(x)
     assert got == (side, main)
+
+
+def _work(L):
+    return tuple(_count(L, "stub_" + k) for k in ("chol", "tree_factors", "eigen", "mallocs"))
+
+
+# every bond at most 16 columns: trees; 24 columns: Gram route while well conditioned,
+# trees behind the first core that is not; 40: Gram route
+@pytest.mark.parametrize("r,kappa", [(10, 1.5), (16, 1e7), (24, 1.5), (24, 1e7), (40, 1.5)])
+@pytest.mark.parametrize("pred", [0, 9, 200, None])
+def test_rounding_without_a_usable_prediction_is_the_plain_one(lib, r, kappa, pred):
+    """A sketch takes at least 9 columns and at most half of the bond's and 128."""
+    if pred == 9 and 2 * (pred + 8) <= r:
+        pytest.skip("the prediction is usable")
+    n, ranks = [50] * 5, [1, r, r, r, r, 1]
+    mr = _ints([1] + [5] * 4 + [1])
+    _set_condition(lib, kappa)
+    got = []
+    for sketch in (0, 0, 1):  # the first one grows the scratch memory
+        x = lib.alloc_ptt(5, _ints(n), _ints(ranks))
+        lib.stub_reset()
+        if sketch:
+            p = None if pred is None else _ints([0] + [pred] * 4 + [0])
+            lib.paratt_amd_truncate_rel_sketch(x, 1e-8, mr, p)
+        else:
+            lib.paratt_amd_truncate_rel(x, 1e-8, mr)
+        got.append(_work(lib))
+        lib.free_ptt(x)
+    assert got[2] == got[1]
+    cnt = (C.c_int * 2)()
+    lib.paratt_amd_last_sketch_counts(cnt)
+    assert list(cnt) == [0, 0]
+
+
+@pytest.mark.parametrize("kappa,trees", [(1.5, 0), (1e7, 3)])
+def test_refused_predictions_round_again_only_where_the_trees_would(lib, kappa, trees):
+    """24 columns, sketches of 12 that the stub's residual refuses: at most one
+    eigensolver call a bond."""
+    x = lib.alloc_ptt(5, _ints([50] * 5), _ints([1, 24, 24, 24, 24, 1]))
+    _set_condition(lib, kappa)
+    lib.stub_reset()
+    lib.paratt_amd_truncate_rel_sketch(x, 1e-8, _ints([1] + [5] * 4 + [1]),
+                                       _ints([0, 4, 4, 4, 4, 0]))
+    cnt = (C.c_int * 2)()
+    lib.paratt_amd_last_sketch_counts(cnt)
+    eigen, factors = _count(lib, "stub_eigen"), _count(lib, "stub_tree_factors")
+    lib.free_ptt(x)
+    assert list(cnt) == [4, 0]
+    assert eigen <= 4 and factors == trees
