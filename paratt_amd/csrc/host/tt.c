@@ -76,9 +76,15 @@ paratt *alloc_ptt(int ndims, int *d, int *ttR) {
     return p;
 }
 
+/* Old cores of a growing train are freed together, for each call that frees waits
+ * for the device, but no more than this many bytes of them wait for that: growing
+ * a train that fills the card takes its new cores and little more. */
+#define GROW_PENDING ((size_t)1 << 30)
+
 attac_tt *rank_change_tt(attac_tt *x, int *ttR) {
     void **old = (void **)xmalloc(sizeof(void *) * (size_t)x->numDim);
     int nold = 0;
+    size_t pending = 0;
     for (int k = 0; k < x->numDim; k++) {
         long need = (long)x->dim[k] * ttR[k] * ttR[k + 1];
         if (x->coreMem[k] < need) {
@@ -86,8 +92,14 @@ attac_tt *rank_change_tt(attac_tt *x, int *ttR) {
             double *nb = (double *)ptt_hip_malloc(sizeof(double) * (size_t)need);
             ptt_hip_d2d(nb, x->coreList[k], sizeof(double) * (size_t)x->coreMem[k]);
             old[nold++] = x->coreList[k];
+            pending += sizeof(double) * (size_t)x->coreMem[k];
             x->coreList[k] = nb;
             x->coreMem[k] = (int)need;
+            if (pending > GROW_PENDING) {
+                ptt_hip_free_many(nold, old);
+                nold = 0;
+                pending = 0;
+            }
         }
         x->ttRank[k] = ttR[k];
     }

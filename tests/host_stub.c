@@ -16,13 +16,14 @@ int stub_deficient = 0;
 long stub_side_inplace; /* in-place products queued on the side stream (Q = A T) */
 long stub_main_inplace; /* the same on the main stream, c x c from the right */
 long stub_chol, stub_tree_factors, stub_eigen, stub_mallocs;
+long stub_frees; /* calls that free (each waits for the device) */
 size_t stub_live, stub_peak;
 
 static int on_side;
 
 void stub_reset(void) {
     stub_side_inplace = stub_main_inplace = 0;
-    stub_chol = stub_tree_factors = stub_eigen = stub_mallocs = 0;
+    stub_chol = stub_tree_factors = stub_eigen = stub_mallocs = stub_frees = 0;
     stub_peak = stub_live;
 }
 
@@ -44,6 +45,7 @@ void ptt_hip_free(void *p) {
 }
 void ptt_hip_free_many(int count, void *const *p) {
     for (int i = 0; i < count; i++) ptt_hip_free(p[i]);
+    if (count > 0) stub_frees++;
 }
 static struct {
     void *p;

@@ -23,6 +23,9 @@ def lib(tmp_path_factory):
     PP, IP = C.POINTER(P.Paratt), C.POINTER(C.c_int)
     L.alloc_ptt.restype = PP
     L.free_ptt.argtypes = [PP]
+    L.alloc_tt.restype = C.POINTER(P.AttacTT)
+    L.free_tt.argtypes = [C.POINTER(P.AttacTT)]
+    L.rank_change_tt.argtypes = [C.POINTER(P.AttacTT), IP]
     L.paratt_amd_truncate_rel.argtypes = [PP, C.c_double, IP]
     L.paratt_amd_truncate_rel_sketch.argtypes = [PP, C.c_double, IP, IP]
     L.paratt_amd_last_sketch_counts.argtypes = [IP]
@@ -104,3 +107,18 @@ def test_refused_predictions_round_again_only_where_the_trees_would(lib, kappa, 
     lib.free_ptt(x)
     assert list(cnt) == [4, 0]
     assert eigen <= 4 and factors == trees
+
+
+def test_growing_a_train_waits_once_and_keeps_little_of_the_old(lib):
+    """Small trains free all of their old cores at once; a large one never holds more
+    than 1 GiB and one core of them besides its new ones."""
+    for n, r, grown in ((20, 10, 12), (1000, 280, 400)):
+        x = lib.alloc_tt(9, _ints([n] * 9), _ints([1] + [r] * 8 + [1]))
+        lib.stub_reset()
+        lib.rank_change_tt(x, _ints([1] + [grown] * 8 + [1]))
+        live = C.c_size_t.in_dll(lib, "stub_live").value
+        peak = C.c_size_t.in_dll(lib, "stub_peak").value
+        frees = _count(lib, "stub_frees")
+        lib.free_tt(x)
+        assert peak - live <= 2 ** 30 + 8 * n * r * r
+        assert frees == 1 if n == 20 else frees <= 6
