@@ -22,16 +22,29 @@ static bool g_side_used[2] = {false, false};
 static bool g_side_on = true;
 // Side work queued since the main stream last joined the side stream.
 static bool g_side_dirty = false;
-// Small uploads queued since the main stream was last waited for (their
-// staging slots are free again after such a wait).
-static int g_h2d_inflight = 0;
+// Small uploads queued so far, and how many of them a wait for the main stream
+// has covered (their staging slots are free again).  The mutex keeps a slot, or a
+// published number (below), and its launch together: calls that share no train
+// and no scratch may come from several threads.
+static std::mutex g_queue_mutex;
+static unsigned long long g_up_queued = 0, g_up_done = 0;
+
+static unsigned long long uploads_queued() {
+    std::lock_guard<std::mutex> lock(g_queue_mutex);
+    return g_up_queued;
+}
+static void uploads_done(unsigned long long upto) {
+    std::lock_guard<std::mutex> lock(g_queue_mutex);
+    if (upto > g_up_done) g_up_done = upto;
+}
 
 // Waits for both streams.
 static void sync_all() {
+    const unsigned long long up = uploads_queued();
     HIPCHECK(hipStreamSynchronize(g_stream));
     if (g_side) HIPCHECK(hipStreamSynchronize(g_side));
     g_side_dirty = false;
-    g_h2d_inflight = 0;
+    uploads_done(up);
 }
 // Host-visible mode (environment PARATT_AMD_HOST_VISIBLE=1, read once at
 // init): every library allocation is pinned host memory that the GPU reads
@@ -79,7 +92,8 @@ static unsigned char *g_stage_d2h = nullptr, *g_stage_h2d = nullptr;
 // that word instead of sleeping in a stream synchronisation, whose wake-up
 // costs tens of microseconds per read.  The spin gives up after a bound and
 // falls back to the stream synchronisation (which also reports a failed
-// launch).
+// launch).  Numbers are launched in order (g_queue_mutex), so a later one in
+// the word, another thread's, says as much.
 static unsigned long long *g_d2h_flag = nullptr;
 static unsigned long long g_d2h_seq = 0;
 constexpr double D2H_SPIN_SECONDS = 0.05;
@@ -107,7 +121,7 @@ __global__ __launch_bounds__(256) void k_copy_publish(unsigned char *__restrict_
 static void wait_published(unsigned long long seq) {
     const auto t0 = std::chrono::steady_clock::now();
     for (unsigned spin = 1;; spin++) {
-        if (__atomic_load_n(g_d2h_flag, __ATOMIC_ACQUIRE) == seq) return;
+        if (__atomic_load_n(g_d2h_flag, __ATOMIC_ACQUIRE) >= seq) return;
         if ((spin & 4095) == 0 &&
             std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count() >
                 D2H_SPIN_SECONDS)
@@ -115,7 +129,7 @@ static void wait_published(unsigned long long seq) {
         __builtin_ia32_pause();
     }
     HIPCHECK(hipStreamSynchronize(g_stream));
-    if (__atomic_load_n(g_d2h_flag, __ATOMIC_ACQUIRE) != seq) {
+    if (__atomic_load_n(g_d2h_flag, __ATOMIC_ACQUIRE) < seq) {
         fprintf(stderr, "paratt_amd: device-to-host read %llu not published\n", seq);
         exit(1);
     }
@@ -145,8 +159,8 @@ void fatal_hip(hipError_t e, const char *what, const char *file, int line) {
 // marginal), and hipMalloc / hipFree cost tens of microseconds a core.  Freed
 // blocks are kept, at most POOL_BYTES in all, and handed out again for requests
 // they fit within a quarter.  A block enters the pool only after the device has
-// finished everything queued so far (ptt_hip_free waits as hipFree does), so it
-// may be used on any stream by any thread.  The pool is emptied when an
+// finished everything queued so far (ptt_hip_free waits as hipFree does), so
+// whoever takes it may use it on any stream.  The pool is emptied when an
 // allocation fails and by ptt_hip_trim.
 constexpr size_t POOL_BYTES = (size_t)8 << 30;
 static std::mutex g_pool_mutex;
@@ -364,8 +378,9 @@ void ptt_hip_h2d(void *dst, const void *src, size_t bytes) {
     if (g_host_visible) return host_mode_copy(dst, src, bytes);
     if (bytes <= STAGE_BYTES) {
         ptt_hip_h2d_queued(dst, src, bytes);
+        const unsigned long long up = uploads_queued();
         HIPCHECK(hipStreamSynchronize(g_stream));
-        g_h2d_inflight = 0;
+        uploads_done(up);
         return;
     }
     HIPCHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, g_stream));
@@ -377,14 +392,15 @@ void ptt_hip_h2d_queued(void *dst, const void *src, size_t bytes) {
     if (!bytes) return;
     if (g_host_visible) return host_mode_copy(dst, src, bytes);
     if (bytes > STAGE_BYTES) return ptt_hip_h2d(dst, src, bytes);
-    if (g_h2d_inflight == H2D_SLOTS) {
+    ProfScope ps_("copy_bytes", 0.0, 2.0 * (double)bytes);
+    std::lock_guard<std::mutex> lock(g_queue_mutex);
+    if (g_up_queued - g_up_done == H2D_SLOTS) {
         HIPCHECK(hipStreamSynchronize(g_stream));
-        g_h2d_inflight = 0;
+        g_up_done = g_up_queued;
     }
-    unsigned char *stage = g_stage_h2d + STAGE_BYTES * (size_t)g_h2d_inflight++;
+    unsigned char *stage = g_stage_h2d + STAGE_BYTES * (size_t)(g_up_queued++ % H2D_SLOTS);
     memcpy(stage, src, bytes);
     unsigned blocks = (unsigned)((bytes / 8 + 255) / 256);
-    ProfScope ps_("copy_bytes", 0.0, 2.0 * (double)bytes);
     hipLaunchKernelGGL(k_copy_bytes, dim3(blocks < 1 ? 1 : blocks), dim3(256), 0, g_stream,
                        (unsigned char *)dst, stage, bytes);
     HIPCHECK(hipGetLastError());
@@ -395,9 +411,11 @@ void ptt_hip_d2h(void *dst, const void *src, size_t bytes) {
     if (!bytes) return;
     if (g_host_visible) return host_mode_copy(dst, src, bytes);
     if (bytes <= STAGE_BYTES) {
-        const unsigned long long seq = ++g_d2h_seq;
+        unsigned long long seq;
         {
-            ProfScope ps_("copy_bytes", 0.0, 2.0 * (double)bytes);
+            ProfScope ps_("copy_bytes", 0.0, 2.0 * (double)bytes);  // may wait: outside the lock
+            std::lock_guard<std::mutex> lock(g_queue_mutex);
+            seq = ++g_d2h_seq;
             hipLaunchKernelGGL(k_copy_publish, dim3(1), dim3(256), 0, g_stream, g_stage_d2h,
                                (const unsigned char *)src, bytes, g_d2h_flag, seq);
             HIPCHECK(hipGetLastError());
@@ -422,8 +440,9 @@ unsigned long long ptt_hip_d2h_begin(const void *src, size_t bytes) {
         host_mode_copy(g_stage_d2h, src, bytes);
         return 0;
     }
-    const unsigned long long seq = ++g_d2h_seq;
     ProfScope ps_("copy_bytes", 0.0, 2.0 * (double)bytes);
+    std::lock_guard<std::mutex> lock(g_queue_mutex);
+    const unsigned long long seq = ++g_d2h_seq;
     hipLaunchKernelGGL(k_copy_publish, dim3(1), dim3(256), 0, g_stream, g_stage_d2h,
                        (const unsigned char *)src, bytes, g_d2h_flag, seq);
     HIPCHECK(hipGetLastError());
@@ -459,11 +478,16 @@ void ptt_hip_sync(void) {
     // host-visible memory needs the stream's own end-of-work release; side
     // work that the main stream has not joined is waited for by itself
     if (g_host_visible || g_side_dirty) return sync_all();
-    const unsigned long long seq = ++g_d2h_seq;
-    hipLaunchKernelGGL(k_publish, dim3(1), dim3(1), 0, g_stream, g_d2h_flag, seq);
-    HIPCHECK(hipGetLastError());
+    unsigned long long seq, up;
+    {
+        std::lock_guard<std::mutex> lock(g_queue_mutex);
+        seq = ++g_d2h_seq;
+        up = g_up_queued;
+        hipLaunchKernelGGL(k_publish, dim3(1), dim3(1), 0, g_stream, g_d2h_flag, seq);
+        HIPCHECK(hipGetLastError());
+    }
     wait_published(seq);
-    g_h2d_inflight = 0;
+    uploads_done(up);
 }
 
 int ptt_hip_side_enabled(void) {
