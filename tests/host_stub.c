@@ -13,6 +13,7 @@
 
 double stub_kappa = 1.5;
 int stub_deficient = 0;
+long stub_bad_chol = -1; /* the factorisation (from 0) that reports a condition of 1e7 */
 long stub_side_inplace; /* in-place products queued on the side stream (Q = A T) */
 long stub_main_inplace; /* the same on the main stream, c x c from the right */
 long stub_chol, stub_tree_factors, stub_eigen, stub_mallocs;
@@ -106,10 +107,10 @@ void ptt_hip_gram32(char t, int c, long n, const double *A, long lda, double *G)
 void ptt_hip_chol_qr_factor(int c, const double *G, double shift, double tiny, double *R, double *T,
                             int *info, double *dinfo, int want) {
     (void)c; (void)G; (void)shift; (void)tiny; (void)R; (void)T; (void)want;
-    stub_chol++;
+    const int bad = stub_chol++ == stub_bad_chol;
     info[0] = stub_deficient;
     dinfo[0] = 0.0;
-    dinfo[1] = stub_kappa;
+    dinfo[1] = bad ? 1e7 : stub_kappa;
     dinfo[2] = stub_deficient;
     dinfo[3] = 1.0;
 }

@@ -122,3 +122,19 @@ def test_growing_a_train_waits_once_and_keeps_little_of_the_old(lib):
         lib.free_tt(x)
         assert peak - live <= 2 ** 30 + 8 * n * r * r
         assert frees == 1 if n == 20 else frees <= 6
+
+
+@pytest.mark.parametrize("bad", [1, 2, 3])
+def test_unformed_qs_are_formed_where_the_trees_take_over(lib, bad):
+    """24 columns: the cores before the first ill-conditioned one after core 0 hold A
+    with Q unformed; the trees take over there and get every one of those Qs."""
+    x = lib.alloc_ptt(5, _ints([50] * 5), _ints([1, 24, 24, 24, 24, 1]))
+    _set_condition(lib, 1.5)
+    lib.stub_reset()
+    C.c_long.in_dll(lib, "stub_bad_chol").value = bad
+    lib.paratt_amd_truncate_rel(x, 1e-8, _ints([1] + [5] * 4 + [1]))
+    C.c_long.in_dll(lib, "stub_bad_chol").value = -1
+    got = tuple(_count(lib, "stub_" + k) for k in ("chol", "main_inplace", "side_inplace",
+                                                   "tree_factors"))
+    lib.free_ptt(x)
+    assert got == (bad + 1, bad, 0, 4 - bad)
