@@ -98,6 +98,31 @@ struct EntryChunk {
     int first;  // 1 if the chunk holds the last core of the TT
 };
 
+// acc plus the first n of W terms x[u ld] v[u] in order, all loads in flight (those
+// beyond n read the last one): an entry is a chain of cores, bound by the latency of
+// its slices.  Measured (us a call; loads one after another; remainders so): d = 20,
+// r = 32: 152 / 35, r = 16: 84 / 35; d = 10, r = 8: 21.4 / 18.5, r = 1: 14.5 / 15.1;
+// d = 40, r = 4: 37.8 / 37.0.
+template <int W, bool FULL>
+__device__ __forceinline__ double entry_terms(const double *__restrict__ x, long ld, int n,
+                                              const double *v, double acc) {
+    // the offsets are formed here: hoisted out of the loops over q, those of all
+    // widths cost every slice some 460 instructions (0.85 us)
+    __asm__ volatile("" : "+s"(ld));
+    double xv[W];
+    long o = 0;
+#pragma unroll
+    for (int u = 0; u < W; u++) {
+        xv[u] = x[o];
+        if (FULL || u + 1 < n) o += ld;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < W; u++)
+        if (FULL || u < n) acc = acc + v[u] * xv[u];
+    return acc;
+}
+
 __global__ __launch_bounds__(ENTRY_NT) void k_tt_entry(EntryChunk ch, double *__restrict__ vec,
                                                        int rmax) {
     extern __shared__ double sh[];
@@ -119,24 +144,16 @@ __global__ __launch_bounds__(ENTRY_NT) void k_tt_entry(EntryChunk ch, double *__
         for (int p = threadIdx.x; p < r0; p += blockDim.x) {
             double acc = 0.0;
             int q = 0;
-            // thirty-two loads in flight (a row's terms are added in order): the
-            // chain of cores is bound by the latency of its slices (d = 20, r =
-            // 32: 116 us with the loads one after another, 43 this way)
-            for (; q + 32 <= r1; q += 32) {
-                double xv[32];
-#pragma unroll
-                for (int u = 0; u < 32; u++) xv[u] = x[p + ld * (q + u)];
-#pragma unroll
-                for (int u = 0; u < 32; u++) acc = acc + va[q + u] * xv[u];
-            }
-            for (; q + 8 <= r1; q += 8) {
-                double xv[8];
-#pragma unroll
-                for (int u = 0; u < 8; u++) xv[u] = x[p + ld * (q + u)];
-#pragma unroll
-                for (int u = 0; u < 8; u++) acc = acc + va[q + u] * xv[u];
-            }
-            for (; q < r1; q++) acc = acc + va[q] * x[p + ld * q];
+            for (; q + 32 <= r1; q += 32)
+                acc = entry_terms<32, true>(x + p + ld * q, ld, 32, va + q, acc);
+            const double *xq = x + p + ld * q;
+            const int n = r1 - q;
+            if (n == 1) acc = acc + va[q] * *xq;
+            else if (n == 2) acc = entry_terms<2, true>(xq, ld, n, va + q, acc);
+            else if (n > 16) acc = entry_terms<32, false>(xq, ld, n, va + q, acc);
+            else if (n > 8) acc = entry_terms<16, false>(xq, ld, n, va + q, acc);
+            else if (n > 4) acc = entry_terms<8, false>(xq, ld, n, va + q, acc);
+            else if (n > 2) acc = entry_terms<4, false>(xq, ld, n, va + q, acc);
             vb[p] = acc;
         }
         __syncthreads();
