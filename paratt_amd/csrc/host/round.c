@@ -1080,8 +1080,15 @@ static void fill_scales(const attac_tt *x, double *inv, double *sq) {
  * us), which take one Cholesky-QR pass and no Jacobi sweeps, and win on
  * ill-conditioned ones (some 600 us a bond there: three to four passes a
  * factorisation): such a train starts on the Cholesky-QR sweep and changes over
- * at the first core after core 0 that one pass does not orthogonalise. */
+ * at the first core after core 0 that one pass does not orthogonalise.  So does one
+ * with an unfolding of 11 to 16 columns and 8192 rows or more, whose blocks fill
+ * the GPU less well than a Gram's (d = 8, us, trees / this way; before the trees):
+ * 16 columns, n = 2048, well-conditioned 1401 / 848 (1129), deficient 1210 / 1331
+ * (2250); 12 columns, n = 2048, 1135 / 802 (1046) and 1038 / 1150 (2083).  With
+ * fewer rows or columns the trees lose nothing to the sweep they replaced. */
 #define TREE_RANK_ALWAYS 16
+#define TREE_RANK_TALL 10
+#define TREE_ROWS_TALL 8192
 #define TREE_RANK 32
 #define TREE_ROWS 65536
 /* 0: not by trees; 1: by trees; 2: by trees once a core is ill-conditioned. */
@@ -1093,6 +1100,9 @@ static int tree_route(const attac_tt *x) {
         const int r0 = x->ttRank[k], r1 = x->ttRank[k + 1];
         if (r0 < 1 || r1 < 1 || (k > 0 && r0 > TREE_RANK)) return 0;
         if (k > 0 && r0 > TREE_RANK_ALWAYS) route = 2;
+        if ((r1 > TREE_RANK_TALL && (long)r0 * x->dim[k] >= TREE_ROWS_TALL) ||
+            (r0 > TREE_RANK_TALL && (long)r1 * x->dim[k] >= TREE_ROWS_TALL))
+            route = 2;
         if ((long)r0 * x->dim[k] > TREE_ROWS || (long)r1 * x->dim[k] > TREE_ROWS) return 0;
     }
     return route;
@@ -1328,8 +1338,8 @@ void paratt_amd_truncate_rel_sketch(paratt *x_ptt, double eps_rel, int *maxRank,
         return;
     }
     /* Refused predictions leave the plain rounding's result.  A train that it would
-     * hand over to the trees (17 to 32 columns and a core of more than one pass;
-     * smaller ones take no sketch) is kept until a step has been accepted. */
+     * hand over to the trees (up to 32 columns and a core of more than one pass) is
+     * kept until a step has been accepted. */
     int *mr = (int *)ptt_host_malloc(sizeof(int) * (size_t)(d + 1));
     memcpy(mr, maxRank, sizeof(int) * (size_t)(d + 1));
     if (tree_route(x)) {

@@ -138,3 +138,17 @@ def test_unformed_qs_are_formed_where_the_trees_take_over(lib, bad):
                                                    "tree_factors"))
     lib.free_ptt(x)
     assert got == (bad + 1, bad, 0, 4 - bad)
+
+
+@pytest.mark.parametrize("n,r,trees", [(50, 16, True), (511, 16, True), (512, 16, False),
+                                       (745, 11, False), (744, 11, True), (4096, 10, True),
+                                       (4096, 16, False), (50, 17, False)])
+def test_trains_that_the_trees_take_from_the_start(lib, n, r, trees):
+    """Up to 16 columns, but not 11 to 16 with 8192 rows or more."""
+    x = lib.alloc_ptt(5, _ints([n] * 5), _ints([1] + [r] * 4 + [1]))
+    _set_condition(lib, 1.5)
+    lib.stub_reset()
+    lib.paratt_amd_truncate_rel(x, 1e-8, _ints([1] + [5] * 4 + [1]))
+    got = (_count(lib, "stub_tree_factors"), _count(lib, "stub_chol") > 0)
+    lib.free_ptt(x)
+    assert got == ((4, False) if trees else (0, True))
