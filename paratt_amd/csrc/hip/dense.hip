@@ -8,8 +8,10 @@
 //
 // ptt_hip_svd_jacobi: one-sided (Hestenes) Jacobi SVD with round-robin
 // parallel pairing; each pair is owned by a lane group that reduces its
-// three inner products with cross-lane shuffles.  Columns live in LDS when
-// they fit (160 KB per CU on gfx950), else in the caller's global buffers.
+// three inner products with cross-lane shuffles.  Up to 56 columns that fit in
+// the LDS of one CU (160 KB on gfx950) are rotated there by one wave or one
+// workgroup; otherwise many workgroups take pairs of blocks of columns into LDS
+// in turn, and columns too long for that stay in global memory.
 // The reference's rank rule (pattac.c:468-481) is applied on the device.
 #include "common.hpp"
 
@@ -20,8 +22,7 @@ using namespace ptt;
 namespace {
 
 constexpr int NT = 1024;
-// The Jacobi kernel holds 24 KB of static LDS (sorting and packing tables),
-// so its dynamic budget is smaller: 17280 doubles + 24.1 KB < 160 KB.
+// Doubles of columns in the one-workgroup Jacobi's LDS (135 KB of the CU's 160).
 constexpr int SVD_LDS_DOUBLES = 17280;
 // Columns beyond which the Jacobi SVD runs over many workgroups.  Measured with
 // V (us; flat spectrum, square): k = 48: 658 on one workgroup, 760 on many;
@@ -159,7 +160,7 @@ __global__ __launch_bounds__(NT) void k_chol_report(int c, const double *__restr
         if (PIT > 0 && c <= CR_REG) {
             // the matrix in registers, rows 12 wv + 3 lg + v, columns li + 16 q; S
             // first, then Ts^T (beyond this order every product reads it from
-            // memory: 246 us at 192 columns)
+            // memory: 635 us at 256 columns)
             const int li = lane & 15, lg = lane >> 4, r0 = 12 * wv + 3 * lg;
             double m[3][12];
             auto load = [&](const double *__restrict__ A, const double *__restrict__ cs,
@@ -921,13 +922,13 @@ __global__ __launch_bounds__(SVD_NT) void k_svd_jacobi(int m, int k, const doubl
     double *Vw = V ? lds + (long)ldw * k : nullptr;
     const int ldvw = k | 1;
     __shared__ int s_rot;
-    __shared__ double s_sig[1024];
-    __shared__ double s_sorted[1024];
-    __shared__ int s_pos[1024];
+    __shared__ double s_sig[SVD_ONE_WG_MAX];
+    __shared__ double s_sorted[SVD_ONE_WG_MAX];
+    __shared__ int s_pos[SVD_ONE_WG_MAX];
 
     // Exactly-zero columns (deficient directions) take no part in the
     // rotations: nonzero columns are packed first, in their original order.
-    __shared__ int s_perm[1024];
+    __shared__ int s_perm[SVD_ONE_WG_MAX];
     __shared__ int s_knz;
     // The columns are scaled by 2^-e (exact) so that the largest entry is
     // O(1): bond matrices of deep trains reach 1e-60 and below, where the

@@ -109,7 +109,7 @@ __device__ __forceinline__ void st_vd(double *p, const Vd<VW> &r) {
 }
 
 // ---- whole trains per launch -------------------------------------------------
-// The formal sum, the Hadamard product and the stencil sum write every core of
+// The formal sum, the stencil sum and the copy write every core of
 // a train independently: one launch takes up to TRAIN_CHUNK cores (descriptors
 // in the kernel arguments), with gridDim.z over the cores, y over a core's
 // columns and x over the rows of a column.  Trains of low rank are bound by
@@ -318,8 +318,9 @@ __global__ void k_stencil_core(int kind, int r0, int n, int r1,
 // with the 3-point periodic stencil of kind 0 applied on the way (same order of
 // operations as k_stencil_core).  Written block by block (the stencil to a
 // buffer, a zero fill, three placements) S was passed over more than twice: the
-// whole operator at d = 20, n = 1024, r = 32 took 739 us and takes 252 us
-// (840 MB read and written once; bound by HBM and the final synchronisation).
+// whole operator at d = 20, n = 1024, r = 32 took 739 us and takes 248 us, 180 of
+// them this kernel (756 MB read and written once, 4.2 TB/s; bound by HBM and the
+// call's launch and wait).
 template <int VW>
 __global__ __launch_bounds__(256) void k_mode_sum_train(ModeSumChunk ch) {
     const ModeSumCore &c = ch.c[blockIdx.z];

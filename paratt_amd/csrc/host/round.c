@@ -668,8 +668,7 @@ static int rtl_step_fast(attac_tt *x, int i, const int *maxr, double delta,
     int rows = r[i];
     long w = (long)n[i] * r[i + 1];
     double *M = x->coreList[i];
-    /* beyond 1024 rows the orthogonal route (its Jacobi SVD keeps the
-     * columns in HBM) handles the bond */
+    /* beyond 1024 rows the orthogonal route handles the bond */
     if (rows > 1024) return -1;
     ptt_hip_gram('N', rows, w, M, rows, ws->G);
     rside_flush(); /* the previous bond's new core beside this bond's eigensolver */
