@@ -60,7 +60,7 @@ def test_formed_q_of_a_rounding_goes_to_the_side_stream(lib, kappa, side, main):
     assert got == (side, main)
 
 
-def _work(L):
+def _queued(L):
     return tuple(_count(L, "stub_" + k) for k in ("chol", "tree_factors", "eigen", "mallocs"))
 
 
@@ -83,7 +83,7 @@ def test_rounding_without_a_usable_prediction_is_the_plain_one(lib, r, kappa, pr
             lib.paratt_amd_truncate_rel_sketch(x, 1e-8, mr, p)
         else:
             lib.paratt_amd_truncate_rel(x, 1e-8, mr)
-        got.append(_work(lib))
+        got.append(_queued(lib))
         lib.free_ptt(x)
     assert got[2] == got[1]
     cnt = (C.c_int * 2)()
